@@ -6,15 +6,14 @@
 // concatenation with the previous frame's twist, FC 134->256 (ReLU), FC 256->6,
 // plus the previous twist (skip connection: the layers predict the change of motion).
 //
-// Layout: activations NHWC (pixel-major, channel fastest), FP32; GEMM operands
-// are BF16 (round to nearest even), accumulation FP32.  A convolution is
-// im2col (rows = output pixels, columns = (ky, kx, cin)) followed by one GEMM
-// against the weight matrix (rows = cout); its backward is two GEMMs (weight
-// gradient with deterministic split-K over pixels, column gradient) and a
-// gather col2im.  The GEMM is one 16x16 output tile per wavefront on
+// Layout: activations NHWC (pixel-major, channel fastest), layers 1-3 as BF16 (the
+// next layer's operand), layer 4 FP32; products are BF16 (round to nearest even) with
+// FP32 accumulation.  The training forward's convolutions read the maps directly
+// (kf_prior_conv.hpp); their backward is two GEMMs (weight gradient from an im2col
+// matrix with deterministic split-K over pixels, column gradient) and a gather
+// col2im.  The GEMM is one 16x16 output tile per wavefront on
 // v_mfma_f32_16x16x32_bf16, four wavefronts per 256-thread block.
-#include "kf_device.hpp"
-#include "kf_internal.hpp"
+#include "kf_prior_conv.hpp"
 
 #include <math.h>
 #include <string.h>
@@ -24,64 +23,6 @@
 
 namespace kf {
 namespace {
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-
-// One 16x16x32 BF16 MFMA step (gfx950): lane l supplies A(l % 16, k0 + 8 (l / 16) + j)
-// and B(k0 + 8 (l / 16) + j, l % 16) for j < 8 as one 16-byte vector each, and holds
-// C(4 (l / 16) + j, l % 16) for j < 4.
-__device__ __forceinline__ v4f mfma32(uint4 a, uint4 b, v4f acc) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), acc, 0,
-                                                 0, 0);
-}
-
-constexpr int kH0 = KF_PRIOR_HEIGHT, kW0 = KF_PRIOR_WIDTH;
-constexpr int kConvs = 4;
-constexpr int kFeat = 128, kTwist = 6, kFc1In = kFeat + kTwist, kHidden = 256;
-
-struct ConvShape {
-  int cin, cout, hin, win, hout, wout, kc;
-};
-constexpr ConvShape kConv[kConvs] = {
-    {2, 32, 120, 160, 60, 80, 18},
-    {32, 64, 60, 80, 30, 40, 288},
-    {64, 64, 30, 40, 15, 20, 576},
-    {64, 128, 15, 20, 8, 10, 576},
-};
-constexpr int kPool = 8 * 10;
-
-// Parameter blob offsets (floats).
-struct ParamLayout {
-  long w[6], b[6], total;
-  ParamLayout() {
-    long o = 0;
-    for (int l = 0; l < kConvs; ++l) {
-      w[l] = o;
-      o += (long)kConv[l].cout * kConv[l].kc;
-      b[l] = o;
-      o += kConv[l].cout;
-    }
-    w[4] = o;
-    o += (long)kHidden * kFc1In;
-    b[4] = o;
-    o += kHidden;
-    w[5] = o;
-    o += (long)kTwist * kHidden;
-    b[5] = o;
-    o += kTwist;
-    total = o;
-  }
-};
-const ParamLayout& layout() {
-  static const ParamLayout L;
-  return L;
-}
-
-__device__ __forceinline__ uint16_t bf16_rne(float f) {
-  const uint32_t u = __float_as_uint(f);
-  return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
-}
 
 // ---------------------------------------------------------------------------
 // GEMM: C[m][n] (+)= sum_k A(m,k) B(k,n); A(m,k) = A[m*sam + k*sak], B(k,n) =
@@ -102,10 +43,6 @@ struct GemmArgs {
   int relu;
   const float* addend;
   uint16_t* Cb;
-  // Convolution operand (convX set): A(m, k) is the im2col element of a 3x3 /
-  // stride-2 / pad-1 convolution read from the BF16 NHWC input convX instead.
-  const uint16_t* convX;
-  int conv_cin, conv_hin, conv_win, conv_hout, conv_wout;
 };
 
 // Each 256-thread block computes a 32x32 tile of C (four 16x16 wave tiles on
@@ -183,44 +120,6 @@ __device__ __forceinline__ void stage(uint16_t (*T)[kPitch], const uint16_t* X, 
   }
 }
 
-// Stages A rows [row0, row0 + 32) of a convolution directly from its BF16 NHWC
-// input: k = (ky * 3 + kx) * cin + ci with cin a multiple of 8, so 8 consecutive k
-// are 8 channels of one tap (one 16-byte load, zero outside the image); the values
-// are those an im2col of the same input would hold.
-__device__ __forceinline__ void stage_conv(uint16_t (*T)[kPitch], const GemmArgs& g, int row0, int kn, int kpad) {
-  const int tid = threadIdx.x;
-  const int vpr = kpad >> 3;
-  const int total = 32 * vpr;
-  const int pix = g.conv_hout * g.conv_wout;
-  uint4 v[kVecPerThread];
-#pragma unroll
-  for (int u = 0; u < kVecPerThread; ++u) {
-    const int e = tid + 256 * u;
-    const int r = e / vpr, c = e - (e / vpr) * vpr;
-    const int m = row0 + r;
-    bool in = e < total && m < g.M && 8 * c < kn;
-    long off = 0;
-    if (in) {
-      const int n = m / pix, q = m - n * pix;
-      const int oy = q / g.conv_wout, ox = q - oy * g.conv_wout;
-      const int tap = (8 * c) / g.conv_cin, ci = 8 * c - tap * g.conv_cin;
-      const int ky = tap / 3, kx = tap - 3 * ky;
-      const int iy = 2 * oy + ky - 1, ix = 2 * ox + kx - 1;
-      in = iy >= 0 && iy < g.conv_hin && ix >= 0 && ix < g.conv_win;
-      off = (((long)n * g.conv_hin + iy) * g.conv_win + ix) * g.conv_cin + ci;
-    }
-    v[u] = in ? *reinterpret_cast<const uint4*>(g.convX + off) : make_uint4(0, 0, 0, 0);
-  }
-#pragma unroll
-  for (int u = 0; u < kVecPerThread; ++u) {
-    const int e = tid + 256 * u;
-    if (e < total) {
-      const int r = e / vpr, c = e - (e / vpr) * vpr;
-      *reinterpret_cast<uint4*>(&T[r][8 * c]) = v[u];
-    }
-  }
-}
-
 __global__ __launch_bounds__(256) void gemm_bf16(GemmArgs g) {
   __shared__ __align__(16) uint16_t As[32][kPitch];
   __shared__ __align__(16) uint16_t Bt[32][kPitch];
@@ -234,10 +133,7 @@ __global__ __launch_bounds__(256) void gemm_bf16(GemmArgs g) {
   for (int kc0 = kbeg; kc0 < kend; kc0 += kKc) {
     const int kn = min(kKc, kend - kc0);
     const int kpad = (kn + 31) & ~31;
-    if (g.convX)  // uniform; the whole K is one chunk for every convolution
-      stage_conv(As, g, mt, kn, kpad);
-    else
-      stage(As, g.A, g.sam, g.sak, mt, g.M, kc0, kn, kpad);
+    stage(As, g.A, g.sam, g.sak, mt, g.M, kc0, kn, kpad);
     stage(Bt, g.B, g.sbn, g.sbk, nt, g.N, kc0, kn, kpad);
     __syncthreads();
     for (int kk = 0; kk < kpad; kk += 32)
@@ -546,7 +442,7 @@ __global__ void im2col_pairs(const float* frames, const int32_t* pairs, int batc
   col[i] = bf16_rne(v);
 }
 
-__global__ void im2col_nhwc(const float* X, int layer, int batch, uint16_t* col) {
+__global__ void im2col_nhwc(const uint16_t* X, int layer, int batch, uint16_t* col) {
   const ConvShape c = kConv[layer];
   const long M = (long)batch * c.hout * c.wout;
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -558,14 +454,14 @@ __global__ void im2col_nhwc(const float* X, int layer, int batch, uint16_t* col)
   const int oy = p / c.wout, ox = p - oy * c.wout;
   const int ky = k / (3 * c.cin), kx = (k / c.cin) % 3, ci = k % c.cin;
   const int iy = 2 * oy + ky - 1, ix = 2 * ox + kx - 1;
-  float v = 0.0f;
+  uint16_t v = 0;
   if (iy >= 0 && iy < c.hin && ix >= 0 && ix < c.win) v = X[(((long)n * c.hin + iy) * c.win + ix) * c.cin + ci];
-  col[i] = bf16_rne(v);
+  col[i] = v;
 }
 
 // dX[n][iy][ix][ci] = sum over (ky,kx) of dcol[(n,oy,ox)][(ky,kx,ci)], times the
 // ReLU mask of the forward activation X (the previous layer's output).
-__global__ void col2im_relu(const float* dcol, const float* X, int layer, int batch, float* dX) {
+__global__ void col2im_relu(const float* dcol, const uint16_t* X, int layer, int batch, float* dX) {
   const ConvShape c = kConv[layer];
   const long total = (long)batch * c.hin * c.win * c.cin;
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -591,7 +487,7 @@ __global__ void col2im_relu(const float* dcol, const float* X, int layer, int ba
       s = s + dcol[m * c.kc + (ky * 3 + kx) * c.cin + ci];
     }
   }
-  dX[i] = X[i] > 0.0f ? s : 0.0f;
+  dX[i] = (int16_t)X[i] > 0 ? s : 0.0f;  // the BF16 map is positive where the FP32 one is
 }
 
 __global__ void to_bf16(const float* x, uint16_t* y, long n) {
@@ -691,8 +587,9 @@ struct kf_prior {
   float* adam_m = nullptr;
   float* adam_v = nullptr;
   long step = 0;
-  // activations (FP32, NHWC) and BF16 im2col buffers, sized for max_batch
-  float* Y[kf::kConvs] = {};
+  // activations (NHWC) and BF16 im2col buffers, sized for max_batch
+  uint16_t* Yb[kf::kConvs - 1] = {};  // layers 1-3, BF16 NHWC
+  float* Y4 = nullptr;                // layer 4, FP32
   uint16_t* col[kf::kConvs] = {};
   float* X5 = nullptr;
   uint16_t* X5b = nullptr;
@@ -728,15 +625,8 @@ struct Epilogue {
 
 kf_status gemm(hipStream_t s, const uint16_t* A, long sam, long sak, const uint16_t* B, long sbk, long sbn, float* C,
                long ldc, int M, int N, int K, bool accumulate, float* part = nullptr, long part_floats = 0,
-               const Epilogue& ep = Epilogue(), const ConvShape* conv = nullptr, const uint16_t* convX = nullptr) {
+               const Epilogue& ep = Epilogue()) {
   GemmArgs g;
-  g.convX = convX;
-  g.conv_cin = conv ? conv->cin : 0;
-  g.conv_hin = conv ? conv->hin : 0;
-  g.conv_win = conv ? conv->win : 0;
-  g.conv_hout = conv ? conv->hout : 0;
-  g.conv_wout = conv ? conv->wout : 0;
-  if (convX) KF_CHECK_ARG(conv->cin % 8 == 0 && K == conv->kc && K <= kKc, "implicit convolution shape");
   g.bias = ep.bias;
   g.relu = ep.relu;
   g.addend = ep.addend;
@@ -785,58 +675,66 @@ kf_status sync_weights(kf_prior* P, hipStream_t s) {
   return check_launch("to_bf16(weights)");
 }
 
-// out: where the twists go (P->O when NULL; training reads P->O).  cols: the
-// im2col matrices of every layer are materialised (training: the weight gradients
-// read them); without, layers 2-4 read their input directly in the GEMM (the
-// previous layer's epilogue leaves its BF16 copy in the next layer's im2col
-// buffer), with the same A values and hence the same outputs.
-kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, const float* prev, int B, hipStream_t s,
-                  float* out = nullptr, bool cols = true) {
+// Inference: the fused kernel (the training forward's outputs, in one launch).
+kf_status infer(kf_prior* P, const float* frames, const int32_t* pairs, const float* prev, int B, float* out,
+                hipStream_t s) {
   const ParamLayout& L = layout();
-  if (!cols) {  // inference: the fused kernel (same outputs, one launch)
-    FuseArgs f;
-    f.frames = frames;
-    f.pairs = pairs;
-    f.prev = prev;
-    f.wbf = P->wbf;
-    f.params = P->params;
-    for (int q = 0; q < 6; ++q) {
-      f.w[q] = L.w[q];
-      f.b[q] = L.b[q];
-    }
-    f.Y4 = P->Y[kConvs - 1];
-    f.X5 = P->X5;
-    f.X5b = P->X5b;
-    f.H = P->Hd;
-    f.Hb = P->Hb;
-    f.out = out ? out : P->O;
-    f.count = P->fuse_count;
-    hipLaunchKernelGGL(prior_infer_fused, dim3(kPool, B), dim3(kFuseThreads), 0, s, f);
-    return check_launch("prior_infer_fused");
+  FuseArgs f;
+  f.frames = frames;
+  f.pairs = pairs;
+  f.prev = prev;
+  f.wbf = P->wbf;
+  f.params = P->params;
+  for (int q = 0; q < 6; ++q) {
+    f.w[q] = L.w[q];
+    f.b[q] = L.b[q];
   }
-  for (int l = 0; l < kConvs; ++l) {
+  f.Y4 = P->Y4;
+  f.X5 = P->X5;
+  f.X5b = P->X5b;
+  f.H = P->Hd;
+  f.Hb = P->Hb;
+  f.out = out;
+  f.count = P->fuse_count;
+  hipLaunchKernelGGL(prior_infer_fused, dim3(kPool, B), dim3(kFuseThreads), 0, s, f);
+  return check_launch("prior_infer_fused");
+}
+
+// One convolution of the training forward: two blocks of four waves a CU hold the
+// weights; a small batch gets one wave per 16-pixel tile and channel group.
+template <int L, int NT, bool F32>
+kf_status launch_conv(kf_prior* P, const uint16_t* X, uint16_t* Yb, float* Y, int B, hipStream_t s) {
+  constexpr ConvShape c = kConv[L];
+  constexpr int GROUPS = c.cout / (16 * NT);
+  const ParamLayout& lay = layout();
+  const int M = B * c.hout * c.wout;
+  const int blocks = std::min(div_up(div_up(M, 16) * GROUPS, kConvWaves), 512);
+  hipLaunchKernelGGL((conv_forward<L, NT, F32>), dim3(blocks), dim3(kConvThreads), 0, s, X, P->wbf + lay.w[L],
+                     (const float*)P->params + lay.b[L], Yb, Y, M);
+  return check_launch("conv_forward");
+}
+
+// Training forward: the activations stay for the backward pass.
+kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, const float* prev, int B, hipStream_t s) {
+  const ParamLayout& L = layout();
+  hipLaunchKernelGGL(conv1_forward, dim3(kConv[0].hout / kL1Rows, B), dim3(kConvThreads), 0, s, frames, pairs,
+                     (const uint16_t*)P->wbf + L.w[0], (const float*)P->params + L.b[0], P->Yb[0]);
+  KF_TRY(check_launch("conv1_forward"));
+  KF_TRY((launch_conv<1, 4, false>(P, P->Yb[0], P->Yb[1], nullptr, B, s)));
+  KF_TRY((launch_conv<2, 2, false>(P, P->Yb[1], P->Yb[2], nullptr, B, s)));
+  KF_TRY((launch_conv<3, 2, true>(P, P->Yb[2], nullptr, P->Y4, B, s)));
+  for (int l = 0; l < kConvs; ++l) {  // the weight gradients' operands
     const ConvShape& c = conv(l);
     const long M = (long)B * c.hout * c.wout;
-    if (l == 0) {
+    if (l == 0)
       hipLaunchKernelGGL(im2col_pairs, dim3(blocks_for(M * kcp(0))), dim3(256), 0, s, frames, pairs, B, P->col[0],
                          kcp(0));
-      KF_TRY(check_launch("im2col_pairs"));
-    } else if (cols) {
-      hipLaunchKernelGGL(im2col_nhwc, dim3(blocks_for(M * c.kc)), dim3(256), 0, s, (const float*)P->Y[l - 1], l, B,
+    else
+      hipLaunchKernelGGL(im2col_nhwc, dim3(blocks_for(M * c.kc)), dim3(256), 0, s, (const uint16_t*)P->Yb[l - 1], l, B,
                          P->col[l]);
-      KF_TRY(check_launch("im2col_nhwc"));
-    }
-    // Y[m][co] = sum_k col[m][k] W[co][k]; the layer-1 padding columns are zero in col.
-    // Y = ReLU(col W^T + b): bias and ReLU in the GEMM epilogue
-    Epilogue ep;
-    ep.bias = (const float*)P->params + L.b[l];
-    ep.relu = 1;
-    if (!cols && l + 1 < kConvs) ep.Cb = P->col[l + 1];  // BF16 NHWC copy, the next layer's input
-    const bool implicit = !cols && l > 0;
-    KF_TRY(gemm(s, P->col[l], kcp(l), 1, P->wbf + L.w[l], 1, c.kc, P->Y[l], c.cout, (int)M, c.cout, c.kc, false,
-                nullptr, 0, ep, implicit ? &c : nullptr, implicit ? P->col[l] : nullptr));
+    KF_TRY(check_launch("im2col"));
   }
-  hipLaunchKernelGGL(pool_concat, dim3(blocks_for((long)B * kFc1In)), dim3(256), 0, s, (const float*)P->Y[3], prev, B,
+  hipLaunchKernelGGL(pool_concat, dim3(blocks_for((long)B * kFc1In)), dim3(256), 0, s, (const float*)P->Y4, prev, B,
                      P->X5, P->X5b);
   KF_TRY(check_launch("pool_concat"));
   {  // FC1: H = ReLU(X5 W5^T + b5), also as BF16 for FC2
@@ -851,7 +749,7 @@ kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, const 
     Epilogue ep;
     ep.bias = (const float*)P->params + L.b[5];
     ep.addend = prev;
-    KF_TRY(gemm(s, P->Hb, kHidden, 1, P->wbf + L.w[5], 1, kHidden, out ? out : P->O, kTwist, B, kTwist, kHidden,
+    KF_TRY(gemm(s, P->Hb, kHidden, 1, P->wbf + L.w[5], 1, kHidden, P->O, kTwist, B, kTwist, kHidden,
                 false, nullptr, 0, ep));
   }
   return KF_OK;
@@ -880,7 +778,7 @@ kf_status backward(kf_prior* P, const float* target, int B, float* loss, hipStre
   float* dY = P->dY;
   float* dYn = P->dY2;
   hipLaunchKernelGGL(pool_backward, dim3(blocks_for((long)B * kPool * kFeat)), dim3(256), 0, s,
-                     (const float*)P->dX5, (const float*)P->Y[3], B, dY);
+                     (const float*)P->dX5, (const float*)P->Y4, B, dY);
   KF_TRY(check_launch("pool_backward"));
   for (int l = kConvs - 1; l >= 0; --l) {
     const ConvShape& c = conv(l);
@@ -897,7 +795,7 @@ kf_status backward(kf_prior* P, const float* target, int B, float* loss, hipStre
     KF_TRY(gemm(s, P->dYb, c.cout, 1, P->wbf + L.w[l], c.kc, 1, P->dcol, c.kc, (int)M, c.kc, c.cout, false));
     const long nin = (long)B * c.hin * c.win * c.cin;
     hipLaunchKernelGGL(col2im_relu, dim3(blocks_for(nin)), dim3(256), 0, s, (const float*)P->dcol,
-                       (const float*)P->Y[l - 1], l, B, dYn);
+                       (const uint16_t*)P->Yb[l - 1], l, B, dYn);
     KF_TRY(check_launch("col2im_relu"));
     std::swap(dY, dYn);
   }
@@ -919,12 +817,12 @@ extern "C" int64_t kf_prior_param_count(void) { return layout().total; }
 
 extern "C" kf_status kf_prior_destroy(kf_prior* P) {
   if (!P) return KF_OK;
-  void* ptrs[] = {P->params, P->wbf, P->grad, P->adam_m, P->adam_v, P->X5, P->X5b, P->Hd, P->Hb, P->O, P->dO,
+  void* ptrs[] = {P->params, P->wbf, P->grad, P->adam_m, P->adam_v, P->Y4, P->X5, P->X5b, P->Hd, P->Hb, P->O, P->dO,
                   P->dOb, P->dH, P->dHb, P->dX5, P->dY, P->dY2, P->dYb, P->dcol, P->part, P->loss_tmp,
                   P->fuse_count};
   for (void* q : ptrs) (void)hipFree(q);
   for (int l = 0; l < kConvs; ++l) {
-    (void)hipFree(P->Y[l]);
+    if (l + 1 < kConvs) (void)hipFree(P->Yb[l]);
     (void)hipFree(P->col[l]);
   }
   delete P;
@@ -951,7 +849,8 @@ extern "C" kf_status kf_prior_create(int32_t max_batch, kf_prior** out) {
   for (int l = 0; l < kConvs; ++l) {
     const ConvShape& c = kConv[l];
     const long M = B * c.hout * c.wout;
-    al((void**)&P->Y[l], M * c.cout * 4);
+    if (l + 1 < kConvs) al((void**)&P->Yb[l], M * c.cout * 2);
+    else al((void**)&P->Y4, M * c.cout * 4);
     al((void**)&P->col[l], M * kcp(l) * 2);
     maxact = std::max(maxact, M * c.cout);
     maxact = std::max(maxact, B * c.hin * c.win * c.cin);
@@ -1033,7 +932,7 @@ extern "C" kf_status kf_prior_forward(kf_prior* P, const float* frames, const in
                                       int32_t B, float* d_out, kf_stream s) {
   KF_TRY(check_batch(P, frames, pairs, prev, B));
   KF_CHECK_ARG(d_out != nullptr, "out is NULL");
-  return forward(P, frames, pairs, prev, B, S(s), d_out, false);
+  return infer(P, frames, pairs, prev, B, d_out, S(s));
 }
 
 extern "C" kf_status kf_prior_gradients(kf_prior* P, const float* frames, const int32_t* pairs, const float* prev,
