@@ -8,10 +8,9 @@
 //
 // Layout: activations NHWC (pixel-major, channel fastest), layers 1-3 as BF16 (the
 // next layer's operand), layer 4 FP32; products are BF16 (round to nearest even) with
-// FP32 accumulation.  The training forward's convolutions read the maps directly
-// (kf_prior_conv.hpp); their backward is two GEMMs (weight gradient from an im2col
-// matrix with deterministic split-K over pixels, column gradient) and a gather
-// col2im.  The GEMM is one 16x16 output tile per wavefront on
+// FP32 accumulation.  The training forward's convolutions and the input gradients read
+// the maps directly (kf_prior_conv.hpp); the weight gradient is a GEMM over an im2col
+// matrix with deterministic split-K over pixels.  The GEMM is one 16x16 output tile per wavefront on
 // v_mfma_f32_16x16x32_bf16, four wavefronts per 256-thread block.
 #include "kf_prior_conv.hpp"
 
@@ -459,37 +458,6 @@ __global__ void im2col_nhwc(const uint16_t* X, int layer, int batch, uint16_t* c
   col[i] = v;
 }
 
-// dX[n][iy][ix][ci] = sum over (ky,kx) of dcol[(n,oy,ox)][(ky,kx,ci)], times the
-// ReLU mask of the forward activation X (the previous layer's output).
-__global__ void col2im_relu(const float* dcol, const uint16_t* X, int layer, int batch, float* dX) {
-  const ConvShape c = kConv[layer];
-  const long total = (long)batch * c.hin * c.win * c.cin;
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  const int ci = (int)(i % c.cin);
-  const long q = i / c.cin;
-  const int ix = (int)(q % c.win);
-  const long q2 = q / c.win;
-  const int iy = (int)(q2 % c.hin);
-  const int n = (int)(q2 / c.hin);
-  float s = 0.0f;
-  for (int ky = 0; ky < 3; ++ky) {
-    const int ty = iy + 1 - ky;
-    if (ty < 0 || (ty & 1)) continue;
-    const int oy = ty >> 1;
-    if (oy >= c.hout) continue;
-    for (int kx = 0; kx < 3; ++kx) {
-      const int tx = ix + 1 - kx;
-      if (tx < 0 || (tx & 1)) continue;
-      const int ox = tx >> 1;
-      if (ox >= c.wout) continue;
-      const long m = ((long)n * c.hout + oy) * c.wout + ox;
-      s = s + dcol[m * c.kc + (ky * 3 + kx) * c.cin + ci];
-    }
-  }
-  dX[i] = (int16_t)X[i] > 0 ? s : 0.0f;  // the BF16 map is positive where the FP32 one is
-}
-
 __global__ void to_bf16(const float* x, uint16_t* y, long n) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) y[i] = bf16_rne(x[i]);
@@ -512,13 +480,42 @@ __global__ void pool_concat(const float* Y4, const float* prev, int batch, float
   X5b[i] = bf16_rne(v);
 }
 
-// dY4[n][p][c] = dX5[n][c] / 80 where Y4 > 0.
-__global__ void pool_backward(const float* dX5, const float* Y4, int batch, float* dY4) {
+// BF16 copies of the parameters: y in the blob's order, and the weights of layers 2-4
+// again as [tap][ci][co] (yt, at the blob's offsets) for the input gradients.
+struct WeightCopyArgs {
+  const float* x;
+  uint16_t *y, *yt;
+  long n, w[kConvs];  // parameter count, weight offsets of the convolutions
+};
+__global__ void copy_weights(WeightCopyArgs a) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long)batch * kPool * kFeat) return;
-  const int c = (int)(i % kFeat);
-  const int n = (int)(i / ((long)kPool * kFeat));
-  dY4[i] = Y4[i] > 0.0f ? dX5[n * kFc1In + c] * (1.0f / (float)kPool) : 0.0f;
+  if (i >= a.n) return;
+  const uint16_t v = bf16_rne(a.x[i]);
+  a.y[i] = v;
+#pragma unroll
+  for (int l = 1; l < kConvs; ++l) {
+    const int e = (int)(i - a.w[l]);
+    if (e >= 0 && e < kConv[l].cout * kConv[l].kc) a.yt[a.w[l] + (e % kConv[l].kc) * kConv[l].cout + e / kConv[l].kc] = v;
+  }
+}
+
+// dY4[n][p][c] = dX5[n][c] / 80 where Y4 > 0, as BF16, and each sample's FP32 sums over
+// its pixels (bpart[n][c]).  One block per sample.
+__global__ __launch_bounds__(2 * kFeat) void pool_backward(const float* dX5, const float* Y4, uint16_t* dY4, float* bpart) {
+  __shared__ float red[kFeat];
+  const int n = blockIdx.x, c = threadIdx.x & (kFeat - 1), half = threadIdx.x / kFeat;
+  const float g = dX5[n * kFc1In + c] * (1.0f / (float)kPool);
+  float s = 0.0f;
+#pragma unroll 8
+  for (int p = half; p < kPool; p += 2) {
+    const long i = ((long)n * kPool + p) * kFeat + c;
+    const float v = Y4[i] > 0.0f ? g : 0.0f;
+    dY4[i] = bf16_rne(v);
+    s = s + v;
+  }
+  if (half == 1) red[c] = s;
+  __syncthreads();
+  if (half == 0) bpart[(long)n * kFeat + c] = s + red[c];
 }
 
 // Loss mean((O - T)^2) and dO = 2 (O - T) / (6 B); one block.
@@ -583,6 +580,7 @@ struct kf_prior {
   long nparams = 0;
   float* params = nullptr;   // FP32 master
   uint16_t* wbf = nullptr;   // BF16 copy
+  uint16_t* wt = nullptr;    // layers 2-4 again as [tap][ci][co], at the same offsets
   float* grad = nullptr;
   float* adam_m = nullptr;
   float* adam_v = nullptr;
@@ -601,10 +599,8 @@ struct kf_prior {
   float* dH = nullptr;
   uint16_t* dHb = nullptr;
   float* dX5 = nullptr;
-  float* dY = nullptr;    // largest activation gradient
-  float* dY2 = nullptr;   // second buffer (ping-pong)
-  uint16_t* dYb = nullptr;
-  float* dcol = nullptr;
+  uint16_t* dYb[kf::kConvs] = {};       // gradients of the layers' outputs, BF16 NHWC
+  float* bpart[kf::kConvs] = {};        // partial bias sums per block (layer 4: per sample)
   float* part = nullptr;  // split-K partial planes
   long part_floats = 0;
   float* loss_tmp = nullptr;
@@ -667,12 +663,17 @@ kf_status gemm(hipStream_t s, const uint16_t* A, long sam, long sak, const uint1
 const ConvShape& conv(int l) { return kConv[l]; }
 int kcp(int l) { return l == 0 ? 32 : kConv[l].kc; }  // im2col row length (layer 1 padded to 32)
 
-// BF16 copy of the weights; every call that changes the FP32 parameters refreshes
-// it, so inference (forward) never converts.
+// BF16 copies of the weights; every call that changes the FP32 parameters refreshes
+// them, so inference (forward) never converts.
 kf_status sync_weights(kf_prior* P, hipStream_t s) {
-  hipLaunchKernelGGL(to_bf16, dim3(blocks_for(P->nparams)), dim3(256), 0, s, (const float*)P->params, P->wbf,
-                     P->nparams);
-  return check_launch("to_bf16(weights)");
+  WeightCopyArgs a;
+  a.x = P->params;
+  a.y = P->wbf;
+  a.yt = P->wt;
+  a.n = P->nparams;
+  for (int l = 0; l < kConvs; ++l) a.w[l] = layout().w[l];
+  hipLaunchKernelGGL(copy_weights, dim3(blocks_for(P->nparams)), dim3(256), 0, s, a);
+  return check_launch("copy_weights");
 }
 
 // Inference: the fused kernel (the training forward's outputs, in one launch).
@@ -700,6 +701,8 @@ kf_status infer(kf_prior* P, const float* frames, const int32_t* pairs, const fl
   return check_launch("prior_infer_fused");
 }
 
+constexpr int kConvBlocks = 512;
+
 // One convolution of the training forward: two blocks of four waves a CU hold the
 // weights; a small batch gets one wave per 16-pixel tile and channel group.
 template <int L, int NT, bool F32>
@@ -708,7 +711,7 @@ kf_status launch_conv(kf_prior* P, const uint16_t* X, uint16_t* Yb, float* Y, in
   constexpr int GROUPS = c.cout / (16 * NT);
   const ParamLayout& lay = layout();
   const int M = B * c.hout * c.wout;
-  const int blocks = std::min(div_up(div_up(M, 16) * GROUPS, kConvWaves), 512);
+  const int blocks = std::min(div_up(div_up(M, 16) * GROUPS, kConvWaves), kConvBlocks);
   hipLaunchKernelGGL((conv_forward<L, NT, F32>), dim3(blocks), dim3(kConvThreads), 0, s, X, P->wbf + lay.w[L],
                      (const float*)P->params + lay.b[L], Yb, Y, M);
   return check_launch("conv_forward");
@@ -755,6 +758,19 @@ kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, const 
   return KF_OK;
 }
 
+// Input gradient of layer L (dYb[L] -> dYb[L - 1], partial sums of layer L - 1's bias
+// gradient; *planes: how many), on the grid of launch_conv.
+template <int L, int NT>
+kf_status launch_dgrad(kf_prior* P, int B, int* planes, hipStream_t s) {
+  constexpr ConvShape c = kConv[L];
+  const int M = B * c.hout * c.wout;
+  *planes = std::min(div_up(div_up(M, 16) * (c.cin / (16 * NT)), kConvWaves), kConvBlocks);
+  hipLaunchKernelGGL((conv_dgrad<L, NT>), dim3(*planes), dim3(kConvThreads), 0, s, (const uint16_t*)P->dYb[L],
+                     (const uint16_t*)P->wt + layout().w[L], (const uint16_t*)P->Yb[L - 1], P->dYb[L - 1],
+                     P->bpart[L - 1], M);
+  return check_launch("conv_dgrad");
+}
+
 kf_status backward(kf_prior* P, const float* target, int B, float* loss, hipStream_t s) {
   const ParamLayout& L = layout();
   float* G = P->grad;
@@ -774,31 +790,34 @@ kf_status backward(kf_prior* P, const float* target, int B, float* loss, hipStre
   KF_TRY(gemm(s, P->dHb, 1, kHidden, P->X5b, kFc1In, 1, G + L.w[4], kFc1In, kHidden, kFc1In, B, false));
   hipLaunchKernelGGL(bias_grad, dim3(kHidden), dim3(256), 0, s, (const float*)P->dH, (long)B, kHidden, G + L.b[4]);
   KF_TRY(gemm(s, P->dHb, kHidden, 1, P->wbf + L.w[4], kFc1In, 1, P->dX5, kFc1In, B, kFeat, kHidden, false));
-  // Pool: dY4.
-  float* dY = P->dY;
-  float* dYn = P->dY2;
-  hipLaunchKernelGGL(pool_backward, dim3(blocks_for((long)B * kPool * kFeat)), dim3(256), 0, s,
-                     (const float*)P->dX5, (const float*)P->Y4, B, dY);
+  hipLaunchKernelGGL(pool_backward, dim3(B), dim3(2 * kFeat), 0, s, (const float*)P->dX5, (const float*)P->Y4,
+                     P->dYb[3], P->bpart[3]);
   KF_TRY(check_launch("pool_backward"));
+  int planes[kConvs] = {0, 0, 0, B};
+  KF_TRY((launch_dgrad<3, 1>(P, B, &planes[2], s)));
+  KF_TRY((launch_dgrad<2, 2>(P, B, &planes[1], s)));
+  KF_TRY((launch_dgrad<1, 2>(P, B, &planes[0], s)));
+  ReduceArgs red;
+  red.jobs = 0;
+  red.block0[0] = 0;
+  auto add = [&](const float* part, int n, int count, float* out) {
+    const int k = red.jobs++;
+    red.part[k] = part;
+    red.planes[k] = n;
+    red.count[k] = count;
+    red.out[k] = out;
+    red.block0[k + 1] = red.block0[k] + div_up(count, 64);
+  };
   for (int l = kConvs - 1; l >= 0; --l) {
     const ConvShape& c = conv(l);
     const long M = (long)B * c.hout * c.wout;
-    hipLaunchKernelGGL(to_bf16, dim3(blocks_for(M * c.cout)), dim3(256), 0, s, (const float*)dY, P->dYb,
-                       M * c.cout);
     // dW[co][k] = sum_m dY[m][co] col[m][k]   (split-K over pixels, deterministic)
-    KF_TRY(gemm(s, P->dYb, 1, c.cout, P->col[l], kcp(l), 1, G + L.w[l], c.kc, c.cout, c.kc, (int)M, false, P->part,
+    KF_TRY(gemm(s, P->dYb[l], 1, c.cout, P->col[l], kcp(l), 1, G + L.w[l], c.kc, c.cout, c.kc, (int)M, false, P->part,
                 P->part_floats));
-    hipLaunchKernelGGL(bias_grad, dim3(c.cout), dim3(256), 0, s, (const float*)dY, M, c.cout, G + L.b[l]);
-    KF_TRY(check_launch("bias_grad"));
-    if (l == 0) break;
-    // dcol[m][k] = sum_co dY[m][co] W[co][k]; dX = col2im(dcol) masked by Y[l-1] > 0.
-    KF_TRY(gemm(s, P->dYb, c.cout, 1, P->wbf + L.w[l], c.kc, 1, P->dcol, c.kc, (int)M, c.kc, c.cout, false));
-    const long nin = (long)B * c.hin * c.win * c.cin;
-    hipLaunchKernelGGL(col2im_relu, dim3(blocks_for(nin)), dim3(256), 0, s, (const float*)P->dcol,
-                       (const uint16_t*)P->Yb[l - 1], l, B, dYn);
-    KF_TRY(check_launch("col2im_relu"));
-    std::swap(dY, dYn);
+    add(P->bpart[l], planes[l], c.cout, G + L.b[l]);
   }
+  hipLaunchKernelGGL(reduce_parts, dim3(red.block0[red.jobs]), dim3(1024), 0, s, red);
+  KF_TRY(check_launch("reduce_parts"));
   return KF_OK;
 }
 
@@ -818,12 +837,14 @@ extern "C" int64_t kf_prior_param_count(void) { return layout().total; }
 extern "C" kf_status kf_prior_destroy(kf_prior* P) {
   if (!P) return KF_OK;
   void* ptrs[] = {P->params, P->wbf, P->grad, P->adam_m, P->adam_v, P->Y4, P->X5, P->X5b, P->Hd, P->Hb, P->O, P->dO,
-                  P->dOb, P->dH, P->dHb, P->dX5, P->dY, P->dY2, P->dYb, P->dcol, P->part, P->loss_tmp,
+                  P->dOb, P->dH, P->dHb, P->dX5, P->wt, P->part, P->loss_tmp,
                   P->fuse_count};
   for (void* q : ptrs) (void)hipFree(q);
   for (int l = 0; l < kConvs; ++l) {
     if (l + 1 < kConvs) (void)hipFree(P->Yb[l]);
     (void)hipFree(P->col[l]);
+    (void)hipFree(P->dYb[l]);
+    (void)hipFree(P->bpart[l]);
   }
   delete P;
   return KF_OK;
@@ -842,19 +863,18 @@ extern "C" kf_status kf_prior_create(int32_t max_batch, kf_prior** out) {
   };
   al((void**)&P->params, P->nparams * 4);
   al((void**)&P->wbf, P->nparams * 2);
+  al((void**)&P->wt, P->nparams * 2);
   al((void**)&P->grad, P->nparams * 4);
   al((void**)&P->adam_m, P->nparams * 4);
   al((void**)&P->adam_v, P->nparams * 4);
-  long maxact = 0, maxdcol = 0;
   for (int l = 0; l < kConvs; ++l) {
     const ConvShape& c = kConv[l];
     const long M = B * c.hout * c.wout;
     if (l + 1 < kConvs) al((void**)&P->Yb[l], M * c.cout * 2);
     else al((void**)&P->Y4, M * c.cout * 4);
     al((void**)&P->col[l], M * kcp(l) * 2);
-    maxact = std::max(maxact, M * c.cout);
-    maxact = std::max(maxact, B * c.hin * c.win * c.cin);
-    if (l > 0) maxdcol = std::max(maxdcol, M * c.kc);
+    al((void**)&P->dYb[l], M * c.cout * 2);
+    al((void**)&P->bpart[l], (l + 1 < kConvs ? kConvBlocks : B) * c.cout * 4);
   }
   al((void**)&P->X5, B * kFc1In * 4);
   al((void**)&P->X5b, B * kFc1In * 2);
@@ -866,10 +886,6 @@ extern "C" kf_status kf_prior_create(int32_t max_batch, kf_prior** out) {
   al((void**)&P->dH, B * kHidden * 4);
   al((void**)&P->dHb, B * kHidden * 2);
   al((void**)&P->dX5, B * kFc1In * 4);
-  al((void**)&P->dY, maxact * 4);
-  al((void**)&P->dY2, maxact * 4);
-  al((void**)&P->dYb, maxact * 2);
-  al((void**)&P->dcol, maxdcol * 4);
   P->part_floats = 64L * 128 * 576;  // up to 64 splits of the largest weight matrix
   al((void**)&P->part, P->part_floats * 4);
   al((void**)&P->loss_tmp, 16);

@@ -123,8 +123,8 @@ __global__ __launch_bounds__(kConvThreads) void conv1_forward(const float* frame
 // Layers 2-4 forward.  Bound by the L1 path of the pixel loads (each map vector is read
 // by up to four taps).  NT is chosen so that every layer's share is 144 weight
 // registers (two waves per SIMD).  Batch 256: 31 / 33 / 23 us for layers 2 / 3 / 4
-// (365 / 172 / 131 TFLOP/s), layer 1 30 us; im2col and the staged GEMM took 1070 us for
-// the four.  NT: 16-channel tiles of a wave (COUT / (16 NT) waves cover a
+// (365 / 172 / 131 TFLOP/s), layer 1 30 us; GEMMs staged through LDS took 570 us for the
+// four.  NT: 16-channel tiles of a wave (COUT / (16 NT) waves cover a
 // pixel's channels); F32: FP32 output (layer 4, which the pooling reads), else BF16.
 template <int L, int NT, bool F32>
 __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* X, const uint16_t* W, const float* bias,
@@ -180,6 +180,143 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* 
     } else {
       store_bf16<4 * NT>(Yb + o, y);
     }
+  }
+}
+
+// Input gradient of layer L (1..3), ReLU mask of the layer below and that layer's bias
+// sums in one pass: dX[n][iy][ix][ci] = sum over the taps (ky, kx) that reach the
+// pixel, in that order, of sum_co dY[n][oy][ox][co] W[co][(ky, kx, ci)]; 0 where the
+// forward map Xb is not positive.  A wave takes 16 2x2 pixel blocks (rows 2j, 2j + 1,
+// columns 2i, 2i + 1): with stride 2 their nine taps read only the four output pixels
+// (j .. j + 1, i .. i + 1), so dY is read four times and every product is needed.
+// The weights ([tap][ci][co], so that eight co are one vector) stay in 144 registers.
+// Each tap's product is an MFMA chain of its own from zero and the taps are added in
+// FP32: the bits of a column-gradient GEMM followed by col2im, without the FP32 column
+// matrix (354 MB for layer 2 at batch 256).  bpart: per block and channel the FP32 sum
+// of the unrounded gradients.  Batch 256: layers 2 / 3 / 4 in 65 / 34 / 27 us (layer 2:
+// 197 MB through memory); the GEMM, col2im, conversion and column sums took 4.3 ms.
+template <int L, int NT>
+__global__ __launch_bounds__(kConvThreads, 2) void conv_dgrad(const uint16_t* dY, const uint16_t* Wt, const uint16_t* Xb,
+                                                              uint16_t* dX, float* bpart, int M) {
+  constexpr ConvShape c = kConv[L];
+  constexpr int KS = c.cout / 32, GROUPS = c.cin / (16 * NT), CH = 4 * NT;
+  static_assert(c.win == 2 * c.wout && (c.hin == 2 * c.hout || c.hin == 2 * c.hout - 1) && kConvWaves % GROUPS == 0,
+                "layer shape");
+  __shared__ float s_b[kConvWaves][16 * NT];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
+  const int gw = blockIdx.x * kConvWaves + wave, group = gw % GROUPS;
+  const int ch0 = group * 16 * NT;
+  uint4 w[9][KS][NT];
+#pragma unroll
+  for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+        w[tap][s][t] = *reinterpret_cast<const uint4*>(Wt + (tap * c.cin + ch0 + tile_channel<NT>(t, r)) * c.cout + 32 * s + 8 * q);
+  float bs[CH];
+#pragma unroll
+  for (int j = 0; j < CH; ++j) bs[j] = 0.0f;
+  const int stride = gridDim.x * kConvWaves / GROUPS;
+  for (int tile = gw / GROUPS; tile * 16 < M; tile += stride) {
+    const bool live = tile * 16 + r < M;
+    const int m = live ? tile * 16 + r : M - 1;
+    const int n = m / (c.hout * c.wout), p = m - n * (c.hout * c.wout);
+    const int j = p / c.wout, i = p - j * c.wout;
+    uint4 a[2][2][KS];  // dY at (j + dj, i + di), 0 outside the map
+#pragma unroll
+    for (int dj = 0; dj < 2; ++dj)
+#pragma unroll
+      for (int di = 0; di < 2; ++di) {
+        const bool in = (dj == 0 || j + 1 < c.hout) && (di == 0 || i + 1 < c.wout);
+        const uint16_t* src = dY + (in ? (m + dj * c.wout + di) * c.cout : 0) + 8 * q;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          a[dj][di][s] = *reinterpret_cast<const uint4*>(src + 32 * s);
+          if (!in) a[dj][di][s] = make_uint4(0u, 0u, 0u, 0u);
+        }
+      }
+#pragma unroll
+    for (int py = 0; py < 2; ++py)
+#pragma unroll
+      for (int px = 0; px < 2; ++px) {
+        float sum[CH];
+#pragma unroll
+        for (int e = 0; e < CH; ++e) sum[e] = 0.0f;
+#pragma unroll
+        for (int ky = 1 - py; ky < 3; ky += 2)
+#pragma unroll
+          for (int kx = 1 - px; kx < 3; kx += 2) {
+            const int dj = ky == 0 ? 1 : 0, di = kx == 0 ? 1 : 0;  // odd pixels: tap 0 is the next output pixel, tap 2 this one
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+              v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+              for (int s = 0; s < KS; ++s) acc = mfma32(w[ky * 3 + kx][s][t], a[dj][di][s], acc);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) sum[4 * t + e] = sum[4 * t + e] + acc[e];
+            }
+          }
+        const int iy = 2 * j + py, ix = 2 * i + px;
+        if (live && (c.hin == 2 * c.hout || iy < c.hin)) {
+          const int o = ((n * c.hin + iy) * c.win + ix) * c.cin + ch0 + CH * q;
+          uint16_t x[CH];
+          __builtin_memcpy(x, __builtin_assume_aligned(Xb + o, 2 * CH), 2 * CH);
+#pragma unroll
+          for (int e = 0; e < CH; ++e) {
+            sum[e] = (int16_t)x[e] > 0 ? sum[e] : 0.0f;
+            bs[e] = bs[e] + sum[e];
+          }
+          store_bf16<CH>(dX + o, sum);
+        }
+      }
+  }
+#pragma unroll
+  for (int e = 0; e < CH; ++e) {
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) bs[e] = bs[e] + __shfl_xor(bs[e], o, kWave);
+    if (r == 0) s_b[wave][CH * q + e] = bs[e];
+  }
+  __syncthreads();
+  if (threadIdx.x < c.cin) {
+    const int g = threadIdx.x / (16 * NT), k = threadIdx.x - g * 16 * NT;
+    float v = s_b[g][k];
+    for (int u = g + GROUPS; u < kConvWaves; u += GROUPS) v = v + s_b[u][k];
+    bpart[(long)blockIdx.x * c.cin + threadIdx.x] = v;
+  }
+}
+
+// Sums of partial planes, several at once: out[i] = sum over p < planes of
+// part[p * count + i].  A block takes 64 outputs; its sixteen waves each add every
+// sixteenth plane (eight loads in flight), and the sixteen sums are added in order.
+constexpr int kReduceJobs = 8;
+struct ReduceArgs {
+  const float* part[kReduceJobs];
+  float* out[kReduceJobs];
+  int planes[kReduceJobs], count[kReduceJobs], block0[kReduceJobs + 1];
+  int jobs;
+};
+
+__global__ __launch_bounds__(1024) void reduce_parts(ReduceArgs a) {
+  __shared__ float s_v[16][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int k = 0;
+  while (k + 1 < a.jobs && (int)blockIdx.x >= a.block0[k + 1]) ++k;
+  const int i = ((int)blockIdx.x - a.block0[k]) * 64 + lane, count = a.count[k], planes = a.planes[k];
+  const float* src = a.part[k] + min(i, count - 1);
+  float sum = 0.0f;
+  for (int p = wave; p < planes; p += 128) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = p + 16 * u < planes ? src[(long)(p + 16 * u) * count] : 0.0f;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) sum = sum + v[u];
+  }
+  s_v[wave][lane] = sum;
+  __syncthreads();
+  if (wave == 0 && i < count) {
+    for (int u = 1; u < 16; ++u) sum = sum + s_v[u][lane];
+    a.out[k][i] = sum;
   }
 }
 
