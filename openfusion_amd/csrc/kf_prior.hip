@@ -8,10 +8,10 @@
 //
 // Layout: activations NHWC (pixel-major, channel fastest), layers 1-3 as BF16 (the
 // next layer's operand), layer 4 FP32; products are BF16 (round to nearest even) with
-// FP32 accumulation.  The training forward's convolutions and the input gradients read
-// the maps directly (kf_prior_conv.hpp); the weight gradient is a GEMM over an im2col
-// matrix with deterministic split-K over pixels.  The GEMM is one 16x16 output tile per wavefront on
-// v_mfma_f32_16x16x32_bf16, four wavefronts per 256-thread block.
+// FP32 accumulation.  Training's convolutions, their input and weight gradients read
+// the maps directly (kf_prior_conv.hpp).  The fully connected layers' GEMM is one 16x16
+// output tile per wavefront on v_mfma_f32_16x16x32_bf16, four wavefronts per 256-thread
+// block.
 #include "kf_prior_conv.hpp"
 
 #include <math.h>
@@ -25,8 +25,7 @@ namespace {
 
 // ---------------------------------------------------------------------------
 // GEMM: C[m][n] (+)= sum_k A(m,k) B(k,n); A(m,k) = A[m*sam + k*sak], B(k,n) =
-// B[k*sbk + n*sbn] (BF16 bits).  Split s of gridDim.z covers k in
-// [s*kps, (s+1)*kps) and, when Cpart is set, writes its own partial plane.
+// B[k*sbk + n*sbn] (BF16 bits).
 struct GemmArgs {
   const uint16_t* A;
   long sam, sak;
@@ -34,9 +33,8 @@ struct GemmArgs {
   long sbk, sbn;
   float* C;
   long ldc;
-  float* Cpart;
-  int M, N, K, kps, accumulate;
-  // Epilogue (no split-K): v = acc [+ bias[n], ReLU] [+ addend[m * N + n]]; C = v and,
+  int M, N, K, accumulate;
+  // Epilogue: v = acc [+ bias[n], ReLU] [+ addend[m * N + n]]; C = v and,
   // with Cb, the BF16 copy (RNE) at the same position.
   const float* bias;
   int relu;
@@ -52,7 +50,7 @@ struct GemmArgs {
 // sequence over k (steps of 32 from 0, zeros beyond K) is the same as a direct k
 // loop, so results do not depend on the chunking; any kernel that runs the same
 // sequence on the same operands gets the same bits.
-constexpr int kKc = 576;        // whole K of every convolution layer fits one chunk
+constexpr int kKc = 576;        // K per chunk
 constexpr int kPitch = kKc + 8;  // LDS row pitch (elements): rows start on different banks
 constexpr int kVecPerThread = (32 * kKc / 8 + 255) / 256;  // 16-byte vectors per thread and operand
 
@@ -125,12 +123,10 @@ __global__ __launch_bounds__(256) void gemm_bf16(GemmArgs g) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int mt = blockIdx.y * 32, nt = blockIdx.x * 32;
   const int wm = (wave >> 1) * 16, wn = (wave & 1) * 16;
-  const int kbeg = blockIdx.z * g.kps;
-  const int kend = min(g.K, kbeg + g.kps);
   const int r = lane & 15, kq = (lane >> 4) * 8;
   v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int kc0 = kbeg; kc0 < kend; kc0 += kKc) {
-    const int kn = min(kKc, kend - kc0);
+  for (int kc0 = 0; kc0 < g.K; kc0 += kKc) {
+    const int kn = min(kKc, g.K - kc0);
     const int kpad = (kn + 31) & ~31;
     stage(As, g.A, g.sam, g.sak, mt, g.M, kc0, kn, kpad);
     stage(Bt, g.B, g.sbn, g.sbk, nt, g.N, kc0, kn, kpad);
@@ -148,9 +144,7 @@ __global__ __launch_bounds__(256) void gemm_bf16(GemmArgs g) {
   for (int j = 0; j < 4; ++j) {
     const int cm = m0 + (lane >> 4) * 4 + j;
     if (cm >= g.M) continue;
-    if (g.Cpart) {
-      g.Cpart[((long)blockIdx.z * g.M + cm) * g.N + cn] = acc[j];
-    } else {
+    {
       float* c = g.C + (long)cm * g.ldc + cn;
       float v = g.accumulate ? *c + acc[j] : acc[j];
       if (g.bias) {
@@ -162,14 +156,6 @@ __global__ __launch_bounds__(256) void gemm_bf16(GemmArgs g) {
       if (g.Cb) g.Cb[(long)cm * g.ldc + cn] = bf16_rne(v);
     }
   }
-}
-
-__global__ void splitk_reduce(const float* part, int splits, long MN, int N, float* C, long ldc) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= MN) return;
-  float s = 0.0f;
-  for (int z = 0; z < splits; ++z) s = s + part[(long)z * MN + i];
-  C[(i / N) * ldc + (i % N)] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -419,45 +405,6 @@ __global__ __launch_bounds__(kFuseThreads) void prior_infer_fused(FuseArgs f) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// im2col.  Layer 1 reads the two depth planes of each pair directly.
-__global__ void im2col_pairs(const float* frames, const int32_t* pairs, int batch, uint16_t* col, int kcp) {
-  const ConvShape c = kConv[0];
-  const long M = (long)batch * c.hout * c.wout;
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= M * kcp) return;
-  const long m = i / kcp;
-  const int k = (int)(i - m * kcp);
-  float v = 0.0f;
-  if (k < c.kc) {
-    const int n = (int)(m / (c.hout * c.wout));
-    const int p = (int)(m - (long)n * c.hout * c.wout);
-    const int oy = p / c.wout, ox = p - oy * c.wout;
-    const int ky = k / (3 * c.cin), kx = (k / c.cin) % 3, ci = k % c.cin;
-    const int iy = 2 * oy + ky - 1, ix = 2 * ox + kx - 1;
-    if (iy >= 0 && iy < c.hin && ix >= 0 && ix < c.win)
-      v = frames[((long)pairs[2 * n + ci] * kH0 + iy) * kW0 + ix];
-  }
-  col[i] = bf16_rne(v);
-}
-
-__global__ void im2col_nhwc(const uint16_t* X, int layer, int batch, uint16_t* col) {
-  const ConvShape c = kConv[layer];
-  const long M = (long)batch * c.hout * c.wout;
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= M * c.kc) return;
-  const long m = i / c.kc;
-  const int k = (int)(i - m * c.kc);
-  const int n = (int)(m / (c.hout * c.wout));
-  const int p = (int)(m - (long)n * c.hout * c.wout);
-  const int oy = p / c.wout, ox = p - oy * c.wout;
-  const int ky = k / (3 * c.cin), kx = (k / c.cin) % 3, ci = k % c.cin;
-  const int iy = 2 * oy + ky - 1, ix = 2 * ox + kx - 1;
-  uint16_t v = 0;
-  if (iy >= 0 && iy < c.hin && ix >= 0 && ix < c.win) v = X[(((long)n * c.hin + iy) * c.win + ix) * c.cin + ci];
-  col[i] = v;
-}
-
 __global__ void to_bf16(const float* x, uint16_t* y, long n) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) y[i] = bf16_rne(x[i]);
@@ -585,10 +532,9 @@ struct kf_prior {
   float* adam_m = nullptr;
   float* adam_v = nullptr;
   long step = 0;
-  // activations (NHWC) and BF16 im2col buffers, sized for max_batch
+  // activations (NHWC), sized for max_batch
   uint16_t* Yb[kf::kConvs - 1] = {};  // layers 1-3, BF16 NHWC
   float* Y4 = nullptr;                // layer 4, FP32
-  uint16_t* col[kf::kConvs] = {};
   float* X5 = nullptr;
   uint16_t* X5b = nullptr;
   float* Hd = nullptr;
@@ -601,16 +547,13 @@ struct kf_prior {
   float* dX5 = nullptr;
   uint16_t* dYb[kf::kConvs] = {};       // gradients of the layers' outputs, BF16 NHWC
   float* bpart[kf::kConvs] = {};        // partial bias sums per block (layer 4: per sample)
-  float* part = nullptr;  // split-K partial planes
-  long part_floats = 0;
+  float* wpart[kf::kConvs] = {};        // partial weight gradients per split
   float* loss_tmp = nullptr;
   unsigned* fuse_count = nullptr;  // [max_batch] finished blocks per sample of the fused inference
 };
 
 namespace kf {
 namespace {
-
-constexpr int kSplitMaxK = 4096;  // pixels per split in weight-gradient GEMMs
 
 struct Epilogue {
   const float* bias = nullptr;
@@ -620,7 +563,7 @@ struct Epilogue {
 };
 
 kf_status gemm(hipStream_t s, const uint16_t* A, long sam, long sak, const uint16_t* B, long sbk, long sbn, float* C,
-               long ldc, int M, int N, int K, bool accumulate, float* part = nullptr, long part_floats = 0,
+               long ldc, int M, int N, int K, bool accumulate,
                const Epilogue& ep = Epilogue()) {
   GemmArgs g;
   g.bias = ep.bias;
@@ -639,29 +582,11 @@ kf_status gemm(hipStream_t s, const uint16_t* A, long sam, long sak, const uint1
   g.N = N;
   g.K = K;
   g.accumulate = accumulate ? 1 : 0;
-  int splits = 1;
-  if (part && K > kSplitMaxK) {
-    splits = (K + kSplitMaxK - 1) / kSplitMaxK;
-    while ((long)splits * M * N > part_floats && splits > 1) splits = (splits + 1) / 2;
-  }
-  g.kps = splits > 1 ? (((K + splits - 1) / splits + 15) / 16) * 16 : ((K + 15) / 16) * 16;
-  if (splits > 1) splits = (K + g.kps - 1) / g.kps;
-  g.Cpart = splits > 1 ? part : nullptr;
-  dim3 grid((N + 31) / 32, (M + 31) / 32, splits);
+  dim3 grid((N + 31) / 32, (M + 31) / 32);
   hipLaunchKernelGGL(gemm_bf16, grid, dim3(256), 0, s, g);
   KF_TRY(check_launch("gemm_bf16"));
-  if (splits > 1) {
-    KF_CHECK_ARG(!accumulate && !ep.bias && !ep.addend && !ep.Cb, "split-K GEMM has no epilogue");
-    const long MN = (long)M * N;
-    hipLaunchKernelGGL(splitk_reduce, dim3(blocks_for(MN)), dim3(256), 0, s, (const float*)part, splits, MN, N, C,
-                       ldc);
-    KF_TRY(check_launch("splitk_reduce"));
-  }
   return KF_OK;
 }
-
-const ConvShape& conv(int l) { return kConv[l]; }
-int kcp(int l) { return l == 0 ? 32 : kConv[l].kc; }  // im2col row length (layer 1 padded to 32)
 
 // BF16 copies of the weights; every call that changes the FP32 parameters refreshes
 // them, so inference (forward) never converts.
@@ -726,17 +651,6 @@ kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, const 
   KF_TRY((launch_conv<1, 4, false>(P, P->Yb[0], P->Yb[1], nullptr, B, s)));
   KF_TRY((launch_conv<2, 2, false>(P, P->Yb[1], P->Yb[2], nullptr, B, s)));
   KF_TRY((launch_conv<3, 2, true>(P, P->Yb[2], nullptr, P->Y4, B, s)));
-  for (int l = 0; l < kConvs; ++l) {  // the weight gradients' operands
-    const ConvShape& c = conv(l);
-    const long M = (long)B * c.hout * c.wout;
-    if (l == 0)
-      hipLaunchKernelGGL(im2col_pairs, dim3(blocks_for(M * kcp(0))), dim3(256), 0, s, frames, pairs, B, P->col[0],
-                         kcp(0));
-    else
-      hipLaunchKernelGGL(im2col_nhwc, dim3(blocks_for(M * c.kc)), dim3(256), 0, s, (const uint16_t*)P->Yb[l - 1], l, B,
-                         P->col[l]);
-    KF_TRY(check_launch("im2col"));
-  }
   hipLaunchKernelGGL(pool_concat, dim3(blocks_for((long)B * kFc1In)), dim3(256), 0, s, (const float*)P->Y4, prev, B,
                      P->X5, P->X5b);
   KF_TRY(check_launch("pool_concat"));
@@ -745,15 +659,14 @@ kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, const 
     ep.bias = (const float*)P->params + L.b[4];
     ep.relu = 1;
     ep.Cb = P->Hb;
-    KF_TRY(gemm(s, P->X5b, kFc1In, 1, P->wbf + L.w[4], 1, kFc1In, P->Hd, kHidden, B, kHidden, kFc1In, false, nullptr,
-                0, ep));
+    KF_TRY(gemm(s, P->X5b, kFc1In, 1, P->wbf + L.w[4], 1, kFc1In, P->Hd, kHidden, B, kHidden, kFc1In, false, ep));
   }
   {  // FC2 plus the skip connection: O = (H W6^T + b6) + previous twist
     Epilogue ep;
     ep.bias = (const float*)P->params + L.b[5];
     ep.addend = prev;
     KF_TRY(gemm(s, P->Hb, kHidden, 1, P->wbf + L.w[5], 1, kHidden, P->O, kTwist, B, kTwist, kHidden,
-                false, nullptr, 0, ep));
+                false, ep));
   }
   return KF_OK;
 }
@@ -771,7 +684,25 @@ kf_status launch_dgrad(kf_prior* P, int B, int* planes, hipStream_t s) {
   return check_launch("conv_dgrad");
 }
 
-kf_status backward(kf_prior* P, const float* target, int B, float* loss, hipStream_t s) {
+// Weight gradient of layer L as *splits partial planes: one block a CU, at least
+// kWgradMinSteps steps of 32 pixels each (a shorter split would mostly write its plane).
+constexpr int kWgradBlocks = 256, kWgradMinSteps = 4;
+template <int L>
+kf_status launch_wgrad(kf_prior* P, int B, int* splits, hipStream_t s) {
+  constexpr int GROUPS = WgradShape<L>::GROUPS;
+  const int M = B * kConv[L].hout * kConv[L].wout, steps = div_up(M, kWgradStep);
+  const int want = std::min(std::max(steps / kWgradMinSteps, 1), kWgradBlocks / GROUPS);
+  const int per = div_up(steps, want);
+  *splits = div_up(steps, per);
+  // eight splits a round (blocks of one split on one XCD): the grid is rounded up, and
+  // the splits past the last write zero planes that nothing reads
+  const int grid = div_up(*splits, 8) * 8 * GROUPS;
+  hipLaunchKernelGGL(conv_wgrad<L>, dim3(grid), dim3(kConvThreads), 0, s, (const uint16_t*)P->dYb[L],
+                     (const uint16_t*)P->Yb[L - 1], P->wpart[L], M, per);
+  return check_launch("conv_wgrad");
+}
+
+kf_status backward(kf_prior* P, const float* frames, const int32_t* pairs, const float* target, int B, float* loss, hipStream_t s) {
   const ParamLayout& L = layout();
   float* G = P->grad;
   hipLaunchKernelGGL(mse_loss, dim3(1), dim3(256), 0, s, (const float*)P->O, target, B, P->dO, loss);
@@ -793,10 +724,18 @@ kf_status backward(kf_prior* P, const float* target, int B, float* loss, hipStre
   hipLaunchKernelGGL(pool_backward, dim3(B), dim3(2 * kFeat), 0, s, (const float*)P->dX5, (const float*)P->Y4,
                      P->dYb[3], P->bpart[3]);
   KF_TRY(check_launch("pool_backward"));
-  int planes[kConvs] = {0, 0, 0, B};
+  int planes[kConvs] = {0, 0, 0, B}, splits[kConvs];
+  KF_TRY(launch_wgrad<3>(P, B, &splits[3], s));
   KF_TRY((launch_dgrad<3, 1>(P, B, &planes[2], s)));
+  KF_TRY(launch_wgrad<2>(P, B, &splits[2], s));
   KF_TRY((launch_dgrad<2, 2>(P, B, &planes[1], s)));
+  KF_TRY(launch_wgrad<1>(P, B, &splits[1], s));
   KF_TRY((launch_dgrad<1, 2>(P, B, &planes[0], s)));
+  const int items = B * (kConv[0].hout / kL1Rows);
+  splits[0] = std::min(items, kConvBlocks);
+  hipLaunchKernelGGL(conv1_wgrad, dim3(splits[0]), dim3(kConvThreads), 0, s, frames, pairs, (const uint16_t*)P->dYb[0],
+                     P->wpart[0], items);
+  KF_TRY(check_launch("conv1_wgrad"));
   ReduceArgs red;
   red.jobs = 0;
   red.block0[0] = 0;
@@ -809,12 +748,8 @@ kf_status backward(kf_prior* P, const float* target, int B, float* loss, hipStre
     red.block0[k + 1] = red.block0[k] + div_up(count, 64);
   };
   for (int l = kConvs - 1; l >= 0; --l) {
-    const ConvShape& c = conv(l);
-    const long M = (long)B * c.hout * c.wout;
-    // dW[co][k] = sum_m dY[m][co] col[m][k]   (split-K over pixels, deterministic)
-    KF_TRY(gemm(s, P->dYb[l], 1, c.cout, P->col[l], kcp(l), 1, G + L.w[l], c.kc, c.cout, c.kc, (int)M, false, P->part,
-                P->part_floats));
-    add(P->bpart[l], planes[l], c.cout, G + L.b[l]);
+    add(P->wpart[l], splits[l], kConv[l].cout * kConv[l].kc, G + L.w[l]);
+    add(P->bpart[l], planes[l], kConv[l].cout, G + L.b[l]);
   }
   hipLaunchKernelGGL(reduce_parts, dim3(red.block0[red.jobs]), dim3(1024), 0, s, red);
   KF_TRY(check_launch("reduce_parts"));
@@ -837,12 +772,12 @@ extern "C" int64_t kf_prior_param_count(void) { return layout().total; }
 extern "C" kf_status kf_prior_destroy(kf_prior* P) {
   if (!P) return KF_OK;
   void* ptrs[] = {P->params, P->wbf, P->grad, P->adam_m, P->adam_v, P->Y4, P->X5, P->X5b, P->Hd, P->Hb, P->O, P->dO,
-                  P->dOb, P->dH, P->dHb, P->dX5, P->wt, P->part, P->loss_tmp,
+                  P->dOb, P->dH, P->dHb, P->dX5, P->wt, P->loss_tmp,
                   P->fuse_count};
   for (void* q : ptrs) (void)hipFree(q);
   for (int l = 0; l < kConvs; ++l) {
     if (l + 1 < kConvs) (void)hipFree(P->Yb[l]);
-    (void)hipFree(P->col[l]);
+    (void)hipFree(P->wpart[l]);
     (void)hipFree(P->dYb[l]);
     (void)hipFree(P->bpart[l]);
   }
@@ -872,7 +807,7 @@ extern "C" kf_status kf_prior_create(int32_t max_batch, kf_prior** out) {
     const long M = B * c.hout * c.wout;
     if (l + 1 < kConvs) al((void**)&P->Yb[l], M * c.cout * 2);
     else al((void**)&P->Y4, M * c.cout * 4);
-    al((void**)&P->col[l], M * kcp(l) * 2);
+    al((void**)&P->wpart[l], (l == 0 ? kConvBlocks : kWgradBlocks / (c.cout / (l == 1 ? 64 : 32))) * c.cout * c.kc * 4);
     al((void**)&P->dYb[l], M * c.cout * 2);
     al((void**)&P->bpart[l], (l + 1 < kConvs ? kConvBlocks : B) * c.cout * 4);
   }
@@ -886,8 +821,6 @@ extern "C" kf_status kf_prior_create(int32_t max_batch, kf_prior** out) {
   al((void**)&P->dH, B * kHidden * 4);
   al((void**)&P->dHb, B * kHidden * 2);
   al((void**)&P->dX5, B * kFc1In * 4);
-  P->part_floats = 64L * 128 * 576;  // up to 64 splits of the largest weight matrix
-  al((void**)&P->part, P->part_floats * 4);
   al((void**)&P->loss_tmp, 16);
   al((void**)&P->fuse_count, B * sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(P->fuse_count, 0, B * sizeof(unsigned));
@@ -956,7 +889,7 @@ extern "C" kf_status kf_prior_gradients(kf_prior* P, const float* frames, const 
   KF_TRY(check_batch(P, frames, pairs, prev, B));
   KF_CHECK_ARG(target && d_grad, "NULL argument");
   KF_TRY(forward(P, frames, pairs, prev, B, S(s)));
-  KF_TRY(backward(P, target, B, d_loss, S(s)));
+  KF_TRY(backward(P, frames, pairs, target, B, d_loss, S(s)));
   KF_HIP(hipMemcpyAsync(d_grad, P->grad, (size_t)P->nparams * 4, hipMemcpyDeviceToDevice, S(s)));
   return KF_OK;
 }
@@ -966,7 +899,7 @@ extern "C" kf_status kf_prior_train_step(kf_prior* P, const float* frames, const
   KF_TRY(check_batch(P, frames, pairs, prev, B));
   KF_CHECK_ARG(target != nullptr, "target is NULL");
   KF_TRY(forward(P, frames, pairs, prev, B, S(s)));
-  KF_TRY(backward(P, target, B, d_loss, S(s)));
+  KF_TRY(backward(P, frames, pairs, target, B, d_loss, S(s)));
   P->step += 1;
   const float b1 = 0.9f, b2 = 0.999f;
   const float c1 = 1.0f - (float)pow(0.9, (double)P->step), c2 = 1.0f - (float)pow(0.999, (double)P->step);

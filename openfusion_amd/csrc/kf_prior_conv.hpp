@@ -193,7 +193,7 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* 
 // Each tap's product is an MFMA chain of its own from zero and the taps are added in
 // FP32: the bits of a column-gradient GEMM followed by col2im, without the FP32 column
 // matrix (354 MB for layer 2 at batch 256).  bpart: per block and channel the FP32 sum
-// of the unrounded gradients.  Batch 256: layers 2 / 3 / 4 in 65 / 34 / 27 us (layer 2:
+// of the unrounded gradients.  Batch 256: layers 2 / 3 / 4 in 50 / 34 / 27 us (layer 2:
 // 197 MB through memory); the GEMM, col2im, conversion and column sums took 4.3 ms.
 template <int L, int NT>
 __global__ __launch_bounds__(kConvThreads, 2) void conv_dgrad(const uint16_t* dY, const uint16_t* Wt, const uint16_t* Xb,
@@ -283,6 +283,160 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_dgrad(const uint16_t* dY
     float v = s_b[g][k];
     for (int u = g + GROUPS; u < kConvWaves; u += GROUPS) v = v + s_b[u][k];
     bpart[(long)blockIdx.x * c.cin + threadIdx.x] = v;
+  }
+}
+
+// Weight gradients contract over pixels, while the maps keep a pixel's channels
+// together.  The tiles are staged in LDS as they lie in memory, one row of channels per
+// pixel, and the operands come from transposing LDS reads (ds_read_b64_tr_b16): of
+// each 16-lane group, lanes 4 i .. 4 i + 3 address the 16 channels of pixel row i, and
+// lane c receives channel c of the four rows.  A fragment is two such reads, pixels
+// 4 q .. 4 q + 3 and 16 + 4 q .. of the 32 staged (both operands in the same order).
+// Row pitches are odd multiples of 8 dwords, so that the eight rows of 32 bytes that
+// a half-wave reads cover all 64 banks.
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4s lds_v4s;
+
+__device__ __forceinline__ uint4 transposed_fragment(const uint16_t* rows, int pitch, int c0, int r, int q) {
+  const uint16_t* p = rows + (4 * q + (r >> 2)) * pitch + c0 + 4 * (r & 3);
+  const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(p));
+  const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(p + 16 * pitch));
+  const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
+  return make_uint4(a.x, a.y, b.x, b.y);
+}
+
+// Weight gradient of layer L (1..3): dW[co][k] = sum_m dY[m][co] col[m][k], col the
+// im2col element read straight from the map X.  A block takes one split of the pixels
+// and COB output channels; a wave 2 x 9 tiles of them, so that eleven fragment reads
+// feed eighteen MFMAs.  Per step of 32 pixels the next step's vectors are in flight
+// while this one's tiles are multiplied.  Each split writes its own plane
+// (reduce_parts adds them in order, 16 us for all).  Bound by the L1 path of the map
+// loads and the LDS reads.  Batch 256: layers 2 / 3 / 4 in 45 / 24 / 15 us (250 / 240 /
+// 198 TFLOP/s); the im2col matrices and the GEMMs over them took 2.3 ms with layer 1.
+constexpr int kWgradStep = 32;
+template <int L>
+struct WgradShape {
+  static constexpr int COB = L == 1 ? 64 : 32;             // output channels of a block
+  static constexpr int GROUPS = kConv[L].cout / COB;
+  static constexpr int NW = kConv[L].kc / (9 * 16);        // waves along the weight columns
+  static_assert(NW * (COB / 32) == kConvWaves && kConv[L].kc % (9 * 16) == 0, "wave tiles");
+};
+
+template <int L>
+__global__ __launch_bounds__(kConvThreads, 2) void conv_wgrad(const uint16_t* dY, const uint16_t* X, float* part, int M,
+                                                              int steps_per_split) {
+  constexpr ConvShape c = kConv[L];
+  constexpr int COB = WgradShape<L>::COB, GROUPS = WgradShape<L>::GROUPS, NW = WgradShape<L>::NW;
+  constexpr int kColPitch = c.kc + 16, kDyPitch = COB + 16;
+  constexpr int kTapVecs = c.cin / 8, kVecs = c.kc / 8, kPer = (kVecs + 7) / 8;  // eight threads per pixel
+  __shared__ __align__(16) uint16_t s_col[kWgradStep * kColPitch];
+  __shared__ __align__(16) uint16_t s_dy[kWgradStep * kDyPitch];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4;
+  // the groups of a split read the same map: keep them on one XCD (blocks go round-robin)
+  const int b = blockIdx.x, split = b / (8 * GROUPS) * 8 + b % 8, group = b / 8 % GROUPS;
+  const int co0 = group * COB;
+  const int px = tid >> 3, v0 = tid & 7;
+  const int first = split * steps_per_split, last = min(first + steps_per_split, (M + kWgradStep - 1) / kWgradStep);
+  uint4 vc[kPer], vd;
+  auto load = [&](int step) {
+    const int m = step * kWgradStep + px;
+    const bool live = m < M;
+    const int mm = live ? m : 0;
+    const int n = mm / (c.hout * c.wout), p = mm - n * (c.hout * c.wout);
+    const int oy = p / c.wout, ox = p - oy * c.wout;
+    const int at = ((n * c.hin + 2 * oy - 1) * c.win + 2 * ox - 1) * c.cin;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int v = v0 + 8 * u, tap = v / kTapVecs, ci = 8 * (v - tap * kTapVecs);
+      const int ky = tap / 3, kx = tap - 3 * ky;
+      const int iy = 2 * oy + ky - 1, ix = 2 * ox + kx - 1;
+      const bool in = live && v < kVecs && iy >= 0 && iy < c.hin && ix >= 0;
+      vc[u] = *reinterpret_cast<const uint4*>(X + (in ? at + (ky * c.win + kx) * c.cin + ci : 0));
+      if (!in) vc[u] = make_uint4(0u, 0u, 0u, 0u);
+    }
+    vd = make_uint4(0u, 0u, 0u, 0u);
+    if (live && v0 < COB / 8) vd = *reinterpret_cast<const uint4*>(dY + m * c.cout + co0 + 8 * v0);
+  };
+  v4f acc[2][9];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int i = 0; i < 9; ++i) acc[t][i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  const int cw = wave / NW * 32, nw = wave % NW * (9 * 16);  // the wave's first channel and column
+  if (first < last) load(first);
+  for (int step = first; step < last; ++step) {
+#pragma unroll
+    for (int u = 0; u < kPer; ++u)
+      if (v0 + 8 * u < kVecs) *reinterpret_cast<uint4*>(&s_col[px * kColPitch + 8 * (v0 + 8 * u)]) = vc[u];
+    if (v0 < COB / 8) *reinterpret_cast<uint4*>(&s_dy[px * kDyPitch + 8 * v0]) = vd;
+    __syncthreads();
+    if (step + 1 < last) load(step + 1);
+    uint4 a[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) a[t] = transposed_fragment(s_dy, kDyPitch, cw + 16 * t, r, q);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+      const uint4 f = transposed_fragment(s_col, kColPitch, nw + 16 * i, r, q);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) acc[t][i] = mfma32(a[t], f, acc[t][i]);
+    }
+    __syncthreads();
+  }
+  float* plane = part + (long)split * (c.cout * c.kc);
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) plane[(co0 + cw + 16 * t + 4 * q + j) * c.kc + nw + 16 * i + r] = acc[t][i][j];
+}
+
+// Weight gradient of layer 1.  A block walks over groups of four output rows: the input
+// rows staged as in the forward, from them the 320 x 18 im2col tile in LDS (columns
+// 18 .. 31 zero), beside it the rows' gradients; each wave one 16 x 16 tile of the
+// 32 x 32 products.  One plane per block.  Batch 256: 32 us (98 MB
+// read).
+constexpr int kL1Pix = kL1Rows * kConv[0].wout;
+__global__ __launch_bounds__(kConvThreads) void conv1_wgrad(const float* frames, const int32_t* pairs, const uint16_t* dY,
+                                                            float* part, int items) {
+  constexpr ConvShape c = kConv[0];
+  constexpr int kPitch = 32 + 16, kGroups = c.hout / kL1Rows;
+  static_assert(kL1Pix % kWgradStep == 0 && c.cout == 32, "layer-1 tiles");
+  __shared__ uint32_t patch[kL1In][kL1Pitch];
+  __shared__ __align__(16) uint16_t s_col[kL1Pix * kPitch];
+  __shared__ __align__(16) uint16_t s_dy[kL1Pix * kPitch];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4;
+  const int cw = (wave >> 1) * 16, nw = (wave & 1) * 16;
+  for (int e = tid; e < kL1Pix * 7; e += kConvThreads)  // columns 18 .. 31
+    *reinterpret_cast<uint32_t*>(&s_col[e / 7 * kPitch + 18 + 2 * (e % 7)]) = 0u;
+  v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int it = blockIdx.x; it < items; it += gridDim.x) {
+    const int n = it / kGroups, oy0 = (it - n * kGroups) * kL1Rows;
+    const uint16_t* src = dY + ((long)n * c.hout + oy0) * c.wout * c.cout;
+    constexpr int PER = kL1Pix * c.cout / 8 / kConvThreads;
+    uint4 v[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) v[u] = *reinterpret_cast<const uint4*>(src + 8 * (tid + kConvThreads * u));
+    stage_l1(patch, frames + (long)pairs[2 * n] * (kH0 * kW0), frames + (long)pairs[2 * n + 1] * (kH0 * kW0), oy0);
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int e = tid + kConvThreads * u;
+      *reinterpret_cast<uint4*>(&s_dy[(e >> 2) * kPitch + 8 * (e & 3)]) = v[u];
+    }
+    __syncthreads();
+    for (int e = tid; e < kL1Pix * 9; e += kConvThreads) {
+      const int p = e / 9, tap = e - 9 * p, oy = p / c.wout, ox = p - oy * c.wout;
+      *reinterpret_cast<uint32_t*>(&s_col[p * kPitch + 2 * tap]) = patch[2 * oy + tap / 3][2 * ox + tap % 3];
+    }
+    __syncthreads();
+    for (int p0 = 0; p0 < kL1Pix; p0 += kWgradStep)
+      acc = mfma32(transposed_fragment(s_dy + p0 * kPitch, kPitch, cw, r, q),
+                   transposed_fragment(s_col + p0 * kPitch, kPitch, nw, r, q), acc);
+    __syncthreads();
+  }
+  if (nw + r < c.kc) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) part[((long)blockIdx.x * c.cout + cw + 4 * q + j) * c.kc + nw + r] = acc[j];
   }
 }
 
