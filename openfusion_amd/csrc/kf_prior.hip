@@ -9,10 +9,9 @@
 // Layout: activations NHWC (pixel-major, channel fastest), layers 1-3 as BF16 (the
 // next layer's operand), layer 4 FP32; products are BF16 (round to nearest even) with
 // FP32 accumulation.  Training's convolutions, their input and weight gradients read
-// the maps directly (kf_prior_conv.hpp).  The fully connected layers' GEMM is one 16x16
-// output tile per wavefront on v_mfma_f32_16x16x32_bf16, four wavefronts per 256-thread
-// block.
-#include "kf_prior_conv.hpp"
+// the maps directly (kf_prior_conv.hpp); its fully connected layers run both ways in one
+// block per sample (kf_prior_head.hpp).
+#include "kf_prior_head.hpp"
 
 #include <math.h>
 #include <string.h>
@@ -24,159 +23,23 @@ namespace kf {
 namespace {
 
 // ---------------------------------------------------------------------------
-// GEMM: C[m][n] (+)= sum_k A(m,k) B(k,n); A(m,k) = A[m*sam + k*sak], B(k,n) =
-// B[k*sbk + n*sbn] (BF16 bits).
-struct GemmArgs {
-  const uint16_t* A;
-  long sam, sak;
-  const uint16_t* B;
-  long sbk, sbn;
-  float* C;
-  long ldc;
-  int M, N, K, accumulate;
-  // Epilogue: v = acc [+ bias[n], ReLU] [+ addend[m * N + n]]; C = v and,
-  // with Cb, the BF16 copy (RNE) at the same position.
-  const float* bias;
-  int relu;
-  const float* addend;
-  uint16_t* Cb;
-};
-
-// Each 256-thread block computes a 32x32 tile of C (four 16x16 wave tiles on
-// v_mfma_f32_16x16x32_bf16).  K is staged through LDS in chunks of kKc: the block
-// loads the 32 x chunk slices of A and B with coalesced accesses (adjacent threads
-// take adjacent addresses along whichever of K or M/N is unit-stride), then runs
-// the chunk's MFMAs from LDS, each operand one 16-byte LDS read per lane.  The MFMA
-// sequence over k (steps of 32 from 0, zeros beyond K) is the same as a direct k
-// loop, so results do not depend on the chunking; any kernel that runs the same
-// sequence on the same operands gets the same bits.
-constexpr int kKc = 576;        // K per chunk
-constexpr int kPitch = kKc + 8;  // LDS row pitch (elements): rows start on different banks
-constexpr int kVecPerThread = (32 * kKc / 8 + 255) / 256;  // 16-byte vectors per thread and operand
-
-// Stages a 32 x kpad operand slice into T[32][kPitch] (row = m or n, column = k)
-// from X(row, k) = X[row * s_row + k * s_k], zero outside rows < nrows, k < kn.
-__device__ __forceinline__ void stage(uint16_t (*T)[kPitch], const uint16_t* X, long s_row, long s_k, int row0,
-                                      int nrows, long k0, int kn, int kpad) {
-  const int tid = threadIdx.x;
-  const bool vec = s_k == 1 && (s_row & 7) == 0 && (k0 & 7) == 0 && (kn & 7) == 0 &&
-                   ((reinterpret_cast<uintptr_t>(X) & 15) == 0);
-  if (vec) {  // 16-byte loads of 8 consecutive k, all issued before any LDS store
-    const int vpr = kpad >> 3;  // vectors per row (the last one may be k padding)
-    const int total = 32 * vpr;
-    uint4 v[kVecPerThread];
-#pragma unroll
-    for (int u = 0; u < kVecPerThread; ++u) {
-      const int e = tid + 256 * u;
-      const int r = e / vpr, c = e - (e / vpr) * vpr;
-      const bool in = e < total && row0 + r < nrows && 8 * c < kn;
-      v[u] = in ? *reinterpret_cast<const uint4*>(X + (long)(row0 + r) * s_row + k0 + 8 * c) : make_uint4(0, 0, 0, 0);
-    }
-#pragma unroll
-    for (int u = 0; u < kVecPerThread; ++u) {
-      const int e = tid + 256 * u;
-      if (e < total) {
-        const int r = e / vpr, c = e - (e / vpr) * vpr;
-        *reinterpret_cast<uint4*>(&T[r][8 * c]) = v[u];
-      }
-    }
-  } else if (s_k == 1) {  // K contiguous: thread e takes (row, k) = (e / kpad, e % kpad)
-    const int total = 32 * kpad;
-    for (int e0 = tid; e0 < total; e0 += 256 * 4) {
-      uint16_t v[4];
-      int rr[4], kk[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int e = e0 + 256 * u;
-        rr[u] = e / kpad;
-        kk[u] = e - rr[u] * kpad;
-        const bool in = e < total && row0 + rr[u] < nrows && kk[u] < kn;
-        v[u] = in ? X[(long)(row0 + rr[u]) * s_row + (k0 + kk[u])] : (uint16_t)0;
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (e0 + 256 * u < total) T[rr[u]][kk[u]] = v[u];
-    }
-  } else {  // rows contiguous (or general): thread e takes (k, row) = (e / 32, e % 32)
-    const int total = 32 * kpad;
-    for (int e0 = tid; e0 < total; e0 += 256 * 4) {
-      uint16_t v[4];
-      int rr[4], kk[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int e = e0 + 256 * u;
-        kk[u] = e >> 5;
-        rr[u] = e & 31;
-        const bool in = e < total && row0 + rr[u] < nrows && kk[u] < kn;
-        v[u] = in ? X[(long)(row0 + rr[u]) * s_row + (k0 + kk[u]) * s_k] : (uint16_t)0;
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (e0 + 256 * u < total) T[rr[u]][kk[u]] = v[u];
-    }
-  }
-}
-
-__global__ __launch_bounds__(256) void gemm_bf16(GemmArgs g) {
-  __shared__ __align__(16) uint16_t As[32][kPitch];
-  __shared__ __align__(16) uint16_t Bt[32][kPitch];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int mt = blockIdx.y * 32, nt = blockIdx.x * 32;
-  const int wm = (wave >> 1) * 16, wn = (wave & 1) * 16;
-  const int r = lane & 15, kq = (lane >> 4) * 8;
-  v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int kc0 = 0; kc0 < g.K; kc0 += kKc) {
-    const int kn = min(kKc, g.K - kc0);
-    const int kpad = (kn + 31) & ~31;
-    stage(As, g.A, g.sam, g.sak, mt, g.M, kc0, kn, kpad);
-    stage(Bt, g.B, g.sbn, g.sbk, nt, g.N, kc0, kn, kpad);
-    __syncthreads();
-    for (int kk = 0; kk < kpad; kk += 32)
-      acc = mfma32(*reinterpret_cast<const uint4*>(&As[wm + r][kk + kq]),
-                   *reinterpret_cast<const uint4*>(&Bt[wn + r][kk + kq]), acc);
-    __syncthreads();
-  }
-  const int m0 = mt + wm, n0 = nt + wn;
-  if (m0 >= g.M || n0 >= g.N) return;  // wave-uniform
-  const int cn = n0 + (lane & 15);
-  if (cn >= g.N) return;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int cm = m0 + (lane >> 4) * 4 + j;
-    if (cm >= g.M) continue;
-    {
-      float* c = g.C + (long)cm * g.ldc + cn;
-      float v = g.accumulate ? *c + acc[j] : acc[j];
-      if (g.bias) {
-        v = v + g.bias[cn];
-        if (g.relu) v = fmaxf(v, 0.0f);
-      }
-      if (g.addend) v = v + g.addend[(long)cm * g.N + cn];
-      *c = v;
-      if (g.Cb) g.Cb[(long)cm * g.ldc + cn] = bf16_rne(v);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Fused inference (kf_prior_forward): one 256-thread block per (layer-4 pixel,
 // sample) carries the pixel's receptive field through the four convolutions in
 // LDS — a 15x15 window of layer 1, 7x7 of layer 2, 3x3 of layer 3, then the pixel
 // (window positions outside a layer's map hold zeros: that layer's padding) — and
-// computes every output with the MFMA sequence gemm_bf16 runs for it (k steps of
+// computes every output with the MFMA sequence training runs for it (k steps of
 // 32 from 0 on the same BF16 operands, the same epilogue), so every activation
 // equals the layer-by-layer forward's bit for bit.  Neighbouring blocks recompute
 // the overlap of their windows (~2.7x the 42 M MACs of one sample) in exchange for
 // one launch instead of eight, with nothing between the layers but LDS.  The last
 // block of a sample to finish (a device counter, cleared again by that block)
 // averages the 80 layer-4 pixels and runs FC1 and FC2 for the sample's row as
-// gemm_bf16 would.  Operands: A from LDS and B (weights, L2-resident) from global
+// head_sample does.  Operands: A from LDS and B (weights, L2-resident) from global
 // memory, one 16-byte vector per lane and MFMA step.
 constexpr int kFuseThreads = 256;
 constexpr int kWin1 = 15, kWin2 = 7, kWin3 = 3;  // window sides of layers 1-3 around one layer-4 pixel
 constexpr int kRows1 = kWin1 * kWin1;            // 225 layer-1 positions
 constexpr int kRows1Pad = 240;                   // 15 MFMA row tiles
-constexpr int kFc1Pad = 160;                     // FC1 K (134) rounded up to the MFMA step
 constexpr int kPatch = 2 * kWin1 + 1;            // 31: input window side
 
 struct FuseArgs {
@@ -187,10 +50,6 @@ struct FuseArgs {
   const float* params;   // FP32 biases
   long w[6], b[6];       // parameter offsets
   float* Y4;             // [B][80][128] layer-4 activations
-  float* X5;             // [B][134] pooled features and previous twist
-  uint16_t* X5b;
-  float* H;              // [B][256] FC1 output
-  uint16_t* Hb;
   float* out;            // [B][6]
   unsigned* count;       // [B] finished blocks of each sample (zero between calls)
 };
@@ -222,7 +81,7 @@ __device__ __forceinline__ uint4 afrag(const uint16_t* act, int p, int k) {
 
 // One convolution layer of the window (layers 2-4): output window side WOUT with
 // origin (y0, x0) in a map of HOUT x WOUT_MAP; wave w takes column tiles w, w + 4,
-// ... and every row tile.  Epilogue as gemm_bf16's (bias, ReLU); layers 2-3 store
+// ... and every row tile.  Epilogue: bias, ReLU; layers 2-3 store
 // the BF16 copy into the output window (zero outside the map), layer 4 (WOUT 1)
 // stores the FP32 value of its one position to y4.
 template <int CIN, int COUT, int WOUT, int HOUT, int WOUT_MAP>
@@ -364,10 +223,7 @@ __global__ __launch_bounds__(kFuseThreads) void prior_infer_fused(FuseArgs f) {
     } else {
       v = f.prev[n * kTwist + (tid - kFeat)];
     }
-    f.X5[n * kFc1In + tid] = v;
-    const uint16_t vb = bf16_rne(v);
-    f.X5b[n * kFc1In + tid] = vb;
-    xs[tid] = vb;
+    xs[tid] = bf16_rne(v);
   } else if (tid < kFc1Pad) {
     xs[tid] = 0;
   }
@@ -382,10 +238,7 @@ __global__ __launch_bounds__(kFuseThreads) void prior_infer_fused(FuseArgs f) {
                    acc);
     if (q == 0) {  // row 0: the sample's row
       const float v = fmaxf(acc[0] + f.params[f.b[4] + nn], 0.0f);
-      f.H[n * kHidden + nn] = v;
-      const uint16_t vb = bf16_rne(v);
-      f.Hb[n * kHidden + nn] = vb;
-      hs[nn] = vb;
+      hs[nn] = bf16_rne(v);
     }
   }
   __syncthreads();
@@ -405,108 +258,14 @@ __global__ __launch_bounds__(kFuseThreads) void prior_infer_fused(FuseArgs f) {
   }
 }
 
-__global__ void to_bf16(const float* x, uint16_t* y, long n) {
+__global__ void copy_weights(WeightCopyArgs a, const float* p) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) y[i] = bf16_rne(x[i]);
+  if (i < a.n) copy_weight(a, i, p[i]);
 }
 
-// feat[n][0..127] = mean over the 80 pooled pixels of Y4; [128..133] = prev twist.
-__global__ void pool_concat(const float* Y4, const float* prev, int batch, float* X5, uint16_t* X5b) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= batch * kFc1In) return;
-  const int n = i / kFc1In, c = i - n * kFc1In;
-  float v;
-  if (c < kFeat) {
-    float s = 0.0f;
-    for (int p = 0; p < kPool; ++p) s = s + Y4[((long)n * kPool + p) * kFeat + c];
-    v = s * (1.0f / (float)kPool);
-  } else {
-    v = prev[n * kTwist + (c - kFeat)];
-  }
-  X5[i] = v;
-  X5b[i] = bf16_rne(v);
-}
-
-// BF16 copies of the parameters: y in the blob's order, and the weights of layers 2-4
-// again as [tap][ci][co] (yt, at the blob's offsets) for the input gradients.
-struct WeightCopyArgs {
-  const float* x;
-  uint16_t *y, *yt;
-  long n, w[kConvs];  // parameter count, weight offsets of the convolutions
-};
-__global__ void copy_weights(WeightCopyArgs a) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
-  const uint16_t v = bf16_rne(a.x[i]);
-  a.y[i] = v;
-#pragma unroll
-  for (int l = 1; l < kConvs; ++l) {
-    const int e = (int)(i - a.w[l]);
-    if (e >= 0 && e < kConv[l].cout * kConv[l].kc) a.yt[a.w[l] + (e % kConv[l].kc) * kConv[l].cout + e / kConv[l].kc] = v;
-  }
-}
-
-// dY4[n][p][c] = dX5[n][c] / 80 where Y4 > 0, as BF16, and each sample's FP32 sums over
-// its pixels (bpart[n][c]).  One block per sample.
-__global__ __launch_bounds__(2 * kFeat) void pool_backward(const float* dX5, const float* Y4, uint16_t* dY4, float* bpart) {
-  __shared__ float red[kFeat];
-  const int n = blockIdx.x, c = threadIdx.x & (kFeat - 1), half = threadIdx.x / kFeat;
-  const float g = dX5[n * kFc1In + c] * (1.0f / (float)kPool);
-  float s = 0.0f;
-#pragma unroll 8
-  for (int p = half; p < kPool; p += 2) {
-    const long i = ((long)n * kPool + p) * kFeat + c;
-    const float v = Y4[i] > 0.0f ? g : 0.0f;
-    dY4[i] = bf16_rne(v);
-    s = s + v;
-  }
-  if (half == 1) red[c] = s;
-  __syncthreads();
-  if (half == 0) bpart[(long)n * kFeat + c] = s + red[c];
-}
-
-// Loss mean((O - T)^2) and dO = 2 (O - T) / (6 B); one block.
-__global__ void mse_loss(const float* O, const float* T, int batch, float* dO, float* loss) {
-  __shared__ float red[256];
-  const int n = batch * kTwist;
-  const float inv = 1.0f / (float)n;
-  float s = 0.0f;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    const float d = O[i] - T[i];
-    dO[i] = 2.0f * d * inv;
-    s = s + d * d;
-  }
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0 && loss) *loss = red[0] * inv;
-}
-
-// db[c] = sum_m dY[m][c]; one block per channel, fixed reduction order.
-__global__ void bias_grad(const float* dY, long M, int C, float* db) {
-  __shared__ float red[256];
-  const int c = blockIdx.x;
-  float s = 0.0f;
-  for (long m = threadIdx.x; m < M; m += blockDim.x) s = s + dY[m * C + c];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) db[c] = red[0];
-}
-
-__global__ void relu_mask(float* dY, const float* Y, long n) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && !(Y[i] > 0.0f)) dY[i] = 0.0f;
-}
-
-__global__ void adam(float* p, const float* g, float* m, float* v, long n, float lr, float b1, float b2, float eps,
-                     float c1, float c2) {
+// One Adam step; the new parameters' BF16 copies are made with it.
+__global__ void adam(WeightCopyArgs w, float* p, const float* g, float* m, float* v, long n, float lr, float b1,
+                     float b2, float eps, float c1, float c2) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const float gi = g[i];
@@ -514,7 +273,9 @@ __global__ void adam(float* p, const float* g, float* m, float* v, long n, float
   const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
   m[i] = mi;
   v[i] = vi;
-  p[i] = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  p[i] = pi;
+  copy_weight(w, i, pi);
 }
 
 inline unsigned blocks_for(long n, int t = 256) { return (unsigned)((n + t - 1) / t); }
@@ -527,7 +288,7 @@ struct kf_prior {
   long nparams = 0;
   float* params = nullptr;   // FP32 master
   uint16_t* wbf = nullptr;   // BF16 copy
-  uint16_t* wt = nullptr;    // layers 2-4 again as [tap][ci][co], at the same offsets
+  uint16_t* wt = nullptr;    // operand copies (WeightCopies)
   float* grad = nullptr;
   float* adam_m = nullptr;
   float* adam_v = nullptr;
@@ -535,16 +296,13 @@ struct kf_prior {
   // activations (NHWC), sized for max_batch
   uint16_t* Yb[kf::kConvs - 1] = {};  // layers 1-3, BF16 NHWC
   float* Y4 = nullptr;                // layer 4, FP32
-  float* X5 = nullptr;
   uint16_t* X5b = nullptr;
-  float* Hd = nullptr;
   uint16_t* Hb = nullptr;
   float* O = nullptr;
   float* dO = nullptr;
   uint16_t* dOb = nullptr;
   float* dH = nullptr;
   uint16_t* dHb = nullptr;
-  float* dX5 = nullptr;
   uint16_t* dYb[kf::kConvs] = {};       // gradients of the layers' outputs, BF16 NHWC
   float* bpart[kf::kConvs] = {};        // partial bias sums per block (layer 4: per sample)
   float* wpart[kf::kConvs] = {};        // partial weight gradients per split
@@ -555,49 +313,22 @@ struct kf_prior {
 namespace kf {
 namespace {
 
-struct Epilogue {
-  const float* bias = nullptr;
-  int relu = 0;
-  const float* addend = nullptr;
-  uint16_t* Cb = nullptr;
-};
-
-kf_status gemm(hipStream_t s, const uint16_t* A, long sam, long sak, const uint16_t* B, long sbk, long sbn, float* C,
-               long ldc, int M, int N, int K, bool accumulate,
-               const Epilogue& ep = Epilogue()) {
-  GemmArgs g;
-  g.bias = ep.bias;
-  g.relu = ep.relu;
-  g.addend = ep.addend;
-  g.Cb = ep.Cb;
-  g.A = A;
-  g.sam = sam;
-  g.sak = sak;
-  g.B = B;
-  g.sbk = sbk;
-  g.sbn = sbn;
-  g.C = C;
-  g.ldc = ldc;
-  g.M = M;
-  g.N = N;
-  g.K = K;
-  g.accumulate = accumulate ? 1 : 0;
-  dim3 grid((N + 31) / 32, (M + 31) / 32);
-  hipLaunchKernelGGL(gemm_bf16, grid, dim3(256), 0, s, g);
-  KF_TRY(check_launch("gemm_bf16"));
-  return KF_OK;
-}
-
 // BF16 copies of the weights; every call that changes the FP32 parameters refreshes
 // them, so inference (forward) never converts.
-kf_status sync_weights(kf_prior* P, hipStream_t s) {
+WeightCopyArgs copy_args(kf_prior* P) {
   WeightCopyArgs a;
-  a.x = P->params;
   a.y = P->wbf;
   a.yt = P->wt;
   a.n = P->nparams;
-  for (int l = 0; l < kConvs; ++l) a.w[l] = layout().w[l];
-  hipLaunchKernelGGL(copy_weights, dim3(blocks_for(P->nparams)), dim3(256), 0, s, a);
+  for (int q = 0; q < 6; ++q) a.w[q] = layout().w[q];
+  a.w5 = weight_copies().w5;
+  a.w5t = weight_copies().w5t;
+  a.w6t = weight_copies().w6t;
+  return a;
+}
+
+kf_status sync_weights(kf_prior* P, hipStream_t s) {
+  hipLaunchKernelGGL(copy_weights, dim3(blocks_for(P->nparams)), dim3(256), 0, s, copy_args(P), (const float*)P->params);
   return check_launch("copy_weights");
 }
 
@@ -616,10 +347,6 @@ kf_status infer(kf_prior* P, const float* frames, const int32_t* pairs, const fl
     f.b[q] = L.b[q];
   }
   f.Y4 = P->Y4;
-  f.X5 = P->X5;
-  f.X5b = P->X5b;
-  f.H = P->Hd;
-  f.Hb = P->Hb;
   f.out = out;
   f.count = P->fuse_count;
   hipLaunchKernelGGL(prior_infer_fused, dim3(kPool, B), dim3(kFuseThreads), 0, s, f);
@@ -642,33 +369,15 @@ kf_status launch_conv(kf_prior* P, const uint16_t* X, uint16_t* Yb, float* Y, in
   return check_launch("conv_forward");
 }
 
-// Training forward: the activations stay for the backward pass.
-kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, const float* prev, int B, hipStream_t s) {
+// Training forward of the convolutions: the activations stay for the backward pass.
+kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, int B, hipStream_t s) {
   const ParamLayout& L = layout();
   hipLaunchKernelGGL(conv1_forward, dim3(kConv[0].hout / kL1Rows, B), dim3(kConvThreads), 0, s, frames, pairs,
                      (const uint16_t*)P->wbf + L.w[0], (const float*)P->params + L.b[0], P->Yb[0]);
   KF_TRY(check_launch("conv1_forward"));
   KF_TRY((launch_conv<1, 4, false>(P, P->Yb[0], P->Yb[1], nullptr, B, s)));
   KF_TRY((launch_conv<2, 2, false>(P, P->Yb[1], P->Yb[2], nullptr, B, s)));
-  KF_TRY((launch_conv<3, 2, true>(P, P->Yb[2], nullptr, P->Y4, B, s)));
-  hipLaunchKernelGGL(pool_concat, dim3(blocks_for((long)B * kFc1In)), dim3(256), 0, s, (const float*)P->Y4, prev, B,
-                     P->X5, P->X5b);
-  KF_TRY(check_launch("pool_concat"));
-  {  // FC1: H = ReLU(X5 W5^T + b5), also as BF16 for FC2
-    Epilogue ep;
-    ep.bias = (const float*)P->params + L.b[4];
-    ep.relu = 1;
-    ep.Cb = P->Hb;
-    KF_TRY(gemm(s, P->X5b, kFc1In, 1, P->wbf + L.w[4], 1, kFc1In, P->Hd, kHidden, B, kHidden, kFc1In, false, ep));
-  }
-  {  // FC2 plus the skip connection: O = (H W6^T + b6) + previous twist
-    Epilogue ep;
-    ep.bias = (const float*)P->params + L.b[5];
-    ep.addend = prev;
-    KF_TRY(gemm(s, P->Hb, kHidden, 1, P->wbf + L.w[5], 1, kHidden, P->O, kTwist, B, kTwist, kHidden,
-                false, ep));
-  }
-  return KF_OK;
+  return launch_conv<3, 2, true>(P, P->Yb[2], nullptr, P->Y4, B, s);
 }
 
 // Input gradient of layer L (dYb[L] -> dYb[L - 1], partial sums of layer L - 1's bias
@@ -686,9 +395,10 @@ kf_status launch_dgrad(kf_prior* P, int B, int* planes, hipStream_t s) {
 
 // Weight gradient of layer L as *splits partial planes: one block a CU, at least
 // kWgradMinSteps steps of 32 pixels each (a shorter split would mostly write its plane).
+// The first such launch of the maps' second layer (L 1) carries the fully connected layers' weight gradients and the loss.
 constexpr int kWgradBlocks = 256, kWgradMinSteps = 4;
 template <int L>
-kf_status launch_wgrad(kf_prior* P, int B, int* splits, hipStream_t s) {
+kf_status launch_wgrad(kf_prior* P, int B, int* splits, hipStream_t s, const FcGradArgs& fc = FcGradArgs{}) {
   constexpr int GROUPS = WgradShape<L>::GROUPS;
   const int M = B * kConv[L].hout * kConv[L].wout, steps = div_up(M, kWgradStep);
   const int want = std::min(std::max(steps / kWgradMinSteps, 1), kWgradBlocks / GROUPS);
@@ -697,63 +407,83 @@ kf_status launch_wgrad(kf_prior* P, int B, int* splits, hipStream_t s) {
   // eight splits a round (blocks of one split on one XCD): the grid is rounded up, and
   // the splits past the last write zero planes that nothing reads
   const int grid = div_up(*splits, 8) * 8 * GROUPS;
-  hipLaunchKernelGGL(conv_wgrad<L>, dim3(grid), dim3(kConvThreads), 0, s, (const uint16_t*)P->dYb[L],
-                     (const uint16_t*)P->Yb[L - 1], P->wpart[L], M, per);
+  hipLaunchKernelGGL(conv_wgrad<L>, dim3(grid + (L == 1 ? kFcBlocks : 0)), dim3(kConvThreads), 0, s, (const uint16_t*)P->dYb[L],
+                     (const uint16_t*)P->Yb[L - 1], P->wpart[L], M, per, fc, grid);
   return check_launch("conv_wgrad");
 }
 
-kf_status backward(kf_prior* P, const float* frames, const int32_t* pairs, const float* target, int B, float* loss, hipStream_t s) {
+// The fully connected layers both ways, then the convolutions' backward; the gradient
+// of every parameter goes to G.
+kf_status backward(kf_prior* P, const float* frames, const int32_t* pairs, const float* prev, const float* target, int B,
+                   float* G, float* loss, hipStream_t s) {
   const ParamLayout& L = layout();
-  float* G = P->grad;
-  hipLaunchKernelGGL(mse_loss, dim3(1), dim3(256), 0, s, (const float*)P->O, target, B, P->dO, loss);
-  hipLaunchKernelGGL(to_bf16, dim3(blocks_for((long)B * kTwist)), dim3(256), 0, s, (const float*)P->dO, P->dOb,
-                     (long)B * kTwist);
-  KF_TRY(check_launch("mse_loss"));
-  // FC2: dW6[j][k] = sum_n dO[n][j] H[n][k]; db6; dH = dO W6, masked by H > 0.
-  KF_TRY(gemm(s, P->dOb, 1, kTwist, P->Hb, kHidden, 1, G + L.w[5], kHidden, kTwist, kHidden, B, false));
-  hipLaunchKernelGGL(bias_grad, dim3(kTwist), dim3(256), 0, s, (const float*)P->dO, (long)B, kTwist, G + L.b[5]);
-  KF_TRY(gemm(s, P->dOb, kTwist, 1, P->wbf + L.w[5], kHidden, 1, P->dH, kHidden, B, kHidden, kTwist, false));
-  hipLaunchKernelGGL(relu_mask, dim3(blocks_for((long)B * kHidden)), dim3(256), 0, s, P->dH, (const float*)P->Hd,
-                     (long)B * kHidden);
-  hipLaunchKernelGGL(to_bf16, dim3(blocks_for((long)B * kHidden)), dim3(256), 0, s, (const float*)P->dH, P->dHb,
-                     (long)B * kHidden);
-  // FC1: dW5[j][k] = sum_n dH[n][j] X5[n][k]; db5; dX5 (features only) = dH W5.
-  KF_TRY(gemm(s, P->dHb, 1, kHidden, P->X5b, kFc1In, 1, G + L.w[4], kFc1In, kHidden, kFc1In, B, false));
-  hipLaunchKernelGGL(bias_grad, dim3(kHidden), dim3(256), 0, s, (const float*)P->dH, (long)B, kHidden, G + L.b[4]);
-  KF_TRY(gemm(s, P->dHb, kHidden, 1, P->wbf + L.w[4], kFc1In, 1, P->dX5, kFc1In, B, kFeat, kHidden, false));
-  hipLaunchKernelGGL(pool_backward, dim3(B), dim3(2 * kFeat), 0, s, (const float*)P->dX5, (const float*)P->Y4,
-                     P->dYb[3], P->bpart[3]);
-  KF_TRY(check_launch("pool_backward"));
+  const WeightCopies& W = weight_copies();
+  HeadArgs h;
+  h.Y4 = P->Y4;
+  h.prev = prev;
+  h.target = target;
+  h.b5 = P->params + L.b[4];
+  h.b6 = P->params + L.b[5];
+  h.w5 = P->wt + W.w5;
+  h.w6 = P->wbf + L.w[5];
+  h.w5t = P->wt + W.w5t;
+  h.w6t = P->wt + W.w6t;
+  h.O = P->O;
+  h.dO = P->dO;
+  h.dH = P->dH;
+  h.X5b = P->X5b;
+  h.Hb = P->Hb;
+  h.dOb = P->dOb;
+  h.dHb = P->dHb;
+  h.dY4 = P->dYb[3];
+  h.bpart = P->bpart[3];
+  h.inv = 1.0f / (float)(B * kTwist);
+  hipLaunchKernelGGL(head_sample, dim3(B), dim3(kConvThreads), 0, s, h);
+  KF_TRY(check_launch("head_sample"));
   int planes[kConvs] = {0, 0, 0, B}, splits[kConvs];
   KF_TRY(launch_wgrad<3>(P, B, &splits[3], s));
   KF_TRY((launch_dgrad<3, 1>(P, B, &planes[2], s)));
   KF_TRY(launch_wgrad<2>(P, B, &splits[2], s));
   KF_TRY((launch_dgrad<2, 2>(P, B, &planes[1], s)));
-  KF_TRY(launch_wgrad<1>(P, B, &splits[1], s));
+  FcGradArgs fc;
+  fc.X5b = P->X5b;
+  fc.Hb = P->Hb;
+  fc.dOb = P->dOb;
+  fc.dHb = P->dHb;
+  fc.O = P->O;
+  fc.target = target;
+  fc.dW5 = G + L.w[4];
+  fc.dW6 = G + L.w[5];
+  fc.loss = loss;
+  fc.batch = B;
+  KF_TRY(launch_wgrad<1>(P, B, &splits[1], s, fc));
   KF_TRY((launch_dgrad<1, 2>(P, B, &planes[0], s)));
   const int items = B * (kConv[0].hout / kL1Rows);
   splits[0] = std::min(items, kConvBlocks);
   hipLaunchKernelGGL(conv1_wgrad, dim3(splits[0]), dim3(kConvThreads), 0, s, frames, pairs, (const uint16_t*)P->dYb[0],
                      P->wpart[0], items);
   KF_TRY(check_launch("conv1_wgrad"));
-  ReduceArgs red;
-  red.jobs = 0;
-  red.block0[0] = 0;
-  auto add = [&](const float* part, int n, int count, float* out) {
-    const int k = red.jobs++;
-    red.part[k] = part;
-    red.planes[k] = n;
-    red.count[k] = count;
-    red.out[k] = out;
-    red.block0[k + 1] = red.block0[k] + div_up(count, 64);
+  ReduceArgs f;
+  f.jobs = 0;
+  f.block0[0] = 0;
+  auto add = [&](const float* part, int n, int pitch, int count, float* out) {
+    const int k = f.jobs++;
+    f.part[k] = part;
+    f.planes[k] = n;
+    f.pitch[k] = pitch;
+    f.count[k] = count;
+    f.out[k] = out;
+    f.block0[k + 1] = f.block0[k] + div_up(count, kReduceOut);
   };
-  for (int l = kConvs - 1; l >= 0; --l) {
-    add(P->wpart[l], splits[l], kConv[l].cout * kConv[l].kc, G + L.w[l]);
-    add(P->bpart[l], planes[l], kConv[l].cout, G + L.b[l]);
+  for (int l = 0; l < kConvs; ++l) {
+    const int nw = kConv[l].cout * kConv[l].kc;
+    add(P->wpart[l], splits[l], nw, nw, G + L.w[l]);
+    add(P->bpart[l], planes[l], kConv[l].cout, kConv[l].cout, G + L.b[l]);
   }
-  hipLaunchKernelGGL(reduce_parts, dim3(red.block0[red.jobs]), dim3(1024), 0, s, red);
-  KF_TRY(check_launch("reduce_parts"));
-  return KF_OK;
+  add(P->dH, B, kHidden, kHidden, G + L.b[4]);
+  add(P->dO, B, kDoSumPitch, kTwist, G + L.b[5]);
+  hipLaunchKernelGGL(reduce_parts, dim3(f.block0[f.jobs]), dim3(kReduceThreads), 0, s, f);
+  return check_launch("reduce_parts");
 }
 
 kf_status check_batch(const kf_prior* P, const float* frames, const int32_t* pairs, const float* prev, int B) {
@@ -771,8 +501,8 @@ extern "C" int64_t kf_prior_param_count(void) { return layout().total; }
 
 extern "C" kf_status kf_prior_destroy(kf_prior* P) {
   if (!P) return KF_OK;
-  void* ptrs[] = {P->params, P->wbf, P->grad, P->adam_m, P->adam_v, P->Y4, P->X5, P->X5b, P->Hd, P->Hb, P->O, P->dO,
-                  P->dOb, P->dH, P->dHb, P->dX5, P->wt, P->loss_tmp,
+  void* ptrs[] = {P->params, P->wbf, P->grad, P->adam_m, P->adam_v, P->Y4, P->X5b, P->Hb, P->O, P->dO,
+                  P->dOb, P->dH, P->dHb, P->wt, P->loss_tmp,
                   P->fuse_count};
   for (void* q : ptrs) (void)hipFree(q);
   for (int l = 0; l < kConvs; ++l) {
@@ -798,7 +528,7 @@ extern "C" kf_status kf_prior_create(int32_t max_batch, kf_prior** out) {
   };
   al((void**)&P->params, P->nparams * 4);
   al((void**)&P->wbf, P->nparams * 2);
-  al((void**)&P->wt, P->nparams * 2);
+  al((void**)&P->wt, weight_copies().total * 2);
   al((void**)&P->grad, P->nparams * 4);
   al((void**)&P->adam_m, P->nparams * 4);
   al((void**)&P->adam_v, P->nparams * 4);
@@ -811,19 +541,17 @@ extern "C" kf_status kf_prior_create(int32_t max_batch, kf_prior** out) {
     al((void**)&P->dYb[l], M * c.cout * 2);
     al((void**)&P->bpart[l], (l + 1 < kConvs ? kConvBlocks : B) * c.cout * 4);
   }
-  al((void**)&P->X5, B * kFc1In * 4);
-  al((void**)&P->X5b, B * kFc1In * 2);
-  al((void**)&P->Hd, B * kHidden * 4);
+  al((void**)&P->X5b, B * kX5Pitch * 2);
   al((void**)&P->Hb, B * kHidden * 2);
   al((void**)&P->O, B * kTwist * 4);
-  al((void**)&P->dO, B * kTwist * 4);
-  al((void**)&P->dOb, B * kTwist * 2);
+  al((void**)&P->dO, B * kDoSumPitch * 4);
+  al((void**)&P->dOb, B * kDoPitch * 2);
   al((void**)&P->dH, B * kHidden * 4);
   al((void**)&P->dHb, B * kHidden * 2);
-  al((void**)&P->dX5, B * kFc1In * 4);
   al((void**)&P->loss_tmp, 16);
   al((void**)&P->fuse_count, B * sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(P->fuse_count, 0, B * sizeof(unsigned));
+  if (e == hipSuccess) e = hipMemset(P->wt, 0, weight_copies().total * 2);  // the copies' padding
   if (e == hipSuccess) e = hipMemset(P->adam_m, 0, P->nparams * 4);
   if (e == hipSuccess) e = hipMemset(P->adam_v, 0, P->nparams * 4);
   if (e == hipSuccess) e = hipMemset(P->params, 0, P->nparams * 4);
@@ -888,23 +616,20 @@ extern "C" kf_status kf_prior_gradients(kf_prior* P, const float* frames, const 
                                         const float* target, int32_t B, float* d_grad, float* d_loss, kf_stream s) {
   KF_TRY(check_batch(P, frames, pairs, prev, B));
   KF_CHECK_ARG(target && d_grad, "NULL argument");
-  KF_TRY(forward(P, frames, pairs, prev, B, S(s)));
-  KF_TRY(backward(P, frames, pairs, target, B, d_loss, S(s)));
-  KF_HIP(hipMemcpyAsync(d_grad, P->grad, (size_t)P->nparams * 4, hipMemcpyDeviceToDevice, S(s)));
-  return KF_OK;
+  KF_TRY(forward(P, frames, pairs, B, S(s)));
+  return backward(P, frames, pairs, prev, target, B, d_grad, d_loss, S(s));
 }
 
 extern "C" kf_status kf_prior_train_step(kf_prior* P, const float* frames, const int32_t* pairs, const float* prev,
                                          const float* target, int32_t B, float lr, float* d_loss, kf_stream s) {
   KF_TRY(check_batch(P, frames, pairs, prev, B));
   KF_CHECK_ARG(target != nullptr, "target is NULL");
-  KF_TRY(forward(P, frames, pairs, prev, B, S(s)));
-  KF_TRY(backward(P, frames, pairs, target, B, d_loss, S(s)));
+  KF_TRY(forward(P, frames, pairs, B, S(s)));
+  KF_TRY(backward(P, frames, pairs, prev, target, B, P->grad, d_loss, S(s)));
   P->step += 1;
   const float b1 = 0.9f, b2 = 0.999f;
   const float c1 = 1.0f - (float)pow(0.9, (double)P->step), c2 = 1.0f - (float)pow(0.999, (double)P->step);
-  hipLaunchKernelGGL(adam, dim3(blocks_for(P->nparams)), dim3(256), 0, S(s), P->params, (const float*)P->grad,
-                     P->adam_m, P->adam_v, P->nparams, lr, b1, b2, 1e-8f, c1, c2);
-  KF_TRY(check_launch("adam"));
-  return sync_weights(P, S(s));
+  hipLaunchKernelGGL(adam, dim3(blocks_for(P->nparams)), dim3(256), 0, S(s), copy_args(P), P->params,
+                     (const float*)P->grad, P->adam_m, P->adam_v, P->nparams, lr, b1, b2, 1e-8f, c1, c2);
+  return check_launch("adam");
 }

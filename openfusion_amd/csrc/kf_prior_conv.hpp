@@ -6,8 +6,8 @@
 // NHWC BF16 map (through L1 / L2, no im2col matrix).  With the weights as A, a lane
 // holds output channels of one pixel; their order over the tiles is chosen so that
 // a lane's channels are contiguous and it stores them as whole vectors.  Each output
-// is one MFMA chain over k = 0, 32, ... from zero, the sequence of gemm_bf16 and
-// prior_infer_fused, so the three give the same bits.
+// is one MFMA chain over k = 0, 32, ... from zero, the sequence of prior_infer_fused, so
+// the two give the same bits.
 #pragma once
 
 #include "kf_prior_net.hpp"
@@ -305,15 +305,115 @@ __device__ __forceinline__ uint4 transposed_fragment(const uint16_t* rows, int p
   return make_uint4(a.x, a.y, b.x, b.y);
 }
 
+constexpr int kWgradStep = 32;  // pixels (or samples) staged at a time
+
+// Weight gradients of the fully connected layers, dW5[j][c] = sum_n dH[n][j] X5[n][c] and
+// dW6[t][k] = sum_n dO[n][t] H[n][k], and the loss mean((O - T)^2): five blocks of their
+// own beside layer 2's weight gradient, which they finish long before (a launch of their
+// own would cost its 4 us, blocks in the final sums 13 us at batch 256).
+constexpr int kX5Pitch = 144;  // row of pooled features and twist, rounded up to MFMA tiles
+constexpr int kDoPitch = 16;   // row of output gradients, rounded up to an MFMA tile
+constexpr int kFcBlocks = 5;   // four of 64 rows of dW5, one of dW6 and the loss
+struct FcGradArgs {
+  const uint16_t *X5b, *Hb, *dOb, *dHb;
+  const float *O, *target;
+  float *dW5, *dW6, *loss;
+  int batch;
+};
+
+// Columns i0 .. of A (WA of them, rows of PA elements) against B's rows of PB: wave w
+// makes row tile w / WPT and column tiles (w % WPT) NT .. of C[i][k] = sum_n A[n][i]
+// B[n][k], 32 samples a step, the next step's vectors in flight.
+template <int PA, int WA, int PB, int NT, int WPT>
+__device__ __forceinline__ void fc_weight_gradient(const uint16_t* A, int i0, const uint16_t* B, int batch, int rows,
+                                                   int cols, float* out, uint16_t* s) {
+  constexpr int pa = WA + 16 + (WA / 16 % 2) * 16, pb = PB + 16 + (PB / 16 % 2) * 16;
+  static_assert(pa / 16 % 2 == 1 && pb / 16 % 2 == 1, "bank-spreading pitches");
+  constexpr int VA = kWgradStep * WA / 8, VB = kWgradStep * PB / 8, PER = (VA + VB + kConvThreads - 1) / kConvThreads;
+  uint16_t* sa = s;
+  uint16_t* sb = s + kWgradStep * pa;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
+  const int it = wave / WPT * 16, k0 = wave % WPT * NT * 16;
+  v4f acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  uint4 v[PER];
+  auto place = [&](int u, bool& isa, int& row, int& col) {  // where vector u of this thread lies; false: it has none
+    const int e = threadIdx.x + kConvThreads * u;
+    isa = e < VA;
+    const int f = isa ? e : e - VA, per = isa ? WA / 8 : PB / 8;
+    row = f / per;
+    col = 8 * (f - row * per);
+    return e < VA + VB;
+  };
+  auto load = [&](int n0) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      bool isa;
+      int row, col;
+      v[u] = make_uint4(0u, 0u, 0u, 0u);
+      if (place(u, isa, row, col) && n0 + row < batch)
+        v[u] = *reinterpret_cast<const uint4*>(isa ? A + (long)(n0 + row) * PA + i0 + col : B + (long)(n0 + row) * PB + col);
+    }
+  };
+  load(0);
+  for (int n0 = 0; n0 < batch; n0 += kWgradStep) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      bool isa;
+      int row, col;
+      if (place(u, isa, row, col)) *reinterpret_cast<uint4*>((isa ? sa : sb) + row * (isa ? pa : pb) + col) = v[u];
+    }
+    if (n0 + kWgradStep < batch) load(n0 + kWgradStep);
+    __syncthreads();
+    const uint4 a = transposed_fragment(sa, pa, it, r, q);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = mfma32(a, transposed_fragment(sb, pb, k0 + 16 * t, r, q), acc[t]);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i = i0 + it + 4 * q + j, k = k0 + 16 * t + r;
+      if (i < rows && k < cols) out[i * cols + k] = acc[t][j];
+    }
+}
+
+// Block b < kFcBlocks of the above; s: kFcLds elements of LDS (dW6's tiles, the larger).
+constexpr int kFcLds = kWgradStep * (kDoPitch + 32 + kHidden + 16);
+static_assert(kFcLds >= kWgradStep * (64 + 16 + kX5Pitch + 32), "dW5's tiles");
+__device__ __forceinline__ void fc_block(const FcGradArgs& a, int b, uint16_t* s) {
+  if (b + 1 < kFcBlocks) {
+    fc_weight_gradient<kHidden, 64, kX5Pitch, kX5Pitch / 16, 1>(a.dHb, 64 * b, a.X5b, a.batch, kHidden, kFc1In, a.dW5, s);
+    return;
+  }
+  fc_weight_gradient<kDoPitch, kDoPitch, kHidden, kHidden / 16 / kConvWaves, kConvWaves>(a.dOb, 0, a.Hb, a.batch, kTwist,
+                                                                                         kHidden, a.dW6, s);
+  float* red = reinterpret_cast<float*>(s);
+  const int n = a.batch * kTwist, tid = threadIdx.x;
+  float v = 0.0f;
+  for (int i = tid; i < n; i += kConvThreads) {
+    const float d = a.O[i] - a.target[i];
+    v = v + d * d;
+  }
+  red[tid] = v;
+  __syncthreads();
+  for (int o = kConvThreads / 2; o > 0; o >>= 1) {
+    if (tid < o) red[tid] += red[tid + o];
+    __syncthreads();
+  }
+  if (tid == 0 && a.loss) *a.loss = red[0] * (1.0f / (float)n);
+}
+
 // Weight gradient of layer L (1..3): dW[co][k] = sum_m dY[m][co] col[m][k], col the
 // im2col element read straight from the map X.  A block takes one split of the pixels
 // and COB output channels; a wave 2 x 9 tiles of them, so that eleven fragment reads
 // feed eighteen MFMAs.  Per step of 32 pixels the next step's vectors are in flight
 // while this one's tiles are multiplied.  Each split writes its own plane
-// (reduce_parts adds them in order, 16 us for all).  Bound by the L1 path of the map
+// (reduce_parts adds them in order).  Bound by the L1 path of the map
 // loads and the LDS reads.  Batch 256: layers 2 / 3 / 4 in 45 / 24 / 15 us (250 / 240 /
 // 198 TFLOP/s); the im2col matrices and the GEMMs over them took 2.3 ms with layer 1.
-constexpr int kWgradStep = 32;
 template <int L>
 struct WgradShape {
   static constexpr int COB = L == 1 ? 64 : 32;             // output channels of a block
@@ -324,13 +424,20 @@ struct WgradShape {
 
 template <int L>
 __global__ __launch_bounds__(kConvThreads, 2) void conv_wgrad(const uint16_t* dY, const uint16_t* X, float* part, int M,
-                                                              int steps_per_split) {
+                                                              int steps_per_split, FcGradArgs fc, int fc_block0) {
   constexpr ConvShape c = kConv[L];
   constexpr int COB = WgradShape<L>::COB, GROUPS = WgradShape<L>::GROUPS, NW = WgradShape<L>::NW;
   constexpr int kColPitch = c.kc + 16, kDyPitch = COB + 16;
   constexpr int kTapVecs = c.cin / 8, kVecs = c.kc / 8, kPer = (kVecs + 7) / 8;  // eight threads per pixel
-  __shared__ __align__(16) uint16_t s_col[kWgradStep * kColPitch];
+  constexpr int kColElems = L == 1 && kFcLds > kWgradStep * kColPitch ? kFcLds : kWgradStep * kColPitch;
+  __shared__ __align__(16) uint16_t s_col[kColElems];
   __shared__ __align__(16) uint16_t s_dy[kWgradStep * kDyPitch];
+  if constexpr (L == 1) {
+    if ((int)blockIdx.x >= fc_block0) {  // uniform
+      fc_block(fc, (int)blockIdx.x - fc_block0, s_col);
+      return;
+    }
+  }
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4;
   // the groups of a split read the same map: keep them on one XCD (blocks go round-robin)
   const int b = blockIdx.x, split = b / (8 * GROUPS) * 8 + b % 8, group = b / 8 % GROUPS;
@@ -437,40 +544,6 @@ __global__ __launch_bounds__(kConvThreads) void conv1_wgrad(const float* frames,
   if (nw + r < c.kc) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) part[((long)blockIdx.x * c.cout + cw + 4 * q + j) * c.kc + nw + r] = acc[j];
-  }
-}
-
-// Sums of partial planes, several at once: out[i] = sum over p < planes of
-// part[p * count + i].  A block takes 64 outputs; its sixteen waves each add every
-// sixteenth plane (eight loads in flight), and the sixteen sums are added in order.
-constexpr int kReduceJobs = 8;
-struct ReduceArgs {
-  const float* part[kReduceJobs];
-  float* out[kReduceJobs];
-  int planes[kReduceJobs], count[kReduceJobs], block0[kReduceJobs + 1];
-  int jobs;
-};
-
-__global__ __launch_bounds__(1024) void reduce_parts(ReduceArgs a) {
-  __shared__ float s_v[16][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int k = 0;
-  while (k + 1 < a.jobs && (int)blockIdx.x >= a.block0[k + 1]) ++k;
-  const int i = ((int)blockIdx.x - a.block0[k]) * 64 + lane, count = a.count[k], planes = a.planes[k];
-  const float* src = a.part[k] + min(i, count - 1);
-  float sum = 0.0f;
-  for (int p = wave; p < planes; p += 128) {
-    float v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = p + 16 * u < planes ? src[(long)(p + 16 * u) * count] : 0.0f;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) sum = sum + v[u];
-  }
-  s_v[wave][lane] = sum;
-  __syncthreads();
-  if (wave == 0 && i < count) {
-    for (int u = 1; u < 16; ++u) sum = sum + s_v[u][lane];
-    a.out[k][i] = sum;
   }
 }
 
