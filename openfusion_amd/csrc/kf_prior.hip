@@ -380,36 +380,35 @@ kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, int B,
   return launch_conv<3, 2, true>(P, P->Yb[2], nullptr, P->Y4, B, s);
 }
 
-// Input gradient of layer L (dYb[L] -> dYb[L - 1], partial sums of layer L - 1's bias
-// gradient; *planes: how many), on the grid of launch_conv.
-template <int L, int NT>
-kf_status launch_dgrad(kf_prior* P, int B, int* planes, hipStream_t s) {
-  constexpr ConvShape c = kConv[L];
-  const int M = B * c.hout * c.wout;
-  *planes = std::min(div_up(div_up(M, 16) * (c.cin / (16 * NT)), kConvWaves), kConvBlocks);
-  hipLaunchKernelGGL((conv_dgrad<L, NT>), dim3(*planes), dim3(kConvThreads), 0, s, (const uint16_t*)P->dYb[L],
-                     (const uint16_t*)P->wt + layout().w[L], (const uint16_t*)P->Yb[L - 1], P->dYb[L - 1],
-                     P->bpart[L - 1], M);
-  return check_launch("conv_dgrad");
-}
-
-// Weight gradient of layer L as *splits partial planes: one block a CU, at least
-// kWgradMinSteps steps of 32 pixels each (a shorter split would mostly write its plane).
-// The first such launch of the maps' second layer (L 1) carries the fully connected layers' weight gradients and the loss.
-constexpr int kWgradBlocks = 256, kWgradMinSteps = 4;
+// Backward pass of layer L: the weight gradient as *splits partial planes, one block a CU
+// and at least kWgradMinSteps steps of 32 pixels each (a shorter split would mostly
+// write its plane), and dYb[L] -> dYb[L - 1] with *planes partial sums of layer L - 1's
+// bias gradient, one block a CU beside the first: two blocks fit a CU, so all are
+// resident at once (512 blocks of input gradient ran a second round: 179 us against 159
+// for the three layers at batch 256).  fc (L = 1): carried along.
+constexpr int kWgradBlocks = 256, kWgradMinSteps = 4, kDgradBlocks = 256;
 template <int L>
-kf_status launch_wgrad(kf_prior* P, int B, int* splits, hipStream_t s, const FcGradArgs& fc = FcGradArgs{}) {
+kf_status launch_backward(kf_prior* P, int B, int* splits, int* planes, hipStream_t s, const FcGradArgs& fc = FcGradArgs{}) {
   constexpr int GROUPS = WgradShape<L>::GROUPS;
   const int M = B * kConv[L].hout * kConv[L].wout, steps = div_up(M, kWgradStep);
   const int want = std::min(std::max(steps / kWgradMinSteps, 1), kWgradBlocks / GROUPS);
-  const int per = div_up(steps, want);
-  *splits = div_up(steps, per);
-  // eight splits a round (blocks of one split on one XCD): the grid is rounded up, and
+  ConvBackArgs a;
+  a.dY = P->dYb[L];
+  a.X = P->Yb[L - 1];
+  a.Wt = P->wt + layout().w[L];
+  a.dX = P->dYb[L - 1];
+  a.wpart = P->wpart[L];
+  a.bpart = P->bpart[L - 1];
+  a.M = M;
+  a.steps_per_split = div_up(steps, want);
+  *splits = div_up(steps, a.steps_per_split);
+  // eight splits a round (blocks of one split on one XCD): the count is rounded up, and
   // the splits past the last write zero planes that nothing reads
-  const int grid = div_up(*splits, 8) * 8 * GROUPS;
-  hipLaunchKernelGGL(conv_wgrad<L>, dim3(grid + (L == 1 ? kFcBlocks : 0)), dim3(kConvThreads), 0, s, (const uint16_t*)P->dYb[L],
-                     (const uint16_t*)P->Yb[L - 1], P->wpart[L], M, per, fc, grid);
-  return check_launch("conv_wgrad");
+  a.wblocks = div_up(*splits, 8) * 8 * GROUPS;
+  a.dblocks = *planes = std::min(div_up(div_up(M, 16) * DgradShape<L>::GROUPS, kConvWaves), kDgradBlocks);
+  a.fc = fc;
+  hipLaunchKernelGGL(conv_backward<L>, dim3(a.wblocks + a.dblocks + (L == 1 ? kFcBlocks : 0)), dim3(kConvThreads), 0, s, a);
+  return check_launch("conv_backward");
 }
 
 // The fully connected layers both ways, then the convolutions' backward; the gradient
@@ -441,10 +440,8 @@ kf_status backward(kf_prior* P, const float* frames, const int32_t* pairs, const
   hipLaunchKernelGGL(head_sample, dim3(B), dim3(kConvThreads), 0, s, h);
   KF_TRY(check_launch("head_sample"));
   int planes[kConvs] = {0, 0, 0, B}, splits[kConvs];
-  KF_TRY(launch_wgrad<3>(P, B, &splits[3], s));
-  KF_TRY((launch_dgrad<3, 1>(P, B, &planes[2], s)));
-  KF_TRY(launch_wgrad<2>(P, B, &splits[2], s));
-  KF_TRY((launch_dgrad<2, 2>(P, B, &planes[1], s)));
+  KF_TRY(launch_backward<3>(P, B, &splits[3], &planes[2], s));
+  KF_TRY(launch_backward<2>(P, B, &splits[2], &planes[1], s));
   FcGradArgs fc;
   fc.X5b = P->X5b;
   fc.Hb = P->Hb;
@@ -456,8 +453,7 @@ kf_status backward(kf_prior* P, const float* frames, const int32_t* pairs, const
   fc.dW6 = G + L.w[5];
   fc.loss = loss;
   fc.batch = B;
-  KF_TRY(launch_wgrad<1>(P, B, &splits[1], s, fc));
-  KF_TRY((launch_dgrad<1, 2>(P, B, &planes[0], s)));
+  KF_TRY(launch_backward<1>(P, B, &splits[1], &planes[0], s, fc));
   const int items = B * (kConv[0].hout / kL1Rows);
   splits[0] = std::min(items, kConvBlocks);
   hipLaunchKernelGGL(conv1_wgrad, dim3(splits[0]), dim3(kConvThreads), 0, s, frames, pairs, (const uint16_t*)P->dYb[0],
@@ -539,7 +535,7 @@ extern "C" kf_status kf_prior_create(int32_t max_batch, kf_prior** out) {
     else al((void**)&P->Y4, M * c.cout * 4);
     al((void**)&P->wpart[l], (l == 0 ? kConvBlocks : kWgradBlocks / (c.cout / (l == 1 ? 64 : 32))) * c.cout * c.kc * 4);
     al((void**)&P->dYb[l], M * c.cout * 2);
-    al((void**)&P->bpart[l], (l + 1 < kConvs ? kConvBlocks : B) * c.cout * 4);
+    al((void**)&P->bpart[l], (l + 1 < kConvs ? kDgradBlocks : B) * c.cout * 4);
   }
   al((void**)&P->X5b, B * kX5Pitch * 2);
   al((void**)&P->Hb, B * kHidden * 2);

@@ -195,16 +195,24 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* 
 // matrix (354 MB for layer 2 at batch 256).  bpart: per block and channel the FP32 sum
 // of the unrounded gradients.  Batch 256: layers 2 / 3 / 4 in 50 / 34 / 27 us (layer 2:
 // 197 MB through memory); the GEMM, col2im, conversion and column sums took 4.3 ms.
-template <int L, int NT>
-__global__ __launch_bounds__(kConvThreads, 2) void conv_dgrad(const uint16_t* dY, const uint16_t* Wt, const uint16_t* Xb,
-                                                              uint16_t* dX, float* bpart, int M) {
+// Block `block` of `blocks`; s_b: kDgradLds floats of LDS.
+template <int L>
+struct DgradShape {
+  static constexpr int NT = L == 3 ? 1 : 2;                // 16-channel tiles of a wave
+  static constexpr int GROUPS = kConv[L].cin / (16 * NT);  // waves that cover a pixel's channels
+};
+constexpr int kDgradLds = kConvWaves * 32;
+
+template <int L>
+__device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* Wt, const uint16_t* Xb, uint16_t* dX,
+                                            float* bpart, int M, int block, int blocks, float* s_sum) {
   constexpr ConvShape c = kConv[L];
-  constexpr int KS = c.cout / 32, GROUPS = c.cin / (16 * NT), CH = 4 * NT;
+  constexpr int NT = DgradShape<L>::NT, KS = c.cout / 32, GROUPS = DgradShape<L>::GROUPS, CH = 4 * NT;
   static_assert(c.win == 2 * c.wout && (c.hin == 2 * c.hout || c.hin == 2 * c.hout - 1) && kConvWaves % GROUPS == 0,
                 "layer shape");
-  __shared__ float s_b[kConvWaves][16 * NT];
+  float (*s_b)[16 * NT] = reinterpret_cast<float (*)[16 * NT]>(s_sum);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
-  const int gw = blockIdx.x * kConvWaves + wave, group = gw % GROUPS;
+  const int gw = block * kConvWaves + wave, group = gw % GROUPS;
   const int ch0 = group * 16 * NT;
   uint4 w[9][KS][NT];
 #pragma unroll
@@ -217,7 +225,7 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_dgrad(const uint16_t* dY
   float bs[CH];
 #pragma unroll
   for (int j = 0; j < CH; ++j) bs[j] = 0.0f;
-  const int stride = gridDim.x * kConvWaves / GROUPS;
+  const int stride = blocks * kConvWaves / GROUPS;
   for (int tile = gw / GROUPS; tile * 16 < M; tile += stride) {
     const bool live = tile * 16 + r < M;
     const int m = live ? tile * 16 + r : M - 1;
@@ -282,7 +290,7 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_dgrad(const uint16_t* dY
     const int g = threadIdx.x / (16 * NT), k = threadIdx.x - g * 16 * NT;
     float v = s_b[g][k];
     for (int u = g + GROUPS; u < kConvWaves; u += GROUPS) v = v + s_b[u][k];
-    bpart[(long)blockIdx.x * c.cin + threadIdx.x] = v;
+    bpart[(long)block * c.cin + threadIdx.x] = v;
   }
 }
 
@@ -309,7 +317,7 @@ constexpr int kWgradStep = 32;  // pixels (or samples) staged at a time
 
 // Weight gradients of the fully connected layers, dW5[j][c] = sum_n dH[n][j] X5[n][c] and
 // dW6[t][k] = sum_n dO[n][t] H[n][k], and the loss mean((O - T)^2): five blocks of their
-// own beside layer 2's weight gradient, which they finish long before (a launch of their
+// own beside layer 2's backward pass, which they finish long before (a launch of their
 // own would cost its 4 us, blocks in the final sums 13 us at batch 256).
 constexpr int kX5Pitch = 144;  // row of pooled features and twist, rounded up to MFMA tiles
 constexpr int kDoPitch = 16;   // row of output gradients, rounded up to an MFMA tile
@@ -419,28 +427,22 @@ struct WgradShape {
   static constexpr int COB = L == 1 ? 64 : 32;             // output channels of a block
   static constexpr int GROUPS = kConv[L].cout / COB;
   static constexpr int NW = kConv[L].kc / (9 * 16);        // waves along the weight columns
+  static constexpr int kColPitch = kConv[L].kc + 16, kDyPitch = COB + 16;
+  static constexpr int kColLds = kWgradStep * kColPitch, kDyLds = kWgradStep * kDyPitch;
   static_assert(NW * (COB / 32) == kConvWaves && kConv[L].kc % (9 * 16) == 0, "wave tiles");
 };
 
+// Block `block`; s_col: kColLds elements, s_dy: kDyLds.
 template <int L>
-__global__ __launch_bounds__(kConvThreads, 2) void conv_wgrad(const uint16_t* dY, const uint16_t* X, float* part, int M,
-                                                              int steps_per_split, FcGradArgs fc, int fc_block0) {
+__device__ __forceinline__ void wgrad_block(const uint16_t* dY, const uint16_t* X, float* part, int M, int steps_per_split,
+                                            int block, uint16_t* s_col, uint16_t* s_dy) {
   constexpr ConvShape c = kConv[L];
   constexpr int COB = WgradShape<L>::COB, GROUPS = WgradShape<L>::GROUPS, NW = WgradShape<L>::NW;
-  constexpr int kColPitch = c.kc + 16, kDyPitch = COB + 16;
+  constexpr int kColPitch = WgradShape<L>::kColPitch, kDyPitch = WgradShape<L>::kDyPitch;
   constexpr int kTapVecs = c.cin / 8, kVecs = c.kc / 8, kPer = (kVecs + 7) / 8;  // eight threads per pixel
-  constexpr int kColElems = L == 1 && kFcLds > kWgradStep * kColPitch ? kFcLds : kWgradStep * kColPitch;
-  __shared__ __align__(16) uint16_t s_col[kColElems];
-  __shared__ __align__(16) uint16_t s_dy[kWgradStep * kDyPitch];
-  if constexpr (L == 1) {
-    if ((int)blockIdx.x >= fc_block0) {  // uniform
-      fc_block(fc, (int)blockIdx.x - fc_block0, s_col);
-      return;
-    }
-  }
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4;
   // the groups of a split read the same map: keep them on one XCD (blocks go round-robin)
-  const int b = blockIdx.x, split = b / (8 * GROUPS) * 8 + b % 8, group = b / 8 % GROUPS;
+  const int b = block, split = b / (8 * GROUPS) * 8 + b % 8, group = b / 8 % GROUPS;
   const int co0 = group * COB;
   const int px = tid >> 3, v0 = tid & 7;
   const int first = split * steps_per_split, last = min(first + steps_per_split, (M + kWgradStep - 1) / kWgradStep);
@@ -496,6 +498,34 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_wgrad(const uint16_t* dY
     for (int i = 0; i < 9; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) plane[(co0 + cw + 16 * t + 4 * q + j) * c.kc + nw + 16 * i + r] = acc[t][i][j];
+}
+
+// The backward pass of layer L: its weight gradient (blocks below wblocks), its input
+// gradient (dblocks more) and, beside layer L = 1, the fully connected layers' blocks.
+// Neither needs the other, and neither fills the chip at small batches: one launch
+// instead of two.  Batch 256: layers 2 / 3 / 4 in 79 / 48 / 32 us (95 / 58 / 42 apart);
+// the whole step at batch 19: 99 us against 120.
+struct ConvBackArgs {
+  const uint16_t *dY, *X, *Wt;
+  uint16_t* dX;
+  float *wpart, *bpart;
+  int M, steps_per_split, wblocks, dblocks;
+  FcGradArgs fc;
+};
+
+template <int L>
+__global__ __launch_bounds__(kConvThreads, 2) void conv_backward(ConvBackArgs a) {
+  using S = WgradShape<L>;
+  constexpr int kCol = L == 1 && kFcLds > S::kColLds ? kFcLds : S::kColLds;
+  __shared__ __align__(16) uint16_t s_col[kCol], s_dy[S::kDyLds];
+  static_assert(sizeof(s_col) >= kDgradLds * sizeof(float), "LDS of the input gradient");
+  const int b = blockIdx.x;  // every branch is uniform
+  if (b < a.wblocks)
+    wgrad_block<L>(a.dY, a.X, a.wpart, a.M, a.steps_per_split, b, s_col, s_dy);
+  else if (b < a.wblocks + a.dblocks)
+    dgrad_block<L>(a.dY, a.Wt, a.X, a.dX, a.bpart, a.M, b - a.wblocks, a.dblocks, reinterpret_cast<float*>(s_col));
+  else if constexpr (L == 1)
+    fc_block(a.fc, b - a.wblocks - a.dblocks, s_col);
 }
 
 // Weight gradient of layer 1.  A block walks over groups of four output rows: the input
