@@ -23,7 +23,7 @@ namespace kf {
 namespace {
 
 // ---------------------------------------------------------------------------
-// Fused inference (kf_prior_forward): one 256-thread block per (layer-4 pixel,
+// Fused inference (kf_prior_forward at small batches): one block per (layer-4 pixel,
 // sample) carries the pixel's receptive field through the four convolutions in
 // LDS — a 15x15 window of layer 1, 7x7 of layer 2, 3x3 of layer 3, then the pixel
 // (window positions outside a layer's map hold zeros: that layer's padding) — and
@@ -31,22 +31,30 @@ namespace {
 // 32 from 0 on the same BF16 operands, the same epilogue), so every activation
 // equals the layer-by-layer forward's bit for bit.  Neighbouring blocks recompute
 // the overlap of their windows (~2.7x the 42 M MACs of one sample) in exchange for
-// one launch instead of eight, with nothing between the layers but LDS.  The last
+// one launch, with nothing between the layers but LDS.  The last
 // block of a sample to finish (a device counter, cleared again by that block)
-// averages the 80 layer-4 pixels and runs FC1 and FC2 for the sample's row as
-// head_sample does.  Operands: A from LDS and B (weights, L2-resident) from global
-// memory, one 16-byte vector per lane and MFMA step.
-constexpr int kFuseThreads = 256;
+// runs the forward head.
+//
+// Bound by latency: at batch 1 there are 80 blocks and every stage waits for the one
+// before.  So the weights are the A operand, held in registers and loaded a layer ahead
+// of their use; eight waves share each layer's tiles; window pixels are padded by 16
+// bytes in LDS (without, the 16 pixels of an operand read lie on the same banks); the
+// layer-4 pixels go to the last block by agent-scope stores and loads (no L2 write-back
+// and invalidation, kf_icp.hip), all of them in flight together.  Batch 1: 17.6 us
+// against 23.7 with four waves, weights loaded where they are used, scalar FC1 weight
+// loads and fences around the hand-over.
+constexpr int kFuseThreads = 512, kFuseWaves = kFuseThreads / kWave;
 constexpr int kWin1 = 15, kWin2 = 7, kWin3 = 3;  // window sides of layers 1-3 around one layer-4 pixel
 constexpr int kRows1 = kWin1 * kWin1;            // 225 layer-1 positions
-constexpr int kRows1Pad = 240;                   // 15 MFMA row tiles
 constexpr int kPatch = 2 * kWin1 + 1;            // 31: input window side
+constexpr int kPix1 = 32 + 8, kPix2 = 64 + 8, kPix3 = 64;  // elements per window pixel in LDS
 
 struct FuseArgs {
   const float* frames;
   const int32_t* pairs;
   const float* prev;
   const uint16_t* wbf;   // BF16 weights
+  const uint16_t* w5;    // FC1 with padded rows (WeightCopies)
   const float* params;   // FP32 biases
   long w[6], b[6];       // parameter offsets
   float* Y4;             // [B][80][128] layer-4 activations
@@ -54,208 +62,177 @@ struct FuseArgs {
   unsigned* count;       // [B] finished blocks of each sample (zero between calls)
 };
 
-// B operand of one MFMA step for output column n: W(n, k .. k + 7) of the row-major
-// [N][kc] BF16 weights, zero for n >= N or beyond kc.
-__device__ __forceinline__ uint4 wfrag(const uint16_t* W, int kc, int N, int n, int k) {
-  if (n >= N || k >= kc) return make_uint4(0u, 0u, 0u, 0u);
-  const uint16_t* row = W + (long)n * kc;
-  if ((kc & 7) == 0) return *reinterpret_cast<const uint4*>(row + k);  // 16-byte aligned rows
-  uint16_t e[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) e[j] = k + j < kc ? row[k + j] : (uint16_t)0;
-  uint4 r;
-  __builtin_memcpy(&r, e, 16);
-  return r;
-}
+// NT tiles of one convolution layer (L 1..3) as a wave computes them: channels ch0 .. of
+// 16 window positions.  Output window side WOUT; input window pixels of PIN elements.
+template <int L, int NT, int WOUT, int PIN>
+struct FuseConv {
+  static constexpr ConvShape c = kConv[L];
+  static constexpr int KS = c.kc / 32, CH = 4 * NT;
+  uint4 w[KS][NT];
+  float b[CH];
 
-// A operand of one MFMA step of a 3x3 / stride-2 convolution over an LDS window of
-// side 2 WOUT + 1 (NHWC, CIN channels): output window position p, k .. k + 7 = eight
-// channels of one tap.
-template <int CIN, int WOUT>
-__device__ __forceinline__ uint4 afrag(const uint16_t* act, int p, int k) {
-  const int tap = k / CIN, ci = k - tap * CIN;
-  const int ky = tap / 3, kx = tap - 3 * ky;
-  const int wy = p / WOUT, wx = p - wy * WOUT;
-  return *reinterpret_cast<const uint4*>(act + ((2 * wy + ky) * (2 * WOUT + 1) + (2 * wx + kx)) * CIN + ci);
-}
-
-// One convolution layer of the window (layers 2-4): output window side WOUT with
-// origin (y0, x0) in a map of HOUT x WOUT_MAP; wave w takes column tiles w, w + 4,
-// ... and every row tile.  Epilogue: bias, ReLU; layers 2-3 store
-// the BF16 copy into the output window (zero outside the map), layer 4 (WOUT 1)
-// stores the FP32 value of its one position to y4.
-template <int CIN, int COUT, int WOUT, int HOUT, int WOUT_MAP>
-__device__ __forceinline__ void fuse_conv(const uint16_t* in, uint16_t* outw, const uint16_t* W, const float* bias,
-                                          int y0, int x0, float* y4) {
-  constexpr int K = 9 * CIN, STEPS = K / 32, ROWS = WOUT * WOUT, MT = (ROWS + 15) / 16, NT = COUT / 16;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, q = lane >> 4;
-  for (int nt = wave; nt < NT; nt += kFuseThreads / kWave) {
-    const int n = nt * 16 + r;
-    uint4 bf[STEPS];
+  __device__ __forceinline__ void load(const uint16_t* W, const float* bias, int ch0) {
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
 #pragma unroll
-    for (int s = 0; s < STEPS; ++s) bf[s] = wfrag(W, K, COUT, n, 32 * s + 8 * q);
-    const float bn = bias[n];
-    for (int mt = 0; mt < MT; ++mt) {
-      const int p = min(mt * 16 + r, ROWS - 1);  // rows beyond the window repeat the last one
-      v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int t = 0; t < NT; ++t) {
+      const uint16_t* row = W + (ch0 + tile_channel<NT>(t, r)) * c.kc + 8 * q;
 #pragma unroll
-      for (int s = 0; s < STEPS; ++s) acc = mfma32(afrag<CIN, WOUT>(in, p, 32 * s + 8 * q), bf[s], acc);
+      for (int s = 0; s < KS; ++s) w[s][t] = *reinterpret_cast<const uint4*>(row + 32 * s);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int row = mt * 16 + 4 * q + j;
-        if (row >= ROWS) continue;
-        float v = acc[j] + bn;
-        v = fmaxf(v, 0.0f);
-        if (y4) {
-          if (row == 0) y4[n] = v;
-        } else {
-          const int wy = row / WOUT, wx = row - wy * WOUT;
-          const int gy = y0 + wy, gx = x0 + wx;
-          const bool in_map = gy >= 0 && gy < HOUT && gx >= 0 && gx < WOUT_MAP;
-          outw[row * COUT + n] = in_map ? bf16_rne(v) : (uint16_t)0;
-        }
-      }
+      for (int j = 0; j < 4; ++j) b[4 * t + j] = bias[ch0 + CH * q + 4 * t + j];
     }
   }
-}
+
+  // Channels ch0 + CH q .. of position p (in the window); y: ReLU(conv + bias).
+  __device__ __forceinline__ void run(const uint16_t* in, int p, float* y) const {
+    const int q = (threadIdx.x & 63) >> 4;
+    const int wy = p / WOUT, wx = p - wy * WOUT;
+    const uint16_t* at = in + (2 * wy * (2 * WOUT + 1) + 2 * wx) * PIN + 8 * q;
+    v4f acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int tap = 32 * s / c.cin, ci = 32 * s % c.cin;
+      const uint4 a = *reinterpret_cast<const uint4*>(at + (tap / 3 * (2 * WOUT + 1) + tap % 3) * PIN + ci);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = mfma32(w[s][t], a, acc[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[4 * t + j] = fmaxf(acc[t][j] + b[4 * t + j], 0.0f);
+  }
+
+  // The same, stored as BF16 into the output window (POUT elements per pixel) with origin
+  // (y0, x0) in the layer's map, zero outside it.
+  template <int POUT>
+  __device__ __forceinline__ void run_store(const uint16_t* in, int tile, uint16_t* out, int ch0, int y0, int x0) const {
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+    const int p = tile * 16 + r;
+    float y[CH];
+    run(in, min(p, WOUT * WOUT - 1), y);
+    if (p >= WOUT * WOUT) return;
+    const int gy = y0 + p / WOUT, gx = x0 + p % WOUT;
+    if (!(gy >= 0 && gy < c.hout && gx >= 0 && gx < c.wout)) {
+#pragma unroll
+      for (int j = 0; j < CH; ++j) y[j] = 0.0f;
+    }
+    store_bf16<CH>(out + p * POUT + ch0 + CH * q, y);
+  }
+};
 
 __global__ __launch_bounds__(kFuseThreads) void prior_infer_fused(FuseArgs f) {
-  __shared__ uint16_t patch[2][kPatch][kPatch];              // input window (two planes), BF16
-  __shared__ __align__(16) uint16_t col1[kRows1Pad * 32];    // layer-1 im2col of the window
-  __shared__ __align__(16) uint16_t act1[kRows1 * 32];       // layer-1 window, NHWC
-  __shared__ __align__(16) uint16_t act2[kWin2 * kWin2 * 64];
-  __shared__ __align__(16) uint16_t act3[kWin3 * kWin3 * 64];
-  __shared__ __align__(16) uint16_t xs[kFc1Pad];
-  __shared__ __align__(16) uint16_t hs[kHidden];
+  __shared__ uint32_t patch[kPatch][kPatch + 1];  // input window, BF16 pairs (previous, current)
+  __shared__ __align__(16) uint16_t act1[kRows1 * kPix1];  // layer windows, NHWC
+  __shared__ __align__(16) uint16_t act2[kWin2 * kWin2 * kPix2];
+  __shared__ __align__(16) uint16_t act3[kWin3 * kWin3 * kPix3];
+  __shared__ __align__(16) uint16_t xs[kFc1Pad], hs[kHidden];
   __shared__ int s_last;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, q = lane >> 4;
   const int n = blockIdx.y, pix = blockIdx.x;
   const int y4 = pix / kConv[3].wout, x4 = pix - y4 * kConv[3].wout;
-  const int f0 = f.pairs[2 * n], f1 = f.pairs[2 * n + 1];
+  const float* f0 = f.frames + (long)f.pairs[2 * n] * (kH0 * kW0);
+  const float* f1 = f.frames + (long)f.pairs[2 * n + 1] * (kH0 * kW0);
 
-  // the 31x31 input window of both planes (zero outside the frame), BF16 as im2col_pairs rounds it
-  {
-    constexpr int E = 2 * kPatch * kPatch, PER = (E + kFuseThreads - 1) / kFuseThreads;
-    float v[PER];
+  // the 31x31 input window (zero outside the frame): the loads first, the weights of
+  // layers 1 and 2 behind them
+  constexpr int E = kPatch * kPatch, PER = (E + kFuseThreads - 1) / kFuseThreads;
+  float v[PER][2];
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = tid + kFuseThreads * u;
-      const int c = e / (kPatch * kPatch), rem = e - c * (kPatch * kPatch);
-      const int py = rem / kPatch, px = rem - py * kPatch;
-      const int iy = 16 * y4 - 15 + py, ix = 16 * x4 - 15 + px;
-      const bool in = e < E && iy >= 0 && iy < kH0 && ix >= 0 && ix < kW0;
-      v[u] = in ? f.frames[((long)(c ? f1 : f0) * kH0 + iy) * kW0 + ix] : 0.0f;
+  for (int u = 0; u < PER; ++u) {
+    const int e = tid + kFuseThreads * u, py = e / kPatch, px = e - py * kPatch;
+    const int iy = 16 * y4 - 15 + py, ix = 16 * x4 - 15 + px;
+    const bool in = e < E && iy >= 0 && iy < kH0 && ix >= 0 && ix < kW0;
+    const int o = in ? iy * kW0 + ix : 0;
+    v[u][0] = in ? f0[o] : 0.0f;
+    v[u][1] = in ? f1[o] : 0.0f;
+  }
+  uint4 w1[2];
+  float b1[8];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    uint16_t e[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      e[j] = 8 * q + j < kConv[0].kc ? f.wbf[f.w[0] + tile_channel<2>(t, r) * kConv[0].kc + 8 * q + j] : (uint16_t)0;
+    __builtin_memcpy(&w1[t], e, 16);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) b1[4 * t + j] = f.params[f.b[0] + 8 * q + 4 * t + j];
+  }
+  FuseConv<1, 2, kWin2, kPix1> c2;  // wave: channels 32 (wave / 4) .., position tile wave % 4
+  const int ch2 = wave / 4 * 32;
+  c2.load(f.wbf + f.w[1], f.params + f.b[1], ch2);
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int e = tid + kFuseThreads * u;
+    if (e < E) patch[e / kPatch][e % kPatch] = pack_bf16(v[u][0], v[u][1]);
+  }
+  __syncthreads();
+  FuseConv<2, 1, kWin3, kPix2> c3;  // waves 0..3: channels 16 wave ..
+  const int ch3 = wave % 4 * 16;
+  c3.load(f.wbf + f.w[2], f.params + f.b[2], ch3);
+  {  // layer 1: one K step, the lane's four taps straight from the patch (tap 8 alone at q = 2)
+    int off[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int tap = min(4 * q + e, 8);
+      off[e] = tap / 3 * (kPatch + 1) + tap % 3;
     }
+    for (int tile = wave; tile < (kRows1 + 15) / 16; tile += kFuseWaves) {
+      const int p = tile * 16 + r, pc = min(p, kRows1 - 1), wy = pc / kWin1, wx = pc - wy * kWin1;
+      const uint32_t* at = &patch[0][0] + 2 * wy * (kPatch + 1) + 2 * wx;
+      uint32_t a[4];
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = tid + kFuseThreads * u;
-      if (e < E) {
-        const int c = e / (kPatch * kPatch), rem = e - c * (kPatch * kPatch);
-        const int py = rem / kPatch, px = rem - py * kPatch;
-        patch[c][py][px] = bf16_rne(v[u]);
+      for (int e = 0; e < 4; ++e) {
+        a[e] = at[off[e]];
+        if (4 * q + e > 8) a[e] = 0u;
       }
-    }
-  }
-  __syncthreads();
-  // layer-1 im2col of the 15x15 window (k = (ky * 3 + kx) * 2 + plane, zero for k >= 18)
-  for (int e = tid; e < kRows1Pad * 32; e += kFuseThreads) {
-    const int p = e >> 5, k = e & 31;
-    uint16_t v = 0;
-    if (p < kRows1 && k < kConv[0].kc) {
-      const int wy = p / kWin1, wx = p - wy * kWin1;
-      const int tap = k >> 1, ky = tap / 3, kx = tap - 3 * ky;
-      v = patch[k & 1][2 * wy + ky][2 * wx + kx];
-    }
-    col1[e] = v;
-  }
-  __syncthreads();
-  // layer 1: M = 225 window positions, N = 32, one K step; wave w: column tile w & 1,
-  // row tiles (w >> 1), (w >> 1) + 2, ...
-  {
-    const int nt = wave & 1, nn = nt * 16 + r;
-    const uint4 bw = wfrag(f.wbf + f.w[0], kConv[0].kc, 32, nn, 8 * q);
-    const float bn = f.params[f.b[0] + nn];
-    for (int mt = wave >> 1; mt < kRows1Pad / 16; mt += 2) {
-      const uint4 a = *reinterpret_cast<const uint4*>(&col1[(mt * 16 + r) * 32 + 8 * q]);
-      v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-      acc = mfma32(a, bw, acc);
+      const int gy = 8 * y4 - 7 + wy, gx = 8 * x4 - 7 + wx;
+      const bool in_map = gy >= 0 && gy < kConv[0].hout && gx >= 0 && gx < kConv[0].wout;
+      float y[8];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int row = mt * 16 + 4 * q + j;
-        if (row >= kRows1) continue;
-        const float v = fmaxf(acc[j] + bn, 0.0f);
-        const int wy = row / kWin1, wx = row - wy * kWin1;
-        const int gy = 8 * y4 - 7 + wy, gx = 8 * x4 - 7 + wx;
-        const bool in_map = gy >= 0 && gy < kConv[0].hout && gx >= 0 && gx < kConv[0].wout;
-        act1[row * 32 + nn] = in_map ? bf16_rne(v) : (uint16_t)0;
+      for (int t = 0; t < 2; ++t) {
+        v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        acc = mfma32(w1[t], make_uint4(a[0], a[1], a[2], a[3]), acc);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) y[4 * t + j] = in_map ? fmaxf(acc[j] + b1[4 * t + j], 0.0f) : 0.0f;
       }
+      if (p < kRows1) store_bf16<8>(act1 + p * kPix1 + 8 * q, y);
     }
   }
   __syncthreads();
-  fuse_conv<32, 64, kWin2, 30, 40>(act1, act2, f.wbf + f.w[1], f.params + f.b[1], 4 * y4 - 3, 4 * x4 - 3, nullptr);
+  c2.run_store<kPix2>(act1, wave % 4, act2, ch2, 4 * y4 - 3, 4 * x4 - 3);
+  FuseConv<3, 1, 1, kPix3> c4;  // wave: channels 16 wave ..
+  const int ch4 = wave * 16;
+  c4.load(f.wbf + f.w[3], f.params + f.b[3], ch4);
   __syncthreads();
-  fuse_conv<64, 64, kWin3, 15, 20>(act2, act3, f.wbf + f.w[2], f.params + f.b[2], 2 * y4 - 1, 2 * x4 - 1, nullptr);
+  if (wave < 4) c3.run_store<kPix3>(act2, 0, act3, ch3, 2 * y4 - 1, 2 * x4 - 1);
   __syncthreads();
-  float* y4row = f.Y4 + ((long)n * kPool + pix) * kFeat;
-  fuse_conv<64, 128, 1, 8, 10>(act3, nullptr, f.wbf + f.w[3], f.params + f.b[3], y4, x4, y4row);
+  {
+    float y[4];
+    c4.run(act3, 0, y);
+    float* o = f.Y4 + ((long)n * kPool + pix) * kFeat + ch4 + 4 * q;
+    if (r == 0) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) __hip_atomic_store(o + j, y[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
 
-  // the last block of the sample: every other block's layer-4 pixel is visible to it
-  __builtin_amdgcn_s_waitcnt(0);  // this thread's stores have completed
+  // the last block of the sample: every block's stores have completed (s_waitcnt 0
+  // counts them) before its arrival, and the loads below are agent-scope too
+  __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  if (tid == 0) {
-    __threadfence();
-    const unsigned done = atomicAdd(&f.count[n], 1u);
-    s_last = done == (unsigned)(kPool - 1);
-    if (s_last) __threadfence();
-  }
+  if (tid == 0)
+    s_last = __hip_atomic_fetch_add(&f.count[n], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(kPool - 1);
   __syncthreads();
   if (!s_last) return;  // uniform
-
-  // pooling and the previous twist (as pool_concat)
-  if (tid < kFc1In) {
-    float v;
-    if (tid < kFeat) {
-      float sum = 0.0f;
-      for (int p = 0; p < kPool; ++p) sum = sum + f.Y4[((long)n * kPool + p) * kFeat + tid];
-      v = sum * (1.0f / (float)kPool);
-    } else {
-      v = f.prev[n * kTwist + (tid - kFeat)];
-    }
-    xs[tid] = bf16_rne(v);
-  } else if (tid < kFc1Pad) {
-    xs[tid] = 0;
-  }
-  __syncthreads();
-  // FC1 (row n only): H = ReLU(X5 W5^T + b5), K = 134 in 5 steps; wave w: column tiles w, w + 4, ...
-  for (int nt = wave; nt < kHidden / 16; nt += kFuseThreads / kWave) {
-    const int nn = nt * 16 + r;
-    v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int k = 0; k < kFc1Pad; k += 32)
-      acc = mfma32(*reinterpret_cast<const uint4*>(&xs[k + 8 * q]), wfrag(f.wbf + f.w[4], kFc1In, kHidden, nn, k + 8 * q),
-                   acc);
-    if (q == 0) {  // row 0: the sample's row
-      const float v = fmaxf(acc[0] + f.params[f.b[4] + nn], 0.0f);
-      hs[nn] = bf16_rne(v);
-    }
-  }
-  __syncthreads();
-  // FC2 plus the skip connection (one wave): O = (H W6^T + b6) + previous twist
-  if (wave == 0) {
-    v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int k = 0; k < kHidden; k += 32)
-      acc = mfma32(*reinterpret_cast<const uint4*>(&hs[k + 8 * q]), wfrag(f.wbf + f.w[5], kHidden, kTwist, r, k + 8 * q),
-                   acc);
-    if (q == 0 && r < kTwist) {
-      float v = acc[0] + f.params[f.b[5] + r];
-      v = v + f.prev[n * kTwist + r];
-      f.out[n * kTwist + r] = v;
-    }
-    if (lane == 0) f.count[n] = 0u;  // ready for the next call
-  }
+  HeadForward<kFuseWaves, true> head;
+  head.load(f.w5, f.wbf + f.w[5], f.params + f.b[4], f.params + f.b[5]);
+  const float o = head.run(f.Y4, f.prev, n, xs, hs);
+  if (tid < kTwist) f.out[n * kTwist + tid] = o;
+  if (tid == 0) f.count[n] = 0u;  // ready for the next call
 }
 
 __global__ void copy_weights(WeightCopyArgs a, const float* p) {
@@ -332,27 +309,6 @@ kf_status sync_weights(kf_prior* P, hipStream_t s) {
   return check_launch("copy_weights");
 }
 
-// Inference: the fused kernel (the training forward's outputs, in one launch).
-kf_status infer(kf_prior* P, const float* frames, const int32_t* pairs, const float* prev, int B, float* out,
-                hipStream_t s) {
-  const ParamLayout& L = layout();
-  FuseArgs f;
-  f.frames = frames;
-  f.pairs = pairs;
-  f.prev = prev;
-  f.wbf = P->wbf;
-  f.params = P->params;
-  for (int q = 0; q < 6; ++q) {
-    f.w[q] = L.w[q];
-    f.b[q] = L.b[q];
-  }
-  f.Y4 = P->Y4;
-  f.out = out;
-  f.count = P->fuse_count;
-  hipLaunchKernelGGL(prior_infer_fused, dim3(kPool, B), dim3(kFuseThreads), 0, s, f);
-  return check_launch("prior_infer_fused");
-}
-
 constexpr int kConvBlocks = 512;
 
 // One convolution of the training forward: two blocks of four waves a CU hold the
@@ -378,6 +334,40 @@ kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, int B,
   KF_TRY((launch_conv<1, 4, false>(P, P->Yb[0], P->Yb[1], nullptr, B, s)));
   KF_TRY((launch_conv<2, 2, false>(P, P->Yb[1], P->Yb[2], nullptr, B, s)));
   return launch_conv<3, 2, true>(P, P->Yb[2], nullptr, P->Y4, B, s);
+}
+
+// Inference, with the training forward's outputs either way.  The fused kernel's blocks
+// (80 a sample, one fits a CU) are all resident up to three samples on 256 CUs; from the
+// fourth on a second round and the recomputed window overlaps cost more than the layered
+// forward's five launches.  Fused / layered at batch 1: 17.7 / 30.6 us, 3: 19.8 / 31.6,
+// 4: 32.1 / 31.9, 8: 45.9 / 33.7, 256: 1106 / 114.
+constexpr int kLayeredBatch = 4;
+kf_status infer(kf_prior* P, const float* frames, const int32_t* pairs, const float* prev, int B, float* out,
+                hipStream_t s) {
+  const ParamLayout& L = layout();
+  if (B >= kLayeredBatch) {
+    KF_TRY(forward(P, frames, pairs, B, s));
+    hipLaunchKernelGGL(head_infer, dim3(B), dim3(kConvThreads), 0, s, (const float*)P->Y4, prev,
+                       (const uint16_t*)P->wt + weight_copies().w5, (const uint16_t*)P->wbf + L.w[5],
+                       (const float*)P->params + L.b[4], (const float*)P->params + L.b[5], out);
+    return check_launch("head_infer");
+  }
+  FuseArgs f;
+  f.frames = frames;
+  f.pairs = pairs;
+  f.prev = prev;
+  f.wbf = P->wbf;
+  f.w5 = P->wt + weight_copies().w5;
+  f.params = P->params;
+  for (int q = 0; q < 6; ++q) {
+    f.w[q] = L.w[q];
+    f.b[q] = L.b[q];
+  }
+  f.Y4 = P->Y4;
+  f.out = out;
+  f.count = P->fuse_count;
+  hipLaunchKernelGGL(prior_infer_fused, dim3(kPool, B), dim3(kFuseThreads), 0, s, f);
+  return check_launch("prior_infer_fused");
 }
 
 // Backward pass of layer L: the weight gradient as *splits partial planes, one block a CU

@@ -50,20 +50,84 @@ __device__ __forceinline__ void copy_weight(const WeightCopyArgs& a, long i, flo
   if (g >= 0 && g < kTwist * kHidden) a.yt[a.w6t + g % kHidden * 8 + g / kHidden] = v;
 }
 
-// Mean of layer 4 over its pixels for feature c of sample n (added in pixel order).
-__device__ __forceinline__ float pooled_feature(const float* Y4, int n, int c) {
-  constexpr int kLoads = 40;  // two rounds of memory latency
-  static_assert(kPool % kLoads == 0, "pooling batches");
-  const float* y = Y4 + (long)n * kPool * kFeat + c;
-  float s = 0.0f;
-  for (int p = 0; p < kPool; p += kLoads) {
-    float v[kLoads];
+// The forward head of sample n: pooling (the 80 pixels added in order), FC1, FC2 and the
+// skip connection, by a block of WAVES wavefronts.  Every product is the MFMA sequence of
+// a GEMM over the batch (k steps of 32 from zero); the sample's row is broadcast to the
+// 16 rows of the A operand and row 0 of the result is used.  load() issues the weights'
+// loads, so that a caller can put them ahead of other latencies.  AGENT: Y4 was written
+// by other blocks of the same launch, with agent-scope stores.
+template <int WAVES, bool AGENT>
+struct HeadForward {
+  static constexpr int NT = kHidden / 16 / WAVES;  // FC1 column tiles of a wave
+  uint4 w5[NT][kFc1Pad / 32], w6[kHidden / 32];
+  float b5[NT], b6;
+
+  __device__ __forceinline__ void load(const uint16_t* W5, const uint16_t* W6, const float* B5, const float* B6) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
 #pragma unroll
-    for (int u = 0; u < kLoads; ++u) v[u] = y[(p + u) * kFeat];
+    for (int t = 0; t < NT; ++t) {
+      const int nn = (wave + WAVES * t) * 16 + r;
 #pragma unroll
-    for (int u = 0; u < kLoads; ++u) s = s + v[u];
+      for (int s = 0; s < kFc1Pad / 32; ++s) w5[t][s] = *reinterpret_cast<const uint4*>(W5 + nn * kFc1Pad + 32 * s + 8 * q);
+      b5[t] = B5[nn];
+    }
+    const int row = min(r, kTwist - 1);  // columns past the six outputs are not used
+#pragma unroll
+    for (int s = 0; s < kHidden / 32; ++s) w6[s] = *reinterpret_cast<const uint4*>(W6 + row * kHidden + 32 * s + 8 * q);
+    b6 = B6[row];
   }
-  return s * (1.0f / (float)kPool);
+
+  // xs[kFc1Pad], hs[kHidden] (LDS): FC1's and FC2's inputs.  Returns output r in the
+  // lanes q = 0, r < 6 of wave 0; hs is published, the output is not.
+  __device__ __forceinline__ float run(const float* Y4, const float* prev, int n, uint16_t* xs, uint16_t* hs) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4;
+    if (tid < kFc1Pad) {
+      float v = 0.0f;
+      if (tid < kFeat) {
+        const float* y = Y4 + (long)n * kPool * kFeat + tid;
+        float e[kPool];  // one round of memory latency
+#pragma unroll
+        for (int p = 0; p < kPool; ++p) {
+          if constexpr (AGENT) e[p] = __hip_atomic_load(const_cast<float*>(y) + p * kFeat, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          else e[p] = y[p * kFeat];
+        }
+#pragma unroll
+        for (int p = 0; p < kPool; ++p) v = v + e[p];
+        v = v * (1.0f / (float)kPool);
+      } else if (tid < kFc1In) {
+        v = prev[n * kTwist + (tid - kFeat)];
+      }
+      xs[tid] = bf16_rne(v);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {  // H = ReLU(X5 W5^T + b5)
+      v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int s = 0; s < kFc1Pad / 32; ++s) acc = mfma32(*reinterpret_cast<const uint4*>(&xs[32 * s + 8 * q]), w5[t][s], acc);
+      if (q == 0) hs[(wave + WAVES * t) * 16 + r] = bf16_rne(fmaxf(acc[0] + b5[t], 0.0f));
+    }
+    __syncthreads();
+    float o = 0.0f;
+    if (wave == 0) {  // O = (H W6^T + b6) + previous twist
+      v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int s = 0; s < kHidden / 32; ++s) acc = mfma32(*reinterpret_cast<const uint4*>(&hs[32 * s + 8 * q]), w6[s], acc);
+      o = acc[0] + b6;
+      o = o + prev[n * kTwist + min(r, kTwist - 1)];
+    }
+    return o;
+  }
+};
+
+// The head alone (batched inference): one sample per block.
+__global__ __launch_bounds__(kConvThreads) void head_infer(const float* Y4, const float* prev, const uint16_t* W5,
+                                                           const uint16_t* W6, const float* B5, const float* B6, float* out) {
+  __shared__ __align__(16) uint16_t xs[kFc1Pad], hs[kHidden];
+  HeadForward<kConvWaves, false> head;
+  head.load(W5, W6, B5, B6);
+  const float o = head.run(Y4, prev, blockIdx.x, xs, hs);
+  if (threadIdx.x < kTwist) out[blockIdx.x * kTwist + threadIdx.x] = o;
 }
 
 struct HeadArgs {
@@ -76,60 +140,32 @@ struct HeadArgs {
   float inv;                     // 1 / (6 B)
 };
 
-// One sample per block: pooling, FC1, FC2 and the skip connection, the loss gradient,
-// and back to layer 4 (dY4[p][c] = dX5[c] / 80 where Y4 > 0).  Every product is the
-// MFMA sequence of a GEMM over the batch (k steps of 32 from zero); the sample's row is
-// broadcast to the 16 rows of the A operand and row 0 of the result is used.  Latency
-// bound (six dependent stages); one launch in place of twelve, 60 us of launches at any
-// batch.  18 us at batch 256.
+// One sample per block: the forward head, the loss gradient, and back to layer 4
+// (dY4[p][c] = dX5[c] / 80 where Y4 > 0).  Latency bound (six dependent stages); one
+// launch in place of twelve, 60 us of launches at any batch.  18 us at batch 256.
 __global__ __launch_bounds__(kConvThreads) void head_sample(HeadArgs a) {
   __shared__ __align__(16) uint16_t xs[kFc1Pad], hs[kHidden], dhs[kHidden];
   __shared__ __align__(16) uint16_t dos[8];
   __shared__ float dx[kFeat], red[kFeat];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4, n = blockIdx.x;
-  if (tid < kFc1Pad) {
-    float v = 0.0f;
-    if (tid < kFeat) v = pooled_feature(a.Y4, n, tid);
-    else if (tid < kFc1In) v = a.prev[n * kTwist + (tid - kFeat)];
-    xs[tid] = bf16_rne(v);
-    if (tid < kX5Pitch) a.X5b[n * kX5Pitch + tid] = xs[tid];
-  }
+  HeadForward<kConvWaves, false> head;
+  head.load(a.w5, a.w6, a.b5, a.b6);
   if (tid < 8) dos[tid] = 0;
-  __syncthreads();
-  for (int nt = wave; nt < kHidden / 16; nt += kConvWaves) {  // H = ReLU(X5 W5^T + b5)
-    const int nn = nt * 16 + r;
-    v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int k = 0; k < kFc1Pad; k += 32)
-      acc = mfma32(*reinterpret_cast<const uint4*>(&xs[k + 8 * q]),
-                   *reinterpret_cast<const uint4*>(a.w5 + nn * kFc1Pad + k + 8 * q), acc);
-    if (q == 0) {
-      hs[nn] = bf16_rne(fmaxf(acc[0] + a.b5[nn], 0.0f));
-      a.Hb[n * kHidden + nn] = hs[nn];
+  const float o = head.run(a.Y4, a.prev, n, xs, hs);
+  if (tid < kX5Pitch) a.X5b[n * kX5Pitch + tid] = xs[tid];
+  a.Hb[n * kHidden + tid] = hs[tid];
+  static_assert(kHidden == kConvThreads, "one hidden unit a thread");
+  if (wave == 0 && q == 0) {  // dLoss/dO
+    uint16_t db = 0;
+    if (r < kTwist) {
+      const float d = o - a.target[n * kTwist + r];
+      const float g = 2.0f * d * a.inv;
+      a.O[n * kTwist + r] = o;
+      a.dO[n * kDoSumPitch + r] = g;
+      db = bf16_rne(g);
+      dos[r] = db;
     }
-  }
-  __syncthreads();
-  if (wave == 0) {  // O = (H W6^T + b6) + previous twist, and dLoss/dO
-    v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    const int row = min(r, kTwist - 1);  // columns past the six outputs are not used
-#pragma unroll
-    for (int k = 0; k < kHidden; k += 32)
-      acc = mfma32(*reinterpret_cast<const uint4*>(&hs[k + 8 * q]),
-                   *reinterpret_cast<const uint4*>(a.w6 + row * kHidden + k + 8 * q), acc);
-    if (q == 0) {
-      uint16_t db = 0;
-      if (r < kTwist) {
-        float v = acc[0] + a.b6[r];
-        v = v + a.prev[n * kTwist + r];
-        const float d = v - a.target[n * kTwist + r];
-        const float g = 2.0f * d * a.inv;
-        a.O[n * kTwist + r] = v;
-        a.dO[n * kDoSumPitch + r] = g;
-        db = bf16_rne(g);
-        dos[r] = db;
-      }
-      a.dOb[n * kDoPitch + r] = db;
-    }
+    a.dOb[n * kDoPitch + r] = db;
   }
   __syncthreads();
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);

@@ -42,3 +42,31 @@ def test_gradients_match_oracle_at_tile_edges(gpu, kf, B):
     prior.gradients(df, dp, dv, dt, B, dg, dl)
     kf.synchronize()
     assert np.array_equal(g, dg.download(np.float32).astype(np.float64))
+
+
+def test_batched_inference_equals_single_samples(gpu, kf):
+    """Batches of 1 and 3 run fused, 4 and 37 layer by layer: the same MFMA sequences, so
+    the same bits per sample."""
+    rng = np.random.default_rng(7)
+    B = 37
+    frames = rng.uniform(0.5, 3.5, size=(B + 1, po.H0, po.W0)).astype(np.float32)
+    pairs = rng.integers(0, B + 1, size=(B, 2)).astype(np.int32)
+    prev = rng.normal(0, 0.5, size=(B, 6)).astype(np.float32)
+    df, dp, dv = [kf.upload(a) for a in (frames, pairs, prev)]
+    prior = kf.Prior(max_batch=B)
+    prior.set_params(po.init_params(3).astype(np.float32))
+    dout = kf.DeviceBuffer(B * 24)
+
+    def run(first, n):
+        print(f"prior forward {first}..{first + n - 1}", flush=True)
+        prior.forward(df, dp.ptr + first * 8, dv.ptr + first * 24, n, dout)
+        kf.synchronize()
+        return dout.download(np.float32, n * 6).reshape(n, 6).view(np.uint32)
+
+    single = np.concatenate([run(i, 1) for i in range(B)])
+    assert np.array_equal(run(0, B), single)
+    assert np.array_equal(run(5, 4), single[5:9])
+    assert np.array_equal(run(11, 3), single[11:14])
+    ref, _ = po.forward(po.init_params(3), frames, pairs, prev, bf=True)
+    out = single.view(np.float32)
+    assert np.max(np.abs(out - ref)) < 2e-3 * np.abs(ref).max()
