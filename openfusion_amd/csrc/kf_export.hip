@@ -29,13 +29,34 @@ __device__ __forceinline__ void vox_fw(const void* vox, size_t i, float& f, floa
   }
 }
 
-template <int FMT>
-__global__ __launch_bounds__(256) void tsdf_export(const void* vox, size_t n3, float trunc, float* out) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n3) return;
-  float f, w;
-  vox_fw<FMT>(vox, i, f, w);
-  out[i] = w > 0.0f ? f * trunc : trunc;
+// Four voxels per thread: one 16-byte load (two for FP32 records) and one 16-byte
+// non-temporal store, no loop.  Bound by memory; 512^3 FP16: 170 us, 6.3 TB/s (a voxel
+// per thread 290 us; four vectors a thread 186, a grid-stride loop 173..192; temporal
+// stores 175).  ALIGNED: d_out is 16-byte aligned, as a device allocation is; a caller's
+// offset into one gets four 4-byte stores.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <int FMT, bool ALIGNED>
+__global__ __launch_bounds__(256) void tsdf_export(const uint4* vox, size_t n4, float trunc, float* out) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  f32x4 o;
+  if (FMT == KF_VOXEL_F16) {
+    const uint4 q = vox[i];
+    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = (w[j] >> 16) ? half_bits_to_float(w[j] & 0xffffu) * trunc : trunc;
+  } else {
+    const uint4 a = vox[2 * i], b = vox[2 * i + 1];
+    const uint32_t f[4] = {a.x, a.z, b.x, b.z}, w[4] = {a.y, a.w, b.y, b.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = __uint_as_float(w[j]) > 0.0f ? __uint_as_float(f[j]) * trunc : trunc;
+  }
+  if (ALIGNED) {
+    __builtin_nontemporal_store(o, reinterpret_cast<f32x4*>(out) + i);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[4 * i + j] = o[j];
+  }
 }
 
 // Freudenthal split: corner i = dx + 2 dy + 4 dz; tetrahedra (0, 7, a, b) for the
@@ -157,14 +178,14 @@ using namespace kf;
 
 extern "C" kf_status kf_volume_export_tsdf(const kf_volume* v, float* d_out, kf_stream s) {
   KF_CHECK_ARG(v && d_out, "NULL argument");
-  const size_t n3 = (size_t)v->desc.n * v->desc.n * v->desc.n;
-  const unsigned blocks = (unsigned)((n3 + 255) / 256);
-  if (v->desc.format == KF_VOXEL_F16)
-    hipLaunchKernelGGL(tsdf_export<KF_VOXEL_F16>, dim3(blocks), dim3(256), 0, S(s), (const void*)v->d_voxels, n3,
-                       v->desc.trunc_m, d_out);
-  else
-    hipLaunchKernelGGL(tsdf_export<KF_VOXEL_F32>, dim3(blocks), dim3(256), 0, S(s), (const void*)v->d_voxels, n3,
-                       v->desc.trunc_m, d_out);
+  const size_t n4 = (size_t)v->desc.n * v->desc.n * v->desc.n / 4;  // n is a multiple of 8
+  const unsigned blocks = (unsigned)((n4 + 255) / 256);
+  const bool aligned = (reinterpret_cast<uintptr_t>(d_out) & 15) == 0;
+  auto kern = v->desc.format == KF_VOXEL_F16
+                  ? (aligned ? tsdf_export<KF_VOXEL_F16, true> : tsdf_export<KF_VOXEL_F16, false>)
+                  : (aligned ? tsdf_export<KF_VOXEL_F32, true> : tsdf_export<KF_VOXEL_F32, false>);
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, S(s), static_cast<const uint4*>(v->d_voxels), n4,
+                     v->desc.trunc_m, d_out);
   return check_launch("tsdf_export");
 }
 

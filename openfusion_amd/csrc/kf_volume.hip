@@ -75,10 +75,12 @@ struct SweepArgs {
   float band;  // T + max(0.01 T, 0.1 mm): half-width of the band where the square root is taken
 };
 
+// One 16-byte store per thread, no loop.  Bound by memory; 512 MB: 78 us, 6.8 TB/s (a
+// grid-stride loop 117 us on 8192 blocks, 96 on 16384; two or more stores a thread 88
+// and up), 128 MB: 20.6 us against 21.9.
 __global__ __launch_bounds__(256) void volume_fill(uint4* p, size_t n16, uint4 word) {
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (; i < n16; i += stride) p[i] = word;
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n16) p[i] = word;
 }
 
 // Raylen extrema of the 8x8 and 32x32 pixel tiles (x = min, y = max).  Pixels
@@ -775,8 +777,7 @@ kf_status launch_volume_reset(kf_volume* v, hipStream_t s) {
     word = make_uint4(one, 0u, one, 0u);
   }
   const size_t n16 = v->bytes / 16;
-  const int blocks = (int)std::min<size_t>((n16 + 255) / 256, 8192);
-  hipLaunchKernelGGL(volume_fill, dim3(blocks), dim3(256), 0, s, static_cast<uint4*>(v->d_voxels), n16,
+  hipLaunchKernelGGL(volume_fill, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, s, static_cast<uint4*>(v->d_voxels), n16,
                      word);
   KF_TRY(check_launch("volume_fill"));
   if (v->d_occ) KF_TRY(clear_occupancy(v, s));  // every voxel is free space: all bricks clear
