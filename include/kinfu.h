@@ -276,9 +276,8 @@ typedef struct kf_icp_params {
   float dist_thresh_m;
   float normal_thresh_deg;
   int32_t compensated;                /* 1: terms accumulated in FP64 (exact products of the FP32 row
-                                         entries, one rounding per term), block partials stored as
-                                         (hi, lo) FP32 pairs keeping ~48 bits (default); 0: plain FP32
-                                         partials */
+                                         entries), block partials in FP64 (default); 0: plain FP32
+                                         sums within a block */
   int32_t single_launch;              /* 1: the whole call is one launch, iterations separated by a
                                          grid barrier (same results as the multi-launch form, bit for
                                          bit, while the barrier works); 0: one launch per iteration

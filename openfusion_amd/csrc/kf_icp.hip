@@ -13,13 +13,13 @@
 // cos_thresh < n.m < 1+1e-6.  Row: A = [m x d, m], b = m.(s-d); after the solve
 // of (A^T A) x = A^T b the rotation is -x[0..2] (ICP.cpp:162-168).
 //
-// Reduction: every thread accumulates the 28 terms (21 A^TA, 6 A^Tb, b^2) over its
-// pixels; waves combine with DPP lane moves (reduce-scatter: row mirrors, quad
-// permutes) and blocks through LDS.  In compensated mode the terms are FP64 (the
-// product of two FP32 row entries is exact in FP64, so a term costs one fused
-// multiply-add with one rounding at 2^-53) and a block partial is stored as a
-// (hi, lo) FP32 pair accurate to ~2^-48 relative; plain mode uses FP32 sums.
-// Each block writes its partial as a slot.  The next launch (the next iteration,
+// Reduction: 28 terms (21 A^TA, 6 A^Tb, b^2).  In compensated mode they are FP64 (the
+// product of two FP32 row entries is exact in FP64): the rows (A, b, inlier flag) of a
+// wave's 64 pixels form an 8 x 64 matrix R, and R R^T holds every term and the inlier
+// count, so they are sums over pixels on the FP64 matrix cores with no lane reduction
+// after them.  Plain mode accumulates FP32 terms per thread and combines waves with DPP
+// lane moves (reduce-scatter: row mirrors, quad permutes).  Blocks combine through LDS.
+// Each block writes its partial as a slot of FP64 values.  The next launch (the next iteration,
 // or the final one-block launch) adds the slots in FP64 in block order, solves by
 // FP64 LDL^T and composes the Euler-ZYX increment onto the FP64 pose; every
 // block of an iteration repeats that solve for itself, so the pose never makes a
@@ -36,14 +36,14 @@ namespace {
 
 constexpr int kTerms = 28;   // 21 + 6 + 1 float terms
 constexpr int kPad = 32;     // terms padded to a power of two for the wave reduction
-constexpr int kSlot = 64;    // floats per block partial: 28 (hi,lo) + 2 int counts + stop marker
-constexpr int kStopAt = 58;  // slot float (int bits): 1 when the block stopped (singular system)
-constexpr int kSums = kTerms + 3;  // slot sums: 28 terms, inliers, candidates, stopped blocks
+constexpr int kSlot = 32;    // doubles per block partial: 28 terms, inliers, candidates, stop marker, unused
+constexpr int kInlAt = kTerms, kCandAt = kTerms + 1;
+constexpr int kStopAt = kTerms + 2;  // 1 when the block stopped (singular system)
+constexpr int kRowPitch = kWave + 4;  // doubles per row entry of a wave's pixels in LDS
 constexpr int kThreads = 256;
 constexpr double kPivotRelEps = 1e-9;
 constexpr int kMinInliers = 6;
-constexpr int kPpt0 = 3;            // pixels per thread of a level-0 tracking step (200 blocks at 640x480)
-constexpr int kFinUnroll = 7;       // slot loads in flight per thread of the slot sum (7 x 32 groups cover 200 slots in one round)
+constexpr int kFinUnroll = 8;       // slot loads in flight per thread of the slot sum (8 x 32 groups: 256 slots in one round)
 constexpr int kStepThreads = 512;    // tracking step: 8 waves per block
 // One-block sums and solves use the step's block size, so that every slot sum (in
 // a step, the final one-block launch or the single-launch kernel) adds in the same
@@ -55,9 +55,10 @@ struct IcpArgs {
   const float *mvx, *mvy, *mvz, *mnx, *mny, *mnz;  // model level maps (world frame)
   int W, H;
   float fx, fy, cx, cy;
-  float dist_thr, cos_thr;
+  float dist_thr2;  // sqrtf(d2) < dist_thresh exactly where d2 < dist_thr2
+  float cos_thr;
   kf_pose* pose;
-  float* partials;
+  double* partials;
   kf_icp_ctrl* ctrl;
   kf_icp_stats* stats;
   double* sums_out;
@@ -70,18 +71,16 @@ struct IcpArgs {
 // a cache write-back or invalidation (the single-launch form); otherwise ordinary
 // accesses, published by a kernel boundary.  The values are the same either way.
 template <bool COH>
-__device__ __forceinline__ void slot_put(float* p, float v) {
+__device__ __forceinline__ void slot_put(double* p, double v) {
   if constexpr (COH) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   else *p = v;
 }
 template <bool COH>
-__device__ __forceinline__ float4 slot_get4(const float4* p) {
+__device__ __forceinline__ double2 slot_get2(const double2* p) {
   if constexpr (COH) {
-    unsigned long long* q = reinterpret_cast<unsigned long long*>(const_cast<float4*>(p));
-    const unsigned long long lo = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned long long hi = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return make_float4(__uint_as_float((unsigned)lo), __uint_as_float((unsigned)(lo >> 32)),
-                       __uint_as_float((unsigned)hi), __uint_as_float((unsigned)(hi >> 32)));
+    double* q = reinterpret_cast<double*>(const_cast<double2*>(p));
+    return make_double2(__hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                        __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
   } else {
     return *p;
   }
@@ -106,13 +105,23 @@ __device__ __forceinline__ PxModel load_model(const IcpArgs& a, int i) {
                  f3{plane_at(a.mnx, o), plane_at(a.mny, o), plane_at(a.mnz, o)}, plane_at(a.lvz, o)};
 }
 
+// 1.0f / z for every z the gate below admits: the hardware reciprocal and one Newton step
+// equal the IEEE quotient for all normal z below 2^126 (checked over every such float);
+// beyond, the division itself.
+__device__ __forceinline__ float reciprocal(float z) {
+  float r = __builtin_amdgcn_rcpf(z);
+  r = fmaf(r, fmaf(-z, r, 1.0f), r);
+  if (__builtin_expect(__any(z >= 0x1p126f), 0)) r = z >= 0x1p126f ? 1.0f / z : r;
+  return r;
+}
+
 // Live pixel the model point projects to, or -1 (0 = not a candidate, 1 = rejected
 // in r when j < 0).  Every value is formed and the tests select the result (a
 // wavefront's lanes differ in which test they fail); lanes out of range convert 0.
 __device__ __forceinline__ int project_model(const IcpArgs& a, const kf_posef& cw, const PxModel& q, int& r) {
   const bool cand = q.lz_here == q.lz_here && finite3(q.s) && finite3(q.m);
   const f3 sc = xform(cw, q.s);
-  const float iz = 1.0f / sc.z;
+  const float iz = reciprocal(sc.z);
   const float u = (a.fx * sc.x + a.cx * sc.z) * iz;
   const float v = (a.fy * sc.y + a.cy * sc.z) * iz;
   const float ru = round_half_up(u), rv = round_half_up(v);
@@ -135,7 +144,7 @@ __device__ __forceinline__ int finish_row(const IcpArgs& a, const kf_posef& wc, 
   const f3 df = sub(d, q.s);
   const f3 m = q.m, s = q.s;
   const float cs = dot(n, m);
-  const bool in = finite3(l.dc) && finite3(l.nc) && sqrtf(dot(df, df)) < a.dist_thr && cs > a.cos_thr &&
+  const bool in = finite3(l.dc) && finite3(l.nc) && dot(df, df) < a.dist_thr2 && cs > a.cos_thr &&
                   cs < 1.0f + 1e-6f;
   A[0] = m.y * d.z - m.z * d.y;
   A[1] = m.z * d.x - m.x * d.z;
@@ -147,86 +156,126 @@ __device__ __forceinline__ int finish_row(const IcpArgs& a, const kf_posef& wc, 
   return j < 0 ? r : (in ? 2 : 1);
 }
 
-// Per-thread accumulator of the 28 terms: FP64 when COMP (the product of two FP32
-// values is exact in FP64, so each term is one fused multiply-add with a single
-// rounding at 2^-53), else FP32 (product rounded, then added).
-template <bool COMP>
-struct AccOf {
-  using T = float;
-};
-template <>
-struct AccOf<true> {
-  using T = double;
-};
-template <bool COMP>
-using acc_t = typename AccOf<COMP>::T;
-
-// Adds the 28 terms of one inlier row: 21 upper-triangle A^T A, 6 A^T b, b^2.
-template <bool COMP>
-__device__ __forceinline__ void accumulate(acc_t<COMP>* s, const float* A, float b) {
-  if constexpr (COMP) {
-    double Ad[6];
+// Plain mode: adds the 28 terms of one inlier row: 21 upper-triangle A^T A, 6 A^T b, b^2.
+__device__ __forceinline__ void accumulate(float* s, const float* A, float b) {
+  int k = 0;
 #pragma unroll
-    for (int p = 0; p < 6; ++p) Ad[p] = A[p];
-    const double bd = b;
-    int k = 0;
+  for (int p = 0; p < 6; ++p)
 #pragma unroll
-    for (int p = 0; p < 6; ++p)
-#pragma unroll
-      for (int q = p; q < 6; ++q) {
-        s[k] = fma(Ad[p], Ad[q], s[k]);
-        ++k;
-      }
-#pragma unroll
-    for (int p = 0; p < 6; ++p) s[21 + p] = fma(Ad[p], bd, s[21 + p]);
-    s[27] = fma(bd, bd, s[27]);
-  } else {
-    int k = 0;
-#pragma unroll
-    for (int p = 0; p < 6; ++p)
-#pragma unroll
-      for (int q = p; q < 6; ++q) {
-        const float v = A[p] * A[q];
-        s[k] = s[k] + v;
-        ++k;
-      }
-#pragma unroll
-    for (int p = 0; p < 6; ++p) {
-      const float v = A[p] * b;
-      s[21 + p] = s[21 + p] + v;
+    for (int q = p; q < 6; ++q) {
+      const float v = A[p] * A[q];
+      s[k] = s[k] + v;
+      ++k;
     }
-    const float v = b * b;
-    s[27] = s[27] + v;
+#pragma unroll
+  for (int p = 0; p < 6; ++p) {
+    const float v = A[p] * b;
+    s[21 + p] = s[21 + p] + v;
   }
+  const float v = b * b;
+  s[27] = s[27] + v;
 }
 
-template <int CTRL, typename T>
-__device__ __forceinline__ T dpp_t(T v) {
-  if constexpr (sizeof(T) == 8) return dpp_d<CTRL>(v);
-  else return dpp_f<CTRL>(v);
-}
-
-// One recursive-halving step of the wave reduction (reduce-scatter): lanes paired
-// by the DPP pattern CTRL hold the same H terms; the lane with `upper` keeps the
+// One recursive-halving step of the plain mode's wave reduction (reduce-scatter): lanes
+// paired by the DPP pattern CTRL hold the same H terms; the lane with `upper` keeps the
 // upper H/2, its partner the lower H/2, and each adds the partner's copy of the
 // half it keeps.
-template <int CTRL, int H, typename T>
-__device__ __forceinline__ void halve(T* s, bool upper) {
+template <int CTRL, int H>
+__device__ __forceinline__ void halve(float* s, bool upper) {
 #pragma unroll
   for (int k = 0; k < H / 2; ++k) {
-    const T ks = upper ? s[k + H / 2] : s[k];
-    const T gs = upper ? s[k] : s[k + H / 2];
-    s[k] = ks + dpp_t<CTRL>(gs);
+    const float ks = upper ? s[k + H / 2] : s[k];
+    const float gs = upper ? s[k] : s[k + H / 2];
+    s[k] = ks + dpp_f<CTRL>(gs);
   }
 }
 
-// Block partial: this block's share of the association (pixels bid*T + tid + k*nblk*T,
-// K per round with their loads in flight together, consumed in index order), the
-// 28 terms per thread, the reduce-scatter wave reduction and the sum over the
-// block's waves, written as one slot: 28 (hi, lo) float pairs — hi the FP32
-// rounding of the term, lo that of the remainder, so hi + lo keeps about 48 bits
-// of an FP64 sum (lo = 0 for FP32 sums) — and the inlier / candidate counts.  The
-// sums do not depend on K.
+// Orders the LDS accesses of one wavefront around this point.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// LDS of block_partial.
+template <int WAVES, int K>
+struct PartialLds {
+  double rows[WAVES][K][8][kRowPitch];  // compensated mode: a wave's row entries, one pixel per column
+  double red[WAVES][kWave];
+  int cand[WAVES];
+};
+
+// FP64 sums of products over pixels on v_mfma_f64_4x4x4 (four 4 x 4 products of depth 4
+// per instruction, lane l: block b = (l / 4) % 4, operand row l % 4, depth l / 16).  A lane
+// reads row entry e = l % 8 of the pixels of its group l / 8 (so 64 lanes hold 8 entries of
+// 8 pixels) and the entry 7 - e of the same pixels.  The first register as both operands
+// gives the products of entries 0..3 and of entries 4..7 with themselves; the second as
+// B the products of 0..3 with 7..4.  Two accumulators each, since a chain waits 24 cycles
+// per step.  The LDS reads bound it (eight 16-byte reads per 64 pixels; a lane move in
+// place of the second read costs more, operands held per 4 x 4 block twice the reads).
+// Against 28 FP64 multiply-adds per thread and a reduce-scatter of 28 doubles over the
+// lanes (32 additions, each with four selects and two lane moves): a coarse step's
+// association 3.5 k cycles instead of 5.4 k.
+struct TermSums {
+  double c[2] = {0.0, 0.0}, x[2] = {0.0, 0.0};
+
+  // rows: the wave's 8 x 64 entries in LDS; the pitch puts a quarter-wave's 16-byte
+  // reads (8 entries, two pixel pairs) on all 64 banks.
+  __device__ __forceinline__ void add(const double (*rows)[kRowPitch]) {
+    const int lane = threadIdx.x & 63, e = lane & 7, group = lane >> 3;
+    const double2* p = reinterpret_cast<const double2*>(&rows[e][2 * group]);
+    const double2* q = reinterpret_cast<const double2*>(&rows[7 - e][2 * group]);
+    double2 v[4], w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {  // pixels 16 u + 2 group, + 1
+      v[u] = p[8 * u];
+      w[u] = q[8 * u];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      c[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(v[u].x, v[u].x, c[0], 0, 0, 0);
+      x[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(v[u].x, w[u].x, x[0], 0, 0, 0);
+      c[1] = __builtin_amdgcn_mfma_f64_4x4x4f64(v[u].y, v[u].y, c[1], 0, 0, 0);
+      x[1] = __builtin_amdgcn_mfma_f64_4x4x4f64(v[u].y, w[u].y, x[1], 0, 0, 0);
+    }
+  }
+  // The wave's totals: 64 values, see term_of.
+  __device__ __forceinline__ void store(double* red) const {
+    const int lane = threadIdx.x & 63, at = (lane >> 4) * 8 + (lane & 7);
+    const double d = c[0] + c[1], o = x[0] + x[1];
+    const double ds = d + dpp_d<0x108>(d), os = o + dpp_d<0x108>(o);  // the two pixel groups of a depth
+    if ((lane & 8) == 0) {
+      red[at] = ds;
+      red[32 + at] = os;
+    }
+  }
+};
+
+// Slot position of the entry (p, q) of R R^T that TermSums leaves at `at`: the term, the
+// inlier count (7, 7), or -1 (lower triangles and the other products with the flag).
+__device__ __forceinline__ int term_of(int at) {
+  const int i = (at >> 3) & 3, b = (at >> 2) & 1, j = at & 3;
+  const int p = at < 32 ? 4 * b + i : (b == 0 ? i : 8), q = at < 32 ? 4 * b + j : 7 - j;
+  if (p > q) return -1;
+  if (q < 6) return p * 6 - p * (p - 1) / 2 + (q - p);
+  if (q == 6) return 21 + p;  // A^T b, then b^2 at 27
+  return p == 7 ? kInlAt : -1;
+}
+
+// Which pixels a block of WAVES waves associates at a time: F full rounds (pixel k nblk T
+// + bid T + tid) and, with H, a half round by the block's first WAVES / 2 waves.  nblk
+// blocks cover nblk kPixels pixels; larger images repeat.
+template <int WAVES, int F, int H>
+struct PixelShape {
+  static constexpr int T = WAVES * kWave, K = F + H, kPixels = F * T + H * (T / 2);
+  // this thread's pixel of round k in pass `pass`; its wave takes part in `rounds` of them
+  static __device__ __forceinline__ int pixel(int bid, int nblk, int pass, int k) {
+    const int base = pass * nblk * kPixels + k * nblk * T, tid = threadIdx.x;
+    return base + (k < F ? bid * T + tid : bid * (T / 2) + tid);
+  }
+  static __device__ __forceinline__ int rounds() { return H && (int)threadIdx.x >= T / 2 ? F : K; }  // uniform per wave
+};
+
 // The model samples of a thread's first K pixels in block_partial; they do not
 // depend on the pose, so a step can load them before it solves for the pose.
 template <int K>
@@ -234,207 +283,201 @@ struct PxPre {
   PxModel q[K];
 };
 
-template <int WAVES, int K>
-__device__ __forceinline__ PxPre<K> prefetch_models(const IcpArgs& a, int bid, int nblk) {
-  constexpr int T = WAVES * kWave;
-  const int P = a.W * a.H, stride = nblk * T;
-  const int i0 = bid * T + (int)threadIdx.x;
-  const int j0 = i0 < P ? i0 : 0;  // in bounds; unused when the block has no pixel here
-  PxPre<K> pre;
+template <typename Shape>
+__device__ __forceinline__ PxPre<Shape::K> load_models(const IcpArgs& a, int bid, int nblk, int pass) {
+  const int P = a.W * a.H, rounds = Shape::rounds();
+  PxPre<Shape::K> pre;
 #pragma unroll
-  for (int k = 0; k < K; ++k) pre.q[k] = load_model(a, i0 + k * stride < P ? i0 + k * stride : j0);
+  for (int k = 0; k < Shape::K; ++k) {
+    const int i = Shape::pixel(bid, nblk, pass, k);
+    if (k < rounds) pre.q[k] = load_model(a, i < P ? i : 0);  // pixel 0: unused
+  }
   return pre;
 }
 
-// One round of a thread's association: pixels i0 + k * stride (k < K) with model
-// samples q, their live loads in flight together, the rows accumulated in order.
-template <bool COMP, int K>
-__device__ __forceinline__ void associate_round(const IcpArgs& a, const kf_posef& wc, const kf_posef& cw, int i0,
-                                                int stride, int P, const PxModel (&q)[K], acc_t<COMP>* s,
-                                                int& n_in, int& n_cand) {
-  int j[K], r[K];
+// Block partial: this block's share of the association (K pixels per thread with their
+// loads in flight together), the sums over the block's waves, written as one slot: 28
+// terms and the inlier and candidate counts.  PRE: the first pass' samples are given.
+template <bool COMP, typename Shape, int WAVES, bool PRE = false, bool COH = false>
+__device__ __forceinline__ void block_partial(const IcpArgs& a, const kf_posef& wc, const kf_posef& cw, int bid,
+                                              int nblk, double* slot, PartialLds<WAVES, Shape::K>& lds,
+                                              PxPre<Shape::K> pre = {}) {
+  constexpr int K = Shape::K;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int P = a.W * a.H, passes = (P + nblk * Shape::kPixels - 1) / (nblk * Shape::kPixels);
+  const int rounds = Shape::rounds();
+  int n_cand = 0, n_in = 0;
+  TermSums sums;
+  float s[kPad];  // plain mode; terms 28..31 stay zero (padding for the halving)
+  if constexpr (!COMP) {
 #pragma unroll
-  for (int k = 0; k < K; ++k) {
-    j[k] = project_model(a, cw, q[k], r[k]);
-    if (i0 + k * stride >= P) {  // no pixel: contributes nothing
-      j[k] = -1;
-      r[k] = 0;
+    for (int k = 0; k < kPad; ++k) s[k] = 0.0f;
+  }
+  double (*rows)[8][kRowPitch] = lds.rows[wave];
+  for (int pass = 0; pass < passes; ++pass) {
+    if (!PRE || pass > 0) pre = load_models<Shape>(a, bid, nblk, pass);
+    int j[K], r[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (k >= rounds) continue;  // uniform
+      j[k] = project_model(a, cw, pre.q[k], r[k]);
+      if (Shape::pixel(bid, nblk, pass, k) >= P) {  // no pixel: contributes nothing
+        j[k] = -1;
+        r[k] = 0;
+      }
+    }
+    PxLive l[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (k < rounds) l[k] = load_live(a, j[k]);
+    if constexpr (COMP) wave_lds_sync();  // the previous pass' reads are done
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (k >= rounds) continue;
+      float A[6], b;
+      r[k] = finish_row(a, wc, pre.q[k], l[k], j[k], r[k], A, b);
+      const int i = Shape::pixel(bid, nblk, pass, k);
+      if (a.mask && i < P) a.mask[i] = (uint8_t)(r[k] == 2);
+      n_cand += (int)__popcll(__ballot(r[k] != 0));  // of the wave
+      // rejected pixels are zero rows: they leave the sums' bits as they are
+      const bool inl = r[k] == 2;
+#pragma unroll
+      for (int p = 0; p < 6; ++p) A[p] = inl ? A[p] : 0.0f;
+      b = inl ? b : 0.0f;
+      if constexpr (COMP) {
+#pragma unroll
+        for (int p = 0; p < 6; ++p) rows[k][p][lane] = (double)A[p];
+        rows[k][6][lane] = (double)b;
+        rows[k][7][lane] = inl ? 1.0 : 0.0;
+      } else {
+        accumulate(s, A, b);
+        n_in += (int)__popcll(__ballot(inl));
+      }
+    }
+    if constexpr (COMP) {
+      wave_lds_sync();
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+        if (k < rounds) sums.add(rows[k]);
     }
   }
-  PxLive l[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) l[k] = load_live(a, j[k]);
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    float A[6], b;
-    r[k] = finish_row(a, wc, q[k], l[k], j[k], r[k], A, b);
-    if (a.mask && i0 + k * stride < P) a.mask[i0 + k * stride] = (uint8_t)(r[k] == 2);
-    n_cand += r[k] != 0 ? 1 : 0;
-    // every lane accumulates, others a zero row: fma(0, 0, s) and s + 0 leave the
-    // sums' bits as they are (a sum that starts at +0 never becomes -0)
-    const bool inl = r[k] == 2;
-    n_in += inl ? 1 : 0;
-#pragma unroll
-    for (int p = 0; p < 6; ++p) A[p] = inl ? A[p] : 0.0f;
-    b = inl ? b : 0.0f;
-    accumulate<COMP>(s, A, b);
-  }
-}
-
-template <bool COMP, int WAVES, int K = 2, bool PRE = false, bool COH = false>
-__device__ __forceinline__ void block_partial(const IcpArgs& a, const kf_posef& wc, const kf_posef& cw, int bid,
-                                              int nblk, float* slot, PxPre<K> pre = {}) {
-  using T_ = acc_t<COMP>;
-  __shared__ T_ red_s[WAVES][kPad];
-  __shared__ int red_n[WAVES][2];
-  constexpr int T = WAVES * kWave;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  T_ s[kPad];  // terms 28..31 stay zero (padding for the halving)
-#pragma unroll
-  for (int k = 0; k < kPad; ++k) s[k] = 0;
-  int n_in = 0, n_cand = 0;
-  const int P = a.W * a.H;
-  const int stride = nblk * T;
-  int i0 = bid * T + tid;
-  if (PRE && i0 < P) {  // first round from the prefetched samples
-    associate_round<COMP, K>(a, wc, cw, i0, stride, P, pre.q, s, n_in, n_cand);
-    i0 += K * stride;
-  }
-  for (; i0 < P; i0 += K * stride) {
-    PxModel q[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) q[k] = load_model(a, i0 + k * stride < P ? i0 + k * stride : i0);
-    associate_round<COMP, K>(a, wc, cw, i0, stride, P, q, s, n_in, n_cand);
-  }
-
-  // Wave reduction by recursive halving (reduce-scatter): five pairings, each
-  // halving the terms a lane holds — row mirror (lane bit 3), half-row mirror
-  // (bit 2), quad xor 2 (bit 1), quad xor 1 (bit 0), xor 16 (bit 4) — then xor 32
-  // adds the two half-waves.  Lane l < 32 ends with the full wave sum of term
-  // 16*b3 + 8*b2 + 4*b1 + 2*b0 + b4 (b = bits of l).  About 1/5 of the work of
-  // reducing all 28 terms down the whole butterfly.
-  halve<0x140, 32>(s, (lane & 8) != 0);
-  halve<0x141, 16>(s, (lane & 4) != 0);
-  halve<0x4E, 8>(s, (lane & 2) != 0);
-  halve<0xB1, 4>(s, (lane & 1) != 0);
-  {
+  if constexpr (COMP) {
+    sums.store(lds.red[wave]);
+  } else {
+    // Wave reduction by recursive halving (reduce-scatter): five pairings, each
+    // halving the terms a lane holds — row mirror (lane bit 3), half-row mirror
+    // (bit 2), quad xor 2 (bit 1), quad xor 1 (bit 0), xor 16 (bit 4) — then xor 32
+    // adds the two half-waves.  Lane l < 32 ends with the full wave sum of term
+    // 16*b3 + 8*b2 + 4*b1 + 2*b0 + b4 (b = bits of l).
+    halve<0x140, 32>(s, (lane & 8) != 0);
+    halve<0x141, 16>(s, (lane & 4) != 0);
+    halve<0x4E, 8>(s, (lane & 2) != 0);
+    halve<0xB1, 4>(s, (lane & 1) != 0);
     const bool up = (lane & 16) != 0;
-    const T_ gs = up ? s[0] : s[1];
-    T_ ks = up ? s[1] : s[0];
+    const float gs = up ? s[0] : s[1];
+    float ks = up ? s[1] : s[0];
     ks = ks + __shfl_xor(gs, 16, kWave);
     ks = ks + __shfl_xor(ks, 32, kWave);
     const int term = ((lane & 8) << 1) | ((lane & 4) << 1) | ((lane & 2) << 1) | ((lane & 1) << 1) | ((lane >> 4) & 1);
-    if (lane < 32) red_s[wave][term] = ks;
+    if (lane < 32 && term < kTerms) lds.red[wave][term] = (double)ks;
+    if (lane == 32) lds.red[wave][kInlAt] = (double)n_in;
   }
-  n_in = wave_sum_i_lane63(n_in);
-  n_cand = wave_sum_i_lane63(n_cand);
-  if (lane == 63) {
-    red_n[wave][0] = n_in;
-    red_n[wave][1] = n_cand;
-  }
+  if (lane == 0) lds.cand[wave] = n_cand;
   __syncthreads();
-  if (tid < kTerms) {
-    T_ S = red_s[0][tid];
-    for (int w = 1; w < WAVES; ++w) S = S + red_s[w][tid];
-    const float hi = (float)S;
-    const float lo = COMP ? (float)(S - (T_)hi) : 0.0f;
-    slot_put<COH>(&slot[2 * tid], hi);
-    slot_put<COH>(&slot[2 * tid + 1], lo);
-  } else if (tid == kTerms) {
-    int ni = 0, nc = 0;
-    for (int w = 0; w < WAVES; ++w) {
-      ni += red_n[w][0];
-      nc += red_n[w][1];
+  if (tid < kWave) {
+    const int at = COMP ? term_of(lane) : (lane <= kInlAt ? lane : -1);
+    if (at >= 0) {
+      if constexpr (COMP) {
+        double S = lds.red[0][lane];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) S = S + lds.red[w][lane];
+        slot_put<COH>(&slot[at], S);
+      } else {  // FP32 sums
+        float S = (float)lds.red[0][lane];
+        for (int w = 1; w < WAVES; ++w) S = S + (float)lds.red[w][lane];
+        slot_put<COH>(&slot[at], (double)S);
+      }
     }
-    slot_put<COH>(&slot[56], __int_as_float(ni));
-    slot_put<COH>(&slot[57], __int_as_float(nc));
-    slot_put<COH>(&slot[kStopAt], __int_as_float(0));
+  } else if (tid == kWave) {
+    int nc = 0;
+    for (int w = 0; w < WAVES; ++w) nc += lds.cand[w];
+    slot_put<COH>(&slot[kCandAt], (double)nc);
+    slot_put<COH>(&slot[kStopAt], 0.0);
   }
 }
 
-// FP64 sum of nb slots into sum[kSums] (LDS, valid after the call for every
-// thread): the 28 terms, inliers, candidates and the number of stopped blocks.
-// Thread (g, j) reads float4 j of the slots of blocks g, g + G, ... (j < 14: terms
-// 2j, 2j + 1 as (hi, lo) pairs; j = 14: the counts) with kFinUnroll loads in
-// flight; the group totals are combined in a fixed order (lane shuffles within a
-// wave, then the waves in order).
-// Split in two so that a caller can issue the first round of slot loads before
-// other loads (loads complete in issue order) and consume them later.  COH: the
-// slots are read with slot_get4<true> (written across a grid barrier).
+// x of the lane 16 (32) away added to this lane's (v_permlane16_swap / 32_swap: the two
+// results are the lower and the upper rows' values in every lane).
+__device__ __forceinline__ double add_rows16(double x) {
+  const uint2 u = __builtin_bit_cast(uint2, x);
+  const auto lo = __builtin_amdgcn_permlane16_swap(u.x, u.x, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(u.y, u.y, false, false);
+  return __builtin_bit_cast(double, make_uint2(lo[0], hi[0])) + __builtin_bit_cast(double, make_uint2(lo[1], hi[1]));
+}
+__device__ __forceinline__ double add_rows32(double x) {
+  const uint2 u = __builtin_bit_cast(uint2, x);
+  const auto lo = __builtin_amdgcn_permlane32_swap(u.x, u.x, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(u.y, u.y, false, false);
+  return __builtin_bit_cast(double, make_uint2(lo[0], hi[0])) + __builtin_bit_cast(double, make_uint2(lo[1], hi[1]));
+}
+
+// FP64 sum of nb slots: thread (g, j) reads doubles 2j, 2j + 1 of slots g, g + G, ...
+// with kFinUnroll loads in flight; the groups of a wave are added by lane moves and
+// each wave leaves its 32 sums in fin[wave] (publish with a barrier, then
+// wave_totals).  Split in two so that a caller can issue the first round of slot loads
+// before other loads (loads complete in issue order) and consume them later.  COH: the
+// slots were written across a grid barrier.
+template <int THREADS>
+struct SlotFin {
+  double w[THREADS / kWave][kSlot];
+};
+
 template <int THREADS, bool COH = false>
 struct SlotSum {
   static constexpr int G = THREADS / 16;
-  float4 v[kFinUnroll];
-  // The first round of loads (blocks g, g + G, ..., g + (kFinUnroll - 1) G; nb >= 1).
+  double2 v[kFinUnroll];
+  // The first round of loads (slots g, g + G, ..., g + (kFinUnroll - 1) G; nb >= 1).
   // Unconditional, from clamped in-bounds addresses, so that nothing waits for
-  // them here; finish() drops the out-of-range ones.
-  __device__ __forceinline__ void load(const float* slots, int nb) {
-    const int tid = threadIdx.x;
-    const int j = tid & 15, g = tid >> 4;
-    const float4* base = reinterpret_cast<const float4*>(slots) + (j < 15 ? j : 0);
+  // them here; reduce() drops the out-of-range ones.
+  __device__ __forceinline__ void load(const double* slots, int nb) {
+    const int j = threadIdx.x & 15, g = threadIdx.x >> 4;
+    const double2* base = reinterpret_cast<const double2*>(slots) + j;
 #pragma unroll
-    for (int u = 0; u < kFinUnroll; ++u) v[u] = slot_get4<COH>(base + (size_t)min(g + G * u, nb - 1) * (kSlot / 4));
+    for (int u = 0; u < kFinUnroll; ++u) v[u] = slot_get2<COH>(base + (size_t)min(g + G * u, nb - 1) * (kSlot / 2));
   }
-  __device__ __forceinline__ void finish(const float* slots, int nb, double* sum);
-};
-
-template <int THREADS, bool COH>
-__device__ __forceinline__ void SlotSum<THREADS, COH>::finish(const float* slots, int nb, double* sum) {
-  constexpr int WV = THREADS / kWave;
-  __shared__ double fin[WV][kSums];
-  const int tid = threadIdx.x;
-  const int j = tid & 15, g = tid >> 4;
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-  if (j < 15) {
-    const float4* base = reinterpret_cast<const float4*>(slots) + j;
-    for (int b0 = g; b0 < nb; b0 += G * kFinUnroll) {
-      if (b0 != g) {
-#pragma unroll
-        for (int u = 0; u < kFinUnroll; ++u) v[u] = slot_get4<COH>(base + (size_t)min(b0 + G * u, nb - 1) * (kSlot / 4));
-      }
+  __device__ __forceinline__ void reduce(const double* slots, int nb, SlotFin<THREADS>& fin) {
+    const int tid = threadIdx.x, j = tid & 15, g = tid >> 4;
+    const double2* base = reinterpret_cast<const double2*>(slots) + j;
+    double a0 = 0.0, a1 = 0.0;
+    for (int b0 = g;;) {
 #pragma unroll
       for (int u = 0; u < kFinUnroll; ++u) {
-        if (b0 + G * u >= nb) v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        // one path for every lane: term lanes add (hi, lo) pairs, the count lane
-        // (j = 14) adds its three integers with +0 in the pairs' second places
-        // (x + 0 = x: a sum that starts at +0 never becomes -0)
-        const bool cnt = j == 14;
-        const double x = cnt ? (double)__float_as_int(v[u].x) : (double)v[u].x;
-        const double y = cnt ? 0.0 : (double)v[u].y;
-        const double z = cnt ? (double)__float_as_int(v[u].y) : (double)v[u].z;
-        const double w = cnt ? 0.0 : (double)v[u].w;
-        a0 = (a0 + x) + y;
-        a1 = (a1 + z) + w;
-        a2 = a2 + (cnt ? (double)__float_as_int(v[u].z) : 0.0);
+        const bool in = b0 + G * u < nb;
+        a0 = a0 + (in ? v[u].x : 0.0);
+        a1 = a1 + (in ? v[u].y : 0.0);
       }
+      b0 += G * kFinUnroll;
+      if (b0 - g >= nb) break;  // uniform
+#pragma unroll
+      for (int u = 0; u < kFinUnroll; ++u) v[u] = slot_get2<COH>(base + (size_t)min(b0 + G * u, nb - 1) * (kSlot / 2));
+    }
+    a0 = add_rows32(add_rows16(a0));
+    a1 = add_rows32(add_rows16(a1));
+    if ((tid & 63) < 16) {
+      fin.w[tid >> 6][2 * j] = a0;
+      fin.w[tid >> 6][2 * j + 1] = a1;
     }
   }
-  // the four groups of a wave (lanes j, j+16, j+32, j+48), then the waves in order
-  a0 = a0 + __shfl_xor(a0, 16, kWave);
-  a1 = a1 + __shfl_xor(a1, 16, kWave);
-  a0 = a0 + __shfl_xor(a0, 32, kWave);
-  a1 = a1 + __shfl_xor(a1, 32, kWave);
-  a2 = a2 + __shfl_xor(a2, 16, kWave);
-  a2 = a2 + __shfl_xor(a2, 32, kWave);
-  if ((tid & 63) < 15) {
-    fin[tid >> 6][2 * j] = a0;
-    fin[tid >> 6][2 * j + 1] = a1;
-  }
-  if ((tid & 63) == 14) fin[tid >> 6][kTerms + 2] = a2;
-  __syncthreads();
-  if (tid < kSums) {
-    double t = fin[0][tid];
-    for (int w = 1; w < WV; ++w) t = t + fin[w][tid];
-    sum[tid] = t;
-  }
-  __syncthreads();
-}
+};
 
+// Slot sum lane % 32, from the waves' sums in order (any wave, after the barrier).
 template <int THREADS>
-__device__ __forceinline__ void sum_slots(const float* slots, int nb, double* sum) {
-  SlotSum<THREADS> L;
-  L.load(slots, nb);
-  L.finish(slots, nb, sum);
+__device__ __forceinline__ double wave_totals(const SlotFin<THREADS>& fin) {
+  const int t = threadIdx.x & (kSlot - 1);
+  double s = fin.w[0][t];
+#pragma unroll
+  for (int w = 1; w < THREADS / kWave; ++w) s = s + fin.w[w][t];
+  return s;
 }
 
 // Lane l's value of v, in every lane (v_readlane: no LDS round trip).
@@ -445,44 +488,49 @@ __device__ __forceinline__ double lane_value(double v, int l) {
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// Solve (A^T A) x = A^T b from sum[30] and compose the Euler-ZYX increment onto
-// Tin (LDS, 16 doubles): Tout (LDS) and the FP32 fields wc / cw (LDS).  Returns
-// false for a singular system (fewer than kMinInliers inliers or an LDL^T pivot
-// not above 1e-9 x the largest diagonal); then the outputs are untouched.  With
-// `st`, the level statistics are written and, when singular, status 1.
-// Called by the whole block; the first wavefront computes, in three stages
-// joined by lane broadcasts (v_readlane) rather than LDS: lane 0 solves with the
-// square-root-free factorisation shared with the host (ldlt_solve6, its system in
-// registers: a 6x6 solve is a short dependent chain); lanes 0..2 take the sine and
-// cosine of one angle each; lane 4i + j forms entry (i, j) of the product with
-// the expressions of the serial helpers, and the FP32 field(s) that entry gives.
-// The statistics (a division and a square root) are written by the second
-// wavefront meanwhile; the final barrier publishes everything.
-__device__ __forceinline__ bool solve_compose(const double* sum, const double* Tin, kf_icp_stats* st, int level,
+// Solve (A^T A) x = A^T b from the slot sums in fin (published) and compose the
+// Euler-ZYX increment onto Tin (LDS, 16 doubles): Tout (LDS) and the FP32 fields
+// wc / cw (LDS).  Returns false, with the outputs untouched, when an earlier solve was
+// singular (a block stopped) or this one is (fewer than kMinInliers inliers or an
+// LDL^T pivot not above 1e-9 x the largest diagonal).  With `st`, the level statistics
+// are written and, when this system is singular, status 1.
+// Called by the whole block; the first wavefront computes, as one chain of dependent
+// FP64 operations: every lane solves with the square-root-free factorisation shared with
+// the host (ldlt_solve6: no branch, and no broadcast of the solution after it), lanes
+// 0..2 take the sine and cosine of one angle each (v_readlane), lane 4i + j forms entry
+// (i, j) of the product with the expressions of the serial helpers, and the FP32
+// field(s) that entry gives; the rigid inverse's translation sums down the columns by
+// DPP row shifts.  The statistics (a division and a square root) are written by the
+// second wavefront meanwhile; the final barrier publishes everything.  3.1 k cycles from
+// the slot sums to the barrier against 4.1 k with lane 0 alone in the factorisation, IEEE
+// divisions and 24 lane broadcasts for the inverse.
+template <int THREADS>
+__device__ __forceinline__ bool solve_compose(const SlotFin<THREADS>& fin, const double* Tin, kf_icp_stats* st, int level,
                                               double* Tout, kf_posef* wc, kf_posef* cw) {
   __shared__ int tok;
+  __shared__ __align__(16) double sum[kSlot];
   const int tid = threadIdx.x;
   if (tid < kWave) {
     const int lane = tid;
     const int i = (lane >> 2) & 3, j = lane & 3;
     // this lane's column of Tin (for the product), loaded before the solve
     const double b0 = Tin[j], b1 = Tin[4 + j], b2 = Tin[8 + j], b3 = Tin[12 + j];
-    double x[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    int ok = 0;
+    const double tot = wave_totals(fin);
+    if (lane < kSlot) sum[lane] = tot;
+    wave_lds_sync();
+    double up[21], g[6], x[6];
+#pragma unroll
+    for (int q = 0; q < 21; ++q) up[q] = sum[q];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) g[q] = sum[21 + q];
+    const bool stopped = sum[kStopAt] != 0.0, few = (int)sum[kInlAt] < kMinInliers;
+    const bool solved = ldlt_solve6(up, g, kPivotRelEps, x) && !few;
+    const int ok = __builtin_amdgcn_readfirstlane(!stopped && solved ? 1 : 0);  // every lane agrees
     if (lane == 0) {
-      double up[21], g[6];
-#pragma unroll
-      for (int q = 0; q < 21; ++q) up[q] = sum[q];
-#pragma unroll
-      for (int q = 0; q < 6; ++q) g[q] = sum[21 + q];
-      ok = ((int)sum[28] >= kMinInliers && ldlt_solve6(up, g, kPivotRelEps, x)) ? 1 : 0;
       tok = ok;
-      if (!ok && st) st->status = 1;
+      if (!stopped && !ok && st) st->status = 1;
     }
-    ok = __builtin_amdgcn_readlane(ok, 0);
     if (ok) {  // uniform
-#pragma unroll
-      for (int q = 0; q < 6; ++q) x[q] = lane_value(x[q], 0);
       // lanes 0, 1, 2: the angle of their axis (the rotation is the negated solution)
       const double ang = -(lane == 0 ? x[0] : (lane == 1 ? x[1] : x[2]));
       double cl, sl;
@@ -510,23 +558,24 @@ __device__ __forceinline__ bool solve_compose(const double* sum, const double* T
           wc->t[i] = f;
         }
       }
-      double Tu[12];
-#pragma unroll
-      for (int e = 0; e < 12; ++e) Tu[e] = lane_value(t, e);
-      if (lane < 3) {
-        const double r0 = rigid_inverse_t(Tu, 0), r1 = rigid_inverse_t(Tu, 1), r2 = rigid_inverse_t(Tu, 2);
-        cw->t[lane] = (float)(lane == 0 ? r0 : (lane == 1 ? r1 : r2));
-      }
+      // -(R^T t), rows 0..2 in rigid_inverse_t's order: R(i, c) t_i, t_i from the quad's
+      // last lane, then rows 1 and 2 of the column from 4 and 8 lanes up
+      const double p = t * dpp_d<0xFF>(t);
+      const double r = (p + dpp_d<0x104>(p)) + dpp_d<0x108>(p);
+      if (lane < 3) cw->t[lane] = (float)-r;
     }
-  } else if (tid == kWave && st) {
-    const double inl = sum[28];
-    const int ni = (int)inl;
-    const double rms = ni > 0 ? sqrt(sum[27] / inl) : 0.0;
-    st->inliers = ni;
-    st->candidates = (int)sum[29];
-    st->residual_rms = rms;
-    st->level_residual[level] = rms;
-    st->level_inliers[level] = ni;
+  } else if (tid < 2 * kWave && st) {
+    const double tot = wave_totals(fin);
+    const double b2 = lane_value(tot, 27), inl = lane_value(tot, kInlAt), cand = lane_value(tot, kCandAt);
+    if (tid == kWave && lane_value(tot, kStopAt) == 0.0) {
+      const int ni = (int)inl;
+      const double rms = ni > 0 ? sqrt(b2 / inl) : 0.0;
+      st->inliers = ni;
+      st->candidates = (int)cand;
+      st->residual_rms = rms;
+      st->level_residual[level] = rms;
+      st->level_inliers[level] = ni;
+    }
   }
   __syncthreads();
   return tok != 0;  // uniform
@@ -543,15 +592,21 @@ __device__ __forceinline__ void copy_pose(const kf_pose* src, kf_pose* dst) {
 // Reduce mode (kf_icp_reduce), pass 1: the block partials at a fixed pose.
 template <bool COMP>
 __global__ __launch_bounds__(kThreads) void icp_partials(IcpArgs a) {
+  using Shape = PixelShape<kThreads / kWave, 2, 0>;
+  __shared__ PartialLds<kThreads / kWave, Shape::K> lds;
   const kf_posef wc = a.pose->wc, cw = a.pose->cw;
-  block_partial<COMP, kThreads / kWave>(a, wc, cw, blockIdx.x, gridDim.x, a.partials + (size_t)blockIdx.x * kSlot);
+  block_partial<COMP, Shape>(a, wc, cw, blockIdx.x, gridDim.x, a.partials + (size_t)blockIdx.x * kSlot, lds);
 }
 
 // Reduce mode, pass 2 (one block): the FP64 sums.
 __global__ __launch_bounds__(kSolveThreads) void icp_sums(IcpArgs a, int nb) {
-  __shared__ double sum[kSums];
-  sum_slots<kSolveThreads>(a.partials, nb, sum);
-  if ((int)threadIdx.x < kTerms + 2) a.sums_out[threadIdx.x] = sum[threadIdx.x];
+  __shared__ SlotFin<kSolveThreads> fin;
+  SlotSum<kSolveThreads> slots;
+  slots.load(a.partials, nb);
+  slots.reduce(a.partials, nb, fin);
+  __syncthreads();
+  const double tot = wave_totals(fin);
+  if ((int)threadIdx.x < kTerms + 2) a.sums_out[threadIdx.x] = tot;
 }
 
 // Tracking: one launch per iteration.  Every block first solves the previous
@@ -564,8 +619,8 @@ __global__ __launch_bounds__(kSolveThreads) void icp_sums(IcpArgs a, int nb) {
 struct StepArgs {
   const kf_pose* pose_in;   // the guess (first step) or the previous step's output
   kf_pose* pose_out;
-  const float* slots_in;    // previous step's slots (unused for the first step)
-  float* slots_out;
+  const double* slots_in;   // previous step's slots (unused for the first step)
+  double* slots_out;
   int nb_in;                // number of slots in slots_in
   int level_in;             // level of the previous step
   int first;
@@ -575,14 +630,20 @@ struct StepArgs {
   kf_icp_stats* st;
 };
 
-// K: pixels per thread at this level's grid (the model samples of all of them are
-// loaded before the solve).
-template <bool COMP, int K>
+// F, H: the pixels a thread takes at this level's grid (PixelShape; the model samples of
+// all of them are loaded before the solve).
+template <int F, int H>
+using StepShape = PixelShape<kStepThreads / kWave, F, H>;
+
+template <bool COMP, int F, int H>
 __global__ __launch_bounds__(kStepThreads) void icp_step(IcpArgs a, StepArgs S) {
-  __shared__ double sum[kSums], Tin[16], Tnew[16];
+  __shared__ double Tin[16], Tnew[16];
   __shared__ kf_posef s_wc, s_cw;
+  __shared__ SlotFin<kStepThreads> fin;
+  using Shape = StepShape<F, H>;
+  __shared__ PartialLds<kStepThreads / kWave, Shape::K> lds;
   const int tid = threadIdx.x;
-  float* slot_out = S.slots_out + (size_t)blockIdx.x * kSlot;
+  double* slot_out = S.slots_out + (size_t)blockIdx.x * kSlot;
   // Every load that does not depend on another is issued up front, in the order
   // they are needed (loads complete in issue order): the previous step's slots
   // and pose, then the model samples.  No flag is read before them: a singular
@@ -593,7 +654,7 @@ __global__ __launch_bounds__(kStepThreads) void icp_step(IcpArgs a, StepArgs S) 
     slots_in.load(S.slots_in, S.nb_in);
     tin = S.pose_in->T_wc[tid & 15];
   }
-  const PxPre<K> pre = prefetch_models<kStepThreads / kWave, K>(a, blockIdx.x, gridDim.x);
+  const PxPre<Shape::K> pre = load_models<Shape>(a, blockIdx.x, gridDim.x, 0);
   if (S.first) {
     if (tid < 12) {
       if (tid < 9) s_wc.r[tid] = S.pose_in->wc.r[tid];
@@ -611,16 +672,14 @@ __global__ __launch_bounds__(kStepThreads) void icp_step(IcpArgs a, StepArgs S) 
       }
     }
   } else {
-    slots_in.finish(S.slots_in, S.nb_in, sum);
+    slots_in.reduce(S.slots_in, S.nb_in, fin);
     if (tid < 16) Tin[tid] = tin;
     __syncthreads();
     // an earlier solve was singular (a previous block stopped), or this one is:
     // keep the pose and pass the stop on
-    bool ok = sum[kTerms + 2] == 0.0;  // uniform
-    if (ok) ok = solve_compose(sum, Tin, blockIdx.x == 0 ? S.st : nullptr, S.level_in, Tnew, &s_wc, &s_cw);
-    if (!ok) {
+    if (!solve_compose(fin, Tin, blockIdx.x == 0 ? S.st : nullptr, S.level_in, Tnew, &s_wc, &s_cw)) {
       if (blockIdx.x == 0) copy_pose(S.pose_in, S.pose_out);
-      if (tid == 0) slot_out[kStopAt] = __int_as_float(1);
+      if (tid == 0) slot_out[kStopAt] = 1.0;
       return;  // uniform
     }
     if (blockIdx.x == 0) {
@@ -638,7 +697,7 @@ __global__ __launch_bounds__(kStepThreads) void icp_step(IcpArgs a, StepArgs S) 
     }
   }
   __syncthreads();
-  block_partial<COMP, kStepThreads / kWave, K, true>(a, s_wc, s_cw, blockIdx.x, gridDim.x, slot_out, pre);
+  block_partial<COMP, Shape, kStepThreads / kWave, true>(a, s_wc, s_cw, blockIdx.x, gridDim.x, slot_out, lds, pre);
 }
 
 // Acceptance test of the finished call (IcpGate), from the window count and thread
@@ -685,7 +744,8 @@ __device__ void gate_decide(const IcpGate& g, int count, double wv, const kf_icp
 __global__ __launch_bounds__(kSolveThreads) void icp_finish(IcpArgs a, StepArgs S, int steps, kf_pose* out,
                                                             kf_icp_stats* user, IcpGate gate, int gated,
                                                             FrameEnd fe, int fe_on) {
-  __shared__ double sum[kSums], Tin[16];
+  __shared__ double Tin[16];
+  __shared__ SlotFin<kSolveThreads> fin;
   // The call's statistics and output pose are assembled in LDS and stored once; the
   // acceptance test reads them there instead of back from memory.
   __shared__ kf_icp_stats s_st;
@@ -724,11 +784,10 @@ __global__ __launch_bounds__(kSolveThreads) void icp_finish(IcpArgs a, StepArgs 
     if (tid == 32) a.ctrl->executed = 0;
     __syncthreads();
   } else {
-    slots_in.finish(S.slots_in, S.nb_in, sum);  // its barriers also publish s_st and s_out
+    slots_in.reduce(S.slots_in, S.nb_in, fin);
     if (tid < 16) Tin[tid] = tin;
-    __syncthreads();
-    ok = sum[kTerms + 2] == 0.0;  // no earlier solve was singular (uniform)
-    if (ok) ok = solve_compose(sum, Tin, &s_st, S.level_in, s_out.T_wc, &s_out.wc, &s_out.cw);
+    __syncthreads();  // also publishes s_st and s_out
+    ok = solve_compose(fin, Tin, &s_st, S.level_in, s_out.T_wc, &s_out.wc, &s_out.cw);
     if (ok && tid == 192) a.ctrl->executed = steps;
   }
   // iterations = updates applied: every step's when the last solve succeeded, else
@@ -780,10 +839,10 @@ struct ChainArgs {
   int levels;
   int iters[KF_MAX_LEVELS];
   int blocks[KF_MAX_LEVELS];  // step grid (slot count) per level, as in the multi-launch chain
-  int ppt[KF_MAX_LEVELS];     // pixels per thread of that grid (4 or 1), as in the multi-launch chain
+  int shape[KF_MAX_LEVELS];   // pixels per thread of that grid (step_shape), as in the multi-launch chain
   const kf_pose* guess;
   kf_pose* out;
-  float* slots[2];
+  double* slots[2];
   kf_icp_stats* user;  // skip flag; receives a copy of the statistics
   kf_icp_stats* st;
   kf_icp_ctrl* ctrl;
@@ -847,40 +906,46 @@ __device__ __forceinline__ bool grid_barrier(kf_icp_ctrl* ctrl, unsigned target,
   return s_ok != 0;
 }
 
-// One iteration of the chain at a level whose step grid has nb blocks of K pixels
-// per thread (as icp_step<COMP, K>): the slot loads of the previous iteration
+// One iteration of the chain at a level whose step grid has nb blocks of Shape's pixels
+// (as icp_step): the slot loads of the previous iteration
 // (solve = true; nb_in slots of level lvl_in), then this block's model samples, both
 // in flight together; the sum, solve and composition onto T[cur]; this block's
 // slots.  Returns false (uniform) when the solve was singular: nothing is written.
-template <bool COMP, int K>
-__device__ __forceinline__ bool chain_iteration(const IcpArgs& a, int nb, bool solve, const float* slots_in,
-                                                int nb_in, int lvl_in, float* slots_out, double* sum,
+template <bool COMP, typename Shape>
+__device__ __forceinline__ bool chain_iteration(const IcpArgs& a, int nb, bool solve, const double* slots_in,
+                                                int nb_in, int lvl_in, double* slots_out,
+                                                SlotFin<kStepThreads>& fin, PartialLds<kStepThreads / kWave, 3>& lds3,
                                                 double (*T)[16], int& cur, kf_posef* wc, kf_posef* cw,
                                                 kf_icp_stats* st) {
   constexpr int WV = kStepThreads / kWave;
+  auto& lds = reinterpret_cast<PartialLds<WV, Shape::K>&>(lds3);  // room for the largest shape
+  static_assert(Shape::K <= 3, "chain LDS");
   SlotSum<kStepThreads, true> L;
   if (solve) L.load(slots_in, nb_in);
   const bool mine = (int)blockIdx.x < nb;
-  PxPre<K> pre = {};
-  if (mine) pre = prefetch_models<WV, K>(a, blockIdx.x, nb);
+  PxPre<Shape::K> pre = {};
+  if (mine) pre = load_models<Shape>(a, blockIdx.x, nb, 0);
   if (solve) {
-    L.finish(slots_in, nb_in, sum);
-    if (!solve_compose(sum, T[cur], st, lvl_in, T[cur ^ 1], wc, cw)) return false;
+    L.reduce(slots_in, nb_in, fin);
+    __syncthreads();
+    if (!solve_compose(fin, T[cur], st, lvl_in, T[cur ^ 1], wc, cw)) return false;
     cur ^= 1;
   }
   __syncthreads();
-  if (mine) block_partial<COMP, WV, K, true, true>(a, *wc, *cw, blockIdx.x, nb, slots_out + (size_t)blockIdx.x * kSlot, pre);
+  if (mine) block_partial<COMP, Shape, WV, true, true>(a, *wc, *cw, blockIdx.x, nb, slots_out + (size_t)blockIdx.x * kSlot, lds, pre);
   for (int vb = blockIdx.x + gridDim.x; vb < nb; vb += gridDim.x) {
     __syncthreads();
-    block_partial<COMP, WV, K, false, true>(a, *wc, *cw, vb, nb, slots_out + (size_t)vb * kSlot);
+    block_partial<COMP, Shape, WV, false, true>(a, *wc, *cw, vb, nb, slots_out + (size_t)vb * kSlot, lds);
   }
   return true;
 }
 
 template <bool COMP>
 __global__ __launch_bounds__(kStepThreads) void icp_chain(ChainArgs C) {
-  __shared__ double sum[kSums], T[2][16];
+  __shared__ double T[2][16];
   __shared__ kf_posef s_wc, s_cw;
+  __shared__ SlotFin<kStepThreads> fin;
+  __shared__ PartialLds<kStepThreads / kWave, 3> lds;
   const int tid = threadIdx.x;
   const bool lead = blockIdx.x == 0;
   if (C.user && C.user->skip) {  // uniform
@@ -941,11 +1006,17 @@ __global__ __launch_bounds__(kStepThreads) void icp_chain(ChainArgs C) {
     for (int it = 0; it < C.iters[l]; ++it) {
       const bool solve = steps > 0;
       kf_icp_stats* sp = lead ? st : nullptr;
-      const bool ok = C.ppt[l] == kPpt0
-          ? chain_iteration<COMP, kPpt0>(a, nb, solve, C.slots[par ^ 1], nb_prev, lvl_prev, C.slots[par], sum, T, cur,
-                                     &s_wc, &s_cw, sp)
-          : chain_iteration<COMP, 1>(a, nb, solve, C.slots[par ^ 1], nb_prev, lvl_prev, C.slots[par], sum, T, cur,
-                                     &s_wc, &s_cw, sp);
+      auto iterate = [&](auto shape) {
+        return chain_iteration<COMP, decltype(shape)>(a, nb, solve, C.slots[par ^ 1], nb_prev, lvl_prev, C.slots[par], fin,
+                                                      lds, T, cur, &s_wc, &s_cw, sp);
+      };
+      bool ok;
+      switch (C.shape[l]) {  // uniform
+        case 0: ok = iterate(StepShape<0, 1>{}); break;
+        case 1: ok = iterate(StepShape<1, 0>{}); break;
+        case 2: ok = iterate(StepShape<2, 1>{}); break;
+        default: ok = iterate(StepShape<3, 0>{}); break;
+      }
       if (!ok) {
         stop = true;  // uniform: every block solved the same system
         break;
@@ -964,8 +1035,9 @@ __global__ __launch_bounds__(kStepThreads) void icp_chain(ChainArgs C) {
   if (!stop && steps > 0) {  // the last iteration's update (as icp_finish)
     SlotSum<kStepThreads, true> L;
     L.load(C.slots[par ^ 1], nb_prev);
-    L.finish(C.slots[par ^ 1], nb_prev, sum);
-    if (solve_compose(sum, T[cur], lead ? st : nullptr, lvl_prev, T[cur ^ 1], &s_wc, &s_cw)) {
+    L.reduce(C.slots[par ^ 1], nb_prev, fin);
+    __syncthreads();
+    if (solve_compose(fin, T[cur], lead ? st : nullptr, lvl_prev, T[cur ^ 1], &s_wc, &s_cw)) {
       cur ^= 1;
       ++executed;
     }
@@ -1010,6 +1082,15 @@ __global__ void pose_copy(const kf_pose* src, kf_pose* dst) {
   if (threadIdx.x == 0) *dst = *src;
 }
 
+// The smallest float whose square root (correctly rounded, so monotone) is not below
+// thr: sqrtf(x) < thr exactly where x < square_gate(thr).
+float square_gate(float thr) {
+  float x = thr * thr;
+  while (x > 0.0f && sqrtf(x) >= thr) x = nextafterf(x, 0.0f);
+  while (sqrtf(x) < thr) x = nextafterf(x, INFINITY);
+  return x;
+}
+
 IcpArgs level_args(const kf_tracker* t, int l, const kf_frame_maps& live, const kf_frame_maps& model) {
   IcpArgs a = {};
   const kf_level_maps& L = live.level[l];
@@ -1023,7 +1104,7 @@ IcpArgs level_args(const kf_tracker* t, int l, const kf_frame_maps& live, const 
   a.fy = kl.fy;
   a.cx = kl.cx;
   a.cy = kl.cy;
-  a.dist_thr = t->params.dist_thresh_m;
+  a.dist_thr2 = square_gate(t->params.dist_thresh_m);
   a.cos_thr = (float)cos((double)t->params.normal_thresh_deg * 3.14159265358979323846 / 180.0);
   a.partials = t->d_partials;
   a.ctrl = t->d_ctrl;
@@ -1031,14 +1112,33 @@ IcpArgs level_args(const kf_tracker* t, int l, const kf_frame_maps& live, const 
   return a;
 }
 
-// Tracking steps: 512-thread blocks, 3 pixels per thread at level 0 (200 blocks at
-// 640x480) and 1 below (150 / 38 blocks): on the coarse levels more blocks beat more
-// pixels per thread.
-int step_ppt(int l) { return l == 0 ? kPpt0 : 1; }
+// Pixels of a tracking step's 512-thread block by the level's size, so that one block per
+// CU (256) covers the level and no SIMD has more pixels than it must: half a block's waves
+// take one pixel per thread up to 65,536 pixels (level 2 of 640x480: 75 blocks, one wave
+// per SIMD), all of them up to 131,072 (level 1: 150), two and a half pixels per thread up
+// to 327,680 (level 0: 240), three beyond (the fewest slots; a step's block sums them all).
+// A step inside the kernel: levels 2 and 1 of 640x480 4.0 us, level 0 6.3 us (7.75 with
+// 200 blocks of three pixels a thread and the per-thread sums, 5.6 below); 1024-thread
+// blocks 5.9 us at level 0 but 4.5 below.
+constexpr int kShapes = 4;
+constexpr int kShapePixels[kShapes] = {StepShape<0, 1>::kPixels, StepShape<1, 0>::kPixels, StepShape<2, 1>::kPixels,
+                                       StepShape<3, 0>::kPixels};
+int step_shape(int W, int H) {
+  int k = 0;
+  while (k + 1 < kShapes && W * H > 256 * kShapePixels[k]) ++k;
+  return k;
+}
 
-int step_blocks(const kf_tracker* t, int W, int H, int l) {
-  int b = div_up(W * H, kStepThreads * step_ppt(l));
+int step_blocks(const kf_tracker* t, int W, int H) {
+  const int b = div_up(W * H, kShapePixels[step_shape(W, H)]);
   return b < t->max_blocks ? b : t->max_blocks;
+}
+
+template <bool COMP>
+void launch_step(int shape, int blocks, hipStream_t s, const IcpArgs& a, const StepArgs& S) {
+  auto kern = shape == 0 ? icp_step<COMP, 0, 1> : shape == 1 ? icp_step<COMP, 1, 0> : shape == 2 ? icp_step<COMP, 2, 1>
+                                                                                                : icp_step<COMP, 3, 0>;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kStepThreads), 0, s, a, S);
 }
 
 int level_blocks(const kf_tracker* t, int W, int H, int l) {
@@ -1071,7 +1171,7 @@ kf_status launch_icp_track(kf_tracker* t, const kf_frame_maps& live, const kf_fr
   const kf_icp_params& p = t->params;
   KF_TRY(check_maps(t, live, model, p.levels));
   kf_icp_stats* st = t->d_stats_tmp;
-  float* slots[2] = {t->d_partials, t->d_partials + (size_t)t->max_blocks * kSlot};
+  double* slots[2] = {t->d_partials, t->d_partials + (size_t)t->max_blocks * kSlot};
   if (single_launch || p.single_launch) {
     ChainArgs C = {};
     C.levels = p.levels;
@@ -1079,8 +1179,8 @@ kf_status launch_icp_track(kf_tracker* t, const kf_frame_maps& live, const kf_fr
     for (int l = 0; l < p.levels; ++l) {
       C.lv[l] = level_args(t, l, live, model);
       C.iters[l] = p.iterations[l];
-      C.blocks[l] = step_blocks(t, C.lv[l].W, C.lv[l].H, l);
-      C.ppt[l] = step_ppt(l);
+      C.blocks[l] = step_blocks(t, C.lv[l].W, C.lv[l].H);
+      C.shape[l] = step_shape(C.lv[l].W, C.lv[l].H);
       if (C.iters[l] > 0 && C.blocks[l] > grid) grid = C.blocks[l];
     }
     if (t->chain_capacity < 0) {  // blocks of this kernel that can be resident at once
@@ -1120,7 +1220,7 @@ kf_status launch_icp_track(kf_tracker* t, const kf_frame_maps& live, const kf_fr
   IcpArgs a = {};
   for (int l = p.levels - 1; l >= 0; --l) {
     a = level_args(t, l, live, model);
-    const int blocks = step_blocks(t, a.W, a.H, l);
+    const int blocks = step_blocks(t, a.W, a.H), shape = step_shape(a.W, a.H);
     for (int it = 0; it < p.iterations[l]; ++it, ++step) {
       S.first = step == 0 ? 1 : 0;
       S.index = step;
@@ -1129,14 +1229,8 @@ kf_status launch_icp_track(kf_tracker* t, const kf_frame_maps& live, const kf_fr
       S.slots_out = slots[step & 1];
       S.nb_in = prev_blocks;
       S.level_in = prev_level;
-      const int K = step_ppt(l);
-      if (p.compensated) {
-        if (K == kPpt0) hipLaunchKernelGGL((icp_step<true, kPpt0>), dim3(blocks), dim3(kStepThreads), 0, s, a, S);
-        else hipLaunchKernelGGL((icp_step<true, 1>), dim3(blocks), dim3(kStepThreads), 0, s, a, S);
-      } else {
-        if (K == kPpt0) hipLaunchKernelGGL((icp_step<false, kPpt0>), dim3(blocks), dim3(kStepThreads), 0, s, a, S);
-        else hipLaunchKernelGGL((icp_step<false, 1>), dim3(blocks), dim3(kStepThreads), 0, s, a, S);
-      }
+      if (p.compensated) launch_step<true>(shape, blocks, s, a, S);
+      else launch_step<false>(shape, blocks, s, a, S);
       KF_TRY(check_launch("icp_step"));
       S.pose_in = S.pose_out;
       prev_blocks = blocks;
@@ -1200,7 +1294,7 @@ namespace {
 
 constexpr int kNoAllocSlots = KF_ICP_NOALLOC_MAX_SLOTS;
 struct NoAllocScratch {
-  float slots[2 * kNoAllocSlots * kSlot];
+  double slots[2 * kNoAllocSlots * kSlot];
   kf_icp_ctrl ctrl;
   kf_pose work[2];
   kf_icp_stats stats;
@@ -1243,7 +1337,7 @@ kf_status launch_icp_track_noalloc(const kf_intrinsics& k0, const kf_icp_params&
   for (int l = 0; l < p.levels; ++l) {
     if (p.iterations[l] == 0) continue;
     const kf_intrinsics kl = kf_intrinsics_level(&k0, l);
-    KF_CHECK_ARG(div_up(kl.width * kl.height, kStepThreads * step_ppt(l)) <= kNoAllocSlots,
+    KF_CHECK_ARG(div_up(kl.width * kl.height, kShapePixels[step_shape(kl.width, kl.height)]) <= kNoAllocSlots,
                  "image too large for kf_icp_track_noalloc (level-0 images up to 786432 pixels)");
   }
   NoAllocScratch* sc = nullptr;

@@ -6,7 +6,7 @@
 // (Source/src/ICP.cu:266-321) with an FP64 Euler-ZYX increment left-multiplied
 // onto the pose.  Operation order is fixed, contraction is off and the fused
 // multiply-adds are explicit (fma, correctly rounded on both sides), so host and
-// device produce identical bits.
+// device produce identical bits but for the solve's reciprocals (pivot_inverse).
 #pragma once
 
 #include <math.h>
@@ -128,6 +128,16 @@ KF_HD void euler_zyx(double a, double b, double g, double tx, double ty, double 
   for (int e = 0; e < 16; ++e) D[e] = euler_zyx_entry(e, ca, sa, cb, sb, cg, sg, tx, ty, tz);
 }
 
+KF_HD double pivot_inverse(double d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double r = __builtin_amdgcn_rcp(d);
+  r = fma(r, fma(-d, r, 1.0), r);
+  return fma(r, fma(-d, r, 1.0), r);
+#else
+  return 1.0 / d;
+#endif
+}
+
 // Solves the 6x6 SPD system A x = g (A given by its 21 upper-triangle entries,
 // row-major i <= j) by the square-root-free Cholesky factorisation A = L D L^T
 // (L unit lower triangular).  Returns false if a pivot D_j is not above
@@ -135,7 +145,9 @@ KF_HD void euler_zyx(double a, double b, double g, double tx, double ty, double 
 // the square root of.  Each column divides once (1 / D_j) and multiplies, so the
 // critical path holds six divisions and no square root.  W holds L D (the
 // unscaled column entries), so no product is formed twice.  The updates are fused
-// multiply-adds (one rounding each, the same bits on host and device).
+// multiply-adds (one rounding each).  On the device 1 / D_j is the hardware reciprocal
+// refined by two Newton steps (within an ulp of the quotient; D_j is a normal number
+// where it counts) and there is no early return: a bad pivot is remembered.
 KF_HD bool ldlt_solve6(const double* upper21, const double* g, double rel_eps, double* x) {
   double A[6][6];
   int k = 0;
@@ -148,12 +160,13 @@ KF_HD bool ldlt_solve6(const double* upper21, const double* g, double rel_eps, d
     }
   for (int i = 0; i < 6; ++i) dmax = A[i][i] > dmax ? A[i][i] : dmax;
   const double thr = rel_eps * dmax;
+  bool ok = true;
   double L[6][6], W[6][6], inv[6];
   for (int j = 0; j < 6; ++j) {
     double d = A[j][j];
     for (int m = 0; m < j; ++m) d = fma(-W[j][m], L[j][m], d);
-    if (!(d > thr)) return false;
-    inv[j] = 1.0 / d;
+    ok = ok && d > thr;
+    inv[j] = pivot_inverse(d);
     for (int i = j + 1; i < 6; ++i) {
       double w = A[i][j];
       for (int m = 0; m < j; ++m) w = fma(-W[i][m], L[j][m], w);
@@ -169,36 +182,41 @@ KF_HD bool ldlt_solve6(const double* upper21, const double* g, double rel_eps, d
   }
   for (int i = 5; i >= 0; --i) {
     double s = z[i] * inv[i];
-    for (int m = i + 1; m < 6; ++m) s = fma(-L[m][i], x[m], s);
+    for (int m = 5; m > i; --m) s = fma(-L[m][i], x[m], s);  // the newest x last: one step of the chain each
     x[i] = s;
   }
-  return true;
+  return ok;
 }
 
 // cos and sin of a small angle: Taylor series through x^14 / x^13 (Horner in x^2)
-// for |x| <= 0.25, where the truncation error is below 1e-20; libm otherwise.
+// for |x| <= 0.25, where the truncation error is below 1e-20; libm otherwise.  On the
+// device the series is formed without a branch, and libm's code is entered only when a
+// lane of the wave needs it (800 cycles against 200 with the test around the series).
 KF_HD void small_sincos(double x, double* c, double* s) {
-  if (fabs(x) <= 0.25) {
-    const double z = x * x;
-    double ps = 1.0 / 6227020800.0, pc = -1.0 / 87178291200.0;  // Horner steps as fused multiply-adds
-    ps = fma(z, ps, -1.0 / 39916800.0);
-    ps = fma(z, ps, 1.0 / 362880.0);
-    ps = fma(z, ps, -1.0 / 5040.0);
-    ps = fma(z, ps, 1.0 / 120.0);
-    ps = fma(z, ps, -1.0 / 6.0);
-    ps = fma(z, ps, 1.0);
-    *s = x * ps;
-    pc = fma(z, pc, 1.0 / 479001600.0);
-    pc = fma(z, pc, -1.0 / 3628800.0);
-    pc = fma(z, pc, 1.0 / 40320.0);
-    pc = fma(z, pc, -1.0 / 720.0);
-    pc = fma(z, pc, 1.0 / 24.0);
-    pc = fma(z, pc, -0.5);
-    *c = fma(z, pc, 1.0);
-  } else {
-    *c = cos(x);
-    *s = sin(x);
-  }
+  const double z = x * x;
+  double ps = 1.0 / 6227020800.0, pc = -1.0 / 87178291200.0;  // Horner steps as fused multiply-adds
+  ps = fma(z, ps, -1.0 / 39916800.0);
+  pc = fma(z, pc, 1.0 / 479001600.0);
+  ps = fma(z, ps, 1.0 / 362880.0);
+  pc = fma(z, pc, -1.0 / 3628800.0);
+  ps = fma(z, ps, -1.0 / 5040.0);
+  pc = fma(z, pc, 1.0 / 40320.0);
+  ps = fma(z, ps, 1.0 / 120.0);
+  pc = fma(z, pc, -1.0 / 720.0);
+  ps = fma(z, ps, -1.0 / 6.0);
+  pc = fma(z, pc, 1.0 / 24.0);
+  ps = fma(z, ps, 1.0);
+  pc = fma(z, pc, -0.5);
+  *s = x * ps;
+  *c = fma(z, pc, 1.0);
+  const bool large = !(fabs(x) <= 0.25);
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (__builtin_expect(__any(large), 0))
+#endif
+    if (large) {
+      *c = cos(x);
+      *s = sin(x);
+    }
 }
 
 }  // namespace kf
