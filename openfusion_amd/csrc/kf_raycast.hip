@@ -19,11 +19,21 @@
 // band of image rows and its L2 sees neighbouring rays.
 //
 // Normals are computed once per wavefront after every ray of it has finished its
-// march: the six central-difference samples of all the wave's hits read a box of
-// voxels that the wave first stages in LDS with coalesced z-row loads (8x8
-// neighbouring rays hit nearby surface points, so the box is small and each voxel
-// serves several rays); a wave whose box is too large (a silhouette) samples the
-// volume directly.  Either way every sample is the same trilinear expression.
+// march: each hit loads the 32 voxels of its six central-difference samples in one
+// round of row loads.
+//
+// What bounds it: issue.  A round of the march is ~225 vector instructions (FP16
+// records) at four cycles each, a wave makes ~9 rounds and its longest ray up to 20, and
+// 4,800 waves of a 640x480 image share 1,024 SIMDs; then the latency of the longest
+// waves' rounds, which end alone (vector pipes busy 57% of the kernel before the
+// instruction counts below were cut, 39% of a wave's time in memory waits).  Hence: no
+// domain check per sample, differences of FP16 halves without conversions, one face per
+// axis in the free-space skip, no division inside the loop.  Measured together with the
+// brick distances, 512^3 FP16 at 640x480: 42.9 -> 34.9 us; 256^3 FP32 at 319x241: 36.2
+// -> 29.0 us.  Looking at the map once per sample and loading corners only where a brick
+// is set (fewer instructions a round, more rounds), corner loads ahead of the map's
+// answer, four or five samples a round, and a wave priority that grows with its rounds
+// were all slower.
 #include <hip/hip_ext.h>
 
 #include <type_traits>
@@ -35,8 +45,6 @@ namespace kf {
 namespace {
 
 constexpr int kXcds = 8;
-constexpr int kRayWaves = 4;      // wavefronts per 256-thread block
-constexpr int kGradBox = 1024;    // voxels of a wavefront's LDS box for the normals
 
 struct RayArgs {
   const void* vox;
@@ -62,13 +70,6 @@ struct RayArgs {
   int blocks_x, blocks_y;
 };
 
-// f of the voxel at byte address p (the TSDF half of the voxel record).
-template <int FMT>
-__device__ __forceinline__ float vox_at(const char* p) {
-  if (FMT == KF_VOXEL_F16) return half_bits_to_float(*reinterpret_cast<const uint32_t*>(p) & 0xffffu);
-  return *reinterpret_cast<const float*>(p);
-}
-
 // Interpolations and points along a ray are fused multiply-adds (one rounding each;
 // the oracle computes them the same way).
 __device__ __forceinline__ float lerp(float a, float b, float t) { return fmaf(b - a, t, a); }
@@ -86,22 +87,29 @@ __device__ __forceinline__ voff_t<OFF32> vox_offset(int n, int ix, int iy, int i
   constexpr unsigned kB = FMT == KF_VOXEL_F16 ? 4u : 8u;
   if constexpr (OFF32) {
     const unsigned un = (unsigned)n;
-    const unsigned row = opaque_u32(__umul24((unsigned)ix, un)) + (unsigned)iy;
-    return (opaque_u32(__umul24(row, un)) + (unsigned)iz) * kB;
+    const unsigned row = opaque_u32(__umul24((unsigned)ix, un) + (unsigned)iy);
+    return opaque_u32(__umul24(row, un) + (unsigned)iz) * kB;
   } else {
     return ((((size_t)ix * (size_t)n) + (size_t)iy) * (size_t)n + (size_t)iz) * kB;
   }
 }
 
-// The eight corners of the trilinear cell whose base voxel is at byte offset o:
-// c[0..7] = f at (x,y,z), (x,y,z+1), (x,y+1,z), (x,y+1,z+1), (x+1,y,z), ...
+// The eight corners of the trilinear cell whose base voxel is at byte offset o.
 // The (z, z+1) pairs are adjacent records, fetched by one load each: 8 bytes for
 // FP16 records, 16 bytes ({f, w} twice) for FP32 records.
 typedef unsigned int u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
+typedef unsigned int u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
 
+template <int FMT>
+using pair_ld = typename std::conditional<FMT == KF_VOXEL_F16, u32x2_a4, f32x4_a8>::type;
+template <int FMT>
+struct Corners {  // the (z, z + 1) pairs at (x, y), (x, y + 1), (x + 1, y), (x + 1, y + 1)
+  pair_ld<FMT> q[4];
+};
+
 template <int FMT, bool OFF32>
-__device__ __forceinline__ void load_corners(const RayArgs& a, voff_t<OFF32> o, float* c) {
+__device__ __forceinline__ Corners<FMT> load_corners(const RayArgs& a, voff_t<OFF32> o) {
   constexpr unsigned kB = FMT == KF_VOXEL_F16 ? 4u : 8u;
   // an opaque 32-bit register keeps the base-register + 32-bit-offset load form
   if constexpr (OFF32) o = opaque_u32(o);
@@ -110,33 +118,37 @@ __device__ __forceinline__ void load_corners(const RayArgs& a, voff_t<OFF32> o, 
   b[1] = b[0] + (size_t)a.n * kB;        // y + 1
   b[2] = b[0] + (size_t)a.n * a.n * kB;  // x + 1
   b[3] = b[2] + (size_t)a.n * kB;        // x + 1, y + 1
-  if constexpr (FMT == KF_VOXEL_F16) {
-    u32x2_a4 q[4];
+  Corners<FMT> c;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) q[i] = *reinterpret_cast<const u32x2_a4*>(b[i] + o);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      c[2 * i] = half_bits_to_float(q[i].x & 0xffffu);
-      c[2 * i + 1] = half_bits_to_float(q[i].y & 0xffffu);
-    }
-  } else {
-    f32x4_a8 q[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) q[i] = *reinterpret_cast<const f32x4_a8*>(b[i] + o);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      c[2 * i] = q[i].x;
-      c[2 * i + 1] = q[i].z;
-    }
-  }
+  for (int i = 0; i < 4; ++i) c.q[i] = *reinterpret_cast<const pair_ld<FMT>*>(b[i] + o);
+  return c;
 }
 
-// Trilinear value from the eight corners and the grid coordinate's fractions.
-__device__ __forceinline__ float trilinear(const float* c, float tx, float ty, float tz) {
-  const float c00 = lerp(c[0], c[1], tz), c01 = lerp(c[2], c[3], tz);
-  const float c10 = lerp(c[4], c[5], tz), c11 = lerp(c[6], c[7], tz);
-  const float c0 = lerp(c00, c01, ty), c1 = lerp(c10, c11, ty);
-  return lerp(c0, c1, tx);
+// lerp of the FP16 halves of two voxel records, converted as they are read: b - a and
+// fma(b - a, t, a), each one rounding to FP32, as lerp() of the converted values (the
+// difference is written as fma(b, 1, -a); two instructions instead of four).
+__device__ __forceinline__ float lerp_h(uint32_t a, uint32_t b, float t) {
+  float d, r;
+  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,1]" : "=v"(d) : "v"(b), "v"(a));
+  asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[0,0,1]" : "=v"(r) : "v"(d), "v"(t), "v"(a));
+  return r;
+}
+
+// Trilinear value from four values interpolated along z and the x and y fractions.
+__device__ __forceinline__ float bilinear(float c00, float c01, float c10, float c11, float tx, float ty) {
+  return lerp(lerp(c00, c01, ty), lerp(c10, c11, ty), tx);
+}
+template <int FMT>
+__device__ __forceinline__ float trilinear(const Corners<FMT>& c, float tx, float ty, float tz) {
+  float z[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (FMT == KF_VOXEL_F16)
+      z[i] = lerp_h(c.q[i].x, c.q[i].y, tz);
+    else
+      z[i] = lerp(c.q[i].x, c.q[i].z, tz);
+  }
+  return bilinear(z[0], z[1], z[2], z[3], tx, ty);
 }
 
 // Inside the trilinear domain: every coordinate in [0, n - 1).
@@ -144,72 +156,62 @@ __device__ __forceinline__ bool in_domain(f3 g, float lim) {
   return fminf(fminf(g.x, g.y), g.z) >= 0.0f && fmaxf(fmaxf(g.x, g.y), g.z) < lim;
 }
 
-// K trilinear samples of f at grid points g[j]; ok[j] is false outside the
-// trilinear domain.  Base voxel floor(g), weights g - floor(g).  When the brick of
-// the base voxel is clear in the occupancy map (its brick distance is not 0), all
-// eight corners hold f == 1 and the interpolation is exactly 1 (a + (b - a) t with
-// a = b = 1), so the voxel loads are skipped: the value is the same.  dclear
-// (optional): the brick distance of each sample whose brick is clear (>= 1), 0
-// otherwise.  Three phases, so that a batch costs about one map latency plus one
-// voxel latency instead of K of each: the distance bytes of all samples, then the
-// corners of all samples (one wave-uniform branch; lanes whose sample needs no
-// corners read voxel 0 instead, which stays cached), then the interpolations.  need_in (optional): samples that must not
-// be taken at all (then fk = 1 and ok as computed).  use_map = false: this lane
-// loads the corners without looking at the map (dclear 0).  Returns the number of
-// samples that loaded corners.
+// Whether any lane's condition holds (the lane mask itself, no vector compare).
+__device__ __forceinline__ bool any_lane(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
+
+// K trilinear samples of f at grid points g[j]: 1 where ok[j] is false (a point outside
+// the trilinear domain, or one that the march does not reach).  Base voxel floor(g),
+// weights g - floor(g).  When the brick of the base voxel is clear in the occupancy map
+// (its brick distance is not 0), all eight corners hold f == 1 and the interpolation is
+// exactly 1 (a + (b - a) t with a = b = 1), so the voxel loads are skipped: the value is
+// the same.  dclear (optional): the brick distance of each sample whose brick is clear
+// (>= 1), 0 otherwise.  Three phases, so that a batch costs about one map latency plus
+// one voxel latency instead of K of each: the distance bytes of all samples, then the
+// corners of all samples (one wave-uniform branch; lanes whose sample needs no corners
+// read voxel 0 instead, which stays cached), then the interpolations.  use_map = false:
+// this lane loads the corners without looking at the map (dclear 0).  need: the samples
+// that loaded corners.
 template <int FMT, bool OFF32, int K>
-__device__ __forceinline__ int sample_points(const RayArgs& a, const f3* g, bool* ok, float* fk,
-                                             int* dclear = nullptr, const bool* need_in = nullptr,
-                                             bool use_map = true) {
-  const float lim = (float)(a.n - 1);
-  int ix[K], iy[K], iz[K];
-  bool need[K];
+__device__ __forceinline__ void sample_points(const RayArgs& a, const f3* g, const bool* ok, float* fk, bool* need,
+                                              int* dclear = nullptr, bool use_map = true) {
+  // positions are finite (finite pose, t inside the slab interval); offsets of samples
+  // with ok false are not used
+  int d[K];
 #pragma unroll
-  for (int j = 0; j < K; ++j) {
-    // positions are finite (finite pose, t inside the slab interval)
-    ok[j] = in_domain(g[j], lim);
-    ix[j] = ok[j] ? (int)g[j].x : 0;
-    iy[j] = ok[j] ? (int)g[j].y : 0;
-    iz[j] = ok[j] ? (int)g[j].z : 0;
-  }
+  for (int j = 0; j < K; ++j) d[j] = 0;
   const bool map_lane = a.bdist != nullptr && use_map;
-  if (__any(map_lane)) {  // uniform
+  if (any_lane(map_lane)) {  // uniform
     // the brick's distance byte (64 per occupancy word of the column): 0 for a set
     // brick (its bit in the occupancy map), else the distance to the nearest set one;
     // lanes that do not use the map load the corners whatever the brick
     const unsigned row = (unsigned)kOccWordBricks * (unsigned)a.occ_words;
-    unsigned dj[K];
+    unsigned o[K];
 #pragma unroll
     for (int j = 0; j < K; ++j) {
-      const unsigned col = opaque_u32(__umul24((unsigned)(ix[j] >> 3), (unsigned)a.occ_nb)) + (unsigned)(iy[j] >> 3);
-      dj[j] = map_lane ? (unsigned)a.bdist[opaque_u32(__umul24(col, row) + (unsigned)(iz[j] >> 3))] : 0u;
+      const int bx = (int)g[j].x >> 3, by = (int)g[j].y >> 3, bz = (int)g[j].z >> 3;
+      const unsigned col = opaque_u32(__umul24((unsigned)bx, (unsigned)a.occ_nb) + (unsigned)by);
+      o[j] = opaque_u32(__umul24(col, row) + (unsigned)bz);
+      o[j] = ok[j] && map_lane ? o[j] : 0u;
     }
 #pragma unroll
-    for (int j = 0; j < K; ++j) {
-      need[j] = ok[j] && dj[j] == 0u;
-      if (dclear) dclear[j] = ok[j] && !need[j] ? (int)dj[j] : 0;
-    }
-  } else {
+    for (int j = 0; j < K; ++j) d[j] = a.bdist[opaque_u32(o[j])];
 #pragma unroll
-    for (int j = 0; j < K; ++j) {
-      need[j] = ok[j];
-      if (dclear) dclear[j] = 0;
-    }
+    for (int j = 0; j < K; ++j) d[j] = ok[j] && map_lane ? d[j] : 0;
   }
-  int loads = 0, any = 0;
+  bool any = false;
 #pragma unroll
   for (int j = 0; j < K; ++j) {
-    if (need_in) need[j] = need[j] && need_in[j];
+    need[j] = ok[j] && d[j] == 0;
     fk[j] = 1.0f;
-    loads += need[j] ? 1 : 0;
-    any |= need[j] ? 1 : 0;
+    any = any || need[j];
+    if (dclear) dclear[j] = d[j];
   }
-  if (__any(any)) {
-    float c[K][8];
+  if (any_lane(any)) {
+    Corners<FMT> c[K];
 #pragma unroll
     for (int j = 0; j < K; ++j) {
-      const voff_t<OFF32> o = vox_offset<FMT, OFF32>(a.n, ix[j], iy[j], iz[j]);
-      load_corners<FMT, OFF32>(a, need[j] ? o : (voff_t<OFF32>)0, c[j]);
+      const voff_t<OFF32> o = vox_offset<FMT, OFF32>(a.n, (int)g[j].x, (int)g[j].y, (int)g[j].z);
+      c[j] = load_corners<FMT, OFF32>(a, need[j] ? o : (voff_t<OFF32>)0);
     }
 #pragma unroll
     for (int j = 0; j < K; ++j) {
@@ -219,7 +221,6 @@ __device__ __forceinline__ int sample_points(const RayArgs& a, const f3* g, bool
       fk[j] = need[j] ? v : 1.0f;
     }
   }
-  return loads;
 }
 
 // Grid position of ray parameter t.
@@ -227,115 +228,87 @@ __device__ __forceinline__ f3 gpos(f3 go, f3 gd, float t) {
   return f3{fmaf(t, gd.x, go.x), fmaf(t, gd.y, go.y), fmaf(t, gd.z, go.z)};
 }
 
-// Wave-wide min / max of an int (every lane gets the result).
-__device__ __forceinline__ int wave_min_i(int v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = min(v, __shfl_xor(v, off, kWave));
-  return v;
-}
-__device__ __forceinline__ int wave_max_i(int v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = max(v, __shfl_xor(v, off, kWave));
-  return v;
-}
-
-// Orders the LDS accesses of one wavefront around this point.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The six central-difference samples at grid point gh (x+1, x-1, y+1, y-1, z+1, z-1)
-// for every lane with `want`, staged through the wave's LDS box when it fits.
-// Returns whether all six are inside the trilinear domain (false without `want`).
+// for every lane with `want`.  Returns whether all six are inside the trilinear domain
+// (false without `want`).  Their 48 corners are 32 voxels in 12 z-rows around the base
+// voxel b of gh: (z-1 .. z+2) of the four rows (x, y), (x, y+1), (x+1, y), (x+1, y+1),
+// and (z, z+1) of the rows next to them along x and y.  The lane loads each row once
+// (FP16 records: one 16-byte or one 8-byte load, 12 in flight together): no pass
+// through LDS, no wave reduction and no index division.  (The wave's samples staged as a
+// box in LDS took ~550 vector instructions and a chain of reductions where this takes
+// ~150: 39.6 -> 37.3 us with the brick distances at 512^3 FP16, 32.1 -> 30.5 at 256^3.)
 template <int FMT, bool OFF32>
-__device__ __forceinline__ bool gradient_samples(const RayArgs& a, bool want, f3 gh, float* box, float* fq) {
+__device__ __forceinline__ bool gradient_samples(const RayArgs& a, bool want, f3 gh, float* fq) {
+  constexpr unsigned kB = FMT == KF_VOXEL_F16 ? 4u : 8u;
   const float lim = (float)(a.n - 1);
   const f3 q[6] = {f3{gh.x + 1.0f, gh.y, gh.z}, f3{gh.x - 1.0f, gh.y, gh.z}, f3{gh.x, gh.y + 1.0f, gh.z},
                    f3{gh.x, gh.y - 1.0f, gh.z}, f3{gh.x, gh.y, gh.z + 1.0f}, f3{gh.x, gh.y, gh.z - 1.0f}};
-  bool all = want;
+  // rounding is monotone, so these six coordinates bound the others
+  const bool all = want && fminf(fminf(q[1].x, q[3].y), q[5].z) >= 0.0f && fmaxf(fmaxf(q[0].x, q[2].y), q[4].z) < lim;
+  const int bx = all ? (int)gh.x : 0, by = all ? (int)gh.y : 0, bz = all ? (int)gh.z : 0;
+  // gh + 1 can round up to the next whole number where the exponent changes: its base
+  // voxel is then not b + 1.  Such a wave takes the samples one by one.
+  const bool plain = !all || ((int)q[0].x == bx + 1 && (int)q[1].x == bx - 1 && (int)q[2].y == by + 1 &&
+                              (int)q[3].y == by - 1 && (int)q[4].z == bz + 1 && (int)q[5].z == bz - 1);
+  if (any_lane(!plain)) {
+    const bool okq[3] = {all, all, all};
+    bool need[3];
+    sample_points<FMT, OFF32, 3>(a, q, okq, fq, need);
+    sample_points<FMT, OFF32, 3>(a, q + 3, okq, fq + 3, need);
+  } else if (all) {
+    typedef pair_ld<FMT> pair_t;
+    voff_t<OFF32> o = vox_offset<FMT, OFF32>(a.n, bx, by, bz);
+    if constexpr (OFF32) o = opaque_u32(o);
+    const ptrdiff_t sy = (ptrdiff_t)a.n * kB, sx = sy * a.n;
+    auto row = [&](ptrdiff_t off) { return static_cast<const char*>(a.vox) + off + o; };
+    struct Row {
+      pair_t m, p;  // (z - 1, z), (z + 1, z + 2)
+    } r[4];         // (x, y), (x, y + 1), (x + 1, y), (x + 1, y + 1)
+    pair_t xm[2], xp[2], ym[2], yp[2];  // (z, z + 1) at x - 1 and x + 2 (y, y + 1), at y - 1 and y + 2 (x, x + 1)
 #pragma unroll
-  for (int j = 0; j < 6; ++j) all = all && in_domain(q[j], lim);
-  // base voxels of the six samples: per axis [min floor, max floor + 1]
-  int lo[3] = {1 << 30, 1 << 30, 1 << 30}, hi[3] = {-1, -1, -1};
-  if (all) {
-#pragma unroll
-    for (int j = 0; j < 6; ++j) {
-      const int b[3] = {(int)q[j].x, (int)q[j].y, (int)q[j].z};
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        lo[k] = min(lo[k], b[k]);
-        hi[k] = max(hi[k], b[k] + 1);
+    for (int i = 0; i < 4; ++i) {
+      const char* p = row((i >> 1) * sx + (i & 1) * sy - (ptrdiff_t)kB);
+      if constexpr (FMT == KF_VOXEL_F16) {
+        const u32x4_a4 w = *reinterpret_cast<const u32x4_a4*>(p);
+        r[i].m = pair_t{w.x, w.y};
+        r[i].p = pair_t{w.z, w.w};
+      } else {
+        r[i].m = *reinterpret_cast<const f32x4_a8*>(p);
+        r[i].p = *reinterpret_cast<const f32x4_a8*>(p + 2 * kB);
       }
     }
-  }
-  int L[3], E[3];
+    auto pair = [&](ptrdiff_t off) { return *reinterpret_cast<const pair_ld<FMT>*>(row(off)); };
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    L[k] = wave_min_i(lo[k]);
-    E[k] = wave_max_i(hi[k]) - L[k] + 1;  // <= 0 when no lane has all six samples
-  }
-  const bool any = __any(all);
-  const int vol = any ? E[0] * E[1] * E[2] : 0;
-  if (any && vol <= kGradBox) {  // uniform
-    // stage the box: voxel (L + (x, y, z)) at box[(x * Ey + y) * Ez + z], z-rows coalesced
-    const int lane = threadIdx.x & (kWave - 1);
-    const char* vb = static_cast<const char*>(a.vox);
-    // the lane's first box voxel, then steps of kWave voxels: kWave = dr Ez + dz and
-    // dr = dx Ey + dy, each with at most one carry
-    int z = lane % E[2], r = lane / E[2];
-    int y = r % E[1], x = r / E[1];
-    const int dz = kWave % E[2], dr = kWave / E[2];
-    const int dy = dr % E[1], dx = dr / E[1];
-    // all of the lane's loads in flight together (one memory latency for the box),
-    // then the LDS stores; voxels past the box read its first voxel instead
-    constexpr int kPer = kGradBox / kWave;
-    float v[kPer];
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const bool in = lane + u * kWave < vol;
-      v[u] = vox_at<FMT>(vb + vox_offset<FMT, OFF32>(a.n, L[0] + (in ? x : 0), L[1] + (in ? y : 0), L[2] + (in ? z : 0)));
-      z += dz;
-      y += dy;
-      x += dx;
-      if (z >= E[2]) {
-        z -= E[2];
-        ++y;
-      }
-      if (y >= E[1]) {
-        y -= E[1];
-        ++x;
-      }
+    for (int i = 0; i < 2; ++i) {
+      xm[i] = pair(i * sy - sx);
+      xp[i] = pair(i * sy + 2 * sx);
+      ym[i] = pair(i * sx - sy);
+      yp[i] = pair(i * sx + 2 * sy);
     }
-#pragma unroll
-    for (int u = 0; u < kPer; ++u)
-      if (lane + u * kWave < vol) box[lane + u * kWave] = v[u];
-    wave_lds_sync();
-    if (all) {
-#pragma unroll
-      for (int j = 0; j < 6; ++j) {
-        const int bx = (int)q[j].x - L[0], by = (int)q[j].y - L[1], bz = (int)q[j].z - L[2];
-        const int i0 = (bx * E[1] + by) * E[2] + bz, sy = E[2], sx = E[1] * E[2];
-        const float c[8] = {box[i0], box[i0 + 1], box[i0 + sy], box[i0 + sy + 1],
-                            box[i0 + sx], box[i0 + sx + 1], box[i0 + sx + sy], box[i0 + sx + sy + 1]};
-        fq[j] = trilinear(c, __builtin_amdgcn_fractf(q[j].x), __builtin_amdgcn_fractf(q[j].y),
-                          __builtin_amdgcn_fractf(q[j].z));
-      }
-    }
-    wave_lds_sync();  // the box is free again
-  } else if (any) {
-    bool okq[6];
-    const bool need[3] = {all, all, all};
-    sample_points<FMT, OFF32, 3>(a, q, okq, fq, nullptr, need);
-    sample_points<FMT, OFF32, 3>(a, q + 3, okq + 3, fq + 3, nullptr, need);
+    // (z, z + 1) of a central row
+    auto mid = [&](int i) {
+      if constexpr (FMT == KF_VOXEL_F16)
+        return pair_t{r[i].m.y, r[i].p.x};
+      else
+        return pair_t{r[i].m.z, r[i].m.w, r[i].p.x, r[i].p.y};
+    };
+    auto take = [&](int j, pair_t c00, pair_t c01, pair_t c10, pair_t c11) {
+      const Corners<FMT> c{{c00, c01, c10, c11}};
+      fq[j] = trilinear(c, __builtin_amdgcn_fractf(q[j].x), __builtin_amdgcn_fractf(q[j].y),
+                        __builtin_amdgcn_fractf(q[j].z));
+    };
+    take(0, mid(2), mid(3), xp[0], xp[1]);
+    take(1, xm[0], xm[1], mid(0), mid(1));
+    take(2, mid(1), yp[0], mid(3), yp[1]);
+    take(3, ym[0], mid(0), ym[1], mid(2));
+    take(4, r[0].p, r[1].p, r[2].p, r[3].p);
+    take(5, r[0].m, r[1].m, r[2].m, r[3].m);
   }
   return all;
 }
 
 template <int FMT, bool OFF32>
 __global__ __launch_bounds__(256) void raycast(RayArgs a) {
-  __shared__ float s_box[kRayWaves][kGradBox];
   // XCD-aware block remap: logical = (xcd band) + (position within band).
   const int nb = a.blocks_x * a.blocks_y;
   const int per = (nb + kXcds - 1) / kXcds;
@@ -394,21 +367,42 @@ __global__ __launch_bounds__(256) void raycast(RayArgs a) {
     // step size stays the same and then consumed in order; a batch ends where the
     // march would change step size or stop, so the result and the step count equal
     // the one-step-at-a-time march while the dependent-load chain is up to kSpec
-    // times shorter.  FP16 records: three samples a batch (88 VGPRs, five waves per
-    // SIMD) beat two (69 VGPRs) once the frame's concurrent kernels leave the
-    // raycast its CU slots.  FP32 records (16-byte corner loads): three would need
-    // 102 VGPRs (four waves per SIMD, fewer than the 4,800 waves), so two.
+    // times shorter.  FP16 records: three samples a batch (80 VGPRs, six waves per
+    // SIMD) as fast as two (70 VGPRs: 35.6 and 34.8 us) when the image is alone on the
+    // chip, and ahead once the frame's concurrent kernels share it.  FP32 records
+    // (16-byte corner loads): three would need 110 VGPRs (four waves per SIMD, fewer
+    // than the 4,800 waves), so two.
     constexpr int kSpec = FMT == KF_VOXEL_F16 ? 3 : 2;
+    const float lim = (float)(a.n - 1);
     float t = tnear, fp;
     bool ok;
+    int last_d;  // brick distance of the sample at t when its brick is clear, else 0
     {
       const f3 g0 = gpos(go, gd, t);
-      sample_points<FMT, OFF32, 1>(a, &g0, &ok, &fp);
+      ok = in_domain(g0, lim);
+      bool need;
+      sample_points<FMT, OFF32, 1>(a, &g0, &ok, &fp, &need, &last_d);
+      // A coordinate of g(t) is a monotone function of t, so the part of [tnear, tfar]
+      // whose points are in the domain is an interval from tnear on: with its end as
+      // tfar (tfar itself but for rounding far outside the volume; else bisected), the
+      // march needs no domain check.
+      if (ok && !in_domain(gpos(go, gd, tfar), lim)) {
+        float in = tnear;
+        for (int k = 0; k < 256; ++k) {
+          const float mid = in + (tfar - in) * 0.5f;
+          if (!(mid > in && mid < tfar)) break;
+          const bool inside = in_domain(gpos(go, gd, mid), lim);
+          in = inside ? mid : in;
+          tfar = inside ? tfar : mid;
+        }
+        tfar = in;
+      }
       ok = ok && fp >= 0.0f;
     }
-    int s = 0;
-    float t0 = t;         // start of the current segment
-    int i = 0;            // steps taken in it
+    float t0 = t;           // start of the current segment
+    int i = 0;              // steps taken in it
+    int imax = a.max_steps;  // steps that may still be taken at its start
+    float fb = 0.0f;         // the sample that ended the march in a crossing
     bool seg_far = fp >= 1.0f;
     // Free-space skip.  From a far-mode position t (sample 1) whose base voxel lies
     // in a brick at distance D >= 1 from the nearest set brick, every brick within
@@ -418,39 +412,55 @@ __global__ __launch_bounds__(256) void raycast(RayArgs a) {
     // coordinate of a position is a monotone function of i on each axis, so if the
     // last one is still in the box (checked with the exact sample arithmetic) every
     // intermediate one is too.  The step count, the position and the value are those
-    // of the step-by-step march.
+    // of the step-by-step march.  A ray can leave the box only through the faces
+    // ahead of it: axes along which it runs down are mirrored (sign and order of
+    // floats negate exactly; brick b becomes ~b), so each axis has one face, above.
+    float gom[3], gdm[3], rd[3], rc[3], top[3];
+    int flip[3];
+    const float go_[3] = {go.x, go.y, go.z}, gd_[3] = {gd.x, gd.y, gd.z};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const bool down = gd_[k] < 0.0f;
+      flip[k] = down ? -1 : 0;
+      top[k] = down ? 0.0f : (float)(a.n - 1);
+      gom[k] = down ? -go_[k] : go_[k];
+      gdm[k] = fabsf(gd_[k]);
+      // exit estimate of a face: face * rd + rc (not a number for an axis the ray does
+      // not move along; the minimum below passes over it)
+      rd[k] = __builtin_amdgcn_rcpf(gdm[k]);
+      rc[k] = -gom[k] * rd[k];
+    }
     auto skip_free = [&](int D) {
       const f3 gp = gpos(go, gd, t);
-      const int bx = (int)gp.x >> 3, by = (int)gp.y >> 3, bz = (int)gp.z >> 3, r = D - 1;
-      const float lim = (float)(a.n - 1);
-      const float lx = (float)(8 * max(bx - r, 0)), hx = fminf((float)(8 * (bx + r + 1)), lim);
-      const float ly = (float)(8 * max(by - r, 0)), hy = fminf((float)(8 * (by + r + 1)), lim);
-      const float lz = (float)(8 * max(bz - r, 0)), hz = fminf((float)(8 * (bz + r + 1)), lim);
-      // Approximate exit parameter of the box, with reciprocals: only the estimate
-      // of k depends on it, and the skip is verified with the exact arithmetic below.
-      auto exit_t = [&](float d, float lo_, float hi_, float g0) {
-        return d != 0.0f ? ((d > 0.0f ? hi_ : lo_) - g0) * __builtin_amdgcn_rcpf(d) : 3.0e38f;
-      };
-      const float te = fminf(fminf(tfar, exit_t(gd.x, lx, hx, go.x)),
-                             fminf(exit_t(gd.y, ly, hy, go.y), exit_t(gd.z, lz, hz, go.z)));
+      const int b[3] = {(int)gp.x >> 3, (int)gp.y >> 3, (int)gp.z >> 3};
+      float face[3], e[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        face[k] = fminf((float)(((b[k] ^ flip[k]) + D) * 8), top[k]);
+        e[k] = fmaf(face[k], rd[k], rc[k]);
+      }
+      // Approximate exit parameter of the box: only the estimate of k depends on it, and
+      // the skip is verified with the exact arithmetic below.
+      const float te = fminf(fminf(tfar, e[0]), fminf(e[1], e[2]));
       int k = (int)fminf((te - t) * a.inv_step_far, (float)a.max_steps) - 1;
-      k = min(k, a.max_steps - s);
+      k = min(k, imax - i);
       if (k <= 0) return;
       const float tt = fmaf((float)(i + k), a.step_far_m, t0);
-      const f3 ge = gpos(go, gd, tt);
-      if (tt <= tfar && ge.x >= lx && ge.x < hx && ge.y >= ly && ge.y < hy && ge.z >= lz && ge.z < hz) {
+      bool in = tt <= tfar;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) in = in && fmaf(tt, gdm[k], gom[k]) < face[k];
+      if (in) {
         t = tt;
         i += k;
-        s += k;
-        nsteps += k;
         n_skipped += k;
       }
     };
-    int last_d = 0;  // brick distance of the sample at t when its brick is clear, else 0
-    while (ok && s < a.max_steps) {
+    bool run = ok && i < imax;
+    while (run) {
       const bool far = fp >= 1.0f;
       if (far != seg_far) {  // the step size changes: a new segment from t
         t0 = t;
+        imax -= i;
         i = 0;
         seg_far = far;
       }
@@ -464,39 +474,34 @@ __global__ __launch_bounds__(256) void raycast(RayArgs a) {
       for (int j = 0; j < kSpec; ++j) {
         tk[j] = fmaf((float)(i + j + 1), st, t0);
         gk[j] = gpos(go, gd, tk[j]);
+        vk[j] = tk[j] <= tfar;
       }
       // Inside the truncation band (near mode) the bricks ahead hold the surface, so
       // the corners are loaded without the map's dependent lookup first: one memory
       // latency per batch instead of two (the values are the same; the map only
       // spares loads).
-      n_loads += sample_points<FMT, OFF32, kSpec>(a, gk, vk, fk, ck, nullptr, far);
-      ++n_batches;
+      bool lk[kSpec];
+      sample_points<FMT, OFF32, kSpec>(a, gk, vk, fk, lk, ck, far);
+      if (a.diag) {  // uniform
+        ++n_batches;
 #pragma unroll
-      for (int j = 0; j < kSpec; ++j) vk[j] = vk[j] && tk[j] <= tfar;
+        for (int j = 0; j < kSpec; ++j) n_loads += lk[j] ? 1 : 0;
+      }
       // Consume the batch in order, as selects rather than branches.  Sample j is
       // examined when every earlier sample of the batch was consumed (valid, no
-      // crossing) and kept the step size; then it is step s + j, taken while
-      // s + j < max_steps.  A step that finds its sample invalid still counts and
-      // ends the march; a crossing ends it, refined between the last consumed
-      // sample (>= 0) and this one (< 0).
-      bool go_on = true, ended = false, cross = false;
-      float ta = t, fa = fp, fb = 0.0f;
-      int taken = 0;
+      // crossing) and kept the step size; then it is step i + j of the segment, taken
+      // while i + j < imax.  A step that finds its sample invalid still counts and
+      // ends the march; a crossing ends it with t and fp at the last consumed sample
+      // (>= 0) and fb at this one (< 0).
+      bool go_on = true;
+      const int left = imax - i;
 #pragma unroll
       for (int j = 0; j < kSpec; ++j) {
-        const bool in = go_on && s + j < a.max_steps;
-        const bool v = in && vk[j];
+        const bool v = go_on && j < left && vk[j];
         const bool x = v && fk[j] < 0.0f;
         const bool c = v && !x;
-        nsteps += in ? 1 : 0;
-        taken += v ? 1 : 0;
-        if (x) {
-          ta = j == 0 ? t : tk[j - 1];
-          fa = j == 0 ? fp : fk[j - 1];
-          fb = fk[j];
-        }
-        cross = cross || x;
-        ended = ended || (go_on && !c);
+        if (x) fb = fk[j];
+        if (go_on && !c) run = false;
         go_on = c && ((fk[j] >= 1.0f) == far);
         if (c) {
           t = tk[j];
@@ -505,12 +510,12 @@ __global__ __launch_bounds__(256) void raycast(RayArgs a) {
           ++i;
         }
       }
-      s += taken;
-      if (cross) {
-        ts = ta + st * (fa / (fa - fb));
-        found = true;
-      }
-      if (ended) break;
+      run = run && i < imax;
+    }
+    if (ok) nsteps = a.max_steps - (imax - i) + (i < imax ? 1 : 0);
+    if (fb < 0.0f) {
+      ts = t + (seg_far ? a.step_far_m : a.step_near_m) * (fp / (fp - fb));
+      found = true;
     }
   }
   // Normals of the wave's hits: trilinear central differences at the refined point.
@@ -518,7 +523,7 @@ __global__ __launch_bounds__(256) void raycast(RayArgs a) {
   {
     const f3 gh = found ? gpos(go, gd, ts) : f3{0.0f, 0.0f, 0.0f};
     float fq[6];
-    if (gradient_samples<FMT, OFF32>(a, found, gh, s_box[wave], fq)) {
+    if (gradient_samples<FMT, OFF32>(a, found, gh, fq)) {
       const f3 gr = f3{fq[0] - fq[1], fq[2] - fq[3], fq[4] - fq[5]};
       const float gl = sqrtf(dot(gr, gr));
       if (gl > 0.0f) {
