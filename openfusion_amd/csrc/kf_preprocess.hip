@@ -5,13 +5,12 @@
 // filter and 3-level pyramid the reference only mentions (CameraHandler.cu:6).
 // Maps are kept in the camera frame; the tracker applies the pose itself.
 //
-//   depth_to_l0   : uint16 -> metres, range gate, raylen = |K^-1 [x,y,1]| * d,
+//   depth_levels  : uint16 -> metres, range gate, raylen = |K^-1 [x,y,1]| * d,
 //                   bilateral filter (LDS tile with halo, spatial weights
 //                   from the kernel arguments, range weights from a
-//                   per-block LDS table)                             [per L0 pixel]
-//   pyr_down      : 2x2 block average gated by |d - centre| < gate, levels 1
-//                   and 2 in one launch (level 2 from the block's level-1
-//                   tile in LDS)                                       [per L1 pixel]
+//                   per-block LDS table); then levels 1 and 2 from the block's
+//                   filtered tile in LDS: 2x2 block average gated by
+//                   |d - centre| < gate                       [two L0 pixels]
 //   vertex_normal : v = d * K^-1 [x,y,1];  n = normalize((v(x,y+1)-v) x (v(x+1,y)-v))
 //                   (points towards the camera), all levels in one launch
 #include <type_traits>
@@ -22,14 +21,17 @@
 namespace kf {
 namespace {
 
-constexpr int kTile = 16;
+constexpr int kTileX = 32, kTileY = 16;  // level-0 pixels of a block
+constexpr int kThreads = kTileX * kTileY / 2;
 constexpr int kMaxRadius = 4;
-constexpr int kHalo = kTile + 2 * kMaxRadius;
 
 struct PreArgs {
   const uint16_t* depth;
   float* raylen;
   float* out;  // filtered level-0 depth
+  float *l1, *l2, *l2_copy;  // filtered depth of levels 1 and 2 (NULL: no such level) and a copy of level 2
+  int W1, H1, W2, H2;
+  float gate;
   int W, H;
   float fx, fy, cx, cy;
   float scale, dmin, dmax;
@@ -39,91 +41,6 @@ struct PreArgs {
   // host with the same exp_neg (kernel arguments: scalar registers in the kernel)
   float ws[(2 * kMaxRadius + 1) * (2 * kMaxRadius + 1)];
 };
-
-// Bilateral weight of a neighbour: exp(-|dp|^2 / 2 sigma_s^2) * exp(-dr^2 / 2 sigma_r^2)
-// with dr = |u_q - u_c| * scale (the integer depth-code difference in metres).  Both
-// factors are exp_neg values: the spatial ones made on the host (kernel arguments),
-// the range ones in a per-block LDS table for code differences below kRangeLut.
-// ZT: the range weight is exactly 0 from kRangeLut on (exp_neg's argument,
-// monotone in the difference, has reached 80 there), so larger differences need no
-// exp_neg of their own.
-constexpr int kRangeLut = 512;
-
-// R: the window half-size (a.radius), fixed per instance so that the window loop
-// unrolls.  Pixels outside the image are stored as code 0 in the tile, so the
-// window needs no bounds test of its own: such taps are skipped like invalid ones.
-template <int R, bool ZT>
-__global__ __launch_bounds__(256) void depth_to_l0(PreArgs a) {
-  __shared__ int tile[kHalo * kHalo];  // depth codes, 0 = invalid
-  __shared__ float wr[kRangeLut];
-  const int span = kTile + 2 * R;
-  const int bx = blockIdx.x * kTile, by = blockIdx.y * kTile;
-  const int tid = threadIdx.y * kTile + threadIdx.x;
-  // the tile and its halo, every load of a thread in flight at once (out-of-image
-  // entries read a clamped pixel and store 0)
-  constexpr int kPer = ((kTile + 2 * R) * (kTile + 2 * R) + kTile * kTile - 1) / (kTile * kTile);
-  int uv[kPer];
-#pragma unroll
-  for (int j = 0; j < kPer; ++j) {
-    const int i = min(tid + j * kTile * kTile, span * span - 1);
-    const int ty = i / span, tx = i - ty * span;
-    const int gx = bx + tx - R, gy = by + ty - R;
-    const int u = a.depth[min(max(gy, 0), a.H - 1) * a.W + min(max(gx, 0), a.W - 1)];
-    uv[j] = (gx >= 0 && gx < a.W && gy >= 0 && gy < a.H) ? u : 0;
-  }
-#pragma unroll
-  for (int j = 0; j < kPer; ++j) {
-    const int i = tid + j * kTile * kTile;
-    if (i < span * span) {
-      const float d = (float)uv[j] * a.scale;
-      tile[i] = (d >= a.dmin && d <= a.dmax) ? uv[j] : 0;
-    }
-  }
-  for (int i = tid; i < kRangeLut; i += kTile * kTile) {
-    const float rm = (float)i * a.scale;
-    wr[i] = exp_neg((rm * rm) * a.inv2sr);
-  }
-  __syncthreads();
-  const int x = bx + threadIdx.x, y = by + threadIdx.y;
-  if (x >= a.W || y >= a.H) return;
-  const int uc = tile[(threadIdx.y + R) * span + threadIdx.x + R];
-  const int idx = y * a.W + x;
-  if (uc == 0) {
-    a.raylen[idx] = 0.0f;
-    a.out[idx] = 0.0f;
-    return;
-  }
-  const float dc = (float)uc * a.scale;
-  const float xn = ((float)x - a.cx) / a.fx;
-  const float yn = ((float)y - a.cy) / a.fy;
-  const float lam = sqrtf((xn * xn + yn * yn) + 1.0f);
-  a.raylen[idx] = dc * lam;
-
-  float sw = 0.0f, swd = 0.0f;
-#pragma unroll
-  for (int dy = -R; dy <= R; ++dy) {
-#pragma unroll
-    for (int dx = -R; dx <= R; ++dx) {
-      const int uq = tile[(threadIdx.y + R + dy) * span + threadIdx.x + R + dx];
-      if (uq == 0) continue;
-      const int du = uq > uc ? uq - uc : uc - uq;
-      float w_r;
-      if (ZT) {
-        w_r = du < kRangeLut ? wr[min(du, kRangeLut - 1)] : 0.0f;
-      } else if (du < kRangeLut) {
-        w_r = wr[du];
-      } else {
-        const float rm = (float)du * a.scale;
-        w_r = exp_neg((rm * rm) * a.inv2sr);
-      }
-      const float w = a.ws[(dy + R) * (2 * R + 1) + (dx + R)] * w_r;
-      const float dq = (float)uq * a.scale;
-      sw = sw + w;
-      swd = swd + w * dq;
-    }
-  }
-  a.out[idx] = swd / sw;
-}
 
 // One coarse pixel: the mean of the valid samples of its 2x2 block (those inside
 // the fine level) within `gate` of the block's top-left sample, 0 when that one is
@@ -152,33 +69,157 @@ __device__ __forceinline__ float pyr_pixel(const Get& get, int x, int y, int Wi,
   return r;
 }
 
-// Levels 1 and 2 of the pyramid in one launch: a kTile x kTile block makes its tile
-// of level 1 from level 0, keeps it in LDS, and makes the (kTile / 2)^2 level-2
-// pixels under it from there (a level-2 block reads only level-1 pixels of its own
-// tile, since tiles start at even coordinates).  l2 == nullptr: level 1 only.
-// l2_copy (optional): a second destination of level 2 (same layout).
-__global__ __launch_bounds__(kTile * kTile) void pyr_down(const float* l0, int W0, int H0, float* l1, int W1, int H1,
-                                                          float* l2, int W2, int H2, float gate, float* l2_copy) {
-  __shared__ float t1[kTile][kTile];
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  const int x = blockIdx.x * kTile + tx, y = blockIdx.y * kTile + ty;
-  float r = 0.0f;
-  if (x < W1 && y < H1) {
-    r = pyr_pixel([&](int sx, int sy) { return l0[sy * W0 + sx]; }, x, y, W0, H0, gate);
-    l1[y * W1 + x] = r;
-  }
-  if (l2 == nullptr) return;  // uniform
-  t1[ty][tx] = r;
-  __syncthreads();
-  constexpr int kHalf = kTile / 2;
-  if (tx >= kHalf || ty >= kHalf) return;
-  const int x2 = blockIdx.x * kHalf + tx, y2 = blockIdx.y * kHalf + ty;
-  if (x2 >= W2 || y2 >= H2) return;
-  const int bx = blockIdx.x * kTile, by = blockIdx.y * kTile;  // the tile's level-1 origin
-  const float r2 = pyr_pixel([&](int sx, int sy) { return t1[sy - by][sx - bx]; }, x2, y2, W1, H1, gate);
-  l2[y2 * W2 + x2] = r2;
-  if (l2_copy) l2_copy[y2 * W2 + x2] = r2;
+// Bilateral weight of a neighbour: exp(-|dp|^2 / 2 sigma_s^2) * exp(-dr^2 / 2 sigma_r^2)
+// with dr = |u_q - u_c| * scale (the integer depth-code difference in metres).  Both
+// factors are exp_neg values: the spatial ones made on the host (kernel arguments),
+// the range ones in a per-block LDS table for code differences below kRangeLut.
+// ZT: the range weight is exactly 0 from kRangeLut on (exp_neg's argument,
+// monotone in the difference, has reached 80 there), so larger differences need no
+// exp_neg of their own: the table ends with a 0 that they all read.
+constexpr int kRangeLut = 512;
+// Codes are held times four, so that a difference is the table's byte offset; an invalid
+// pixel's is farther than any table entry from every valid one.
+constexpr int kInvalid = 1 << 24;
+
+// |a - b| in one instruction.
+__device__ __forceinline__ unsigned abs_diff(unsigned a, unsigned b) {
+  unsigned d;
+  asm("v_sad_u32 %0, %1, %2, 0" : "=v"(d) : "v"(a), "v"(b));
+  return d;
 }
+
+// A block filters kTileX x kTileY pixels, a pair of neighbours per thread (the 2R + 2
+// codes of a window row are read once for both), and makes the coarser levels' pixels
+// under them (tiles start at multiples of 4, so they need no other block's).  R: the
+// window half-size (a.radius), fixed per instance so that the window loop unrolls.
+// Pixels outside the image are invalid in the tile, so the window needs no bounds test
+// of its own; an invalid tap has weight 0, which adds exactly nothing (sums are >= 0).
+//
+// Bound by latency: a wavefront lives 7 us, half of it waiting (the frame's first touch,
+// the LDS reads, the barriers before the coarser levels), with vector pipes busy for 3.8
+// and LDS for 2.4 us of a 640x480 frame.  In one launch and with a window row's codes and
+// metres read once for two pixels 9.6 us, where a pixel per thread and a second launch for
+// the coarser levels took 10.9 + 3.7.  A table of weight products per window distance
+// (no products per tap) took as long.
+template <int R, bool ZT>
+__global__ __launch_bounds__(kThreads) void depth_levels(PreArgs a) {
+  constexpr int kSpanX = kTileX + 2 * R, kSpanY = kTileY + 2 * R, kSpan = kSpanX * kSpanY;
+  __shared__ __align__(8) int tile[kSpan];      // four times the depth codes
+  __shared__ __align__(8) float metres[kSpan];  // the same in metres, 0 = invalid
+  __shared__ float wr[kRangeLut + 1], s_xn[kTileX], s_yn[kTileY];
+  __shared__ float t0[kTileY][kTileX], t1[kTileY / 2][kTileX / 2];
+  const int bx = blockIdx.x * kTileX, by = blockIdx.y * kTileY;
+  const int tid = threadIdx.x;
+  // the tile and its halo, a row per wavefront and pass, every load of a thread in flight
+  // at once (out-of-image entries read a clamped pixel and are dropped)
+  constexpr int kWaves = kThreads / kWave, kPer = (kSpanY + kWaves - 1) / kWaves;
+  static_assert(kSpanX <= kWave, "a row per wavefront");
+  const int lane = tid & (kWave - 1), wave = tid / kWave;
+  const int gx = bx + lane - R;
+  const bool col = gx >= 0 && gx < a.W;
+  int uv[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int gy = by + wave + j * kWaves - R;
+    const int u = a.depth[min(max(gy, 0), a.H - 1) * a.W + min(max(gx, 0), a.W - 1)];
+    uv[j] = col && gy >= 0 && gy < a.H ? u : 0;
+  }
+  for (int i = tid; i <= kRangeLut; i += kThreads) {
+    const float rm = (float)i * a.scale;
+    wr[i] = i < kRangeLut ? exp_neg((rm * rm) * a.inv2sr) : 0.0f;
+  }
+  if (tid < kTileX)
+    s_xn[tid] = ((float)(bx + tid) - a.cx) / a.fx;
+  else if (tid < kTileX + kTileY)
+    s_yn[tid - kTileX] = ((float)(by + tid - kTileX) - a.cy) / a.fy;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int ty = wave + j * kWaves;
+    if (lane < kSpanX && ty < kSpanY) {
+      const float d = (float)uv[j] * a.scale;
+      const bool ok = uv[j] != 0 && d >= a.dmin && d <= a.dmax;
+      tile[ty * kSpanX + lane] = ok ? 4 * uv[j] : kInvalid;
+      metres[ty * kSpanX + lane] = ok ? d : 0.0f;
+    }
+  }
+  __syncthreads();
+  const int px = 2 * (tid % (kTileX / 2)), py = tid / (kTileX / 2);  // the pair's first pixel in the tile
+  int uc[2];
+  float sw[2] = {0.0f, 0.0f}, swd[2] = {0.0f, 0.0f};
+#pragma unroll
+  for (int p = 0; p < 2; ++p) uc[p] = tile[(py + R) * kSpanX + px + p + R];
+#pragma unroll
+  for (int dy = -R; dy <= R; ++dy) {
+    int u[2 * R + 2];
+    float m[2 * R + 2];
+    const int row = (py + R + dy) * kSpanX + px;
+#pragma unroll
+    for (int i = 0; i < 2 * R + 2; i += 2) {
+      const int2 u2 = *reinterpret_cast<const int2*>(&tile[row + i]);
+      const float2 m2 = *reinterpret_cast<const float2*>(&metres[row + i]);
+      u[i] = u2.x;
+      u[i + 1] = u2.y;
+      m[i] = m2.x;
+      m[i + 1] = m2.y;
+    }
+#pragma unroll
+    for (int dx = -R; dx <= R; ++dx) {
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int uq = u[dx + R + p];
+        const unsigned du4 = abs_diff((unsigned)uq, (unsigned)uc[p]);
+        float w_r = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(wr) + min(du4, 4u * kRangeLut));
+        if (!ZT && du4 >= 4u * kRangeLut && uq != kInvalid) {
+          const float rm = (float)(du4 / 4u) * a.scale;
+          w_r = exp_neg((rm * rm) * a.inv2sr);
+        }
+        const float w = a.ws[(dy + R) * (2 * R + 1) + (dx + R)] * w_r;
+        sw[p] = sw[p] + w;
+        swd[p] = swd[p] + w * m[dx + R + p];
+      }
+    }
+  }
+  const int x = bx + px, y = by + py;
+  const float yn = s_yn[py];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const bool ok = uc[p] != kInvalid;
+    const float f = ok ? swd[p] / sw[p] : 0.0f;
+    t0[py][px + p] = f;
+    if (x + p < a.W && y < a.H) {
+      const float xn = s_xn[px + p];
+      const float lam = sqrtf((xn * xn + yn * yn) + 1.0f);
+      const int idx = y * a.W + x + p;
+      a.raylen[idx] = ok ? metres[(py + R) * kSpanX + px + p + R] * lam : 0.0f;
+      a.out[idx] = f;
+    }
+  }
+  if (!a.l1) return;  // uniform
+  __syncthreads();
+  if (tid < kThreads / 2) {
+    const int tx = tid % (kTileX / 2), ty = tid / (kTileX / 2);
+    const int x1 = bx / 2 + tx, y1 = by / 2 + ty;
+    float r = 0.0f;
+    if (x1 < a.W1 && y1 < a.H1) {
+      r = pyr_pixel([&](int sx, int sy) { return t0[sy - by][sx - bx]; }, x1, y1, a.W, a.H, a.gate);
+      a.l1[y1 * a.W1 + x1] = r;
+    }
+    t1[ty][tx] = r;
+  }
+  if (!a.l2) return;  // uniform
+  __syncthreads();
+  if (tid < kThreads / 8) {
+    const int tx = tid % (kTileX / 4), ty = tid / (kTileX / 4);
+    const int x2 = bx / 4 + tx, y2 = by / 4 + ty;
+    if (x2 < a.W2 && y2 < a.H2) {
+      const float r = pyr_pixel([&](int sx, int sy) { return t1[sy - by / 2][sx - bx / 2]; }, x2, y2, a.W1, a.H1, a.gate);
+      a.l2[y2 * a.W2 + x2] = r;
+      if (a.l2_copy) a.l2_copy[y2 * a.W2 + x2] = r;
+    }
+  }
+}
+
+constexpr int kMapX = 64, kMapY = 4;
 
 struct LevelMapArgs {
   const float* depth;
@@ -193,15 +234,12 @@ struct MapArgs {
   int levels;
 };
 
-__device__ __forceinline__ f3 backproject(const LevelMapArgs& a, int x, int y) {
-  const float d = a.depth[y * a.W + x];
-  if (d == 0.0f) return f3{nanf_(), nanf_(), nanf_()};
-  const float xn = ((float)x - a.cx) / a.fx;
-  const float yn = ((float)y - a.cy) / a.fy;
-  return f3{xn * d, yn * d, d};
-}
-
-__global__ __launch_bounds__(256) void vertex_normal(MapArgs m) {
+// Vertices and normals, one pixel per thread, a wavefront per kMapX pixels of a row (its
+// six planes' stores are whole lines).  x and y in camera units are divided once per
+// block, not four times per pixel.  Bound by its stores; 640x480 and two coarser levels:
+// 4.8 us (16x16 blocks that divided per pixel: 6.1).
+__global__ __launch_bounds__(kMapX * kMapY) void vertex_normal(MapArgs m) {
+  __shared__ float s_xn[kMapX + 1], s_yn[kMapY + 1];
   int b = blockIdx.x;
   int l = 0;
   for (int i = 1; i < m.levels; ++i)
@@ -209,19 +247,26 @@ __global__ __launch_bounds__(256) void vertex_normal(MapArgs m) {
   const LevelMapArgs& a = m.lv[l];
   b -= a.block_begin;
   const int by = b / a.blocks_x, bx = b - by * a.blocks_x;
-  const int x = bx * kTile + (threadIdx.x & (kTile - 1));
-  const int y = by * kTile + (threadIdx.x >> 4);
-  if (x >= a.W || y >= a.H) return;
-  const int idx = y * a.W + x;
-  const f3 v = backproject(a, x, y);
-  a.vx[idx] = v.x;
-  a.vy[idx] = v.y;
-  a.vz[idx] = v.z;
-  f3 n = f3{nanf_(), nanf_(), nanf_()};
-  if (v.z == v.z && x + 1 < a.W && y + 1 < a.H) {
-    const f3 vr = backproject(a, x + 1, y);
-    const f3 vd = backproject(a, x, y + 1);
-    if (vr.z == vr.z && vd.z == vd.z) {
+  const int tx = threadIdx.x % kMapX, ty = threadIdx.x / kMapX;
+  const int x = bx * kMapX + tx, y = by * kMapY + ty;
+  // the pixel's depth and its right and lower neighbours' (clamped, dropped at the edges)
+  const bool in = x < a.W && y < a.H, edge = x + 1 >= a.W || y + 1 >= a.H;
+  const int idx = in ? y * a.W + x : 0;
+  const float d = a.depth[idx], dr = a.depth[edge ? idx : idx + 1], dd = a.depth[edge ? idx : idx + a.W];
+  for (int i = threadIdx.x; i < kMapX + kMapY + 2; i += kMapX * kMapY) {
+    if (i <= kMapX)
+      s_xn[i] = ((float)(bx * kMapX + i) - a.cx) / a.fx;
+    else
+      s_yn[i - kMapX - 1] = ((float)(by * kMapY + i - kMapX - 1) - a.cy) / a.fy;
+  }
+  __syncthreads();
+  if (!in) return;
+  const float xn = s_xn[tx], yn = s_yn[ty];
+  f3 v = f3{nanf_(), nanf_(), nanf_()}, n = v;
+  if (d != 0.0f) {
+    v = f3{xn * d, yn * d, d};
+    if (!edge && dr != 0.0f && dd != 0.0f) {
+      const f3 vr = f3{s_xn[tx + 1] * dr, yn * dr, dr}, vd = f3{xn * dd, s_yn[ty + 1] * dd, dd};
       const f3 c = cross(sub(vd, v), sub(vr, v));
       const float len = sqrtf(dot(c, c));
       if (len > 0.0f) {
@@ -230,6 +275,9 @@ __global__ __launch_bounds__(256) void vertex_normal(MapArgs m) {
       }
     }
   }
+  a.vx[idx] = v.x;
+  a.vy[idx] = v.y;
+  a.vz[idx] = v.z;
   a.nx[idx] = n.x;
   a.ny[idx] = n.y;
   a.nz[idx] = n.z;
@@ -273,36 +321,29 @@ kf_status launch_preprocess(const kf_intrinsics& k0, const kf_preprocess_params&
       a.ws[(dy + R) * (2 * R + 1) + (dx + R)] = exp_neg((float)(dx * dx + dy * dy) * a.inv2ss);
   const float rm_lut = (float)kRangeLut * a.scale;
   const bool zt = exp_neg((rm_lut * rm_lut) * a.inv2sr) == 0.0f;
-  dim3 blk(kTile, kTile);
-  dim3 grd(div_up(k0.width, kTile), div_up(k0.height, kTile));
+  const bool one = live.levels > 1, two = live.levels > 2;
+  a.l1 = one ? live.level[1].depth : nullptr;
+  a.l2 = two ? live.level[2].depth : nullptr;
+  a.l2_copy = two ? l2_copy : nullptr;
+  a.W1 = one ? live.level[1].width : 0;
+  a.H1 = one ? live.level[1].height : 0;
+  a.W2 = two ? live.level[2].width : 0;
+  a.H2 = two ? live.level[2].height : 0;
+  a.gate = p.pyramid_gate_m;
+  const dim3 grd(div_up(k0.width, kTileX), div_up(k0.height, kTileY));
   auto pick = [&](auto zt_tag) {
     constexpr bool Z = decltype(zt_tag)::value;
     switch (R) {
-      case 0: return depth_to_l0<0, Z>;
-      case 1: return depth_to_l0<1, Z>;
-      case 2: return depth_to_l0<2, Z>;
-      case 3: return depth_to_l0<3, Z>;
-      default: return depth_to_l0<4, Z>;
+      case 0: return depth_levels<0, Z>;
+      case 1: return depth_levels<1, Z>;
+      case 2: return depth_levels<2, Z>;
+      case 3: return depth_levels<3, Z>;
+      default: return depth_levels<4, Z>;
     }
   };
   auto kern = zt ? pick(std::true_type{}) : pick(std::false_type{});
-  hipLaunchKernelGGL(kern, grd, blk, 0, s, a);
-  KF_TRY(check_launch("depth_to_l0"));
-
-  if (live.levels > 1) {  // levels 1 and 2 together; level 2's tiles lie under level 1's
-    const kf_level_maps& m0 = live.level[0];
-    const kf_level_maps& m1 = live.level[1];
-    const bool two = live.levels > 2;
-    const kf_level_maps* m2 = two ? &live.level[2] : nullptr;
-    KF_CHECK_ARG(!two || (div_up(m2->width, kTile / 2) <= div_up(m1.width, kTile) &&
-                          div_up(m2->height, kTile / 2) <= div_up(m1.height, kTile)),
-                 "level 2 larger than half of level 1");
-    dim3 g1(div_up(m1.width, kTile), div_up(m1.height, kTile));
-    hipLaunchKernelGGL(pyr_down, g1, blk, 0, s, (const float*)m0.depth, m0.width, m0.height, m1.depth, m1.width,
-                       m1.height, two ? m2->depth : nullptr, two ? m2->width : 0, two ? m2->height : 0,
-                       p.pyramid_gate_m, two ? l2_copy : nullptr);
-    KF_TRY(check_launch("pyr_down"));
-  }
+  hipLaunchKernelGGL(kern, grd, dim3(kThreads), 0, s, a);
+  KF_TRY(check_launch("depth_levels"));
 
   MapArgs m;
   int blocks = 0;
@@ -316,11 +357,11 @@ kf_status launch_preprocess(const kf_intrinsics& k0, const kf_preprocess_params&
     la.nx = lm.nx; la.ny = lm.ny; la.nz = lm.nz;
     la.W = kl.width; la.H = kl.height;
     la.fx = kl.fx; la.fy = kl.fy; la.cx = kl.cx; la.cy = kl.cy;
-    la.blocks_x = div_up(kl.width, kTile);
+    la.blocks_x = div_up(kl.width, kMapX);
     la.block_begin = blocks;
-    blocks += la.blocks_x * div_up(kl.height, kTile);
+    blocks += la.blocks_x * div_up(kl.height, kMapY);
   }
-  hipLaunchKernelGGL(vertex_normal, dim3(blocks), dim3(256), 0, s, m);
+  hipLaunchKernelGGL(vertex_normal, dim3(blocks), dim3(kMapX * kMapY), 0, s, m);
   return check_launch("vertex_normal");
 }
 
