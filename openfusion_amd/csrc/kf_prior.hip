@@ -272,6 +272,7 @@ struct kf_prior {
   long step = 0;
   // activations (NHWC), sized for max_batch
   uint16_t* Yb[kf::kConvs - 1] = {};  // layers 1-3, BF16 NHWC
+  uint8_t* signs[kf::kConvs - 1] = {};  // bit i of byte b: value 8 b + i of Yb is positive
   float* Y4 = nullptr;                // layer 4, FP32
   uint16_t* X5b = nullptr;
   uint16_t* Hb = nullptr;
@@ -314,26 +315,29 @@ constexpr int kConvBlocks = 512;
 // One convolution of the training forward: two blocks of four waves a CU hold the
 // weights; a small batch gets one wave per 16-pixel tile and channel group.
 template <int L, int NT, bool F32>
-kf_status launch_conv(kf_prior* P, const uint16_t* X, uint16_t* Yb, float* Y, int B, hipStream_t s) {
+kf_status launch_conv(kf_prior* P, const uint16_t* X, uint16_t* Yb, float* Y, uint8_t* signs, int B, hipStream_t s) {
   constexpr ConvShape c = kConv[L];
   constexpr int GROUPS = c.cout / (16 * NT);
   const ParamLayout& lay = layout();
   const int M = B * c.hout * c.wout;
   const int blocks = std::min(div_up(div_up(M, 16) * GROUPS, kConvWaves), kConvBlocks);
   hipLaunchKernelGGL((conv_forward<L, NT, F32>), dim3(blocks), dim3(kConvThreads), 0, s, X, P->wbf + lay.w[L],
-                     (const float*)P->params + lay.b[L], Yb, Y, M);
+                     (const float*)P->params + lay.b[L], Yb, Y, signs, M);
   return check_launch("conv_forward");
 }
 
-// Training forward of the convolutions: the activations stay for the backward pass.
-kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, int B, hipStream_t s) {
+// Training forward of the convolutions: the activations stay for the backward pass, and
+// (train) the signs of layers 1-3.
+kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, int B, bool train, hipStream_t s) {
   const ParamLayout& L = layout();
+  uint8_t* none[kConvs - 1] = {};
+  uint8_t* const* signs = train ? P->signs : none;
   hipLaunchKernelGGL(conv1_forward, dim3(kConv[0].hout / kL1Rows, B), dim3(kConvThreads), 0, s, frames, pairs,
-                     (const uint16_t*)P->wbf + L.w[0], (const float*)P->params + L.b[0], P->Yb[0]);
+                     (const uint16_t*)P->wbf + L.w[0], (const float*)P->params + L.b[0], P->Yb[0], signs[0]);
   KF_TRY(check_launch("conv1_forward"));
-  KF_TRY((launch_conv<1, 4, false>(P, P->Yb[0], P->Yb[1], nullptr, B, s)));
-  KF_TRY((launch_conv<2, 2, false>(P, P->Yb[1], P->Yb[2], nullptr, B, s)));
-  return launch_conv<3, 2, true>(P, P->Yb[2], nullptr, P->Y4, B, s);
+  KF_TRY((launch_conv<1, 4, false>(P, P->Yb[0], P->Yb[1], nullptr, signs[1], B, s)));
+  KF_TRY((launch_conv<2, 2, false>(P, P->Yb[1], P->Yb[2], nullptr, signs[2], B, s)));
+  return launch_conv<3, 2, true>(P, P->Yb[2], nullptr, P->Y4, nullptr, B, s);
 }
 
 // Inference, with the training forward's outputs either way.  The fused kernel's blocks
@@ -346,7 +350,7 @@ kf_status infer(kf_prior* P, const float* frames, const int32_t* pairs, const fl
                 hipStream_t s) {
   const ParamLayout& L = layout();
   if (B >= kLayeredBatch) {
-    KF_TRY(forward(P, frames, pairs, B, s));
+    KF_TRY(forward(P, frames, pairs, B, false, s));
     hipLaunchKernelGGL(head_infer, dim3(B), dim3(kConvThreads), 0, s, (const float*)P->Y4, prev,
                        (const uint16_t*)P->wt + weight_copies().w5, (const uint16_t*)P->wbf + L.w[5],
                        (const float*)P->params + L.b[4], (const float*)P->params + L.b[5], out);
@@ -385,6 +389,7 @@ kf_status launch_backward(kf_prior* P, int B, int* splits, int* planes, hipStrea
   ConvBackArgs a;
   a.dY = P->dYb[L];
   a.X = P->Yb[L - 1];
+  a.signs = P->signs[L - 1];
   a.Wt = P->wt + layout().w[L];
   a.dX = P->dYb[L - 1];
   a.wpart = P->wpart[L];
@@ -492,7 +497,10 @@ extern "C" kf_status kf_prior_destroy(kf_prior* P) {
                   P->fuse_count};
   for (void* q : ptrs) (void)hipFree(q);
   for (int l = 0; l < kConvs; ++l) {
-    if (l + 1 < kConvs) (void)hipFree(P->Yb[l]);
+    if (l + 1 < kConvs) {
+      (void)hipFree(P->Yb[l]);
+      (void)hipFree(P->signs[l]);
+    }
     (void)hipFree(P->wpart[l]);
     (void)hipFree(P->dYb[l]);
     (void)hipFree(P->bpart[l]);
@@ -521,7 +529,10 @@ extern "C" kf_status kf_prior_create(int32_t max_batch, kf_prior** out) {
   for (int l = 0; l < kConvs; ++l) {
     const ConvShape& c = kConv[l];
     const long M = B * c.hout * c.wout;
-    if (l + 1 < kConvs) al((void**)&P->Yb[l], M * c.cout * 2);
+    if (l + 1 < kConvs) {
+      al((void**)&P->Yb[l], M * c.cout * 2);
+      al((void**)&P->signs[l], M * c.cout / 8);
+    }
     else al((void**)&P->Y4, M * c.cout * 4);
     al((void**)&P->wpart[l], (l == 0 ? kConvBlocks : kWgradBlocks / (c.cout / (l == 1 ? 64 : 32))) * c.cout * c.kc * 4);
     al((void**)&P->dYb[l], M * c.cout * 2);
@@ -602,7 +613,7 @@ extern "C" kf_status kf_prior_gradients(kf_prior* P, const float* frames, const 
                                         const float* target, int32_t B, float* d_grad, float* d_loss, kf_stream s) {
   KF_TRY(check_batch(P, frames, pairs, prev, B));
   KF_CHECK_ARG(target && d_grad, "NULL argument");
-  KF_TRY(forward(P, frames, pairs, B, S(s)));
+  KF_TRY(forward(P, frames, pairs, B, true, S(s)));
   return backward(P, frames, pairs, prev, target, B, d_grad, d_loss, S(s));
 }
 
@@ -610,7 +621,7 @@ extern "C" kf_status kf_prior_train_step(kf_prior* P, const float* frames, const
                                          const float* target, int32_t B, float lr, float* d_loss, kf_stream s) {
   KF_TRY(check_batch(P, frames, pairs, prev, B));
   KF_CHECK_ARG(target != nullptr, "target is NULL");
-  KF_TRY(forward(P, frames, pairs, B, S(s)));
+  KF_TRY(forward(P, frames, pairs, B, true, S(s)));
   KF_TRY(backward(P, frames, pairs, prev, target, B, P->grad, d_loss, S(s)));
   P->step += 1;
   const float b1 = 0.9f, b2 = 0.999f;

@@ -24,23 +24,48 @@ __device__ __forceinline__ int tile_channel(int t, int i) {
   return (i >> 2) * 4 * NT + 4 * t + (i & 3);
 }
 
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
-  return (uint32_t)bf16_rne(lo) | ((uint32_t)bf16_rne(hi) << 16);
-}
-
 // Stores N (a multiple of 4) floats as BF16 to p (8-byte aligned; 16-byte aligned when N is a multiple of 8).
 template <int N>
-__device__ __forceinline__ void store_bf16(uint16_t* p, const float* v) {
+__device__ __forceinline__ void store_words(uint16_t* p, const uint32_t* w) {
   if constexpr (N % 8 == 0) {
 #pragma unroll
-    for (int i = 0; i < N; i += 8)
-      *reinterpret_cast<uint4*>(p + i) = make_uint4(pack_bf16(v[i], v[i + 1]), pack_bf16(v[i + 2], v[i + 3]),
-                                                    pack_bf16(v[i + 4], v[i + 5]), pack_bf16(v[i + 6], v[i + 7]));
+    for (int i = 0; i < N / 2; i += 4) *reinterpret_cast<uint4*>(p + 2 * i) = make_uint4(w[i], w[i + 1], w[i + 2], w[i + 3]);
   } else {
 #pragma unroll
-    for (int i = 0; i < N; i += 4)
-      *reinterpret_cast<uint2*>(p + i) = make_uint2(pack_bf16(v[i], v[i + 1]), pack_bf16(v[i + 2], v[i + 3]));
+    for (int i = 0; i < N / 2; i += 2) *reinterpret_cast<uint2*>(p + 2 * i) = make_uint2(w[i], w[i + 1]);
   }
+}
+template <int N>
+__device__ __forceinline__ void store_bf16(uint16_t* p, const float* v) {
+  uint32_t w[N / 2];
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) w[i] = pack_bf16(v[2 * i], v[2 * i + 1]);
+  store_words<N>(p, w);
+}
+
+// The same, and (bits not NULL) which of the N (8 or 16) stored values are positive, value
+// i in bit i: all that the backward pass needs of them under a ReLU, in a sixteenth of
+// the bytes.
+template <int N>
+__device__ __forceinline__ void store_bf16_signs(uint16_t* p, uint8_t* bits, const float* v) {
+  typedef short s2 __attribute__((ext_vector_type(2)));
+  typedef unsigned short u2 __attribute__((ext_vector_type(2)));
+  uint32_t w[N / 2], m = 0;
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) w[i] = pack_bf16(v[2 * i], v[2 * i + 1]);
+  store_words<N>(p, w);
+  if (!bits) return;  // uniform
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) {
+    const s2 pos = __builtin_elementwise_max(__builtin_bit_cast(s2, w[i]), (s2){0, 0});
+    const u2 one = __builtin_elementwise_min(__builtin_bit_cast(u2, pos), (u2){1, 1});
+    m |= __builtin_bit_cast(uint32_t, one) << 2 * i;  // value 2 i in bit 2 i, 2 i + 1 in bit 16 + 2 i
+  }
+  m |= m >> 15;
+  if constexpr (N == 8)
+    *bits = (uint8_t)m;
+  else
+    *reinterpret_cast<uint16_t*>(bits) = (uint16_t)m;
 }
 
 // Layer 1 forward: a block makes four output rows of one sample.  The nine input rows
@@ -73,7 +98,8 @@ __device__ __forceinline__ void stage_l1(uint32_t (*patch)[kL1Pitch], const floa
 }
 
 __global__ __launch_bounds__(kConvThreads) void conv1_forward(const float* frames, const int32_t* pairs,
-                                                              const uint16_t* W, const float* bias, uint16_t* Yb) {
+                                                              const uint16_t* W, const float* bias, uint16_t* Yb,
+                                                              uint8_t* signs) {
   constexpr ConvShape c = kConv[0];
   __shared__ uint32_t patch[kL1In][kL1Pitch];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
@@ -116,7 +142,8 @@ __global__ __launch_bounds__(kConvThreads) void conv1_forward(const float* frame
 #pragma unroll
       for (int j = 0; j < 4; ++j) y[4 * t + j] = fmaxf(acc[j] + b[4 * t + j], 0.0f);
     }
-    store_bf16<8>(Yb + (((long)n * c.hout + oy0 + oy) * c.wout + ox) * c.cout + 8 * q, y);
+    const long o = (((long)n * c.hout + oy0 + oy) * c.wout + ox) * c.cout + 8 * q;
+    store_bf16_signs<8>(Yb + o, signs ? signs + o / 8 : nullptr, y);
   }
 }
 
@@ -128,7 +155,7 @@ __global__ __launch_bounds__(kConvThreads) void conv1_forward(const float* frame
 // pixel's channels); F32: FP32 output (layer 4, which the pooling reads), else BF16.
 template <int L, int NT, bool F32>
 __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* X, const uint16_t* W, const float* bias,
-                                                                uint16_t* Yb, float* Y, int M) {
+                                                                uint16_t* Yb, float* Y, uint8_t* signs, int M) {
   constexpr ConvShape c = kConv[L];
   constexpr int KS = c.kc / 32, GROUPS = c.cout / (16 * NT);
   static_assert(2 * c.wout == c.win && c.kc == 9 * c.cin && c.cin % 32 == 0, "layer shape");
@@ -178,7 +205,7 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* 
 #pragma unroll
       for (int i = 0; i < 4 * NT; i += 4) *reinterpret_cast<float4*>(Y + o + i) = make_float4(y[i], y[i + 1], y[i + 2], y[i + 3]);
     } else {
-      store_bf16<4 * NT>(Yb + o, y);
+      store_bf16_signs<4 * NT>(Yb + o, signs ? signs + o / 8 : nullptr, y);
     }
   }
 }
@@ -186,15 +213,16 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* 
 // Input gradient of layer L (1..3), ReLU mask of the layer below and that layer's bias
 // sums in one pass: dX[n][iy][ix][ci] = sum over the taps (ky, kx) that reach the
 // pixel, in that order, of sum_co dY[n][oy][ox][co] W[co][(ky, kx, ci)]; 0 where the
-// forward map Xb is not positive.  A wave takes 16 2x2 pixel blocks (rows 2j, 2j + 1,
+// forward map is not positive (its signs, one bit a value).  A wave takes 16 2x2 pixel blocks (rows 2j, 2j + 1,
 // columns 2i, 2i + 1): with stride 2 their nine taps read only the four output pixels
 // (j .. j + 1, i .. i + 1), so dY is read four times and every product is needed.
 // The weights ([tap][ci][co], so that eight co are one vector) stay in 144 registers.
 // Each tap's product is an MFMA chain of its own from zero and the taps are added in
 // FP32: the bits of a column-gradient GEMM followed by col2im, without the FP32 column
 // matrix (354 MB for layer 2 at batch 256).  bpart: per block and channel the FP32 sum
-// of the unrounded gradients.  Batch 256: layers 2 / 3 / 4 in 50 / 34 / 27 us (layer 2:
-// 197 MB through memory); the GEMM, col2im, conversion and column sums took 4.3 ms.
+// of the unrounded gradients.  Bound by memory: layer 2 at batch 256 moves 123 MB (197 with
+// the forward map in place of its signs: the three layers' backward passes 160 us, now
+// 140); the GEMM, col2im, conversion and column sums took 4.3 ms.
 // Block `block` of `blocks`; s_b: kDgradLds floats of LDS.
 template <int L>
 struct DgradShape {
@@ -204,7 +232,7 @@ struct DgradShape {
 constexpr int kDgradLds = kConvWaves * 32;
 
 template <int L>
-__device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* Wt, const uint16_t* Xb, uint16_t* dX,
+__device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* Wt, const uint8_t* signs, uint16_t* dX,
                                             float* bpart, int M, int block, int blocks, float* s_sum) {
   constexpr ConvShape c = kConv[L];
   constexpr int NT = DgradShape<L>::NT, KS = c.cout / 32, GROUPS = DgradShape<L>::GROUPS, CH = 4 * NT;
@@ -231,6 +259,17 @@ __device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* 
     const int m = live ? tile * 16 + r : M - 1;
     const int n = m / (c.hout * c.wout), p = m - n * (c.hout * c.wout);
     const int j = p / c.wout, i = p - j * c.wout;
+    // the four pixels' sign bits of the lane's channels
+    uint32_t sign[2][2];
+    int out[2][2];
+#pragma unroll
+    for (int py = 0; py < 2; ++py)
+#pragma unroll
+      for (int px = 0; px < 2; ++px) {
+        const int iy = min(2 * j + py, c.hin - 1), ix = 2 * i + px;
+        out[py][px] = ((n * c.hin + iy) * c.win + ix) * c.cin + ch0 + CH * q;
+        sign[py][px] = (uint32_t)signs[(unsigned)out[py][px] / 8u] >> (out[py][px] & 4);
+      }
     uint4 a[2][2][KS];  // dY at (j + dj, i + di), 0 outside the map
 #pragma unroll
     for (int dj = 0; dj < 2; ++dj)
@@ -265,17 +304,14 @@ __device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* 
               for (int e = 0; e < 4; ++e) sum[4 * t + e] = sum[4 * t + e] + acc[e];
             }
           }
-        const int iy = 2 * j + py, ix = 2 * i + px;
-        if (live && (c.hin == 2 * c.hout || iy < c.hin)) {
-          const int o = ((n * c.hin + iy) * c.win + ix) * c.cin + ch0 + CH * q;
-          uint16_t x[CH];
-          __builtin_memcpy(x, __builtin_assume_aligned(Xb + o, 2 * CH), 2 * CH);
+        if (live && (c.hin == 2 * c.hout || 2 * j + py < c.hin)) {
 #pragma unroll
           for (int e = 0; e < CH; ++e) {
-            sum[e] = (int16_t)x[e] > 0 ? sum[e] : 0.0f;
+            const int keep = (int)(sign[py][px] << (31 - e)) >> 31;  // 0 or all ones
+            sum[e] = __int_as_float(__float_as_int(sum[e]) & keep);
             bs[e] = bs[e] + sum[e];
           }
-          store_bf16<CH>(dX + o, sum);
+          store_bf16<CH>(dX + out[py][px], sum);
         }
       }
   }
@@ -503,10 +539,11 @@ __device__ __forceinline__ void wgrad_block(const uint16_t* dY, const uint16_t* 
 // The backward pass of layer L: its weight gradient (blocks below wblocks), its input
 // gradient (dblocks more) and, beside layer L = 1, the fully connected layers' blocks.
 // Neither needs the other, and neither fills the chip at small batches: one launch
-// instead of two.  Batch 256: layers 2 / 3 / 4 in 79 / 48 / 32 us (95 / 58 / 42 apart);
-// the whole step at batch 19: 99 us against 120.
+// instead of two.  Batch 256: layers 2 / 3 / 4 in 74 / 38 / 28 us (before the input
+// gradient read signs 79 / 48 / 32, and in launches apart 95 / 58 / 42).
 struct ConvBackArgs {
   const uint16_t *dY, *X, *Wt;
+  const uint8_t* signs;  // of X
   uint16_t* dX;
   float *wpart, *bpart;
   int M, steps_per_split, wblocks, dblocks;
@@ -523,7 +560,7 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_backward(ConvBackArgs a)
   if (b < a.wblocks)
     wgrad_block<L>(a.dY, a.X, a.wpart, a.M, a.steps_per_split, b, s_col, s_dy);
   else if (b < a.wblocks + a.dblocks)
-    dgrad_block<L>(a.dY, a.Wt, a.X, a.dX, a.bpart, a.M, b - a.wblocks, a.dblocks, reinterpret_cast<float*>(s_col));
+    dgrad_block<L>(a.dY, a.Wt, a.signs, a.dX, a.bpart, a.M, b - a.wblocks, a.dblocks, reinterpret_cast<float*>(s_col));
   else if constexpr (L == 1)
     fc_block(a.fc, b - a.wblocks - a.dblocks, s_col);
 }
