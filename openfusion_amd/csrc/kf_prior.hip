@@ -382,7 +382,8 @@ kf_status infer(kf_prior* P, const float* frames, const int32_t* pairs, const fl
 // for the three layers at batch 256).  fc (L = 1): carried along.
 constexpr int kWgradBlocks = 256, kWgradMinSteps = 4, kDgradBlocks = 256;
 template <int L>
-kf_status launch_backward(kf_prior* P, int B, int* splits, int* planes, hipStream_t s, const FcGradArgs& fc = FcGradArgs{}) {
+kf_status launch_backward(kf_prior* P, int B, int* splits, int* planes, hipStream_t s, const FcGradArgs& fc = FcGradArgs{},
+                          const Conv1Grad& first = Conv1Grad{}) {
   constexpr int GROUPS = WgradShape<L>::GROUPS;
   const int M = B * kConv[L].hout * kConv[L].wout, steps = div_up(M, kWgradStep);
   const int want = std::min(std::max(steps / kWgradMinSteps, 1), kWgradBlocks / GROUPS);
@@ -402,6 +403,7 @@ kf_status launch_backward(kf_prior* P, int B, int* splits, int* planes, hipStrea
   a.wblocks = div_up(*splits, 8) * 8 * GROUPS;
   a.dblocks = *planes = std::min(div_up(div_up(M, 16) * DgradShape<L>::GROUPS, kConvWaves), kDgradBlocks);
   a.fc = fc;
+  a.first = first;
   hipLaunchKernelGGL(conv_backward<L>, dim3(a.wblocks + a.dblocks + (L == 1 ? kFcBlocks : 0)), dim3(kConvThreads), 0, s, a);
   return check_launch("conv_backward");
 }
@@ -448,12 +450,8 @@ kf_status backward(kf_prior* P, const float* frames, const int32_t* pairs, const
   fc.dW6 = G + L.w[5];
   fc.loss = loss;
   fc.batch = B;
-  KF_TRY(launch_backward<1>(P, B, &splits[1], &planes[0], s, fc));
-  const int items = B * (kConv[0].hout / kL1Rows);
-  splits[0] = std::min(items, kConvBlocks);
-  hipLaunchKernelGGL(conv1_wgrad, dim3(splits[0]), dim3(kConvThreads), 0, s, frames, pairs, (const uint16_t*)P->dYb[0],
-                     P->wpart[0], items);
-  KF_TRY(check_launch("conv1_wgrad"));
+  KF_TRY(launch_backward<1>(P, B, &splits[1], &planes[0], s, fc, Conv1Grad{frames, pairs, P->wpart[0]}));
+  splits[0] = planes[0];
   ReduceArgs f;
   f.jobs = 0;
   f.block0[0] = 0;
@@ -534,8 +532,8 @@ extern "C" kf_status kf_prior_create(int32_t max_batch, kf_prior** out) {
       al((void**)&P->signs[l], M * c.cout / 8);
     }
     else al((void**)&P->Y4, M * c.cout * 4);
-    al((void**)&P->wpart[l], (l == 0 ? kConvBlocks : kWgradBlocks / (c.cout / (l == 1 ? 64 : 32))) * c.cout * c.kc * 4);
-    al((void**)&P->dYb[l], M * c.cout * 2);
+    al((void**)&P->wpart[l], (l == 0 ? kDgradBlocks : kWgradBlocks / (c.cout / (l == 1 ? 64 : 32))) * c.cout * c.kc * 4);
+    if (l > 0) al((void**)&P->dYb[l], M * c.cout * 2);  // layer 1's stays in the kernel that makes it
     al((void**)&P->bpart[l], (l + 1 < kConvs ? kDgradBlocks : B) * c.cout * 4);
   }
   al((void**)&P->X5b, B * kX5Pitch * 2);

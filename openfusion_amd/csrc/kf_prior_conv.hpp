@@ -210,6 +210,149 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* 
   }
 }
 
+// Weight gradients contract over pixels, while the maps keep a pixel's channels
+// together.  The tiles are staged in LDS as they lie in memory, one row of channels per
+// pixel, and the operands come from transposing LDS reads (ds_read_b64_tr_b16): of
+// each 16-lane group, lanes 4 i .. 4 i + 3 address the 16 channels of pixel row i, and
+// lane c receives channel c of the four rows.  A fragment is two such reads, pixels
+// 4 q .. 4 q + 3 and 16 + 4 q .. of the 32 staged (both operands in the same order).
+// Row pitches are odd multiples of 8 dwords, so that the eight rows of 32 bytes that
+// a half-wave reads cover all 64 banks.
+constexpr int kWgradStep = 32;  // pixels (or samples) staged at a time
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4s lds_v4s;
+
+__device__ __forceinline__ uint4 transposed_fragment(const uint16_t* rows, int pitch, int c0, int r, int q) {
+  const uint16_t* p = rows + (4 * q + (r >> 2)) * pitch + c0 + 4 * (r & 3);
+  const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(p));
+  const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(p + 16 * pitch));
+  const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
+  return make_uint4(a.x, a.y, b.x, b.y);
+}
+
+// Orders the LDS accesses of one wavefront around this point.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Layer 1's weight gradient, taken where layer 2's input gradient makes layer 1's output
+// gradient, which then never goes to memory: dW1[co][k] = sum_m dY1[m][co] col[m][k], col
+// the im2col element of the two frames.  A wave's tile is 8 x 2 2x2 blocks; it holds the
+// 9 x 33 input pixels under them as BF16 pairs (previous, current) in LDS, writes its
+// gradients there row by row of the blocks, and makes the 32 x 18 products of 32 pixels
+// from transposing reads of the gradients and 16-bit reads of the pairs.  The gradient
+// (79 MB at batch 256) was written by one launch and read by another: layer 2's backward
+// pass 74 us and 31 more, now 66 for both.
+struct Conv1Grad {
+  const float* frames;
+  const int32_t* pairs;
+  float* part;  // a plane per block
+};
+constexpr int kC1Pitch = 36;                        // pairs of a row: column -1 at 3, columns 0 .. 31 from 4 (16-byte aligned)
+constexpr int kC1Patch = 9 * kC1Pitch;              // pairs of a wave
+constexpr int kC1DyPitch = 32 + 16;                 // gradients of a pixel, bank-spreading
+constexpr int kC1Wave = 2 * kC1Patch + kWgradStep * kC1DyPitch;  // a wave's LDS, in 16-bit elements
+static_assert(kC1Wave % 8 == 0 && kC1Patch % 4 == 0, "16-byte alignment");
+
+struct Conv1GradWave {
+  uint32_t* patch;
+  uint16_t* dy;
+  int base[2];  // of the lane's column of the 16-column tiles, in 16-bit elements
+  v4f acc[2][2];
+
+  __device__ __forceinline__ Conv1GradWave(uint16_t* lds, int lane) {
+    patch = reinterpret_cast<uint32_t*>(lds);
+    dy = lds + 2 * kC1Patch;
+    const int r = lane & 15, q = lane >> 4;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int k = min(16 * t + r, kConv[0].kc - 1), tap = k >> 1;  // columns past the kernel are not kept
+      base[t] = 2 * ((4 * (q >> 1) + tap / 3) * kC1Pitch + 16 * (q & 1) + tap % 3 + 3) + (k & 1);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) acc[c][t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+  }
+
+  // The input pixels of rows 8 jt - 1 .. 8 jt + 7 and columns 32 it - 1 .. 32 it + 31 of
+  // sample n (0 outside the frames): 72 vectors of four columns and nine pixels left of
+  // them.  The loads are issued by load(), the pairs go to LDS in stage().
+  typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+  f4 v[2][2];
+  __device__ __forceinline__ void load(const Conv1Grad& g, int lane, int n, int jt, int it) {
+    const float* f[2] = {g.frames + (long)g.pairs[2 * n] * (kH0 * kW0), g.frames + (long)g.pairs[2 * n + 1] * (kH0 * kW0)};
+    const int y0 = 8 * jt - 1, y1 = lane < 8 ? y0 + 8 : y0 + lane - 8;
+    const int at = (y0 + (lane >> 3)) * kW0 + 32 * it + 4 * (lane & 7);
+    const int left = y1 * kW0 + 32 * it - 1, last = y1 * kW0 + 32 * it + 4 * lane;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      v[0][c] = v[1][c] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (at >= 0) v[0][c] = *reinterpret_cast<const f4*>(f[c] + at);
+      if (lane < 8)
+        v[1][c] = *reinterpret_cast<const f4*>(f[c] + last);
+      else if (lane < 17 && y1 >= 0 && it > 0)
+        v[1][c].x = f[c][left];
+    }
+  }
+  __device__ __forceinline__ void stage(int lane) {
+    uint32_t w[2][4];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[u][e] = pack_bf16(v[u][0][e], v[u][1][e]);
+    *reinterpret_cast<uint4*>(patch + (lane >> 3) * kC1Pitch + 4 + 4 * (lane & 7)) = make_uint4(w[0][0], w[0][1], w[0][2], w[0][3]);
+    if (lane < 8)
+      *reinterpret_cast<uint4*>(patch + 8 * kC1Pitch + 4 + 4 * lane) = make_uint4(w[1][0], w[1][1], w[1][2], w[1][3]);
+    else if (lane < 17)
+      patch[(lane - 8) * kC1Pitch + 3] = w[1][0];
+  }
+
+  // The products of pixel row py of the blocks: dy holds its pixels px = 0, then px = 1.
+  __device__ __forceinline__ void add_row(int lane, int py) {
+    const int r = lane & 15, q = lane >> 4;
+    const uint16_t* pairs = reinterpret_cast<const uint16_t*>(patch);
+    uint4 a[2], b[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) a[c] = transposed_fragment(dy, kC1DyPitch, 16 * c, r, q);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      uint32_t w[4];  // pixels 4 q .. 4 q + 3 of px = 0, then of px = 1, as the fragments order them
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint16_t* p = pairs + base[t] + 4 * py * kC1Pitch + 4 * (i >> 1) + 16 * (i & 1);
+        w[i] = (uint32_t)p[0] | (uint32_t)p[8] << 16;
+      }
+      b[t] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) acc[c][t] = mfma32(a[c], b[t], acc[c][t]);
+  }
+
+  // The block's plane: the sum over its waves, in order.  s: kConvWaves 1024 floats.
+  __device__ __forceinline__ void finish(const Conv1Grad& g, int block, float* s) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[wave * 1024 + (16 * c + 4 * q + j) * 32 + 16 * t + r] = acc[c][t][j];
+    __syncthreads();
+    constexpr int kc = kConv[0].kc;
+    for (int e = threadIdx.x; e < kConv[0].cout * kc; e += kConvThreads) {
+      const int i = e / kc * 32 + e % kc;
+      float v = s[i];
+#pragma unroll
+      for (int u = 1; u < kConvWaves; ++u) v = v + s[u * 1024 + i];
+      g.part[(long)block * (kConv[0].cout * kc) + e] = v;
+    }
+  }
+};
+
 // Input gradient of layer L (1..3), ReLU mask of the layer below and that layer's bias
 // sums in one pass: dX[n][iy][ix][ci] = sum over the taps (ky, kx) that reach the
 // pixel, in that order, of sum_co dY[n][oy][ox][co] W[co][(ky, kx, ci)]; 0 where the
@@ -220,9 +363,9 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* 
 // Each tap's product is an MFMA chain of its own from zero and the taps are added in
 // FP32: the bits of a column-gradient GEMM followed by col2im, without the FP32 column
 // matrix (354 MB for layer 2 at batch 256).  bpart: per block and channel the FP32 sum
-// of the unrounded gradients.  Bound by memory: layer 2 at batch 256 moves 123 MB (197 with
-// the forward map in place of its signs: the three layers' backward passes 160 us, now
-// 140); the GEMM, col2im, conversion and column sums took 4.3 ms.
+// of the unrounded gradients.  Layer 2's output stays on the chip (Conv1Grad).  Bound by
+// memory: with the forward map in place of its signs (layer 2 at batch 256: 79 MB) the
+// three layers' backward passes took 160 us instead of 140; the GEMM, col2im, conversion and column sums took 4.3 ms.
 // Block `block` of `blocks`; s_b: kDgradLds floats of LDS.
 template <int L>
 struct DgradShape {
@@ -233,7 +376,8 @@ constexpr int kDgradLds = kConvWaves * 32;
 
 template <int L>
 __device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* Wt, const uint8_t* signs, uint16_t* dX,
-                                            float* bpart, int M, int block, int blocks, float* s_sum) {
+                                            float* bpart, int M, int block, int blocks, float* s_sum,
+                                            const Conv1Grad& g, uint16_t* lds) {
   constexpr ConvShape c = kConv[L];
   constexpr int NT = DgradShape<L>::NT, KS = c.cout / 32, GROUPS = DgradShape<L>::GROUPS, CH = 4 * NT;
   static_assert(c.win == 2 * c.wout && (c.hin == 2 * c.hout || c.hin == 2 * c.hout - 1) && kConvWaves % GROUPS == 0,
@@ -254,11 +398,27 @@ __device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* 
 #pragma unroll
   for (int j = 0; j < CH; ++j) bs[j] = 0.0f;
   const int stride = blocks * kConvWaves / GROUPS;
+  [[maybe_unused]] Conv1GradWave first(lds + wave * kC1Wave, lane);
   for (int tile = gw / GROUPS; tile * 16 < M; tile += stride) {
-    const bool live = tile * 16 + r < M;
-    const int m = live ? tile * 16 + r : M - 1;
-    const int n = m / (c.hout * c.wout), p = m - n * (c.hout * c.wout);
-    const int j = p / c.wout, i = p - j * c.wout;
+    bool live = true;
+    int m, n, j, i;
+    if constexpr (L == 1) {  // 8 x 2 blocks, 75 tiles of a sample
+      static_assert(c.wout % 8 == 0 && c.hout % 2 == 0, "layer shape");
+      const int at = __builtin_amdgcn_readfirstlane(tile);
+      n = at / (c.hout * c.wout / 16);
+      const int t = at - n * (c.hout * c.wout / 16), jt = t / (c.wout / 8), it = t - jt * (c.wout / 8);
+      j = 2 * jt + (r >> 3);
+      i = 8 * it + (r & 7);
+      m = (n * c.hout + j) * c.wout + i;
+      first.load(g, lane, n, jt, it);
+    } else {
+      live = tile * 16 + r < M;
+      m = live ? tile * 16 + r : M - 1;
+      n = m / (c.hout * c.wout);
+      const int p = m - n * (c.hout * c.wout);
+      j = p / c.wout;
+      i = p - j * c.wout;
+    }
     // the four pixels' sign bits of the lane's channels
     uint32_t sign[2][2];
     int out[2][2];
@@ -283,8 +443,9 @@ __device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* 
           if (!in) a[dj][di][s] = make_uint4(0u, 0u, 0u, 0u);
         }
       }
+    if constexpr (L == 1) first.stage(lane);
 #pragma unroll
-    for (int py = 0; py < 2; ++py)
+    for (int py = 0; py < 2; ++py) {
 #pragma unroll
       for (int px = 0; px < 2; ++px) {
         float sum[CH];
@@ -311,9 +472,18 @@ __device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* 
             sum[e] = __int_as_float(__float_as_int(sum[e]) & keep);
             bs[e] = bs[e] + sum[e];
           }
-          store_bf16<CH>(dX + out[py][px], sum);
+          if constexpr (L == 1)
+            store_bf16<CH>(first.dy + (16 * px + r) * kC1DyPitch + CH * q, sum);
+          else
+            store_bf16<CH>(dX + out[py][px], sum);
         }
       }
+      if constexpr (L == 1) {
+        wave_lds_sync();
+        first.add_row(lane, py);
+        wave_lds_sync();
+      }
+    }
   }
 #pragma unroll
   for (int e = 0; e < CH; ++e) {
@@ -328,28 +498,8 @@ __device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* 
     for (int u = g + GROUPS; u < kConvWaves; u += GROUPS) v = v + s_b[u][k];
     bpart[(long)block * c.cin + threadIdx.x] = v;
   }
+  if constexpr (L == 1) first.finish(g, block, reinterpret_cast<float*>(lds));
 }
-
-// Weight gradients contract over pixels, while the maps keep a pixel's channels
-// together.  The tiles are staged in LDS as they lie in memory, one row of channels per
-// pixel, and the operands come from transposing LDS reads (ds_read_b64_tr_b16): of
-// each 16-lane group, lanes 4 i .. 4 i + 3 address the 16 channels of pixel row i, and
-// lane c receives channel c of the four rows.  A fragment is two such reads, pixels
-// 4 q .. 4 q + 3 and 16 + 4 q .. of the 32 staged (both operands in the same order).
-// Row pitches are odd multiples of 8 dwords, so that the eight rows of 32 bytes that
-// a half-wave reads cover all 64 banks.
-typedef short v4s __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4s lds_v4s;
-
-__device__ __forceinline__ uint4 transposed_fragment(const uint16_t* rows, int pitch, int c0, int r, int q) {
-  const uint16_t* p = rows + (4 * q + (r >> 2)) * pitch + c0 + 4 * (r & 3);
-  const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(p));
-  const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(p + 16 * pitch));
-  const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
-  return make_uint4(a.x, a.y, b.x, b.y);
-}
-
-constexpr int kWgradStep = 32;  // pixels (or samples) staged at a time
 
 // Weight gradients of the fully connected layers, dW5[j][c] = sum_n dH[n][j] X5[n][c] and
 // dW6[t][k] = sum_n dO[n][t] H[n][k], and the loss mean((O - T)^2): five blocks of their
@@ -539,8 +689,8 @@ __device__ __forceinline__ void wgrad_block(const uint16_t* dY, const uint16_t* 
 // The backward pass of layer L: its weight gradient (blocks below wblocks), its input
 // gradient (dblocks more) and, beside layer L = 1, the fully connected layers' blocks.
 // Neither needs the other, and neither fills the chip at small batches: one launch
-// instead of two.  Batch 256: layers 2 / 3 / 4 in 74 / 38 / 28 us (before the input
-// gradient read signs 79 / 48 / 32, and in launches apart 95 / 58 / 42).
+// instead of two.  Batch 256: layers 2 (with layer 1's weight gradient) / 3 / 4 in 66 / 38 /
+// 28 us (in launches apart 126 / 58 / 42).
 struct ConvBackArgs {
   const uint16_t *dY, *X, *Wt;
   const uint8_t* signs;  // of X
@@ -548,6 +698,7 @@ struct ConvBackArgs {
   float *wpart, *bpart;
   int M, steps_per_split, wblocks, dblocks;
   FcGradArgs fc;
+  Conv1Grad first;
 };
 
 template <int L>
@@ -555,63 +706,17 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_backward(ConvBackArgs a)
   using S = WgradShape<L>;
   constexpr int kCol = L == 1 && kFcLds > S::kColLds ? kFcLds : S::kColLds;
   __shared__ __align__(16) uint16_t s_col[kCol], s_dy[S::kDyLds];
-  static_assert(sizeof(s_col) >= kDgradLds * sizeof(float), "LDS of the input gradient");
+  static_assert(sizeof(s_dy) >= kDgradLds * sizeof(float) && kCol >= kConvWaves * (L == 1 ? kC1Wave : 0) &&
+                    sizeof(s_col) >= (L == 1 ? kConvWaves * 1024 * sizeof(float) : 0),
+                "LDS of the input gradient");
   const int b = blockIdx.x;  // every branch is uniform
   if (b < a.wblocks)
     wgrad_block<L>(a.dY, a.X, a.wpart, a.M, a.steps_per_split, b, s_col, s_dy);
   else if (b < a.wblocks + a.dblocks)
-    dgrad_block<L>(a.dY, a.Wt, a.signs, a.dX, a.bpart, a.M, b - a.wblocks, a.dblocks, reinterpret_cast<float*>(s_col));
+    dgrad_block<L>(a.dY, a.Wt, a.signs, a.dX, a.bpart, a.M, b - a.wblocks, a.dblocks, reinterpret_cast<float*>(s_dy), a.first,
+                   s_col);
   else if constexpr (L == 1)
     fc_block(a.fc, b - a.wblocks - a.dblocks, s_col);
-}
-
-// Weight gradient of layer 1.  A block walks over groups of four output rows: the input
-// rows staged as in the forward, from them the 320 x 18 im2col tile in LDS (columns
-// 18 .. 31 zero), beside it the rows' gradients; each wave one 16 x 16 tile of the
-// 32 x 32 products.  One plane per block.  Batch 256: 32 us (98 MB
-// read).
-constexpr int kL1Pix = kL1Rows * kConv[0].wout;
-__global__ __launch_bounds__(kConvThreads) void conv1_wgrad(const float* frames, const int32_t* pairs, const uint16_t* dY,
-                                                            float* part, int items) {
-  constexpr ConvShape c = kConv[0];
-  constexpr int kPitch = 32 + 16, kGroups = c.hout / kL1Rows;
-  static_assert(kL1Pix % kWgradStep == 0 && c.cout == 32, "layer-1 tiles");
-  __shared__ uint32_t patch[kL1In][kL1Pitch];
-  __shared__ __align__(16) uint16_t s_col[kL1Pix * kPitch];
-  __shared__ __align__(16) uint16_t s_dy[kL1Pix * kPitch];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4;
-  const int cw = (wave >> 1) * 16, nw = (wave & 1) * 16;
-  for (int e = tid; e < kL1Pix * 7; e += kConvThreads)  // columns 18 .. 31
-    *reinterpret_cast<uint32_t*>(&s_col[e / 7 * kPitch + 18 + 2 * (e % 7)]) = 0u;
-  v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int it = blockIdx.x; it < items; it += gridDim.x) {
-    const int n = it / kGroups, oy0 = (it - n * kGroups) * kL1Rows;
-    const uint16_t* src = dY + ((long)n * c.hout + oy0) * c.wout * c.cout;
-    constexpr int PER = kL1Pix * c.cout / 8 / kConvThreads;
-    uint4 v[PER];
-#pragma unroll
-    for (int u = 0; u < PER; ++u) v[u] = *reinterpret_cast<const uint4*>(src + 8 * (tid + kConvThreads * u));
-    stage_l1(patch, frames + (long)pairs[2 * n] * (kH0 * kW0), frames + (long)pairs[2 * n + 1] * (kH0 * kW0), oy0);
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = tid + kConvThreads * u;
-      *reinterpret_cast<uint4*>(&s_dy[(e >> 2) * kPitch + 8 * (e & 3)]) = v[u];
-    }
-    __syncthreads();
-    for (int e = tid; e < kL1Pix * 9; e += kConvThreads) {
-      const int p = e / 9, tap = e - 9 * p, oy = p / c.wout, ox = p - oy * c.wout;
-      *reinterpret_cast<uint32_t*>(&s_col[p * kPitch + 2 * tap]) = patch[2 * oy + tap / 3][2 * ox + tap % 3];
-    }
-    __syncthreads();
-    for (int p0 = 0; p0 < kL1Pix; p0 += kWgradStep)
-      acc = mfma32(transposed_fragment(s_dy + p0 * kPitch, kPitch, cw, r, q),
-                   transposed_fragment(s_col + p0 * kPitch, kPitch, nw, r, q), acc);
-    __syncthreads();
-  }
-  if (nw + r < c.kc) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) part[((long)blockIdx.x * c.cout + cw + 4 * q + j) * c.kc + nw + r] = acc[j];
-  }
 }
 
 }  // namespace kf
