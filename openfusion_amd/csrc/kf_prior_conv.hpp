@@ -68,6 +68,35 @@ __device__ __forceinline__ void store_bf16_signs(uint16_t* p, uint8_t* bits, con
     *reinterpret_cast<uint16_t*>(bits) = (uint16_t)m;
 }
 
+// v of the lane below (CTRL 0x111) or above (0x101) in its row of 16, `edge` in the row's
+// last lane on that side.
+template <int CTRL>
+__device__ __forceinline__ uint4 neighbour(uint4 v, uint4 edge) {
+  auto mv = [](uint32_t e, uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)e, (int)x, CTRL, 0xf, 0xf, false);
+  };
+  return make_uint4(mv(edge.x, v.x), mv(edge.y, v.y), mv(edge.z, v.z), mv(edge.w, v.w));
+}
+
+// The 16-pixel tiles of wave group `unit` of `units` in a block, of `blocks` blocks: first,
+// first + step, ... below last.  Blocks go to the eight XCDs (each with its own L2) in
+// turn, and neighbouring tiles read the same rows, so each XCD takes a run of them.
+struct TileRun {
+  int first, last, step;
+  __device__ __forceinline__ TileRun(int tiles, int block, int blocks, int unit, int units) {
+    if (blocks % 8 == 0) {
+      const int x = block % 8;
+      first = (int)((long)tiles * x / 8) + block / 8 * units + unit;
+      last = (int)((long)tiles * (x + 1) / 8);
+      step = blocks / 8 * units;
+    } else {
+      first = block * units + unit;
+      last = tiles;
+      step = blocks * units;
+    }
+  }
+};
+
 // Layer 1 forward: a block makes four output rows of one sample.  The nine input rows
 // of both planes are staged in LDS as BF16 pairs (previous, current), so that one
 // 32-bit LDS read is one tap's two channels.
@@ -172,21 +201,42 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* 
 #pragma unroll
     for (int j = 0; j < 4; ++j) b[4 * t + j] = bias[ch0 + 4 * NT * q + 4 * t + j];
   }
-  const int stride = gridDim.x * kConvWaves / GROUPS;
-  for (int tile = gw / GROUPS; tile * 16 < M; tile += stride) {
+  const TileRun run((M + 15) / 16, blockIdx.x, gridDim.x, wave / GROUPS, kConvWaves / GROUPS);
+  for (int tile = run.first; tile < run.last; tile += run.step) {
     const int m = min(tile * 16 + r, M - 1);  // rows past the end repeat the last one
     const int n = m / (c.hout * c.wout), p = m - n * (c.hout * c.wout);
     const int oy = p / c.wout, ox = p - oy * c.wout;
     const int at = ((n * c.hin + 2 * oy - 1) * c.win + 2 * ox - 1) * c.cin;
+    // A pixel's left column is its left neighbour's right one (stride 2): that operand
+    // comes from the lane below, and only the tile's first pixel loads its own.
+    constexpr int CS = c.cin / 32;
     uint4 a[KS];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const int tap = 32 * s / c.cin, ky = tap / 3, kx = tap % 3, ci = 32 * s % c.cin + 8 * q;
-      const int iy = 2 * oy + ky - 1, ix = 2 * ox + kx - 1;
-      const bool in = (ky > 0 || iy >= 0) && (2 * c.hout <= c.hin || iy < c.hin) && (kx > 0 || ix >= 0);
-      a[s] = *reinterpret_cast<const uint4*>(X + (in ? at + (ky * c.win + kx) * c.cin + ci : 0));
-      if (!in) a[s] = make_uint4(0u, 0u, 0u, 0u);
+    for (int ky = 0; ky < 3; ++ky) {
+      const int iy = 2 * oy + ky - 1;
+      const bool row = (ky > 0 || iy >= 0) && (2 * c.hout <= c.hin || iy < c.hin);
+      const uint16_t* src = X + (row ? at + (ky * c.win + 1) * c.cin : 0) + 8 * q;
+#pragma unroll
+      for (int k = 0; k < CS; ++k) {
+        uint4 own = make_uint4(0u, 0u, 0u, 0u);
+        if (r == 0 && row && ox > 0) own = *reinterpret_cast<const uint4*>(src - c.cin + 32 * k);
+        a[(3 * ky) * CS + k] = own;
+#pragma unroll
+        for (int kx = 1; kx < 3; ++kx) {
+          uint4& v = a[(3 * ky + kx) * CS + k];
+          v = *reinterpret_cast<const uint4*>(src + (kx - 1) * c.cin + 32 * k);
+          if (!row) v = make_uint4(0u, 0u, 0u, 0u);
+        }
+      }
     }
+#pragma unroll
+    for (int ky = 0; ky < 3; ++ky)
+#pragma unroll
+      for (int k = 0; k < CS; ++k) {
+        uint4& v = a[(3 * ky) * CS + k];
+        v = neighbour<0x111>(a[(3 * ky + 2) * CS + k], v);
+        if (ox == 0) v = make_uint4(0u, 0u, 0u, 0u);
+      }
     v4f acc[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -397,9 +447,9 @@ __device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* 
   float bs[CH];
 #pragma unroll
   for (int j = 0; j < CH; ++j) bs[j] = 0.0f;
-  const int stride = blocks * kConvWaves / GROUPS;
+  const TileRun run((M + 15) / 16, block, blocks, wave / GROUPS, kConvWaves / GROUPS);
   [[maybe_unused]] Conv1GradWave first(lds + wave * kC1Wave, lane);
-  for (int tile = gw / GROUPS; tile * 16 < M; tile += stride) {
+  for (int tile = run.first; tile < run.last; tile += run.step) {
     bool live = true;
     int m, n, j, i;
     if constexpr (L == 1) {  // 8 x 2 blocks, 75 tiles of a sample
@@ -431,17 +481,29 @@ __device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* 
         sign[py][px] = (uint32_t)signs[(unsigned)out[py][px] / 8u] >> (out[py][px] & 4);
       }
     uint4 a[2][2][KS];  // dY at (j + dj, i + di), 0 outside the map
+    // (the column to the right is the next lane's, but for the last pixel of the tile's row)
+    constexpr int kEnd = L == 1 ? 7 : 15;
+#pragma unroll
+    for (int dj = 0; dj < 2; ++dj) {
+      const bool in = dj == 0 || j + 1 < c.hout;
+      const uint16_t* src = dY + (in ? (m + dj * c.wout) * c.cout : 0) + 8 * q;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        a[dj][0][s] = *reinterpret_cast<const uint4*>(src + 32 * s);
+        if (!in) a[dj][0][s] = make_uint4(0u, 0u, 0u, 0u);
+        a[dj][1][s] = make_uint4(0u, 0u, 0u, 0u);
+        if ((r & kEnd) == kEnd && in && i + 1 < c.wout) a[dj][1][s] = *reinterpret_cast<const uint4*>(src + c.cout + 32 * s);
+      }
+    }
 #pragma unroll
     for (int dj = 0; dj < 2; ++dj)
 #pragma unroll
-      for (int di = 0; di < 2; ++di) {
-        const bool in = (dj == 0 || j + 1 < c.hout) && (di == 0 || i + 1 < c.wout);
-        const uint16_t* src = dY + (in ? (m + dj * c.wout + di) * c.cout : 0) + 8 * q;
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-          a[dj][di][s] = *reinterpret_cast<const uint4*>(src + 32 * s);
-          if (!in) a[dj][di][s] = make_uint4(0u, 0u, 0u, 0u);
-        }
+      for (int s = 0; s < KS; ++s) {
+        const uint4 own = a[dj][1][s];
+        uint4 v = neighbour<0x101>(a[dj][0][s], own);
+        if (i + 1 >= c.wout) v = make_uint4(0u, 0u, 0u, 0u);
+        if (kEnd < 15 && (r & kEnd) == kEnd) v = own;
+        a[dj][1][s] = v;
       }
     if constexpr (L == 1) first.stage(lane);
 #pragma unroll
