@@ -2,8 +2,8 @@
 //
 // A wavefront keeps its share of a layer's weights in registers (144 of them) as
 // the A operand of v_mfma_f32_16x16x32_bf16 and takes 16 pixels at a time as the B
-// operand, one 16-byte load of eight channels per lane and step straight from the
-// NHWC BF16 map (through L1 / L2, no im2col matrix).  With the weights as A, a lane
+// operand, sixteen bytes of eight channels per lane and step (no im2col matrix).  With
+// the weights as A, a lane
 // holds output channels of one pixel; their order over the tiles is chosen so that
 // a lane's channels are contiguous and it stores them as whole vectors.  Each output
 // is one MFMA chain over k = 0, 32, ... from zero, the sequence of prior_infer_fused, so
@@ -176,21 +176,96 @@ __global__ __launch_bounds__(kConvThreads) void conv1_forward(const float* frame
   }
 }
 
-// Layers 2-4 forward.  Bound by the L1 path of the pixel loads (each map vector is read
-// by up to four taps).  NT is chosen so that every layer's share is 144 weight
-// registers (two waves per SIMD).  Batch 256: 31 / 33 / 23 us for layers 2 / 3 / 4
-// (365 / 172 / 131 TFLOP/s), layer 1 30 us; GEMMs staged through LDS took 570 us for the
-// four.  NT: 16-channel tiles of a wave (COUT / (16 NT) waves cover a
-// pixel's channels); F32: FP32 output (layer 4, which the pooling reads), else BF16.
+// Orders the LDS accesses of one wavefront around this point.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The operand tile of 16 pixels of layer L's forward: the rows of input pixels under them,
+// a wavefront's own in LDS.  The map is read as it lies in memory (a pixel's two columns 2 ox
+// and 2 ox + 1 are 2 cin channels on end: a quarter wave touches two lines, where operands
+// loaded straight from the map touch sixteen, and the L1's lookups bound the kernel), and
+// the tile's left neighbour once.  Column 2 ox - 1 is the pixel before's second one.  A
+// pixel's 16-byte chunks are permuted by its index so that the operand reads' eight
+// pixels at a time meet no bank twice.
+template <int L>
+struct ConvTile {
+  static constexpr ConvShape c = kConv[L];
+  static constexpr int PC = c.cin / 8, U = 2 * PC;      // chunks of an input pixel, of an output pixel's two columns
+  static constexpr int PER = 16 * U / kWave;            // loads of an input row
+  static constexpr int kChunks = 3 * (16 * U + PC);     // LDS of a wave: three rows, and the pixels left of them
+  static_assert(U == 8 || U == 16, "32 or 64 input channels");
+  uint4 v[3][PER], left;
+  bool in[3][PER], left_in;
+
+  static __device__ __forceinline__ int chunk(int pixel, int i) { return pixel * U + (i ^ (U == 8 ? pixel >> 1 : pixel)); }
+  static __device__ __forceinline__ bool row_in(int oy, int ky) {
+    const int iy = 2 * oy + ky - 1;
+    return iy >= 0 && (2 * c.hout <= c.hin || iy < c.hin);
+  }
+
+  __device__ __forceinline__ void load(const uint16_t* X, int tile, int M, int lane) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int e = u * kWave + lane, i = e % U;
+      const int m = min(tile * 16 + e / U, M - 1);
+      const int n = m / (c.hout * c.wout), p = m - n * (c.hout * c.wout), oy = p / c.wout, ox = p - oy * c.wout;
+      const int at = ((n * c.hin + 2 * oy - 1) * c.win + 2 * ox) * c.cin + 8 * i;
+#pragma unroll
+      for (int ky = 0; ky < 3; ++ky) {
+        in[ky][u] = row_in(oy, ky);
+        v[ky][u] = *reinterpret_cast<const uint4*>(X + (in[ky][u] ? at + ky * c.win * c.cin : 0));
+      }
+    }
+    const int m = tile * 16, ky = lane / PC;
+    const int n = m / (c.hout * c.wout), p = m - n * (c.hout * c.wout), oy = p / c.wout, ox = p - oy * c.wout;
+    left = make_uint4(0u, 0u, 0u, 0u);
+    if (lane < 3 * PC && ox > 0 && row_in(oy, ky))
+      left = *reinterpret_cast<const uint4*>(X + ((n * c.hin + 2 * oy - 1 + ky) * c.win + 2 * ox - 1) * c.cin + 8 * (lane % PC));
+  }
+
+  __device__ __forceinline__ void stage(uint4* lds, int lane) {
+#pragma unroll
+    for (int ky = 0; ky < 3; ++ky)
+#pragma unroll
+      for (int u = 0; u < PER; ++u) {
+        const int e = u * kWave + lane;
+        lds[ky * 16 * U + chunk(e / U, e % U)] = in[ky][u] ? v[ky][u] : make_uint4(0u, 0u, 0u, 0u);
+      }
+    if (lane < 3 * PC) lds[3 * 16 * U + lane] = left;
+  }
+
+  // The operand of tap (ky, kx) and channels 32 k .. of pixel r, chunk q of four; ox: its column.
+  static __device__ __forceinline__ uint4 operand(const uint4* lds, int ky, int kx, int k, int r, int q, int ox) {
+    if (kx > 0) return lds[ky * 16 * U + chunk(r, (kx - 1) * PC + 4 * k + q)];
+    const uint4 a = lds[r > 0 ? ky * 16 * U + chunk(r - 1, PC + 4 * k + q) : 3 * 16 * U + ky * PC + 4 * k + q];
+    return ox > 0 ? a : make_uint4(0u, 0u, 0u, 0u);
+  }
+};
+
+// Layers 2-4 forward.  NT: 16-channel tiles of a wave (COUT / (16 NT) waves cover a
+// pixel's channels), chosen so that every layer's share is 144 weight registers (two
+// waves per SIMD); F32: FP32 output (layer 4, which the pooling reads), else BF16.  The
+// next tile's loads are in flight while this one is multiplied.  Bound by memory (layer 2
+// at batch 256: 120 MB), the narrower layers by the weights' loads.  Batch 256: layers 2 /
+// 3 / 4 in 27 / 23 / 17 us (operands straight from the map, the left column from the
+// neighbouring lane: 27 / 27 / 20; all nine from the map: 32 / 33 / 23; GEMMs staged
+// through LDS took 570 us with layer 1's 30).
 template <int L, int NT, bool F32>
 __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* X, const uint16_t* W, const float* bias,
                                                                 uint16_t* Yb, float* Y, uint8_t* signs, int M) {
   constexpr ConvShape c = kConv[L];
-  constexpr int KS = c.kc / 32, GROUPS = c.cout / (16 * NT);
+  using T = ConvTile<L>;
+  constexpr int KS = c.kc / 32, CS = c.cin / 32, GROUPS = c.cout / (16 * NT);
   static_assert(2 * c.wout == c.win && c.kc == 9 * c.cin && c.cin % 32 == 0, "layer shape");
+  __shared__ uint4 s_in[kConvWaves][T::kChunks];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
-  const int gw = blockIdx.x * kConvWaves + wave, group = gw % GROUPS;
-  const int ch0 = group * 16 * NT;
+  const int group = wave % GROUPS, ch0 = group * 16 * NT;
+  const TileRun run((M + 15) / 16, blockIdx.x, gridDim.x, wave / GROUPS, kConvWaves / GROUPS);
+  T in;
+  if (run.first < run.last) in.load(X, run.first, M, lane);
   uint4 w[KS][NT];
   float b[4 * NT];
 #pragma unroll
@@ -201,49 +276,23 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* 
 #pragma unroll
     for (int j = 0; j < 4; ++j) b[4 * t + j] = bias[ch0 + 4 * NT * q + 4 * t + j];
   }
-  const TileRun run((M + 15) / 16, blockIdx.x, gridDim.x, wave / GROUPS, kConvWaves / GROUPS);
+  uint4* lds = s_in[wave];
   for (int tile = run.first; tile < run.last; tile += run.step) {
+    in.stage(lds, lane);
+    if (tile + run.step < run.last) in.load(X, tile + run.step, M, lane);
+    wave_lds_sync();
     const int m = min(tile * 16 + r, M - 1);  // rows past the end repeat the last one
-    const int n = m / (c.hout * c.wout), p = m - n * (c.hout * c.wout);
-    const int oy = p / c.wout, ox = p - oy * c.wout;
-    const int at = ((n * c.hin + 2 * oy - 1) * c.win + 2 * ox - 1) * c.cin;
-    // A pixel's left column is its left neighbour's right one (stride 2): that operand
-    // comes from the lane below, and only the tile's first pixel loads its own.
-    constexpr int CS = c.cin / 32;
-    uint4 a[KS];
-#pragma unroll
-    for (int ky = 0; ky < 3; ++ky) {
-      const int iy = 2 * oy + ky - 1;
-      const bool row = (ky > 0 || iy >= 0) && (2 * c.hout <= c.hin || iy < c.hin);
-      const uint16_t* src = X + (row ? at + (ky * c.win + 1) * c.cin : 0) + 8 * q;
-#pragma unroll
-      for (int k = 0; k < CS; ++k) {
-        uint4 own = make_uint4(0u, 0u, 0u, 0u);
-        if (r == 0 && row && ox > 0) own = *reinterpret_cast<const uint4*>(src - c.cin + 32 * k);
-        a[(3 * ky) * CS + k] = own;
-#pragma unroll
-        for (int kx = 1; kx < 3; ++kx) {
-          uint4& v = a[(3 * ky + kx) * CS + k];
-          v = *reinterpret_cast<const uint4*>(src + (kx - 1) * c.cin + 32 * k);
-          if (!row) v = make_uint4(0u, 0u, 0u, 0u);
-        }
-      }
-    }
-#pragma unroll
-    for (int ky = 0; ky < 3; ++ky)
-#pragma unroll
-      for (int k = 0; k < CS; ++k) {
-        uint4& v = a[(3 * ky) * CS + k];
-        v = neighbour<0x111>(a[(3 * ky + 2) * CS + k], v);
-        if (ox == 0) v = make_uint4(0u, 0u, 0u, 0u);
-      }
+    const int ox = m % c.wout;
     v4f acc[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int s = 0; s < KS; ++s)
+    for (int s = 0; s < KS; ++s) {
+      const uint4 a = T::operand(lds, s / CS / 3, s / CS % 3, s % CS, r, q, ox);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t] = mfma32(w[s][t], a[s], acc[t]);
+      for (int t = 0; t < NT; ++t) acc[t] = mfma32(w[s][t], a, acc[t]);
+    }
+    wave_lds_sync();
     if (tile * 16 + r >= M) continue;
     float y[4 * NT];
 #pragma unroll
@@ -278,13 +327,6 @@ __device__ __forceinline__ uint4 transposed_fragment(const uint16_t* rows, int p
   const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(p + 16 * pitch));
   const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
   return make_uint4(a.x, a.y, b.x, b.y);
-}
-
-// Orders the LDS accesses of one wavefront around this point.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Layer 1's weight gradient, taken where layer 2's input gradient makes layer 1's output
