@@ -40,9 +40,9 @@ namespace {
 // of their use; eight waves share each layer's tiles; window pixels are padded by 16
 // bytes in LDS (without, the 16 pixels of an operand read lie on the same banks); the
 // layer-4 pixels go to the last block by agent-scope stores and loads (no L2 write-back
-// and invalidation, kf_icp.hip), all of them in flight together.  Batch 1: 17.6 us
-// against 23.7 with four waves, weights loaded where they are used, scalar FC1 weight
-// loads and fences around the hand-over.
+// and invalidation, kf_icp.hip), all of them in flight together.  Batch 1: 12.0 us (17.6
+// with the weights' rows on end; 23.7 with four waves, weights loaded where they are used,
+// scalar FC1 weight loads and fences around the hand-over).
 constexpr int kFuseThreads = 512, kFuseWaves = kFuseThreads / kWave;
 constexpr int kWin1 = 15, kWin2 = 7, kWin3 = 3;  // window sides of layers 1-3 around one layer-4 pixel
 constexpr int kRows1 = kWin1 * kWin1;            // 225 layer-1 positions
@@ -54,7 +54,7 @@ struct FuseArgs {
   const int32_t* pairs;
   const float* prev;
   const uint16_t* wbf;   // BF16 weights
-  const uint16_t* w5;    // FC1 with padded rows (WeightCopies)
+  const uint16_t* w5;    // FC1's operand copy (WeightCopies)
   const float* params;   // FP32 biases
   long w[6], b[6];       // parameter offsets
   float* Y4;             // [B][80][128] layer-4 activations
@@ -75,9 +75,9 @@ struct FuseConv {
     const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const uint16_t* row = W + (ch0 + tile_channel<NT>(t, r)) * c.kc + 8 * q;
 #pragma unroll
-      for (int s = 0; s < KS; ++s) w[s][t] = *reinterpret_cast<const uint4*>(row + 32 * s);
+      for (int s = 0; s < KS; ++s)
+        w[s][t] = *reinterpret_cast<const uint4*>(W + operand_at(c.cout, ch0 + tile_channel<NT>(t, r), 32 * s + 8 * q));
 #pragma unroll
       for (int j = 0; j < 4; ++j) b[4 * t + j] = bias[ch0 + CH * q + 4 * t + j];
     }
@@ -343,8 +343,8 @@ kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, int B,
 // Inference, with the training forward's outputs either way.  The fused kernel's blocks
 // (80 a sample, one fits a CU) are all resident up to three samples on 256 CUs; from the
 // fourth on a second round and the recomputed window overlaps cost more than the layered
-// forward's five launches.  Fused / layered at batch 1: 17.7 / 30.6 us, 3: 19.8 / 31.6,
-// 4: 32.1 / 31.9, 8: 45.9 / 33.7, 256: 1106 / 114.
+// forward's five launches.  Fused / layered at batch 1: 11.9 / 20.8 us, 3: 14.2 / 21.2,
+// 4: 21.0 / 21.7, 6: 23.4 / 22.0, 8: 30.0 / 23.1, 256: 666 / 82.
 constexpr int kLayeredBatch = 4;
 kf_status infer(kf_prior* P, const float* frames, const int32_t* pairs, const float* prev, int B, float* out,
                 hipStream_t s) {

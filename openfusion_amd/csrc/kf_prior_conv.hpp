@@ -249,10 +249,10 @@ struct ConvTile {
 // pixel's channels), chosen so that every layer's share is 144 weight registers (two
 // waves per SIMD); F32: FP32 output (layer 4, which the pooling reads), else BF16.  The
 // next tile's loads are in flight while this one is multiplied.  Bound by memory (layer 2
-// at batch 256: 120 MB), the narrower layers by the weights' loads.  Batch 256: layers 2 /
-// 3 / 4 in 27 / 23 / 17 us (operands straight from the map, the left column from the
-// neighbouring lane: 27 / 27 / 20; all nine from the map: 32 / 33 / 23; GEMMs staged
-// through LDS took 570 us with layer 1's 30).
+// at batch 256: 120 MB).  Batch 256: layers 2 / 3 / 4 in 26 / 18 / 13 us (with weight rows on
+// end: 27 / 23 / 17; operands straight from the map, the left column from the neighbouring
+// lane: 27 / 27 / 20; all nine from the map: 32 / 33 / 23; GEMMs staged through LDS took
+// 570 us with layer 1's 30).
 template <int L, int NT, bool F32>
 __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* X, const uint16_t* W, const float* bias,
                                                                 uint16_t* Yb, float* Y, uint8_t* signs, int M) {
@@ -270,9 +270,9 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_forward(const uint16_t* 
   float b[4 * NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const uint16_t* row = W + (ch0 + tile_channel<NT>(t, r)) * c.kc + 8 * q;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) w[s][t] = *reinterpret_cast<const uint4*>(row + 32 * s);
+    for (int s = 0; s < KS; ++s)
+      w[s][t] = *reinterpret_cast<const uint4*>(W + operand_at(c.cout, ch0 + tile_channel<NT>(t, r), 32 * s + 8 * q));
 #pragma unroll
     for (int j = 0; j < 4; ++j) b[4 * t + j] = bias[ch0 + 4 * NT * q + 4 * t + j];
   }
@@ -451,7 +451,7 @@ struct Conv1GradWave {
 // forward map is not positive (its signs, one bit a value).  A wave takes 16 2x2 pixel blocks (rows 2j, 2j + 1,
 // columns 2i, 2i + 1): with stride 2 their nine taps read only the four output pixels
 // (j .. j + 1, i .. i + 1), so dY is read four times and every product is needed.
-// The weights ([tap][ci][co], so that eight co are one vector) stay in 144 registers.
+// The weights (per tap an operand copy with rows ci) stay in 144 registers.
 // Each tap's product is an MFMA chain of its own from zero and the taps are added in
 // FP32: the bits of a column-gradient GEMM followed by col2im, without the FP32 column
 // matrix (354 MB for layer 2 at batch 256).  bpart: per block and channel the FP32 sum
@@ -485,7 +485,8 @@ __device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* 
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int s = 0; s < KS; ++s)
-        w[tap][s][t] = *reinterpret_cast<const uint4*>(Wt + (tap * c.cin + ch0 + tile_channel<NT>(t, r)) * c.cout + 32 * s + 8 * q);
+        w[tap][s][t] = *reinterpret_cast<const uint4*>(Wt + tap * c.cin * c.cout +
+                                                       operand_at(c.cin, ch0 + tile_channel<NT>(t, r), 32 * s + 8 * q));
   float bs[CH];
 #pragma unroll
   for (int j = 0; j < CH; ++j) bs[j] = 0.0f;
@@ -793,8 +794,8 @@ __device__ __forceinline__ void wgrad_block(const uint16_t* dY, const uint16_t* 
 // The backward pass of layer L: its weight gradient (blocks below wblocks), its input
 // gradient (dblocks more) and, beside layer L = 1, the fully connected layers' blocks.
 // Neither needs the other, and neither fills the chip at small batches: one launch
-// instead of two.  Batch 256: layers 2 (with layer 1's weight gradient) / 3 / 4 in 66 / 38 /
-// 28 us (in launches apart 126 / 58 / 42).
+// instead of two.  Batch 256: layers 2 (with layer 1's weight gradient) / 3 / 4 in 64 / 35 /
+// 22 us (in launches apart 126 / 58 / 42).
 struct ConvBackArgs {
   const uint16_t *dY, *X, *Wt;
   const uint8_t* signs;  // of X

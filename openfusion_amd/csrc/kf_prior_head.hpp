@@ -10,9 +10,10 @@ namespace kf {
 constexpr int kFc1Pad = 160;      // FC1 K (134) rounded up to the MFMA step
 constexpr int kDoSumPitch = 8;    // row of FP32 output gradients (their sums take four at a time)
 
-// Second BF16 copies of weights, laid out as operands (padding zero): the convolutions'
-// [tap][ci][co] at the blob's offsets, then FC1 with rows of 160, FC1 transposed
-// ([feature][hidden]) and FC2 transposed with rows of 8.
+// BF16 copies of the weights.  The first holds the blob, layers 2-4 of the convolutions as
+// operands (operand_at).  The second (padding zero): per tap of the convolutions an operand
+// copy with rows ci and k = co at the blob's offsets, then operand copies of FC1 with 160
+// columns and of FC1 transposed, and FC2 transposed with rows of 8.
 struct WeightCopies {
   long w5, w5t, w6t, total;
   WeightCopies() {
@@ -28,24 +29,29 @@ inline const WeightCopies& weight_copies() {
 }
 
 struct WeightCopyArgs {
-  uint16_t *y, *yt;  // the blob as BF16; the operand copies
+  uint16_t *y, *yt;  // the two copies
   long n, w[6], w5, w5t, w6t;
 };
 
 // Parameter i has the value x: its BF16 copies.
 __device__ __forceinline__ void copy_weight(const WeightCopyArgs& a, long i, float x) {
   const uint16_t v = bf16_rne(x);
-  a.y[i] = v;
+  long at = i;
 #pragma unroll
   for (int l = 1; l < kConvs; ++l) {
-    const int e = (int)(i - a.w[l]);
-    if (e >= 0 && e < kConv[l].cout * kConv[l].kc) a.yt[a.w[l] + (e % kConv[l].kc) * kConv[l].cout + e / kConv[l].kc] = v;
+    const int e = (int)(i - a.w[l]), co = e / kConv[l].kc, k = e - co * kConv[l].kc;
+    if (e >= 0 && e < kConv[l].cout * kConv[l].kc) {
+      const int tap = k / kConv[l].cin, ci = k - tap * kConv[l].cin;
+      at = a.w[l] + operand_at(kConv[l].cout, co, k);
+      a.yt[a.w[l] + tap * kConv[l].cin * kConv[l].cout + operand_at(kConv[l].cin, ci, co)] = v;
+    }
   }
+  a.y[at] = v;
   const int f = (int)(i - a.w[4]), g = (int)(i - a.w[5]);
   if (f >= 0 && f < kHidden * kFc1In) {
     const int row = f / kFc1In, col = f - row * kFc1In;
-    a.yt[a.w5 + row * kFc1Pad + col] = v;
-    if (col < kFeat) a.yt[a.w5t + col * kHidden + row] = v;
+    a.yt[a.w5 + operand_at(kHidden, row, col)] = v;
+    if (col < kFeat) a.yt[a.w5t + operand_at(kFeat, col, row)] = v;
   }
   if (g >= 0 && g < kTwist * kHidden) a.yt[a.w6t + g % kHidden * 8 + g / kHidden] = v;
 }
@@ -68,7 +74,7 @@ struct HeadForward {
     for (int t = 0; t < NT; ++t) {
       const int nn = (wave + WAVES * t) * 16 + r;
 #pragma unroll
-      for (int s = 0; s < kFc1Pad / 32; ++s) w5[t][s] = *reinterpret_cast<const uint4*>(W5 + nn * kFc1Pad + 32 * s + 8 * q);
+      for (int s = 0; s < kFc1Pad / 32; ++s) w5[t][s] = *reinterpret_cast<const uint4*>(W5 + operand_at(kHidden, nn, 32 * s + 8 * q));
       b5[t] = B5[nn];
     }
     const int row = min(r, kTwist - 1);  // columns past the six outputs are not used
@@ -142,7 +148,7 @@ struct HeadArgs {
 
 // One sample per block: the forward head, the loss gradient, and back to layer 4
 // (dY4[p][c] = dX5[c] / 80 where Y4 > 0).  Latency bound (six dependent stages); one
-// launch in place of twelve, 60 us of launches at any batch.  18 us at batch 256.
+// launch in place of twelve, 60 us of launches at any batch.  12 us at batch 256.
 __global__ __launch_bounds__(kConvThreads) void head_sample(HeadArgs a) {
   __shared__ __align__(16) uint16_t xs[kFc1Pad], hs[kHidden], dhs[kHidden];
   __shared__ __align__(16) uint16_t dos[8];
@@ -188,7 +194,7 @@ __global__ __launch_bounds__(kConvThreads) void head_sample(HeadArgs a) {
 #pragma unroll
     for (int k = 0; k < kHidden; k += 32)
       acc = mfma32(*reinterpret_cast<const uint4*>(&dhs[k + 8 * q]),
-                   *reinterpret_cast<const uint4*>(a.w5t + nn * kHidden + k + 8 * q), acc);
+                   *reinterpret_cast<const uint4*>(a.w5t + operand_at(kFeat, nn, k + 8 * q)), acc);
     if (q == 0) dx[nn] = acc[0];
   }
   __syncthreads();

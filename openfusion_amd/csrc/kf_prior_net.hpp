@@ -60,6 +60,13 @@ inline const ParamLayout& layout() {
   return L;
 }
 
+// Position of element (row, k) in an operand copy of a weight matrix of `rows` rows: a
+// lane's operand vector is eight k of one row, and the lanes of a quarter wave read
+// neighbouring rows of the same k, so the rows of a vector position lie together.  (Rows on
+// end: a quarter wave's sixteen vectors lie on sixteen lines, and the L1 looks each up:
+// inference at batch 1 17.6 us instead of 12.0, gradients at batch 19 84 instead of 69.)
+__host__ __device__ __forceinline__ int operand_at(int rows, int row, int k) { return ((k >> 3) * rows + row) * 8 + (k & 7); }
+
 // Rounds to the nearest BF16, ties to even: v_cvt_pk_bf16_f32, one instruction for two
 // values (as integer arithmetic on their bits, about nine; the bits are the same for every
 // number and the usual quiet NaN).
