@@ -40,7 +40,7 @@ namespace {
 // of their use; eight waves share each layer's tiles; window pixels are padded by 16
 // bytes in LDS (without, the 16 pixels of an operand read lie on the same banks); the
 // layer-4 pixels go to the last block by agent-scope stores and loads (no L2 write-back
-// and invalidation, kf_icp.hip), all of them in flight together.  Batch 1: 12.0 us (17.6
+// and invalidation, kf_icp.hip), all of them in flight together.  Batch 1: 11.1 us (17.6
 // with the weights' rows on end; 23.7 with four waves, weights loaded where they are used,
 // scalar FC1 weight loads and fences around the hand-over).
 constexpr int kFuseThreads = 512, kFuseWaves = kFuseThreads / kWave;
@@ -54,7 +54,7 @@ struct FuseArgs {
   const int32_t* pairs;
   const float* prev;
   const uint16_t* wbf;   // BF16 weights
-  const uint16_t* w5;    // FC1's operand copy (WeightCopies)
+  const uint16_t *w1, *w5;  // operand copies of layer 1 and FC1 (WeightCopies)
   const float* params;   // FP32 biases
   long w[6], b[6];       // parameter offsets
   float* Y4;             // [B][80][128] layer-4 activations
@@ -153,11 +153,7 @@ __global__ __launch_bounds__(kFuseThreads) void prior_infer_fused(FuseArgs f) {
   float b1[8];
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
-    uint16_t e[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      e[j] = 8 * q + j < kConv[0].kc ? f.wbf[f.w[0] + tile_channel<2>(t, r) * kConv[0].kc + 8 * q + j] : (uint16_t)0;
-    __builtin_memcpy(&w1[t], e, 16);
+    w1[t] = conv1_weights(f.w1, t, r, q);
 #pragma unroll
     for (int j = 0; j < 4; ++j) b1[4 * t + j] = f.params[f.b[0] + 8 * q + 4 * t + j];
   }
@@ -299,6 +295,7 @@ WeightCopyArgs copy_args(kf_prior* P) {
   a.yt = P->wt;
   a.n = P->nparams;
   for (int q = 0; q < 6; ++q) a.w[q] = layout().w[q];
+  a.w1 = weight_copies().w1;
   a.w5 = weight_copies().w5;
   a.w5t = weight_copies().w5t;
   a.w6t = weight_copies().w6t;
@@ -333,7 +330,7 @@ kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, int B,
   uint8_t* none[kConvs - 1] = {};
   uint8_t* const* signs = train ? P->signs : none;
   hipLaunchKernelGGL(conv1_forward, dim3(kConv[0].hout / kL1Rows, B), dim3(kConvThreads), 0, s, frames, pairs,
-                     (const uint16_t*)P->wbf + L.w[0], (const float*)P->params + L.b[0], P->Yb[0], signs[0]);
+                     (const uint16_t*)P->wt + weight_copies().w1, (const float*)P->params + L.b[0], P->Yb[0], signs[0]);
   KF_TRY(check_launch("conv1_forward"));
   KF_TRY((launch_conv<1, 4, false>(P, P->Yb[0], P->Yb[1], nullptr, signs[1], B, s)));
   KF_TRY((launch_conv<2, 2, false>(P, P->Yb[1], P->Yb[2], nullptr, signs[2], B, s)));
@@ -361,6 +358,7 @@ kf_status infer(kf_prior* P, const float* frames, const int32_t* pairs, const fl
   f.pairs = pairs;
   f.prev = prev;
   f.wbf = P->wbf;
+  f.w1 = P->wt + weight_copies().w1;
   f.w5 = P->wt + weight_copies().w5;
   f.params = P->params;
   for (int q = 0; q < 6; ++q) {

@@ -102,54 +102,61 @@ struct TileRun {
 // 32-bit LDS read is one tap's two channels.
 constexpr int kL1Rows = 4;                      // output rows of a block
 constexpr int kL1In = 2 * kL1Rows + 1;          // input rows under them
-constexpr int kL1Pitch = kW0 + 2;               // columns -1 .. 159 (and one of padding)
+constexpr int kL1Pitch = kW0 + 4;               // columns -1 .. 159 from 3 on
 static_assert(kConv[0].hout % kL1Rows == 0, "layer-1 row groups");
 
-// The input rows under output rows oy0 .. oy0 + kL1Rows - 1 (zero outside the frame).
-__device__ __forceinline__ void stage_l1(uint32_t (*patch)[kL1Pitch], const float* f0, const float* f1, int oy0) {
-  constexpr int E = kL1In * kL1Pitch, PER = (E + kConvThreads - 1) / kConvThreads;
-  float v[PER][2];
-#pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int e = threadIdx.x + kConvThreads * u;
-    const int row = e / kL1Pitch, col = e - row * kL1Pitch;
-    const int iy = 2 * oy0 - 1 + row, ix = col - 1;
-    const bool in = e < E && iy >= 0 && iy < kH0 && ix >= 0 && ix < kW0;
-    const int o = in ? iy * kW0 + ix : 0;
-    v[u][0] = in ? f0[o] : 0.0f;
-    v[u][1] = in ? f1[o] : 0.0f;
-  }
-#pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int e = threadIdx.x + kConvThreads * u;
-    if (e < E) patch[e / kL1Pitch][e % kL1Pitch] = pack_bf16(v[u][0], v[u][1]);
-  }
+// One operand tile of layer 1's weights (WeightCopies::w1), its 18 columns padded to 32.
+__device__ __forceinline__ uint4 conv1_weights(const uint16_t* W1, int t, int r, int q) {
+  return *reinterpret_cast<const uint4*>(W1 + operand_at(kConv[0].cout, tile_channel<2>(t, r), 8 * q));
 }
 
+// Bound by the map's stores (79 MB at batch 256).  A row of the patch is loaded as 16-byte
+// vectors of both frames and written as whole vectors (column 0 at 4, so that they are
+// aligned; column -1 at 3 is always outside the frame).  Batch 256: 22.5 us; with single pixels,
+// two divisions each, and the weights as 16-bit loads 31.
 __global__ __launch_bounds__(kConvThreads) void conv1_forward(const float* frames, const int32_t* pairs,
-                                                              const uint16_t* W, const float* bias, uint16_t* Yb,
+                                                              const uint16_t* W1, const float* bias, uint16_t* Yb,
                                                               uint8_t* signs) {
   constexpr ConvShape c = kConv[0];
-  __shared__ uint32_t patch[kL1In][kL1Pitch];
+  typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+  __shared__ __align__(16) uint32_t patch[kL1In][kL1Pitch];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
   const int n = blockIdx.y, oy0 = blockIdx.x * kL1Rows;
-  stage_l1(patch, frames + (long)pairs[2 * n] * (kH0 * kW0), frames + (long)pairs[2 * n + 1] * (kH0 * kW0), oy0);
+  const float* f0 = frames + (long)pairs[2 * n] * (kH0 * kW0);
+  const float* f1 = frames + (long)pairs[2 * n + 1] * (kH0 * kW0);
+  constexpr int V = kW0 / 4, E = kL1In * V, PER = (E + kConvThreads - 1) / kConvThreads;
+  f4 v[PER][2];
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int e = threadIdx.x + kConvThreads * u, o = (2 * oy0 - 1) * kW0 + 4 * e;  // row 2 oy0 - 1 + e / V
+    v[u][0] = v[u][1] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (e < E && o >= 0) {
+      v[u][0] = *reinterpret_cast<const f4*>(f0 + o);
+      v[u][1] = *reinterpret_cast<const f4*>(f1 + o);
+    }
+  }
   uint4 w[2];
   float b[8];
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
-    uint16_t e[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) e[j] = 8 * q + j < c.kc ? W[tile_channel<2>(t, r) * c.kc + 8 * q + j] : (uint16_t)0;
-    __builtin_memcpy(&w[t], e, 16);
+    w[t] = conv1_weights(W1, t, r, q);
 #pragma unroll
     for (int j = 0; j < 4; ++j) b[4 * t + j] = bias[8 * q + 4 * t + j];
   }
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int e = threadIdx.x + kConvThreads * u;
+    if (e < E)
+      *reinterpret_cast<uint4*>(&patch[e / V][4 + 4 * (e % V)]) =
+          make_uint4(pack_bf16(v[u][0].x, v[u][1].x), pack_bf16(v[u][0].y, v[u][1].y), pack_bf16(v[u][0].z, v[u][1].z),
+                     pack_bf16(v[u][0].w, v[u][1].w));
+  }
+  if (threadIdx.x < kL1In) patch[threadIdx.x][3] = 0u;
   int off[4];  // the lane's four taps (4 q ..), tap 8 standing in for those past the kernel
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int tap = min(4 * q + e, 8);
-    off[e] = (tap / 3) * kL1Pitch + tap % 3;
+    off[e] = (tap / 3) * kL1Pitch + tap % 3 + 3;
   }
   __syncthreads();
   const uint32_t* flat = &patch[0][0];

@@ -12,12 +12,13 @@ constexpr int kDoSumPitch = 8;    // row of FP32 output gradients (their sums ta
 
 // BF16 copies of the weights.  The first holds the blob, layers 2-4 of the convolutions as
 // operands (operand_at).  The second (padding zero): per tap of the convolutions an operand
-// copy with rows ci and k = co at the blob's offsets, then operand copies of FC1 with 160
-// columns and of FC1 transposed, and FC2 transposed with rows of 8.
+// copy with rows ci and k = co at the blob's offsets, then operand copies of layer 1 with 32
+// columns, of FC1 with 160 and of FC1 transposed, and FC2 transposed with rows of 8.
 struct WeightCopies {
-  long w5, w5t, w6t, total;
+  long w1, w5, w5t, w6t, total;
   WeightCopies() {
-    w5 = (layout().total + 7) / 8 * 8;
+    w1 = (layout().total + 7) / 8 * 8;
+    w5 = w1 + kConv[0].cout * 32;
     w5t = w5 + kHidden * kFc1Pad;
     w6t = w5t + kFeat * kHidden;
     total = w6t + kHidden * 8;
@@ -30,7 +31,7 @@ inline const WeightCopies& weight_copies() {
 
 struct WeightCopyArgs {
   uint16_t *y, *yt;  // the two copies
-  long n, w[6], w5, w5t, w6t;
+  long n, w[6], w1, w5, w5t, w6t;
 };
 
 // Parameter i has the value x: its BF16 copies.
@@ -47,7 +48,9 @@ __device__ __forceinline__ void copy_weight(const WeightCopyArgs& a, long i, flo
     }
   }
   a.y[at] = v;
-  const int f = (int)(i - a.w[4]), g = (int)(i - a.w[5]);
+  const int f = (int)(i - a.w[4]), g = (int)(i - a.w[5]), h = (int)(i - a.w[0]);
+  if (h >= 0 && h < kConv[0].cout * kConv[0].kc)
+    a.yt[a.w1 + operand_at(kConv[0].cout, h / kConv[0].kc, h % kConv[0].kc)] = v;
   if (f >= 0 && f < kHidden * kFc1In) {
     const int row = f / kFc1In, col = f - row * kFc1In;
     a.yt[a.w5 + operand_at(kHidden, row, col)] = v;
