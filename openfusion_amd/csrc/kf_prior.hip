@@ -378,13 +378,19 @@ kf_status infer(kf_prior* P, const float* frames, const int32_t* pairs, const fl
 // bias gradient, one block a CU beside the first: two blocks fit a CU, so all are
 // resident at once (512 blocks of input gradient ran a second round: 179 us against 159
 // for the three layers at batch 256).  fc (L = 1): carried along.
-constexpr int kWgradBlocks = 256, kWgradMinSteps = 4, kDgradBlocks = 256;
+// Layer 2's input gradient, which also makes layer 1's weight gradient, takes longer than
+// its weight gradient: from eight tiles a wave on it gets 320 of the 512 blocks (batch 256:
+// 58.9 us against 66.8; with few tiles a block mostly loads its weights, and 256 are the
+// better: batch 19 11.6 us against 12.6).
+constexpr int kWgradBlocks = 256, kWgradMinSteps = 4, kDgradBlocks = 256, kDgradMore = 320;
 template <int L>
 kf_status launch_backward(kf_prior* P, int B, int* splits, int* planes, hipStream_t s, const FcGradArgs& fc = FcGradArgs{},
                           const Conv1Grad& first = Conv1Grad{}) {
   constexpr int GROUPS = WgradShape<L>::GROUPS;
   const int M = B * kConv[L].hout * kConv[L].wout, steps = div_up(M, kWgradStep);
-  const int want = std::min(std::max(steps / kWgradMinSteps, 1), kWgradBlocks / GROUPS);
+  const int units = div_up(div_up(M, 16) * DgradShape<L>::GROUPS, kConvWaves);  // blocks at one tile a wave
+  const int most = L == 1 && units >= 8 * kDgradMore ? kDgradMore : kDgradBlocks;
+  const int want = std::min(std::max(steps / kWgradMinSteps, 1), (kWgradBlocks + kDgradBlocks - most) / GROUPS);
   ConvBackArgs a;
   a.dY = P->dYb[L];
   a.X = P->Yb[L - 1];
@@ -399,7 +405,7 @@ kf_status launch_backward(kf_prior* P, int B, int* splits, int* planes, hipStrea
   // eight splits a round (blocks of one split on one XCD): the count is rounded up, and
   // the splits past the last write zero planes that nothing reads
   a.wblocks = div_up(*splits, 8) * 8 * GROUPS;
-  a.dblocks = *planes = std::min(div_up(div_up(M, 16) * DgradShape<L>::GROUPS, kConvWaves), kDgradBlocks);
+  a.dblocks = *planes = std::min(units, most);
   a.fc = fc;
   a.first = first;
   hipLaunchKernelGGL(conv_backward<L>, dim3(a.wblocks + a.dblocks + (L == 1 ? kFcBlocks : 0)), dim3(kConvThreads), 0, s, a);
@@ -530,9 +536,9 @@ extern "C" kf_status kf_prior_create(int32_t max_batch, kf_prior** out) {
       al((void**)&P->signs[l], M * c.cout / 8);
     }
     else al((void**)&P->Y4, M * c.cout * 4);
-    al((void**)&P->wpart[l], (l == 0 ? kDgradBlocks : kWgradBlocks / (c.cout / (l == 1 ? 64 : 32))) * c.cout * c.kc * 4);
+    al((void**)&P->wpart[l], (l == 0 ? kDgradMore : kWgradBlocks / (c.cout / (l == 1 ? 64 : 32))) * c.cout * c.kc * 4);
     if (l > 0) al((void**)&P->dYb[l], M * c.cout * 2);  // layer 1's stays in the kernel that makes it
-    al((void**)&P->bpart[l], (l + 1 < kConvs ? kDgradBlocks : B) * c.cout * 4);
+    al((void**)&P->bpart[l], (l + 1 < kConvs ? kDgradMore : B) * c.cout * 4);
   }
   al((void**)&P->X5b, B * kX5Pitch * 2);
   al((void**)&P->Hb, B * kHidden * 2);

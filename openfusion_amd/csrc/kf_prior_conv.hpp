@@ -24,6 +24,13 @@ __device__ __forceinline__ int tile_channel(int t, int i) {
   return (i >> 2) * 4 * NT + 4 * t + (i & 3);
 }
 
+// The 16 bytes at element `at` of a map, element 0 if not `in`.  The offset goes through an
+// opaque register: otherwise the compiler sees that the value will not be used, and
+// branches around each load.
+__device__ __forceinline__ uint4 load_vec(const uint16_t* p, bool in, int at) {
+  return *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(p) + opaque_u32(in ? 2u * (unsigned)at : 0u));
+}
+
 // Stores N (a multiple of 4) floats as BF16 to p (8-byte aligned; 16-byte aligned when N is a multiple of 8).
 template <int N>
 __device__ __forceinline__ void store_words(uint16_t* p, const uint32_t* w) {
@@ -223,7 +230,7 @@ struct ConvTile {
 #pragma unroll
       for (int ky = 0; ky < 3; ++ky) {
         in[ky][u] = row_in(oy, ky);
-        v[ky][u] = *reinterpret_cast<const uint4*>(X + (in[ky][u] ? at + ky * c.win * c.cin : 0));
+        v[ky][u] = load_vec(X, in[ky][u], at + ky * c.win * c.cin);
       }
     }
     const int m = tile * 16, ky = lane / PC;
@@ -539,8 +546,7 @@ __device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* 
       const uint16_t* src = dY + (in ? (m + dj * c.wout) * c.cout : 0) + 8 * q;
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
-        a[dj][0][s] = *reinterpret_cast<const uint4*>(src + 32 * s);
-        if (!in) a[dj][0][s] = make_uint4(0u, 0u, 0u, 0u);
+        a[dj][0][s] = load_vec(dY, in, (m + dj * c.wout) * c.cout + 8 * q + 32 * s);
         a[dj][1][s] = make_uint4(0u, 0u, 0u, 0u);
         if ((r & kEnd) == kEnd && in && i + 1 < c.wout) a[dj][1][s] = *reinterpret_cast<const uint4*>(src + c.cout + 32 * s);
       }
@@ -549,6 +555,8 @@ __device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* 
     for (int dj = 0; dj < 2; ++dj)
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
+        // (selects only here: before, each would wait for its load)
+        if (dj == 1 && j + 1 >= c.hout) a[dj][0][s] = make_uint4(0u, 0u, 0u, 0u);
         const uint4 own = a[dj][1][s];
         uint4 v = neighbour<0x101>(a[dj][0][s], own);
         if (i + 1 >= c.wout) v = make_uint4(0u, 0u, 0u, 0u);
@@ -745,6 +753,7 @@ __device__ __forceinline__ void wgrad_block(const uint16_t* dY, const uint16_t* 
   const int px = tid >> 3, v0 = tid & 7;
   const int first = split * steps_per_split, last = min(first + steps_per_split, (M + kWgradStep - 1) / kWgradStep);
   uint4 vc[kPer], vd;
+  bool in[kPer], in_dy;  // vectors outside the map (zeroed when staged: a select here would wait for the load)
   auto load = [&](int step) {
     const int m = step * kWgradStep + px;
     const bool live = m < M;
@@ -757,12 +766,11 @@ __device__ __forceinline__ void wgrad_block(const uint16_t* dY, const uint16_t* 
       const int v = v0 + 8 * u, tap = v / kTapVecs, ci = 8 * (v - tap * kTapVecs);
       const int ky = tap / 3, kx = tap - 3 * ky;
       const int iy = 2 * oy + ky - 1, ix = 2 * ox + kx - 1;
-      const bool in = live && v < kVecs && iy >= 0 && iy < c.hin && ix >= 0;
-      vc[u] = *reinterpret_cast<const uint4*>(X + (in ? at + (ky * c.win + kx) * c.cin + ci : 0));
-      if (!in) vc[u] = make_uint4(0u, 0u, 0u, 0u);
+      in[u] = live && v < kVecs && iy >= 0 && iy < c.hin && ix >= 0;
+      vc[u] = load_vec(X, in[u], at + (ky * c.win + kx) * c.cin + ci);
     }
-    vd = make_uint4(0u, 0u, 0u, 0u);
-    if (live && v0 < COB / 8) vd = *reinterpret_cast<const uint4*>(dY + m * c.cout + co0 + 8 * v0);
+    in_dy = live && v0 < COB / 8;
+    vd = load_vec(dY, in_dy, m * c.cout + co0 + 8 * v0);
   };
   v4f acc[2][9];
 #pragma unroll
@@ -774,8 +782,9 @@ __device__ __forceinline__ void wgrad_block(const uint16_t* dY, const uint16_t* 
   for (int step = first; step < last; ++step) {
 #pragma unroll
     for (int u = 0; u < kPer; ++u)
-      if (v0 + 8 * u < kVecs) *reinterpret_cast<uint4*>(&s_col[px * kColPitch + 8 * (v0 + 8 * u)]) = vc[u];
-    if (v0 < COB / 8) *reinterpret_cast<uint4*>(&s_dy[px * kDyPitch + 8 * v0]) = vd;
+      if (v0 + 8 * u < kVecs) *reinterpret_cast<uint4*>(&s_col[px * kColPitch + 8 * (v0 + 8 * u)]) =
+            in[u] ? vc[u] : make_uint4(0u, 0u, 0u, 0u);
+    if (v0 < COB / 8) *reinterpret_cast<uint4*>(&s_dy[px * kDyPitch + 8 * v0]) = in_dy ? vd : make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
     if (step + 1 < last) load(step + 1);
     uint4 a[2];
@@ -801,8 +810,8 @@ __device__ __forceinline__ void wgrad_block(const uint16_t* dY, const uint16_t* 
 // The backward pass of layer L: its weight gradient (blocks below wblocks), its input
 // gradient (dblocks more) and, beside layer L = 1, the fully connected layers' blocks.
 // Neither needs the other, and neither fills the chip at small batches: one launch
-// instead of two.  Batch 256: layers 2 (with layer 1's weight gradient) / 3 / 4 in 64 / 35 /
-// 22 us (in launches apart 126 / 58 / 42).
+// instead of two.  Batch 256: layers 2 (with layer 1's weight gradient) / 3 / 4 in 59 / 33 /
+// 21 us (in launches apart 126 / 58 / 42).
 struct ConvBackArgs {
   const uint16_t *dY, *X, *Wt;
   const uint8_t* signs;  // of X

@@ -1,6 +1,7 @@
 """The prior's training kernels against the FP64 oracle (BF16 operand rounding emulated)
 at batches where their tilings end: one sample (layer 3's 300 pixels are no multiple of
-a 16-pixel tile), an odd batch, and one where every wave takes several tiles."""
+a 16-pixel tile), odd batches, one where every wave takes several tiles, and the first
+where layer 2's input gradient gets more blocks than its weight gradient."""
 import numpy as np
 import pytest
 
@@ -9,7 +10,7 @@ from oracle import prior_oracle as po
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("B", [1, 3, 37])
+@pytest.mark.parametrize("B", [1, 3, 37, 137])
 def test_gradients_match_oracle_at_tile_edges(gpu, kf, B):
     rng = np.random.default_rng(100 + B)
     F = B + 1
