@@ -37,13 +37,10 @@ constexpr int kWavesPerBlock = 4;
 constexpr int kSweepMaxBlocks = 4096;  // 16384 waves: two full waves of residency on 256 CUs
 // The sweep's blocks (their waves stride over the brick list): more than can be
 // resident at once, so that the sweep keeps taking the CU slots that the frame's
-// concurrent preprocessing and prior inference leave free.  Up to 64 bricks per
-// axis the frame's two streams end close together and twice the blocks pay in the
-// frame (measured at 512^3: +0.8 % fps, though the sweep alone takes 87 instead of
-// 54 us); beyond that the sweep's stream is the longer by far and its own speed
-// decides (768^3: 3072 blocks 0.5 % faster than 6144).
+// concurrent preprocessing and prior inference leave free.  512^3, 300-frame stream:
+// 3072 blocks 4482-4494 frames/s and 54 us for the sweep alone, 6144 blocks 4489-4490 and
+// 87 us, 1536 blocks 4374-4377 and 49 us.
 constexpr int kSweepListBlocks = 3072;
-constexpr int kSweepListBlocksSmall = 6144;  // volumes of at most 64 bricks per axis
 constexpr uint32_t kSweepXcdChunk = 16;  // consecutive sweep blocks kept on one XCD
 // x-slices of a brick whose loads a wavefront issues together: four (70 VGPRs, seven
 // waves per SIMD) beat all eight at once (98 VGPRs, five waves per SIMD)
@@ -893,8 +890,7 @@ kf_status launch_integrate(kf_volume* v, const kf_intrinsics& k0, const kf_integ
   hipLaunchKernelGGL(brick_classify, dim3(div_up(nbricks, 256)), dim3(256), 0, s, a);
   KF_TRY(check_launch("brick_classify"));
   if (between) KF_HIP(hipEventRecord(between, s));
-  const int list_blocks = a.nb <= 64 ? kSweepListBlocksSmall : kSweepListBlocks;
-  const int blocks = std::min(div_up(nbricks, kWavesPerBlock), list_blocks);
+  const int blocks = std::min(div_up(nbricks, kWavesPerBlock), kSweepListBlocks);
   auto kern = d.format == KF_VOXEL_F16 ? integrate<KF_VOXEL_F16> : integrate<KF_VOXEL_F32>;
   if (kernel_start && kernel_stop)
     hipExtLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, s, kernel_start, kernel_stop, 0, a);
