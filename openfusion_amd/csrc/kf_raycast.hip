@@ -13,10 +13,10 @@
 // centre and gd the ray direction in voxel units, one fused multiply-add per axis
 // and sample; g = floor(g) + fract(g) gives the trilinear cell and weights.
 //
-// Ray/tile mapping: a 256-thread block covers 16x16 pixels, each wavefront an
-// 8x8 tile (rays in a wave stay coherent in the volume).  Block ids are remapped
-// so each of the 8 XCDs (which receive blocks round-robin) owns a contiguous
-// band of image rows and its L2 sees neighbouring rays.
+// Ray/tile mapping: each wavefront of a 256-thread block takes an 8x8 pixel tile (rays
+// in a wave stay coherent in the volume), the four together or a quarter of the image
+// apart.  Block ids are remapped so that each of the 8 XCDs (which receive blocks
+// round-robin) owns contiguous bands of tiles and its L2 sees neighbouring rays.
 //
 // Normals are computed once per wavefront after every ray of it has finished its
 // march: each hit loads the 32 voxels of its six central-difference samples in one
@@ -45,6 +45,14 @@ namespace kf {
 namespace {
 
 constexpr int kXcds = 8;
+// Long rays lie together in the image, and the waves of a block share a CU's L1, whose
+// line lookups a round of corner loads takes 800 of: from 384 blocks (1.5 a CU) on, a
+// block's four tiles are a quarter of the image apart.  512^3 FP16, together / apart:
+// 480x360 30.7 / 28.2 us, 640x480 35.0 / 34.5, 800x600 45.2 / 42.8; late in a 300-frame
+// stream, beside the frame's other kernels, 4,496 / 4,568 frames/s.  With about a block a CU
+// there is nothing to balance and the tiles' shared lines count: 319x241 26.1 / 26.5 us
+// (256^3 FP32 29.2 / 30.0).
+constexpr int kSpreadBlocks = 384;
 
 struct RayArgs {
   const void* vox;
@@ -68,6 +76,7 @@ struct RayArgs {
   float inv_step_far;  // 1 / step_far_m (estimates only)
   int max_steps;
   int blocks_x, blocks_y;
+  int spread;  // a block's wavefronts take tiles a quarter of the image apart
 };
 
 // Interpolations and points along a ray are fused multiply-adds (one rounding each;
@@ -317,8 +326,14 @@ __global__ __launch_bounds__(256) void raycast(RayArgs a) {
   if (logical >= nb) return;  // whole block
   const int by = logical / a.blocks_x, bx = logical - by * a.blocks_x;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int x = bx * 16 + (wave & 1) * 8 + (lane & 7);
-  const int y = by * 16 + (wave >> 1) * 8 + (lane >> 3);
+  int x = bx * 16 + (wave & 1) * 8, y = by * 16 + (wave >> 1) * 8;
+  if (a.spread) {
+    const int tile = logical + wave * nb, tx = 2 * a.blocks_x;
+    x = tile % tx * 8;
+    y = tile / tx * 8;
+  }
+  x += lane & 7;
+  y += lane >> 3;
   const bool active = x < a.W && y < a.H;  // no early return: the step count is wave-reduced
   const int idx = active ? y * a.W + x : 0;
   const kf_posef P = a.pose->wc;
@@ -642,6 +657,7 @@ kf_status launch_raycast(const kf_volume* v, const kf_intrinsics& k0, const kf_r
   a.blocks_y = div_up(k0.height, 16);
   const int nb = a.blocks_x * a.blocks_y;
   const int grid = ((nb + kXcds - 1) / kXcds) * kXcds;
+  a.spread = nb >= kSpreadBlocks;
   // 32-bit voxel offsets when every byte offset of the volume fits in 32 bits
   const bool off32 = v->bytes <= 0xffffffffull && d.n <= 1024;
   auto kern = d.format == KF_VOXEL_F16 ? (off32 ? raycast<KF_VOXEL_F16, true> : raycast<KF_VOXEL_F16, false>)

@@ -64,3 +64,25 @@ def test_raycast_edges(gpu, kf, orc, n, fmt, view):
                 assert same_bits(model.plane(lvl, nm), om.plane(lvl, nm)), (far, most, lvl, nm)
         if view not in ("past", "farther") and n == 72 and far == 0.8 and most == 2048:
             assert (~np.isnan(om.plane(0, "vz"))).sum() > 200
+
+
+@pytest.mark.parametrize("w,h", [(319, 304), (313, 309)])
+def test_raycast_block_maps(gpu, kf, orc, w, h):
+    """380 and 400 blocks: the last image whose blocks cover 16x16 pixels, and an odd-sized
+    one whose blocks' tiles are a quarter of the image apart; every pixel once."""
+    d, f = _field(72, 1)
+    raw = fill_volume(d, f, 1.0)
+    vol = kf.Volume(72, 1.0, d.trunc_m, 128.0, 1, origin=(d.origin_m[0], d.origin_m[1], d.origin_m[2]))
+    vol.upload_raw(raw)
+    k, p = intr(w, h, 240.0, 240.0), ray_params()
+    T = pose(0.6, -2.3, 0.4)
+    T[:3, 3] = np.array([0.2, 0.0, 0.0]) - 1.2 * T[:3, 2]
+    model, steps = kf.DeviceMaps(k, 3, False), kf.DeviceBuffer(8)
+    steps.zero()
+    kf.Raycaster(k, p).Raycast(vol, kf.DevicePose(T), model, steps=steps)
+    kf.synchronize()
+    om, osteps = orc.raycast(d, 1, raw, k, p, T, 3)
+    assert int(steps.download(np.uint64)[0]) == osteps
+    for lvl in range(3):
+        for nm in PLANES:
+            assert same_bits(model.plane(lvl, nm), om.plane(lvl, nm)), (lvl, nm)
