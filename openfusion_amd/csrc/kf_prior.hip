@@ -40,7 +40,7 @@ namespace {
 // of their use; eight waves share each layer's tiles; window pixels are padded by 16
 // bytes in LDS (without, the 16 pixels of an operand read lie on the same banks); the
 // layer-4 pixels go to the last block by agent-scope stores and loads (no L2 write-back
-// and invalidation, kf_icp.hip), all of them in flight together.  Batch 1: 11.1 us (17.6
+// and invalidation, kf_icp.hip), all of them in flight together.  Batch 1: 10.6 us (17.6
 // with the weights' rows on end; 23.7 with four waves, weights loaded where they are used,
 // scalar FC1 weight loads and fences around the hand-over).
 constexpr int kFuseThreads = 512, kFuseWaves = kFuseThreads / kWave;
