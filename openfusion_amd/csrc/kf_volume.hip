@@ -29,6 +29,7 @@
 
 #include "kf_device.hpp"
 #include "kf_internal.hpp"
+#include "kf_launch.hpp"
 
 namespace kf {
 namespace {
@@ -73,11 +74,11 @@ struct SweepArgs {
   float band;  // T + max(0.01 T, 0.1 mm): half-width of the band where the square root is taken
 };
 
-// One 16-byte store per thread, no loop.  Bound by memory; 512 MB: 78 us, 6.8 TB/s (a
-// grid-stride loop 117 us on 8192 blocks, 96 on 16384; two or more stores a thread 88
-// and up), 128 MB: 20.6 us against 21.9.
-__global__ __launch_bounds__(256) void volume_fill(uint4* p, size_t n16, uint4 word) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+// One 16-byte store per thread, no loop (launch_items: more than 2^31 take several
+// launches).  Bound by memory; 512 MB: 78 us, 6.8 TB/s (a grid-stride loop 117 us on 8192
+// blocks, 96 on 16384; two or more stores a thread 88 and up), 128 MB: 20.6 us against 21.9.
+__global__ __launch_bounds__(kItemThreads) void volume_fill(uint4* p, size_t n16, uint4 word) {
+  const size_t i = (size_t)blockIdx.x * kItemThreads + threadIdx.x;
   if (i < n16) p[i] = word;
 }
 
@@ -786,10 +787,11 @@ kf_status launch_volume_reset(kf_volume* v, hipStream_t s) {
     const uint32_t one = 0x3F800000u;  // 1.0f, weight 0.0f
     word = make_uint4(one, 0u, one, 0u);
   }
-  const size_t n16 = v->bytes / 16;
-  hipLaunchKernelGGL(volume_fill, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, s, static_cast<uint4*>(v->d_voxels), n16,
-                     word);
-  KF_TRY(check_launch("volume_fill"));
+  KF_TRY(launch_items(v->bytes / 16, [&](size_t first, size_t count, unsigned blocks) {
+    hipLaunchKernelGGL(volume_fill, dim3(blocks), dim3(kItemThreads), 0, s, static_cast<uint4*>(v->d_voxels) + first, count,
+                       word);
+    return check_launch("volume_fill");
+  }));
   if (v->d_occ) KF_TRY(clear_occupancy(v, s));  // every voxel is free space: all bricks clear
   v->occ_stale = false;
   return KF_OK;
