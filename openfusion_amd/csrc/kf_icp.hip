@@ -197,10 +197,13 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// LDS of block_partial.
-template <int WAVES, int K>
+// LDS of block_partial.  Compensated mode: the row entries of one round of a wave, one
+// pixel per column; the rounds take turns in it (34 KB for eight waves, so that a CU holds
+// as many blocks as the registers allow; three rounds' rows side by side, 104 KB, left room
+// for one).  Plain mode has no rows.
+template <bool COMP, int WAVES>
 struct PartialLds {
-  double rows[WAVES][K][8][kRowPitch];  // compensated mode: a wave's row entries, one pixel per column
+  double rows[COMP ? WAVES : 1][COMP ? 8 : 1][COMP ? kRowPitch : 1];
   double red[WAVES][kWave];
   int cand[WAVES];
 };
@@ -300,7 +303,7 @@ __device__ __forceinline__ PxPre<Shape::K> load_models(const IcpArgs& a, int bid
 // terms and the inlier and candidate counts.  PRE: the first pass' samples are given.
 template <bool COMP, typename Shape, int WAVES, bool PRE = false, bool COH = false>
 __device__ __forceinline__ void block_partial(const IcpArgs& a, const kf_posef& wc, const kf_posef& cw, int bid,
-                                              int nblk, double* slot, PartialLds<WAVES, Shape::K>& lds,
+                                              int nblk, double* slot, PartialLds<COMP, WAVES>& lds,
                                               PxPre<Shape::K> pre = {}) {
   constexpr int K = Shape::K;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -313,7 +316,6 @@ __device__ __forceinline__ void block_partial(const IcpArgs& a, const kf_posef& 
 #pragma unroll
     for (int k = 0; k < kPad; ++k) s[k] = 0.0f;
   }
-  double (*rows)[8][kRowPitch] = lds.rows[wave];
   for (int pass = 0; pass < passes; ++pass) {
     if (!PRE || pass > 0) pre = load_models<Shape>(a, bid, nblk, pass);
     int j[K], r[K];
@@ -330,7 +332,6 @@ __device__ __forceinline__ void block_partial(const IcpArgs& a, const kf_posef& 
 #pragma unroll
     for (int k = 0; k < K; ++k)
       if (k < rounds) l[k] = load_live(a, j[k]);
-    if constexpr (COMP) wave_lds_sync();  // the previous pass' reads are done
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       if (k >= rounds) continue;
@@ -345,20 +346,18 @@ __device__ __forceinline__ void block_partial(const IcpArgs& a, const kf_posef& 
       for (int p = 0; p < 6; ++p) A[p] = inl ? A[p] : 0.0f;
       b = inl ? b : 0.0f;
       if constexpr (COMP) {
+        double (*rows)[kRowPitch] = lds.rows[wave];
+        wave_lds_sync();  // the previous round's reads are done
 #pragma unroll
-        for (int p = 0; p < 6; ++p) rows[k][p][lane] = (double)A[p];
-        rows[k][6][lane] = (double)b;
-        rows[k][7][lane] = inl ? 1.0 : 0.0;
+        for (int p = 0; p < 6; ++p) rows[p][lane] = (double)A[p];
+        rows[6][lane] = (double)b;
+        rows[7][lane] = inl ? 1.0 : 0.0;
+        wave_lds_sync();
+        sums.add(rows);
       } else {
         accumulate(s, A, b);
         n_in += (int)__popcll(__ballot(inl));
       }
-    }
-    if constexpr (COMP) {
-      wave_lds_sync();
-#pragma unroll
-      for (int k = 0; k < K; ++k)
-        if (k < rounds) sums.add(rows[k]);
     }
   }
   if constexpr (COMP) {
@@ -593,7 +592,7 @@ __device__ __forceinline__ void copy_pose(const kf_pose* src, kf_pose* dst) {
 template <bool COMP>
 __global__ __launch_bounds__(kThreads) void icp_partials(IcpArgs a) {
   using Shape = PixelShape<kThreads / kWave, 2, 0>;
-  __shared__ PartialLds<kThreads / kWave, Shape::K> lds;
+  __shared__ PartialLds<COMP, kThreads / kWave> lds;
   const kf_posef wc = a.pose->wc, cw = a.pose->cw;
   block_partial<COMP, Shape>(a, wc, cw, blockIdx.x, gridDim.x, a.partials + (size_t)blockIdx.x * kSlot, lds);
 }
@@ -641,7 +640,7 @@ __global__ __launch_bounds__(kStepThreads) void icp_step(IcpArgs a, StepArgs S) 
   __shared__ kf_posef s_wc, s_cw;
   __shared__ SlotFin<kStepThreads> fin;
   using Shape = StepShape<F, H>;
-  __shared__ PartialLds<kStepThreads / kWave, Shape::K> lds;
+  __shared__ PartialLds<COMP, kStepThreads / kWave> lds;
   const int tid = threadIdx.x;
   double* slot_out = S.slots_out + (size_t)blockIdx.x * kSlot;
   // Every load that does not depend on another is issued up front, in the order
@@ -914,12 +913,10 @@ __device__ __forceinline__ bool grid_barrier(kf_icp_ctrl* ctrl, unsigned target,
 template <bool COMP, typename Shape>
 __device__ __forceinline__ bool chain_iteration(const IcpArgs& a, int nb, bool solve, const double* slots_in,
                                                 int nb_in, int lvl_in, double* slots_out,
-                                                SlotFin<kStepThreads>& fin, PartialLds<kStepThreads / kWave, 3>& lds3,
+                                                SlotFin<kStepThreads>& fin, PartialLds<COMP, kStepThreads / kWave>& lds,
                                                 double (*T)[16], int& cur, kf_posef* wc, kf_posef* cw,
                                                 kf_icp_stats* st) {
   constexpr int WV = kStepThreads / kWave;
-  auto& lds = reinterpret_cast<PartialLds<WV, Shape::K>&>(lds3);  // room for the largest shape
-  static_assert(Shape::K <= 3, "chain LDS");
   SlotSum<kStepThreads, true> L;
   if (solve) L.load(slots_in, nb_in);
   const bool mine = (int)blockIdx.x < nb;
@@ -945,7 +942,7 @@ __global__ __launch_bounds__(kStepThreads) void icp_chain(ChainArgs C) {
   __shared__ double T[2][16];
   __shared__ kf_posef s_wc, s_cw;
   __shared__ SlotFin<kStepThreads> fin;
-  __shared__ PartialLds<kStepThreads / kWave, 3> lds;
+  __shared__ PartialLds<COMP, kStepThreads / kWave> lds;
   const int tid = threadIdx.x;
   const bool lead = blockIdx.x == 0;
   if (C.user && C.user->skip) {  // uniform
@@ -1112,11 +1109,13 @@ IcpArgs level_args(const kf_tracker* t, int l, const kf_frame_maps& live, const 
   return a;
 }
 
-// Pixels of a tracking step's 512-thread block by the level's size, so that one block per
-// CU (256) covers the level and no SIMD has more pixels than it must: half a block's waves
+// Pixels of a tracking step's 512-thread block by the level's size, so that a block per CU
+// (256) covers the level and no SIMD has more pixels than it must: half a block's waves
 // take one pixel per thread up to 65,536 pixels (level 2 of 640x480: 75 blocks, one wave
 // per SIMD), all of them up to 131,072 (level 1: 150), two and a half pixels per thread up
-// to 327,680 (level 0: 240), three beyond (the fewest slots; a step's block sums them all).
+// to 327,680 (level 0: 240), three beyond (the fewest slots; a step's block sums them all;
+// from 393,217 pixels on some CUs hold two blocks: 800x600 10/5/4 iterations 177 us, plain
+// 168, with room for one 216 and 212).
 // A step inside the kernel: levels 2 and 1 of 640x480 4.0 us, level 0 6.3 us (7.75 with
 // 200 blocks of three pixels a thread and the per-thread sums, 5.6 below); 1024-thread
 // blocks 5.9 us at level 0 but 4.5 below.

@@ -1,0 +1,31 @@
+"""Registers, LDS and scratch of the built kernels (from their metadata, no GPU): what a
+kernel was designed to fit beside on a compute unit."""
+import pytest
+
+from tests import kernel_info as ki
+
+STEP_THREADS, REDUCE_THREADS = 512, 256
+
+
+@pytest.mark.parametrize("shape", ["Li0ELi1E", "Li1ELi0E", "Li2ELi1E", "Li3ELi0E"])
+@pytest.mark.parametrize("comp", [0, 1])
+def test_tracking_step_lds_does_not_limit_its_blocks(comp, shape):
+    k = ki.find(f"icp_stepILb{comp}E{shape}")
+    assert ki.blocks_by_lds(k) >= ki.blocks_by_registers(k, STEP_THREADS) >= 2
+    if not comp:
+        assert k[".group_segment_fixed_size"] <= 8192  # no rows for the matrix cores
+
+
+@pytest.mark.parametrize("comp", [0, 1])
+def test_reduce_lds_does_not_limit_its_blocks(comp):
+    k = ki.find(f"icp_partialsILb{comp}E")
+    assert ki.blocks_by_lds(k) >= ki.blocks_by_registers(k, REDUCE_THREADS)
+    if not comp:
+        assert k[".group_segment_fixed_size"] <= 4096
+
+
+@pytest.mark.parametrize("comp", [0, 1])
+def test_single_launch_tracking_has_no_scratch(comp):
+    k = ki.find(f"icp_chainILb{comp}E")
+    assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0
+    assert ki.blocks_by_lds(k) >= 3
