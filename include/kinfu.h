@@ -285,7 +285,12 @@ typedef struct kf_icp_params {
                                          (the device is shared with other work that keeps blocks from
                                          being co-resident), the call returns the guess with status 2,
                                          and so does every later single-launch call of the tracker
-                                         until kf_tracker_reset (kf_pipeline_reset calls it). */
+                                         until kf_tracker_reset (kf_pipeline_reset calls it).
+                                         Single-launch calls that overlap on one device (several
+                                         trackers, several streams) need all their blocks resident
+                                         together, one per compute unit: ceil(pixels / 1536) per call
+                                         up to 196,608 pixels at the finest level (320x240: 50), up to
+                                         256 beyond, where such calls must not overlap. */
 } kf_icp_params;
 
 /* Per-call tracking statistics (device struct; read back with kf_memcpy_dtoh). */

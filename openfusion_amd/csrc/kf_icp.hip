@@ -24,10 +24,12 @@
 // FP64 LDL^T and composes the Euler-ZYX increment onto the FP64 pose; every
 // block of an iteration repeats that solve for itself, so the pose never makes a
 // round trip through the host and an iteration is a single launch.
+#include <algorithm>
 #include <mutex>
 
 #include "kf_device.hpp"
 #include "kf_frame_end.hpp"
+#include "kf_icp_grid.hpp"
 #include "kf_internal.hpp"
 #include "kf_pose_math.hpp"
 
@@ -44,7 +46,6 @@ constexpr int kThreads = 256;
 constexpr double kPivotRelEps = 1e-9;
 constexpr int kMinInliers = 6;
 constexpr int kFinUnroll = 8;       // slot loads in flight per thread of the slot sum (8 x 32 groups: 256 slots in one round)
-constexpr int kStepThreads = 512;    // tracking step: 8 waves per block
 // One-block sums and solves use the step's block size, so that every slot sum (in
 // a step, the final one-block launch or the single-launch kernel) adds in the same
 // order: 32 groups x 16 float4 columns of the slots.
@@ -200,12 +201,12 @@ __device__ __forceinline__ void wave_lds_sync() {
 // LDS of block_partial.  Compensated mode: the row entries of one round of a wave, one
 // pixel per column; the rounds take turns in it (34 KB for eight waves, so that a CU holds
 // as many blocks as the registers allow; three rounds' rows side by side, 104 KB, left room
-// for one).  Plain mode has no rows.
-template <bool COMP, int WAVES>
+// for one).  Plain mode has no rows.  SETS: sets of wave sums kept at a time.
+template <bool COMP, int WAVES, int SETS = 1>
 struct PartialLds {
   double rows[COMP ? WAVES : 1][COMP ? 8 : 1][COMP ? kRowPitch : 1];
-  double red[WAVES][kWave];
-  int cand[WAVES];
+  double red[SETS][WAVES][kWave];
+  int cand[SETS][WAVES];
 };
 
 // FP64 sums of products over pixels on v_mfma_f64_4x4x4 (four 4 x 4 products of depth 4
@@ -271,12 +272,27 @@ __device__ __forceinline__ int term_of(int at) {
 template <int WAVES, int F, int H>
 struct PixelShape {
   static constexpr int T = WAVES * kWave, K = F + H, kPixels = F * T + H * (T / 2);
+  __device__ __forceinline__ int pixels() const { return kPixels; }
   // this thread's pixel of round k in pass `pass`; its wave takes part in `rounds` of them
-  static __device__ __forceinline__ int pixel(int bid, int nblk, int pass, int k) {
+  __device__ __forceinline__ int pixel(int bid, int nblk, int pass, int k) const {
     const int base = pass * nblk * kPixels + k * nblk * T, tid = threadIdx.x;
     return base + (k < F ? bid * T + tid : bid * (T / 2) + tid);
   }
-  static __device__ __forceinline__ int rounds() { return H && (int)threadIdx.x >= T / 2 ? F : K; }  // uniform per wave
+  __device__ __forceinline__ int rounds() const { return H && (int)threadIdx.x >= T / 2 ? F : K; }  // uniform per wave
+};
+
+// PixelShape<WAVES, 2, 1> (half) or <WAVES, 3, 0>, chosen at run time: one copy of the code
+// in the single-launch kernel, which has little room for registers.
+template <int WAVES>
+struct WideShape {
+  static constexpr int T = WAVES * kWave, K = 3;
+  bool half;
+  __device__ __forceinline__ int pixels() const { return half ? 2 * T + T / 2 : 3 * T; }
+  __device__ __forceinline__ int pixel(int bid, int nblk, int pass, int k) const {
+    const int base = pass * nblk * pixels() + k * nblk * T, tid = threadIdx.x;
+    return base + (k == 2 && half ? bid * (T / 2) + tid : bid * T + tid);
+  }
+  __device__ __forceinline__ int rounds() const { return half && (int)threadIdx.x >= T / 2 ? 2 : 3; }
 };
 
 // The model samples of a thread's first K pixels in block_partial; they do not
@@ -287,43 +303,130 @@ struct PxPre {
 };
 
 template <typename Shape>
-__device__ __forceinline__ PxPre<Shape::K> load_models(const IcpArgs& a, int bid, int nblk, int pass) {
-  const int P = a.W * a.H, rounds = Shape::rounds();
+__device__ __forceinline__ PxPre<Shape::K> load_models(const IcpArgs& a, const Shape& sh, int bid, int nblk, int pass) {
+  const int P = a.W * a.H, rounds = sh.rounds();
   PxPre<Shape::K> pre;
 #pragma unroll
   for (int k = 0; k < Shape::K; ++k) {
-    const int i = Shape::pixel(bid, nblk, pass, k);
+    const int i = sh.pixel(bid, nblk, pass, k);
     if (k < rounds) pre.q[k] = load_model(a, i < P ? i : 0);  // pixel 0: unused
   }
   return pre;
 }
 
+// The sums of one wave over the pixels of its rounds.
+template <bool COMP>
+struct WaveSums {
+  TermSums terms;
+  float s[COMP ? 1 : kPad];  // plain mode; terms 28..31 stay zero (padding for the halving)
+  int n_in = 0, n_cand = 0;  // of the wave (n_in: plain mode)
+
+  __device__ __forceinline__ WaveSums() {
+    if constexpr (!COMP) {
+#pragma unroll
+      for (int k = 0; k < kPad; ++k) s[k] = 0.0f;
+    }
+  }
+
+  // The row of a pixel with outcome r (finish_row).  Rejected pixels are zero rows: they
+  // leave the sums' bits as they are.  rows: the wave's buffer (compensated mode).
+  template <typename Rows>
+  __device__ __forceinline__ void add(float* A, float b, int r, Rows& rows) {
+    n_cand += (int)__popcll(__ballot(r != 0));
+    const bool inl = r == 2;
+#pragma unroll
+    for (int p = 0; p < 6; ++p) A[p] = inl ? A[p] : 0.0f;
+    b = inl ? b : 0.0f;
+    if constexpr (COMP) {
+      const int lane = threadIdx.x & 63;
+      wave_lds_sync();  // the previous round's reads are done
+#pragma unroll
+      for (int p = 0; p < 6; ++p) rows[p][lane] = (double)A[p];
+      rows[6][lane] = (double)b;
+      rows[7][lane] = inl ? 1.0 : 0.0;
+      wave_lds_sync();
+      terms.add(rows);
+    } else {
+      accumulate(s, A, b);
+      n_in += (int)__popcll(__ballot(inl));
+    }
+  }
+
+  // The wave's totals to red[kWave] and *cand.
+  __device__ __forceinline__ void store(double* red, int* cand) {
+    const int lane = threadIdx.x & 63;
+    if constexpr (COMP) {
+      terms.store(red);
+    } else {
+      // Wave reduction by recursive halving (reduce-scatter): five pairings, each
+      // halving the terms a lane holds — row mirror (lane bit 3), half-row mirror
+      // (bit 2), quad xor 2 (bit 1), quad xor 1 (bit 0), xor 16 (bit 4) — then xor 32
+      // adds the two half-waves.  Lane l < 32 ends with the full wave sum of term
+      // 16*b3 + 8*b2 + 4*b1 + 2*b0 + b4 (b = bits of l).
+      halve<0x140, 32>(s, (lane & 8) != 0);
+      halve<0x141, 16>(s, (lane & 4) != 0);
+      halve<0x4E, 8>(s, (lane & 2) != 0);
+      halve<0xB1, 4>(s, (lane & 1) != 0);
+      const bool up = (lane & 16) != 0;
+      const float gs = up ? s[0] : s[1];
+      float ks = up ? s[1] : s[0];
+      ks = ks + __shfl_xor(gs, 16, kWave);
+      ks = ks + __shfl_xor(ks, 32, kWave);
+      const int term = ((lane & 8) << 1) | ((lane & 4) << 1) | ((lane & 2) << 1) | ((lane & 1) << 1) | ((lane >> 4) & 1);
+      if (lane < 32 && term < kTerms) red[term] = (double)ks;
+      if (lane == 32) red[kInlAt] = (double)n_in;
+    }
+    if (lane == 0) *cand = n_cand;
+  }
+};
+
+// A slot's terms and inlier count: the sums of its waves' totals, in order (one wave).
+template <bool COMP, bool COH>
+__device__ __forceinline__ void slot_terms(const double (*red)[kWave], int waves, double* slot) {
+  const int lane = threadIdx.x & 63;
+  const int at = COMP ? term_of(lane) : (lane <= kInlAt ? lane : -1);
+  if (at < 0) return;
+  if constexpr (COMP) {
+    double S = red[0][lane];
+#pragma unroll
+    for (int w = 1; w < waves; ++w) S = S + red[w][lane];
+    slot_put<COH>(&slot[at], S);
+  } else {  // FP32 sums
+    float S = (float)red[0][lane];
+    for (int w = 1; w < waves; ++w) S = S + (float)red[w][lane];
+    slot_put<COH>(&slot[at], (double)S);
+  }
+}
+
+// Its candidate count and stop marker (one thread).
+template <bool COH>
+__device__ __forceinline__ void slot_counts(const int* cand, int waves, double* slot) {
+  int nc = 0;
+  for (int w = 0; w < waves; ++w) nc += cand[w];
+  slot_put<COH>(&slot[kCandAt], (double)nc);
+  slot_put<COH>(&slot[kStopAt], 0.0);
+}
+
 // Block partial: this block's share of the association (K pixels per thread with their
 // loads in flight together), the sums over the block's waves, written as one slot: 28
 // terms and the inlier and candidate counts.  PRE: the first pass' samples are given.
-template <bool COMP, typename Shape, int WAVES, bool PRE = false, bool COH = false>
-__device__ __forceinline__ void block_partial(const IcpArgs& a, const kf_posef& wc, const kf_posef& cw, int bid,
-                                              int nblk, double* slot, PartialLds<COMP, WAVES>& lds,
+template <bool COMP, bool PRE = false, bool COH = false, typename Shape, int WAVES, int SETS>
+__device__ __forceinline__ void block_partial(const IcpArgs& a, const Shape& sh, const kf_posef& wc, const kf_posef& cw,
+                                              int bid, int nblk, double* slot, PartialLds<COMP, WAVES, SETS>& lds,
                                               PxPre<Shape::K> pre = {}) {
   constexpr int K = Shape::K;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int P = a.W * a.H, passes = (P + nblk * Shape::kPixels - 1) / (nblk * Shape::kPixels);
-  const int rounds = Shape::rounds();
-  int n_cand = 0, n_in = 0;
-  TermSums sums;
-  float s[kPad];  // plain mode; terms 28..31 stay zero (padding for the halving)
-  if constexpr (!COMP) {
-#pragma unroll
-    for (int k = 0; k < kPad; ++k) s[k] = 0.0f;
-  }
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const int P = a.W * a.H, passes = (P + nblk * sh.pixels() - 1) / (nblk * sh.pixels());
+  const int rounds = sh.rounds();
+  WaveSums<COMP> sums;
   for (int pass = 0; pass < passes; ++pass) {
-    if (!PRE || pass > 0) pre = load_models<Shape>(a, bid, nblk, pass);
+    if (!PRE || pass > 0) pre = load_models(a, sh, bid, nblk, pass);
     int j[K], r[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       if (k >= rounds) continue;  // uniform
       j[k] = project_model(a, cw, pre.q[k], r[k]);
-      if (Shape::pixel(bid, nblk, pass, k) >= P) {  // no pixel: contributes nothing
+      if (sh.pixel(bid, nblk, pass, k) >= P) {  // no pixel: contributes nothing
         j[k] = -1;
         r[k] = 0;
       }
@@ -337,71 +440,86 @@ __device__ __forceinline__ void block_partial(const IcpArgs& a, const kf_posef& 
       if (k >= rounds) continue;
       float A[6], b;
       r[k] = finish_row(a, wc, pre.q[k], l[k], j[k], r[k], A, b);
-      const int i = Shape::pixel(bid, nblk, pass, k);
+      const int i = sh.pixel(bid, nblk, pass, k);
       if (a.mask && i < P) a.mask[i] = (uint8_t)(r[k] == 2);
-      n_cand += (int)__popcll(__ballot(r[k] != 0));  // of the wave
-      // rejected pixels are zero rows: they leave the sums' bits as they are
-      const bool inl = r[k] == 2;
-#pragma unroll
-      for (int p = 0; p < 6; ++p) A[p] = inl ? A[p] : 0.0f;
-      b = inl ? b : 0.0f;
-      if constexpr (COMP) {
-        double (*rows)[kRowPitch] = lds.rows[wave];
-        wave_lds_sync();  // the previous round's reads are done
-#pragma unroll
-        for (int p = 0; p < 6; ++p) rows[p][lane] = (double)A[p];
-        rows[6][lane] = (double)b;
-        rows[7][lane] = inl ? 1.0 : 0.0;
-        wave_lds_sync();
-        sums.add(rows);
-      } else {
-        accumulate(s, A, b);
-        n_in += (int)__popcll(__ballot(inl));
-      }
+      sums.add(A, b, r[k], lds.rows[COMP ? wave : 0]);
     }
   }
-  if constexpr (COMP) {
-    sums.store(lds.red[wave]);
-  } else {
-    // Wave reduction by recursive halving (reduce-scatter): five pairings, each
-    // halving the terms a lane holds — row mirror (lane bit 3), half-row mirror
-    // (bit 2), quad xor 2 (bit 1), quad xor 1 (bit 0), xor 16 (bit 4) — then xor 32
-    // adds the two half-waves.  Lane l < 32 ends with the full wave sum of term
-    // 16*b3 + 8*b2 + 4*b1 + 2*b0 + b4 (b = bits of l).
-    halve<0x140, 32>(s, (lane & 8) != 0);
-    halve<0x141, 16>(s, (lane & 4) != 0);
-    halve<0x4E, 8>(s, (lane & 2) != 0);
-    halve<0xB1, 4>(s, (lane & 1) != 0);
-    const bool up = (lane & 16) != 0;
-    const float gs = up ? s[0] : s[1];
-    float ks = up ? s[1] : s[0];
-    ks = ks + __shfl_xor(gs, 16, kWave);
-    ks = ks + __shfl_xor(ks, 32, kWave);
-    const int term = ((lane & 8) << 1) | ((lane & 4) << 1) | ((lane & 2) << 1) | ((lane & 1) << 1) | ((lane >> 4) & 1);
-    if (lane < 32 && term < kTerms) lds.red[wave][term] = (double)ks;
-    if (lane == 32) lds.red[wave][kInlAt] = (double)n_in;
-  }
-  if (lane == 0) lds.cand[wave] = n_cand;
+  sums.store(lds.red[0][wave], &lds.cand[0][wave]);
   __syncthreads();
-  if (tid < kWave) {
-    const int at = COMP ? term_of(lane) : (lane <= kInlAt ? lane : -1);
-    if (at >= 0) {
-      if constexpr (COMP) {
-        double S = lds.red[0][lane];
+  if (tid < kWave)
+    slot_terms<COMP, COH>(lds.red[0], WAVES, slot);
+  else if (tid == kWave)
+    slot_counts<COH>(lds.cand[0], WAVES, slot);
+}
+
+// The partials of several slots by one block, for the shapes of one pixel per thread: a
+// round makes one slot or, where a slot has half a block's waves (half), two of them side
+// by side; kSlotRounds rounds with their loads in flight together.  Slot i of the block's
+// is number first + i * step; those below nb are made, as their own blocks would make them.
+constexpr int kSlotRounds = 3;
+struct SlotRounds {
+  bool half;
+  int first, step, nb;
+  __device__ __forceinline__ int waves() const { return kStepThreads / kWave >> (int)half; }
+  __device__ __forceinline__ int slots() const { return half ? 2 * kSlotRounds : kSlotRounds; }
+  __device__ __forceinline__ int number(int i) const { return first + step * i; }
+  // this wave's slot in round k, and the thread's pixel of a slot
+  __device__ __forceinline__ int slot(int k) const {
+    return number(half ? 2 * k + (int)(threadIdx.x / (kStepThreads / 2)) : k);
+  }
+  __device__ __forceinline__ int pixel(int v) const {
+    return half ? v * (kStepThreads / 2) + (int)threadIdx.x % (kStepThreads / 2) : v * kStepThreads + (int)threadIdx.x;
+  }
+};
+
+__device__ __forceinline__ PxPre<kSlotRounds> load_slot_models(const IcpArgs& a, const SlotRounds& sr) {
+  const int P = a.W * a.H;
+  PxPre<kSlotRounds> pre;
 #pragma unroll
-        for (int w = 1; w < WAVES; ++w) S = S + lds.red[w][lane];
-        slot_put<COH>(&slot[at], S);
-      } else {  // FP32 sums
-        float S = (float)lds.red[0][lane];
-        for (int w = 1; w < WAVES; ++w) S = S + (float)lds.red[w][lane];
-        slot_put<COH>(&slot[at], (double)S);
-      }
+  for (int k = 0; k < kSlotRounds; ++k) {
+    const int v = sr.slot(k), i = sr.pixel(v);
+    if (v < sr.nb) pre.q[k] = load_model(a, i < P ? i : 0);  // uniform per wave; pixel 0: unused
+  }
+  return pre;
+}
+
+template <bool COMP, int WAVES>
+__device__ __forceinline__ void slot_partials(const IcpArgs& a, const SlotRounds& sr, const kf_posef& wc, const kf_posef& cw,
+                                              double* slots, PartialLds<COMP, WAVES, kSlotRounds>& lds,
+                                              const PxPre<kSlotRounds>& pre) {
+  static_assert(WAVES * kWave == kStepThreads && 2 * kSlotRounds <= WAVES, "a wave per slot at the end");
+  const int wave = threadIdx.x >> 6, P = a.W * a.H;
+  int j[kSlotRounds], r[kSlotRounds];
+#pragma unroll
+  for (int k = 0; k < kSlotRounds; ++k) {
+    const int v = sr.slot(k);
+    if (v >= sr.nb) continue;  // uniform per wave
+    j[k] = project_model(a, cw, pre.q[k], r[k]);
+    if (sr.pixel(v) >= P) {
+      j[k] = -1;
+      r[k] = 0;
     }
-  } else if (tid == kWave) {
-    int nc = 0;
-    for (int w = 0; w < WAVES; ++w) nc += lds.cand[w];
-    slot_put<COH>(&slot[kCandAt], (double)nc);
-    slot_put<COH>(&slot[kStopAt], 0.0);
+  }
+  PxLive l[kSlotRounds];
+#pragma unroll
+  for (int k = 0; k < kSlotRounds; ++k)
+    if (sr.slot(k) < sr.nb) l[k] = load_live(a, j[k]);
+#pragma unroll
+  for (int k = 0; k < kSlotRounds; ++k) {
+    if (sr.slot(k) >= sr.nb) continue;
+    float A[6], b;
+    r[k] = finish_row(a, wc, pre.q[k], l[k], j[k], r[k], A, b);
+    WaveSums<COMP> sums;
+    sums.add(A, b, r[k], lds.rows[COMP ? wave : 0]);
+    sums.store(lds.red[k][wave], &lds.cand[k][wave]);
+  }
+  __syncthreads();
+  if (wave < sr.slots() && sr.number(wave) < sr.nb) {
+    const int k = sr.half ? wave / 2 : wave, w0 = sr.half ? wave % 2 * (WAVES / 2) : 0;
+    double* slot = slots + (size_t)sr.number(wave) * kSlot;
+    slot_terms<COMP, true>(lds.red[k] + w0, sr.waves(), slot);
+    if ((threadIdx.x & 63) == 0) slot_counts<true>(lds.cand[k] + w0, sr.waves(), slot);
   }
 }
 
@@ -591,10 +709,10 @@ __device__ __forceinline__ void copy_pose(const kf_pose* src, kf_pose* dst) {
 // Reduce mode (kf_icp_reduce), pass 1: the block partials at a fixed pose.
 template <bool COMP>
 __global__ __launch_bounds__(kThreads) void icp_partials(IcpArgs a) {
-  using Shape = PixelShape<kThreads / kWave, 2, 0>;
+  const PixelShape<kThreads / kWave, 2, 0> shape;
   __shared__ PartialLds<COMP, kThreads / kWave> lds;
   const kf_posef wc = a.pose->wc, cw = a.pose->cw;
-  block_partial<COMP, Shape>(a, wc, cw, blockIdx.x, gridDim.x, a.partials + (size_t)blockIdx.x * kSlot, lds);
+  block_partial<COMP>(a, shape, wc, cw, blockIdx.x, gridDim.x, a.partials + (size_t)blockIdx.x * kSlot, lds);
 }
 
 // Reduce mode, pass 2 (one block): the FP64 sums.
@@ -639,7 +757,7 @@ __global__ __launch_bounds__(kStepThreads) void icp_step(IcpArgs a, StepArgs S) 
   __shared__ double Tin[16], Tnew[16];
   __shared__ kf_posef s_wc, s_cw;
   __shared__ SlotFin<kStepThreads> fin;
-  using Shape = StepShape<F, H>;
+  const StepShape<F, H> shape;
   __shared__ PartialLds<COMP, kStepThreads / kWave> lds;
   const int tid = threadIdx.x;
   double* slot_out = S.slots_out + (size_t)blockIdx.x * kSlot;
@@ -653,7 +771,7 @@ __global__ __launch_bounds__(kStepThreads) void icp_step(IcpArgs a, StepArgs S) 
     slots_in.load(S.slots_in, S.nb_in);
     tin = S.pose_in->T_wc[tid & 15];
   }
-  const PxPre<Shape::K> pre = load_models<Shape>(a, blockIdx.x, gridDim.x, 0);
+  const PxPre<F + H> pre = load_models(a, shape, blockIdx.x, gridDim.x, 0);
   if (S.first) {
     if (tid < 12) {
       if (tid < 9) s_wc.r[tid] = S.pose_in->wc.r[tid];
@@ -696,7 +814,7 @@ __global__ __launch_bounds__(kStepThreads) void icp_step(IcpArgs a, StepArgs S) 
     }
   }
   __syncthreads();
-  block_partial<COMP, Shape, kStepThreads / kWave, true>(a, s_wc, s_cw, blockIdx.x, gridDim.x, slot_out, lds, pre);
+  block_partial<COMP, true>(a, shape, s_wc, s_cw, blockIdx.x, gridDim.x, slot_out, lds, pre);
 }
 
 // Acceptance test of the finished call (IcpGate), from the window count and thread
@@ -817,15 +935,15 @@ __global__ __launch_bounds__(kSolveThreads) void icp_finish(IcpArgs a, StepArgs 
 // ---------------------------------------------------------------------------
 // Single-launch tracking: the iterations of the icp_step chain and icp_finish in
 // one launch.  Block b computes the slots b, b + G, ... of each iteration's step
-// grid (same grid size, same pixels per thread and block_partial arguments, hence
-// the same slots), every block sums the previous iteration's slots and solves as
+// grid (the same pixels and sums per slot, hence the same slots), every block sums the previous iteration's slots and solves as
 // icp_step does, and a grid barrier replaces the kernel boundary between
 // iterations, so poses and statistics are those of the multi-launch chain bit for
 // bit.  Every block keeps the pose in LDS; only the lead block writes it, then runs
 // the acceptance test (when gated) and the frame-end bookkeeping, as icp_finish.
 //
 // The barrier needs all G blocks resident at once: the launcher caps G at the
-// device's co-resident block count for this kernel.  Its wait is bounded: a block
+// device's co-resident block count for this kernel, and keeps it well below where
+// several calls of one size fit together (chain_blocks).  Its wait is bounded: a block
 // that waits longer than the control block's poll limit (kBarrierPolls unless set
 // with kf_tracker_set_barrier_polls) gives up, the control block is marked
 // broken and that call and every later single-launch call of the tracker report
@@ -905,23 +1023,31 @@ __device__ __forceinline__ bool grid_barrier(kf_icp_ctrl* ctrl, unsigned target,
   return s_ok != 0;
 }
 
-// One iteration of the chain at a level whose step grid has nb blocks of Shape's pixels
+// One iteration of the chain at a level whose step grid has nb blocks of the given shape
 // (as icp_step): the slot loads of the previous iteration
 // (solve = true; nb_in slots of level lvl_in), then this block's model samples, both
-// in flight together; the sum, solve and composition onto T[cur]; this block's
-// slots.  Returns false (uniform) when the solve was singular: nothing is written.
-template <bool COMP, typename Shape>
-__device__ __forceinline__ bool chain_iteration(const IcpArgs& a, int nb, bool solve, const double* slots_in,
+// in flight together; the sum, solve and composition onto T[cur]; this block's slots,
+// several at once in the shapes of one pixel per thread (WIDE = false).  half: the shape
+// ends in half a block's pixels.  Returns false (uniform) when the solve was singular:
+// nothing is written.
+template <bool COMP, bool WIDE, typename Lds>
+__device__ __forceinline__ bool chain_iteration(const IcpArgs& a, bool half, int nb, bool solve, const double* slots_in,
                                                 int nb_in, int lvl_in, double* slots_out,
-                                                SlotFin<kStepThreads>& fin, PartialLds<COMP, kStepThreads / kWave>& lds,
+                                                SlotFin<kStepThreads>& fin, Lds& lds,
                                                 double (*T)[16], int& cur, kf_posef* wc, kf_posef* cw,
                                                 kf_icp_stats* st) {
-  constexpr int WV = kStepThreads / kWave;
+  const WideShape<kStepThreads / kWave> shape{half};
+  SlotRounds sr{half, (int)blockIdx.x, (int)gridDim.x, nb};
   SlotSum<kStepThreads, true> L;
   if (solve) L.load(slots_in, nb_in);
-  const bool mine = (int)blockIdx.x < nb;
-  PxPre<Shape::K> pre = {};
-  if (mine) pre = load_models<Shape>(a, blockIdx.x, nb, 0);
+  PxPre<3> pre = {};
+  auto load = [&]() {
+    if constexpr (WIDE)
+      pre = load_models(a, shape, sr.first, nb, 0);
+    else
+      pre = load_slot_models(a, sr);
+  };
+  if (sr.first < nb) load();
   if (solve) {
     L.reduce(slots_in, nb_in, fin);
     __syncthreads();
@@ -929,10 +1055,16 @@ __device__ __forceinline__ bool chain_iteration(const IcpArgs& a, int nb, bool s
     cur ^= 1;
   }
   __syncthreads();
-  if (mine) block_partial<COMP, Shape, WV, true, true>(a, *wc, *cw, blockIdx.x, nb, slots_out + (size_t)blockIdx.x * kSlot, lds, pre);
-  for (int vb = blockIdx.x + gridDim.x; vb < nb; vb += gridDim.x) {
-    __syncthreads();
-    block_partial<COMP, Shape, WV, false, true>(a, *wc, *cw, vb, nb, slots_out + (size_t)vb * kSlot, lds);
+  while (sr.first < nb) {  // uniform
+    if constexpr (WIDE)
+      block_partial<COMP, true, true>(a, shape, *wc, *cw, sr.first, nb, slots_out + (size_t)sr.first * kSlot, lds, pre);
+    else
+      slot_partials<COMP>(a, sr, *wc, *cw, slots_out, lds, pre);
+    sr.first += sr.step * (WIDE ? 1 : sr.slots());
+    if (sr.first < nb) {
+      load();
+      __syncthreads();
+    }
   }
   return true;
 }
@@ -942,7 +1074,7 @@ __global__ __launch_bounds__(kStepThreads) void icp_chain(ChainArgs C) {
   __shared__ double T[2][16];
   __shared__ kf_posef s_wc, s_cw;
   __shared__ SlotFin<kStepThreads> fin;
-  __shared__ PartialLds<COMP, kStepThreads / kWave> lds;
+  __shared__ PartialLds<COMP, kStepThreads / kWave, kSlotRounds> lds;
   const int tid = threadIdx.x;
   const bool lead = blockIdx.x == 0;
   if (C.user && C.user->skip) {  // uniform
@@ -1003,17 +1135,12 @@ __global__ __launch_bounds__(kStepThreads) void icp_chain(ChainArgs C) {
     for (int it = 0; it < C.iters[l]; ++it) {
       const bool solve = steps > 0;
       kf_icp_stats* sp = lead ? st : nullptr;
-      auto iterate = [&](auto shape) {
-        return chain_iteration<COMP, decltype(shape)>(a, nb, solve, C.slots[par ^ 1], nb_prev, lvl_prev, C.slots[par], fin,
-                                                      lds, T, cur, &s_wc, &s_cw, sp);
-      };
-      bool ok;
-      switch (C.shape[l]) {  // uniform
-        case 0: ok = iterate(StepShape<0, 1>{}); break;
-        case 1: ok = iterate(StepShape<1, 0>{}); break;
-        case 2: ok = iterate(StepShape<2, 1>{}); break;
-        default: ok = iterate(StepShape<3, 0>{}); break;
-      }
+      const int shape = C.shape[l];  // uniform
+      const bool half = shape == 0 || shape == 2;
+      const bool ok = shape < 2 ? chain_iteration<COMP, false>(a, half, nb, solve, C.slots[par ^ 1], nb_prev, lvl_prev,
+                                                               C.slots[par], fin, lds, T, cur, &s_wc, &s_cw, sp)
+                                : chain_iteration<COMP, true>(a, half, nb, solve, C.slots[par ^ 1], nb_prev, lvl_prev,
+                                                              C.slots[par], fin, lds, T, cur, &s_wc, &s_cw, sp);
       if (!ok) {
         stop = true;  // uniform: every block solved the same system
         break;
@@ -1109,29 +1236,9 @@ IcpArgs level_args(const kf_tracker* t, int l, const kf_frame_maps& live, const 
   return a;
 }
 
-// Pixels of a tracking step's 512-thread block by the level's size, so that a block per CU
-// (256) covers the level and no SIMD has more pixels than it must: half a block's waves
-// take one pixel per thread up to 65,536 pixels (level 2 of 640x480: 75 blocks, one wave
-// per SIMD), all of them up to 131,072 (level 1: 150), two and a half pixels per thread up
-// to 327,680 (level 0: 240), three beyond (the fewest slots; a step's block sums them all;
-// from 393,217 pixels on some CUs hold two blocks: 800x600 10/5/4 iterations 177 us, plain
-// 168, with room for one 216 and 212).
-// A step inside the kernel: levels 2 and 1 of 640x480 4.0 us, level 0 6.3 us (7.75 with
-// 200 blocks of three pixels a thread and the per-thread sums, 5.6 below); 1024-thread
-// blocks 5.9 us at level 0 but 4.5 below.
-constexpr int kShapes = 4;
-constexpr int kShapePixels[kShapes] = {StepShape<0, 1>::kPixels, StepShape<1, 0>::kPixels, StepShape<2, 1>::kPixels,
-                                       StepShape<3, 0>::kPixels};
-int step_shape(int W, int H) {
-  int k = 0;
-  while (k + 1 < kShapes && W * H > 256 * kShapePixels[k]) ++k;
-  return k;
-}
-
-int step_blocks(const kf_tracker* t, int W, int H) {
-  const int b = div_up(W * H, kShapePixels[step_shape(W, H)]);
-  return b < t->max_blocks ? b : t->max_blocks;
-}
+static_assert(StepShape<0, 1>::kPixels == kShapePixels[0] && StepShape<1, 0>::kPixels == kShapePixels[1] &&
+                  StepShape<2, 1>::kPixels == kShapePixels[2] && StepShape<3, 0>::kPixels == kShapePixels[3],
+              "step shapes");
 
 template <bool COMP>
 void launch_step(int shape, int blocks, hipStream_t s, const IcpArgs& a, const StepArgs& S) {
@@ -1178,9 +1285,10 @@ kf_status launch_icp_track(kf_tracker* t, const kf_frame_maps& live, const kf_fr
     for (int l = 0; l < p.levels; ++l) {
       C.lv[l] = level_args(t, l, live, model);
       C.iters[l] = p.iterations[l];
-      C.blocks[l] = step_blocks(t, C.lv[l].W, C.lv[l].H);
-      C.shape[l] = step_shape(C.lv[l].W, C.lv[l].H);
-      if (C.iters[l] > 0 && C.blocks[l] > grid) grid = C.blocks[l];
+      const int pixels = C.lv[l].W * C.lv[l].H;
+      C.blocks[l] = step_blocks(pixels, t->max_blocks);
+      C.shape[l] = step_shape(pixels);
+      if (C.iters[l] > 0) grid = std::max(grid, chain_blocks(pixels, l, t->max_blocks));
     }
     if (t->chain_capacity < 0) {  // blocks of this kernel that can be resident at once
       int dev = 0, per_cu = 0, cus = 0;
@@ -1219,7 +1327,7 @@ kf_status launch_icp_track(kf_tracker* t, const kf_frame_maps& live, const kf_fr
   IcpArgs a = {};
   for (int l = p.levels - 1; l >= 0; --l) {
     a = level_args(t, l, live, model);
-    const int blocks = step_blocks(t, a.W, a.H), shape = step_shape(a.W, a.H);
+    const int blocks = step_blocks(a.W * a.H, t->max_blocks), shape = step_shape(a.W * a.H);
     for (int it = 0; it < p.iterations[l]; ++it, ++step) {
       S.first = step == 0 ? 1 : 0;
       S.index = step;
@@ -1336,7 +1444,8 @@ kf_status launch_icp_track_noalloc(const kf_intrinsics& k0, const kf_icp_params&
   for (int l = 0; l < p.levels; ++l) {
     if (p.iterations[l] == 0) continue;
     const kf_intrinsics kl = kf_intrinsics_level(&k0, l);
-    KF_CHECK_ARG(div_up(kl.width * kl.height, kShapePixels[step_shape(kl.width, kl.height)]) <= kNoAllocSlots,
+    const int pixels = kl.width * kl.height;
+    KF_CHECK_ARG(div_up(pixels, kShapePixels[step_shape(pixels)]) <= kNoAllocSlots,
                  "image too large for kf_icp_track_noalloc (level-0 images up to 786432 pixels)");
   }
   NoAllocScratch* sc = nullptr;
