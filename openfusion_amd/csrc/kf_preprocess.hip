@@ -91,16 +91,22 @@ __device__ __forceinline__ unsigned abs_diff(unsigned a, unsigned b) {
 // A block filters kTileX x kTileY pixels, a pair of neighbours per thread (the 2R + 2
 // codes of a window row are read once for both), and makes the coarser levels' pixels
 // under them (tiles start at multiples of 4, so they need no other block's).  R: the
-// window half-size (a.radius), fixed per instance so that the window loop unrolls.
+// window half-size (a.radius), fixed per instance so that a window row's loop unrolls.
 // Pixels outside the image are invalid in the tile, so the window needs no bounds test
 // of its own; an invalid tap has weight 0, which adds exactly nothing (sums are >= 0).
 //
-// Bound by latency: a wavefront lives 7 us, half of it waiting (the frame's first touch,
-// the LDS reads, the barriers before the coarser levels), with vector pipes busy for 3.8
-// and LDS for 2.4 us of a 640x480 frame.  In one launch and with a window row's codes and
-// metres read once for two pixels 9.6 us, where a pixel per thread and a second launch for
-// the coarser levels took 10.9 + 3.7.  A table of weight products per window distance
-// (no products per tap) took as long.
+// Bound by latency: waiting (the frame's first touch, the LDS reads, the barriers before the
+// coarser levels) is half of a wavefront's life.  In one launch and with a window row's codes
+// and metres read once for two pixels; the rows are a loop of their own, since the compiler
+// otherwise loads all of them first (radius 3: 167 VGPRs, three waves per SIMD instead of
+// eight; radius 4 256).  The whole of kf_preprocess, three levels, against a pixel per thread
+// and a second launch for the coarser levels, and in parentheses the rows unrolled:
+//   640x480   radius 1 10.7 / 14.0 us (10.8), 3 13.4 / 18.5 (13.9), 4 15.2 / 22.1 (20.0)
+//   1280x960  radius 3 29.2 / 40.8 (37.2), 4 33.8 / 51.3 (51.3)
+//   319x241   radius 3 10.6 / 16.1 (10.2), 4 12.1 / 18.9 (11.5)
+//   range weights that do not reach zero in the table, 640x480: radius 3 15.8 / 19.4 (15.7),
+//   4 19.7 / 23.8 (40); 1280x960: 34.5 / 42.6 (47), 43.4 / 57.0 (130)
+// A table of weight products per window distance (no products per tap) took as long.
 template <int R, bool ZT>
 __global__ __launch_bounds__(kThreads) void depth_levels(PreArgs a) {
   constexpr int kSpanX = kTileX + 2 * R, kSpanY = kTileY + 2 * R, kSpan = kSpanX * kSpanY;
@@ -148,7 +154,7 @@ __global__ __launch_bounds__(kThreads) void depth_levels(PreArgs a) {
   float sw[2] = {0.0f, 0.0f}, swd[2] = {0.0f, 0.0f};
 #pragma unroll
   for (int p = 0; p < 2; ++p) uc[p] = tile[(py + R) * kSpanX + px + p + R];
-#pragma unroll
+#pragma unroll 1
   for (int dy = -R; dy <= R; ++dy) {
     int u[2 * R + 2];
     float m[2 * R + 2];

@@ -29,3 +29,11 @@ def test_single_launch_tracking_has_no_scratch(comp):
     k = ki.find(f"icp_chainILb{comp}E")
     assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0
     assert ki.blocks_by_lds(k) >= 3
+
+
+@pytest.mark.parametrize("zero_tail", [0, 1])
+@pytest.mark.parametrize("radius", [0, 1, 2, 3, 4])
+def test_depth_filter_fills_the_simds(radius, zero_tail):
+    k = ki.find(f"depth_levelsILi{radius}ELb{zero_tail}E")
+    assert ki.waves_by_registers(k) == ki.MAX_WAVES
+    assert ki.blocks_by_lds(k) * 256 >= ki.MAX_WAVES * ki.SIMDS * 64
