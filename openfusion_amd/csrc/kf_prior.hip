@@ -339,10 +339,10 @@ kf_status forward(kf_prior* P, const float* frames, const int32_t* pairs, int B,
 
 // Inference, with the training forward's outputs either way.  The fused kernel's blocks
 // (80 a sample, one fits a CU) are all resident up to three samples on 256 CUs; from the
-// fourth on a second round and the recomputed window overlaps cost more than the layered
-// forward's five launches.  Fused / layered at batch 1: 11.9 / 20.8 us, 3: 14.2 / 21.2,
-// 4: 21.0 / 21.7, 6: 23.4 / 22.0, 8: 30.0 / 23.1, 256: 666 / 82.
-constexpr int kLayeredBatch = 4;
+// fourth on they take a second round, and from the sixth on that and the recomputed window
+// overlaps cost more than the layered forward's five launches.  Fused / layered at batch 1:
+// 10.7 / 19.5 us, 3: 12.8 / 19.9, 4: 18.4 / 20.1, 5: 19.2 / 20.4, 6: 21.1 / 20.7, 8: 26.0 / 20.9.
+constexpr int kLayeredBatch = 6;
 kf_status infer(kf_prior* P, const float* frames, const int32_t* pairs, const float* prev, int B, float* out,
                 hipStream_t s) {
   const ParamLayout& L = layout();
