@@ -334,8 +334,8 @@ kf_status kf_icp_track(kf_tracker* t, const kf_frame_maps* live, const kf_frame_
  * tracker's scratch (block slots, control block, step poses, statistics) is a
  * fixed device array of the library of about 257 KiB per GPU, held until the
  * process ends.  It has slots for KF_ICP_NOALLOC_MAX_SLOTS blocks, i.e. level-0
- * images of up to 786,432 pixels; larger images are rejected with
- * KF_ERR_INVALID_ARGUMENT.  Every call on one GPU shares that GPU's array: calls
+ * images of up to 786,432 pixels (262,144 at a coarser level, where level 0 has no
+ * iterations); larger images are rejected with KF_ERR_INVALID_ARGUMENT.  Every call on one GPU shares that GPU's array: calls
  * that overlap on one GPU (two streams, two host threads) race. */
 #define KF_ICP_NOALLOC_MAX_SLOTS 512
 kf_status kf_icp_track_noalloc(const kf_intrinsics* k0, const kf_icp_params* p, const kf_frame_maps* live,

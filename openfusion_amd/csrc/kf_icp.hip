@@ -1439,13 +1439,13 @@ __global__ void clear_ctrl(kf_icp_ctrl* c) {
 kf_status launch_icp_track_noalloc(const kf_intrinsics& k0, const kf_icp_params& p, const kf_frame_maps& live,
                                    const kf_frame_maps& model, const kf_pose* d_guess, kf_pose* d_out,
                                    kf_icp_stats* d_stats, hipStream_t s) {
-  // A step grid larger than the slots is rejected (a tracker would cap it at its own
-  // slot count, which would change the block partition and the sums' rounding).
+  // Images beyond 512 slots of three pixels a thread (one below the finest level) are
+  // rejected: a step grid of more blocks than slots would have to be capped, which changes
+  // the block partition and the sums' rounding.
   for (int l = 0; l < p.levels; ++l) {
     if (p.iterations[l] == 0) continue;
     const kf_intrinsics kl = kf_intrinsics_level(&k0, l);
-    const int pixels = kl.width * kl.height;
-    KF_CHECK_ARG(div_up(pixels, kShapePixels[step_shape(pixels)]) <= kNoAllocSlots,
+    KF_CHECK_ARG(kl.width * kl.height <= kNoAllocSlots * kStepThreads * (l == 0 ? 3 : 1),
                  "image too large for kf_icp_track_noalloc (level-0 images up to 786432 pixels)");
   }
   NoAllocScratch* sc = nullptr;
