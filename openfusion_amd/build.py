@@ -4,6 +4,7 @@
 * ``openfusion_amd/libkfsynth.so`` — host frame sources: synthetic streams and the
   recorded-stream format (g++, OpenMP)
 * ``oracle/libkforacle.so``        — the CPU oracle (g++, OpenMP), via oracle/Makefile
+* ``tests/libdevicemath.so``       — device helpers for the tests that check them (hipcc)
 
 Every call recompiles.  Usage: ``python -m openfusion_amd.build [--no-oracle]``.
 """
@@ -87,9 +88,18 @@ def build_oracle() -> str:
     return os.path.join(ROOT, "oracle", "libkforacle.so")
 
 
+def build_device_math() -> str:
+    src = os.path.join(ROOT, "tests", "csrc", "device_math.hip")
+    out = os.path.join(ROOT, "tests", "libdevicemath.so")
+    tmp = out + ".tmp"
+    _run([HIPCC, *HIP_FLAGS, "-shared", "-o", tmp, src])
+    os.replace(tmp, out)
+    return out
+
+
 def build_all(oracle: bool = True) -> None:
-    with ThreadPoolExecutor(max_workers=3) as ex:
-        futs = [ex.submit(build_kinfu), ex.submit(build_synth)]
+    with ThreadPoolExecutor(max_workers=4) as ex:
+        futs = [ex.submit(build_kinfu), ex.submit(build_synth), ex.submit(build_device_math)]
         if oracle:
             futs.append(ex.submit(build_oracle))
         for f in futs:

@@ -67,6 +67,16 @@ __host__ __device__ __forceinline__ float exp_neg(float x) {
 
 __device__ __forceinline__ float nanf_() { return __builtin_nanf(""); }
 
+// 1.0f / z for positive normal z: the hardware reciprocal and one Newton step give the IEEE
+// quotient below 2^126 (tests/test_gpu_device_math.py compares every mantissa); beyond,
+// where the quotient is subnormal, the division itself.
+__device__ __forceinline__ float reciprocal(float z) {
+  float r = __builtin_amdgcn_rcpf(z);
+  r = fmaf(r, fmaf(-z, r, 1.0f), r);
+  if (__builtin_expect(__any(z >= 0x1p126f), 0)) r = z >= 0x1p126f ? 1.0f / z : r;
+  return r;
+}
+
 // Packed FP16 voxel: low 16 bits = half(tsdf/T), high 16 bits = uint16 weight.
 __device__ __forceinline__ float half_bits_to_float(uint32_t h) {
   _Float16 v = __builtin_bit_cast(_Float16, (uint16_t)h);

@@ -106,16 +106,6 @@ __device__ __forceinline__ PxModel load_model(const IcpArgs& a, int i) {
                  f3{plane_at(a.mnx, o), plane_at(a.mny, o), plane_at(a.mnz, o)}, plane_at(a.lvz, o)};
 }
 
-// 1.0f / z for every z the gate below admits: the hardware reciprocal and one Newton step
-// equal the IEEE quotient for all normal z below 2^126 (checked over every such float);
-// beyond, the division itself.
-__device__ __forceinline__ float reciprocal(float z) {
-  float r = __builtin_amdgcn_rcpf(z);
-  r = fmaf(r, fmaf(-z, r, 1.0f), r);
-  if (__builtin_expect(__any(z >= 0x1p126f), 0)) r = z >= 0x1p126f ? 1.0f / z : r;
-  return r;
-}
-
 // Live pixel the model point projects to, or -1 (0 = not a candidate, 1 = rejected
 // in r when j < 0).  Every value is formed and the tests select the result (a
 // wavefront's lanes differ in which test they fail); lanes out of range convert 0.
