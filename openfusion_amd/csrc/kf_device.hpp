@@ -132,6 +132,13 @@ __device__ __forceinline__ unsigned wave_or_u32(unsigned v) {
   return (unsigned)__builtin_amdgcn_readlane(x, 63);
 }
 
+// Orders the LDS accesses of one wavefront around this point.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // x returned through an empty asm statement: the compiler cannot see its range, so
 // it neither widens the arithmetic that uses it to 64 bits nor fuses a 24-bit
 // multiply and add into a 64-bit multiply-add.

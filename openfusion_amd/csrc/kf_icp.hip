@@ -48,7 +48,7 @@ constexpr int kMinInliers = 6;
 constexpr int kFinUnroll = 8;       // slot loads in flight per thread of the slot sum (8 x 32 groups: 256 slots in one round)
 // One-block sums and solves use the step's block size, so that every slot sum (in
 // a step, the final one-block launch or the single-launch kernel) adds in the same
-// order: 32 groups x 16 float4 columns of the slots.
+// order: 32 groups x 16 columns of two doubles of the slots.
 constexpr int kSolveThreads = kStepThreads;
 
 struct IcpArgs {
@@ -179,13 +179,6 @@ __device__ __forceinline__ void halve(float* s, bool upper) {
     const float gs = upper ? s[k] : s[k + H / 2];
     s[k] = ks + dpp_f<CTRL>(gs);
   }
-}
-
-// Orders the LDS accesses of one wavefront around this point.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // LDS of block_partial.  Compensated mode: the row entries of one round of a wave, one

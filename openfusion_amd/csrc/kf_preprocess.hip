@@ -35,8 +35,7 @@ struct PreArgs {
   int W, H;
   float fx, fy, cx, cy;
   float scale, dmin, dmax;
-  int radius;
-  float inv2ss, inv2sr;  // 0.5/sigma_s^2, 0.5/sigma_r^2
+  float inv2sr;  // 0.5/sigma_r^2
   // spatial weight of each window offset, row-major (2 radius + 1)^2, made on the
   // host with the same exp_neg (kernel arguments: scalar registers in the kernel)
   float ws[(2 * kMaxRadius + 1) * (2 * kMaxRadius + 1)];
@@ -91,7 +90,7 @@ __device__ __forceinline__ unsigned abs_diff(unsigned a, unsigned b) {
 // A block filters kTileX x kTileY pixels, a pair of neighbours per thread (the 2R + 2
 // codes of a window row are read once for both), and makes the coarser levels' pixels
 // under them (tiles start at multiples of 4, so they need no other block's).  R: the
-// window half-size (a.radius), fixed per instance so that a window row's loop unrolls.
+// window half-size, fixed per instance so that a window row's loop unrolls.
 // Pixels outside the image are invalid in the tile, so the window needs no bounds test
 // of its own; an invalid tap has weight 0, which adds exactly nothing (sums are >= 0).
 //
@@ -318,13 +317,12 @@ kf_status launch_preprocess(const kf_intrinsics& k0, const kf_preprocess_params&
   a.scale = p.depth_scale;
   a.dmin = p.min_depth_m;
   a.dmax = p.max_depth_m;
-  a.radius = p.bilateral_radius;
-  a.inv2ss = 0.5f / (p.sigma_space_px * p.sigma_space_px);
+  const float inv2ss = 0.5f / (p.sigma_space_px * p.sigma_space_px);
   a.inv2sr = 0.5f / (p.sigma_range_m * p.sigma_range_m);
-  const int R = a.radius;
+  const int R = p.bilateral_radius;
   for (int dy = -R; dy <= R; ++dy)
     for (int dx = -R; dx <= R; ++dx)
-      a.ws[(dy + R) * (2 * R + 1) + (dx + R)] = exp_neg((float)(dx * dx + dy * dy) * a.inv2ss);
+      a.ws[(dy + R) * (2 * R + 1) + (dx + R)] = exp_neg((float)(dx * dx + dy * dy) * inv2ss);
   const float rm_lut = (float)kRangeLut * a.scale;
   const bool zt = exp_neg((rm_lut * rm_lut) * a.inv2sr) == 0.0f;
   const bool one = live.levels > 1, two = live.levels > 2;

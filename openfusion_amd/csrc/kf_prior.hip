@@ -280,7 +280,6 @@ struct kf_prior {
   uint16_t* dYb[kf::kConvs] = {};       // gradients of the layers' outputs, BF16 NHWC
   float* bpart[kf::kConvs] = {};        // partial bias sums per block (layer 4: per sample)
   float* wpart[kf::kConvs] = {};        // partial weight gradients per split
-  float* loss_tmp = nullptr;
   unsigned* fuse_count = nullptr;  // [max_batch] finished blocks per sample of the fused inference
 };
 
@@ -495,8 +494,7 @@ extern "C" int64_t kf_prior_param_count(void) { return layout().total; }
 extern "C" kf_status kf_prior_destroy(kf_prior* P) {
   if (!P) return KF_OK;
   void* ptrs[] = {P->params, P->wbf, P->grad, P->adam_m, P->adam_v, P->Y4, P->X5b, P->Hb, P->O, P->dO,
-                  P->dOb, P->dH, P->dHb, P->wt, P->loss_tmp,
-                  P->fuse_count};
+                  P->dOb, P->dH, P->dHb, P->wt, P->fuse_count};
   for (void* q : ptrs) (void)hipFree(q);
   for (int l = 0; l < kConvs; ++l) {
     if (l + 1 < kConvs) {
@@ -547,7 +545,6 @@ extern "C" kf_status kf_prior_create(int32_t max_batch, kf_prior** out) {
   al((void**)&P->dOb, B * kDoPitch * 2);
   al((void**)&P->dH, B * kHidden * 4);
   al((void**)&P->dHb, B * kHidden * 2);
-  al((void**)&P->loss_tmp, 16);
   al((void**)&P->fuse_count, B * sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(P->fuse_count, 0, B * sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(P->wt, 0, weight_copies().total * 2);  // the copies' padding

@@ -31,7 +31,8 @@ __device__ __forceinline__ uint4 load_vec(const uint16_t* p, bool in, int at) {
   return *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(p) + opaque_u32(in ? 2u * (unsigned)at : 0u));
 }
 
-// Stores N (a multiple of 4) floats as BF16 to p (8-byte aligned; 16-byte aligned when N is a multiple of 8).
+// Stores N (a multiple of 4) BF16 values, two in a word, to p (8-byte aligned; 16-byte
+// aligned when N is a multiple of 8).
 template <int N>
 __device__ __forceinline__ void store_words(uint16_t* p, const uint32_t* w) {
   if constexpr (N % 8 == 0) {
@@ -42,6 +43,7 @@ __device__ __forceinline__ void store_words(uint16_t* p, const uint32_t* w) {
     for (int i = 0; i < N / 2; i += 2) *reinterpret_cast<uint2*>(p + 2 * i) = make_uint2(w[i], w[i + 1]);
   }
 }
+// The same from floats, rounded to nearest even.
 template <int N>
 __device__ __forceinline__ void store_bf16(uint16_t* p, const float* v) {
   uint32_t w[N / 2];
@@ -75,12 +77,10 @@ __device__ __forceinline__ void store_bf16_signs(uint16_t* p, uint8_t* bits, con
     *reinterpret_cast<uint16_t*>(bits) = (uint16_t)m;
 }
 
-// v of the lane below (CTRL 0x111) or above (0x101) in its row of 16, `edge` in the row's
-// last lane on that side.
-template <int CTRL>
-__device__ __forceinline__ uint4 neighbour(uint4 v, uint4 edge) {
+// v of the lane above in its row of 16, `edge` in the row's last lane.
+__device__ __forceinline__ uint4 lane_above(uint4 v, uint4 edge) {
   auto mv = [](uint32_t e, uint32_t x) {
-    return (uint32_t)__builtin_amdgcn_update_dpp((int)e, (int)x, CTRL, 0xf, 0xf, false);
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)e, (int)x, 0x101, 0xf, 0xf, false);
   };
   return make_uint4(mv(edge.x, v.x), mv(edge.y, v.y), mv(edge.z, v.z), mv(edge.w, v.w));
 }
@@ -188,13 +188,6 @@ __global__ __launch_bounds__(kConvThreads) void conv1_forward(const float* frame
     const long o = (((long)n * c.hout + oy0 + oy) * c.wout + ox) * c.cout + 8 * q;
     store_bf16_signs<8>(Yb + o, signs ? signs + o / 8 : nullptr, y);
   }
-}
-
-// Orders the LDS accesses of one wavefront around this point.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // The operand tile of 16 pixels of layer L's forward: the rows of input pixels under them,
@@ -558,7 +551,7 @@ __device__ __forceinline__ void dgrad_block(const uint16_t* dY, const uint16_t* 
         // (selects only here: before, each would wait for its load)
         if (dj == 1 && j + 1 >= c.hout) a[dj][0][s] = make_uint4(0u, 0u, 0u, 0u);
         const uint4 own = a[dj][1][s];
-        uint4 v = neighbour<0x101>(a[dj][0][s], own);
+        uint4 v = lane_above(a[dj][0][s], own);
         if (i + 1 >= c.wout) v = make_uint4(0u, 0u, 0u, 0u);
         if (kEnd < 15 && (r & kEnd) == kEnd) v = own;
         a[dj][1][s] = v;
