@@ -43,8 +43,10 @@ constexpr int kSweepMaxBlocks = 4096;  // 16384 waves: two full waves of residen
 // 87 us, 1536 blocks 4374-4377 and 49 us.
 constexpr int kSweepListBlocks = 3072;
 constexpr uint32_t kSweepXcdChunk = 16;  // consecutive sweep blocks kept on one XCD
-// x-slices of a brick whose loads a wavefront issues together: four (70 VGPRs, seven
-// waves per SIMD) beat all eight at once (98 VGPRs, five waves per SIMD)
+// x-slices of a brick whose loads a wavefront issues together: four (70 VGPRs for FP16, 72
+// for FP32 voxels, seven waves per SIMD) beat all eight at once (98 VGPRs, five waves per
+// SIMD).  A wave's first list entry loaded beside the counts takes FP32 to 74, six waves,
+// and gave nothing.
 constexpr int kSlicePass = 4;
 constexpr uint8_t kBrickSkip = 0, kBrickFree = 1, kBrickExact = 2;
 constexpr int kRowPass = 2;  // tile rows loaded together
@@ -151,8 +153,7 @@ __device__ __forceinline__ bool tile_range(const SweepArgs& a, int u0, int u1, i
   mx = 0.0f;
   // A row of the range holds at most 6 (8x8) or 8 (32x32) tiles: the loads of kRowPass
   // rows are issued together, one wait for them (past the range: its last tile again).
-  // Classing is a chain of latencies: with this and the sweep's early entry an 8-frame
-  // run at 256^3 takes 174 us instead of 181 (512^3: 336 and 337; three rows 174 and 338).
+  // Classing is a chain of latencies: an 8-frame run at 256^3 takes 175 us instead of 181.
   const int tx0 = u0 >> sh, tx1 = u1 >> sh, ty1 = v1 >> sh;
   for (int ty = v0 >> sh; ty <= ty1; ty += kRowPass) {
     float2 e[kRowPass][kTileRow];
@@ -380,12 +381,9 @@ __global__ __launch_bounds__(256) void integrate(SweepArgs a) {
     const uint32_t x = blockIdx.x % 8u, j = blockIdx.x / 8u;
     lb = ((j / kSweepXcdChunk) * 8u + x) * kSweepXcdChunk + j % kSweepXcdChunk;
   }
-  // the wave's first entry, were it exact, beside the counts that tell
-  const uint32_t i0 = lb * kWavesPerBlock + wave;
-  const uint32_t front = a.list[min(i0, a.cap - 1u)];
   const uint32_t n_exact = a.count[0], items = n_exact + a.count[1];
-  for (uint32_t i = i0; i < items; i += G * kWavesPerBlock) {
-    const uint32_t e = i == i0 && i < n_exact ? front : a.list[i < n_exact ? i : a.cap - 1u - (i - n_exact)];
+  for (uint32_t i = lb * kWavesPerBlock + wave; i < items; i += G * kWavesPerBlock) {
+    const uint32_t e = a.list[i < n_exact ? i : a.cap - 1u - (i - n_exact)];
     const int bx = (int)(e >> 24), by = (int)((e >> 16) & 255u), bz = (int)((e >> 8) & 255u);
     const bool exact = (e & 255u) == kBrickExact;  // uniform
     const int y = 8 * by + yy, z = 8 * bz + zz;

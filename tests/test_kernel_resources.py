@@ -37,3 +37,8 @@ def test_depth_filter_fills_the_simds(radius, zero_tail):
     k = ki.find(f"depth_levelsILi{radius}ELb{zero_tail}E")
     assert ki.waves_by_registers(k) == ki.MAX_WAVES
     assert ki.blocks_by_lds(k) * 256 >= ki.MAX_WAVES * ki.SIMDS * 64
+
+
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_sweep_keeps_seven_waves(fmt):
+    assert ki.waves_by_registers(ki.find(f"integrateILi{fmt}E")) >= 7
