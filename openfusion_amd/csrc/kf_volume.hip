@@ -49,8 +49,12 @@ constexpr uint32_t kSweepXcdChunk = 16;  // consecutive sweep blocks kept on one
 // and gave nothing.
 constexpr int kSlicePass = 4;
 constexpr uint8_t kBrickSkip = 0, kBrickFree = 1, kBrickExact = 2;
-constexpr int kRowPass = 2;  // tile rows loaded together
 constexpr int kTileRow = 8;  // most raylen tiles in one row of a footprint (tile_range)
+// Bricks whose classing waves (64 bricks each) the chip holds at once, three per SIMD: 1,024
+// x 3 x 64.  Eight kf_integrate calls over four rooms, two rows a wait / one: 256^3 146-152 /
+// 151-155 us, 384^3 149-170 / 152-170, 448^3 159-179 / 157-178, 480^3 168-195 / 165-188, 512^3
+// 170-208 / 169-203, 768^3 291-385 / 289-387.
+constexpr int kLatencyBricks = 196608;
 
 struct SweepArgs {
   void* vox;
@@ -133,6 +137,13 @@ __global__ __launch_bounds__(256) void raylen_tiles(const float* rl, int W, int 
 // Raylen extrema over the pixels [u0, u1] x [v0, v1] (a superset: whole tiles), from
 // the 8x8 tiles when the range is small, else the 32x32 ones; false when it is too
 // large for either.
+//
+// A row of the range holds at most 6 (8x8) or 8 (32x32) tiles: its loads are issued
+// together, one wait for them.  LATENCY: those of two rows, all lanes taking part (past the
+// range: its last tile again); else a row's, lanes past their range taking no part.  Classing
+// few bricks is a chain of latencies, where the first form is the faster; once the bricks'
+// waves no longer fit the chip together its extra loads cost more (kLatencyBricks).
+template <bool LATENCY>
 __device__ __forceinline__ bool tile_range(const SweepArgs& a, int u0, int u1, int v0, int v1, float& mn,
                                            float& mx) {
   int sh;
@@ -151,20 +162,23 @@ __device__ __forceinline__ bool tile_range(const SweepArgs& a, int u0, int u1, i
   }
   mn = 3.0e38f;
   mx = 0.0f;
-  // A row of the range holds at most 6 (8x8) or 8 (32x32) tiles: the loads of kRowPass
-  // rows are issued together, one wait for them (past the range: its last tile again).
-  // Classing is a chain of latencies: an 8-frame run at 256^3 takes 175 us instead of 181.
+  constexpr int ROWS = LATENCY ? 2 : 1;
   const int tx0 = u0 >> sh, tx1 = u1 >> sh, ty1 = v1 >> sh;
-  for (int ty = v0 >> sh; ty <= ty1; ty += kRowPass) {
-    float2 e[kRowPass][kTileRow];
+  for (int ty = v0 >> sh; ty <= ty1; ty += ROWS) {
+    float2 e[ROWS][kTileRow];
 #pragma unroll
-    for (int i = 0; i < kRowPass; ++i) {
+    for (int i = 0; i < ROWS; ++i) {
       const float2* row = t + min(ty + i, ty1) * w;
 #pragma unroll
-      for (int j = 0; j < kTileRow; ++j) e[i][j] = row[min(tx0 + j, tx1)];
+      for (int j = 0; j < kTileRow; ++j) {
+        if constexpr (LATENCY)
+          e[i][j] = row[min(tx0 + j, tx1)];
+        else
+          e[i][j] = tx0 + j <= tx1 ? row[tx0 + j] : make_float2(3.0e38f, 0.0f);
+      }
     }
 #pragma unroll
-    for (int i = 0; i < kRowPass; ++i) {
+    for (int i = 0; i < ROWS; ++i) {
 #pragma unroll
       for (int j = 0; j < kTileRow; ++j) {
         mn = fminf(mn, e[i][j].x);
@@ -193,6 +207,7 @@ __device__ __forceinline__ bool tile_range(const SweepArgs& a, int u0, int u1, i
 //   exact: otherwise.
 // Margins: 0.05 px, 1e-4 m in depth, 2e-4 m in distance, against FP32 errors of the
 // per-voxel path below 4e-3 px and 2e-6 m.
+template <bool LATENCY>
 __device__ __forceinline__ uint8_t classify_brick(const SweepArgs& a, int bx, int by, int bz) {
   const kf_posef P = a.pose->cw;
   double R[9], t[3];
@@ -249,7 +264,7 @@ __device__ __forceinline__ uint8_t classify_brick(const SweepArgs& a, int bx, in
       const int pu0 = (int)fmax(2.0, floor(umin + 0.5)), pu1 = (int)fmin((double)(a.W - 3), floor(umax + 0.5));
       const int pv0 = (int)fmax(2.0, floor(vmin + 0.5)), pv1 = (int)fmin((double)(a.H - 3), floor(vmax + 0.5));
       float rmin, rmax;
-      if (pu0 <= pu1 && pv0 <= pv1 && tile_range(a, pu0, pu1, pv0, pv1, rmin, rmax)) {
+      if (pu0 <= pu1 && pv0 <= pv1 && tile_range<LATENCY>(a, pu0, pu1, pv0, pv1, rmin, rmax)) {
         const bool inside = umin >= ulo && umax < uhi && vmin >= vlo && vmax < vhi;
         // nearest point of the box to the camera centre -R^T t
         double dn2 = 0.0;
@@ -273,12 +288,13 @@ __device__ __forceinline__ uint8_t classify_brick(const SweepArgs& a, int bx, in
 // One thread per brick; exact bricks are appended to the front of the work list and
 // free ones to its back (one atomic per block and class; entries in brick order
 // within a block), so that the sweep can deal each wavefront its share of both.
+template <bool LATENCY>
 __global__ __launch_bounds__(256) void brick_classify(SweepArgs a) {
   __shared__ uint32_t s_cnt[2][4], s_base[2];
   const int nb = a.nb;
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   const int bx = b / (nb * nb), r = b - bx * (nb * nb), by = r / nb, bz = r - by * nb;
-  const uint8_t cls = b < nb * nb * nb ? classify_brick(a, bx, by, bz) : kBrickSkip;
+  const uint8_t cls = b < nb * nb * nb ? classify_brick<LATENCY>(a, bx, by, bz) : kBrickSkip;
   const int c = cls == kBrickExact ? 0 : 1;  // list part: 0 exact, 1 free
   const unsigned long long m[2] = {__ballot(cls == kBrickExact), __ballot(cls == kBrickFree)};
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & (kWave - 1);
@@ -887,7 +903,8 @@ kf_status launch_integrate(kf_volume* v, const kf_intrinsics& k0, const kf_integ
     KF_TRY(check_launch("raylen_tiles"));
   }
   const int nbricks = a.nb * a.nb * a.nb;
-  hipLaunchKernelGGL(brick_classify, dim3(div_up(nbricks, 256)), dim3(256), 0, s, a);
+  auto classify = nbricks <= kLatencyBricks ? brick_classify<true> : brick_classify<false>;
+  hipLaunchKernelGGL(classify, dim3(div_up(nbricks, 256)), dim3(256), 0, s, a);
   KF_TRY(check_launch("brick_classify"));
   if (between) KF_HIP(hipEventRecord(between, s));
   const int blocks = std::min(div_up(nbricks, kWavesPerBlock), kSweepListBlocks);

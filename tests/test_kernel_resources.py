@@ -42,3 +42,8 @@ def test_depth_filter_fills_the_simds(radius, zero_tail):
 @pytest.mark.parametrize("fmt", [0, 1])
 def test_sweep_keeps_seven_waves(fmt):
     assert ki.waves_by_registers(ki.find(f"integrateILi{fmt}E")) >= 7
+
+
+@pytest.mark.parametrize("latency", [0, 1])
+def test_brick_classes_keep_three_waves(latency):
+    assert ki.waves_by_registers(ki.find(f"brick_classifyILb{latency}E")) >= 3  # kLatencyBricks counts on them
