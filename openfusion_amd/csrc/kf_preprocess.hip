@@ -96,18 +96,22 @@ __device__ __forceinline__ unsigned abs_diff(unsigned a, unsigned b) {
 //
 // Bound by latency: waiting (the frame's first touch, the LDS reads, the barriers before the
 // coarser levels) is half of a wavefront's life.  In one launch and with a window row's codes
-// and metres read once for two pixels; the rows are a loop of their own, since the compiler
-// otherwise loads all of them first (radius 3: 167 VGPRs, three waves per SIMD instead of
-// eight; radius 4 256).  The whole of kf_preprocess, three levels, against a pixel per thread
-// and a second launch for the coarser levels, and in parentheses the rows unrolled:
-//   640x480   radius 1 10.7 / 14.0 us (10.8), 3 13.4 / 18.5 (13.9), 4 15.2 / 22.1 (20.0)
-//   1280x960  radius 3 29.2 / 40.8 (37.2), 4 33.8 / 51.3 (51.3)
-//   319x241   radius 3 10.6 / 16.1 (10.2), 4 12.1 / 18.9 (11.5)
-//   range weights that do not reach zero in the table, 640x480: radius 3 15.8 / 19.4 (15.7),
-//   4 19.7 / 23.8 (40); 1280x960: 34.5 / 42.6 (47), 43.4 / 57.0 (130)
-// A table of weight products per window distance (no products per tap) took as long.
+// and metres read once for two pixels; kf_preprocess with three levels, against a pixel per
+// thread and a second launch for the coarser levels: radius 3 640x480 13.9 / 18.5 us, 319x241
+// 10.2 / 16.1, 1280x960 37.2 / 40.8.  A table of weight products per window distance (no
+// products per tap) took as long.
+//
+// kUnroll: the window's rows unrolled, the compiler loads all of them first, which takes
+// registers (radius 3: 167, three waves per SIMD); as a loop every instance has eight waves.
+// Where the range weights do not end in the table, or at radius 4, the loop is far ahead:
+// radius 4 640x480 15.2 us (unrolled 20.0, before 22.1), 2560x1440 77 (133, 126); weights
+// beyond the table, 640x480 radius 4 19.7 (40, 23.8), 1280x960 radius 3 34.5 (47, 42.6).  At
+// the frame driver's radius 3 it is too when alone (640x480 13.4 us), but beside the raycast
+// its many waves take the CU slots that the raycast waits for: 512^3 stream 4,466 frames/s
+// against 4,560.
 template <int R, bool ZT>
 __global__ __launch_bounds__(kThreads) void depth_levels(PreArgs a) {
+  constexpr int kUnroll = ZT && R <= 3 ? 2 * R + 1 : 1;
   constexpr int kSpanX = kTileX + 2 * R, kSpanY = kTileY + 2 * R, kSpan = kSpanX * kSpanY;
   __shared__ __align__(8) int tile[kSpan];      // four times the depth codes
   __shared__ __align__(8) float metres[kSpan];  // the same in metres, 0 = invalid
@@ -153,7 +157,7 @@ __global__ __launch_bounds__(kThreads) void depth_levels(PreArgs a) {
   float sw[2] = {0.0f, 0.0f}, swd[2] = {0.0f, 0.0f};
 #pragma unroll
   for (int p = 0; p < 2; ++p) uc[p] = tile[(py + R) * kSpanX + px + p + R];
-#pragma unroll 1
+#pragma unroll kUnroll
   for (int dy = -R; dy <= R; ++dy) {
     int u[2 * R + 2];
     float m[2 * R + 2];
