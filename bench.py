@@ -176,7 +176,8 @@ def kernel_rooflines(kf, d, sr: dict, prior: bool) -> dict:
     icp_bytes = 0.0
     for lvl in range(icp.levels):
         Pl = P >> (2 * lvl)
-        blocks = min(1024, -(-Pl // (512 * (3 if lvl == 0 else 1))))
+        per = next((p for p in (256, 512, 1280) if Pl <= 256 * p), 1536)  # pixels of a step's block
+        blocks = min(1024, -(-Pl // per))
         icp_bytes += icp.iterations[lvl] * (Pl * 49 + 2 * blocks * 256)
     t = float(ms[:, 1].mean())
     out["icp"] = {"kernel": "guess + icp_step (per frame, "

@@ -28,9 +28,11 @@
 // waves' rounds, which end alone (vector pipes busy 57% of the kernel before the
 // instruction counts below were cut, 39% of a wave's time in memory waits).  Hence: no
 // domain check per sample, differences of FP16 halves without conversions, one face per
-// axis in the free-space skip, no division inside the loop.  Measured together with the
-// brick distances, 512^3 FP16 at 640x480: 42.9 -> 34.9 us; 256^3 FP32 at 319x241: 36.2
-// -> 29.0 us.  Looking at the map once per sample and loading corners only where a brick
+// axis in the free-space skip, no division inside the loop.  The time depends on the scene
+// and the pose.  With the brick distances, over seven rooms: 512^3 FP16 at 640x480 37..68 us
+// before, 31..56 now (the first room 43.0 and 34.8); 256^3 FP32 at 319x241 23..42 and 20..36.
+// (One of 35 rooms and sizes is slower, by the spread below: 768^3 FP16 at 640x480 49 -> 54.)
+// Looking at the map once per sample and loading corners only where a brick
 // is set (fewer instructions a round, more rounds), corner loads ahead of the map's
 // answer, four or five samples a round, and a wave priority that grows with its rounds
 // were all slower.
@@ -47,11 +49,12 @@ namespace {
 constexpr int kXcds = 8;
 // Long rays lie together in the image, and the waves of a block share a CU's L1, whose
 // line lookups a round of corner loads takes 800 of: from 384 blocks (1.5 a CU) on, a
-// block's four tiles are a quarter of the image apart.  512^3 FP16, together / apart:
-// 480x360 30.7 / 28.2 us, 640x480 35.0 / 34.5, 800x600 45.2 / 42.8; late in a 300-frame
-// stream, beside the frame's other kernels, 4,496 / 4,568 frames/s.  With about a block a CU
-// there is nothing to balance and the tiles' shared lines count: 319x241 26.1 / 26.5 us
-// (256^3 FP32 29.2 / 30.0).
+// block's four tiles are a quarter of the image apart.  512^3 FP16 over seven rooms,
+// together / apart: 480x360 28.8..48.8 / 25.5..48.5 us, 640x480 31.5..64.4 / 31.5..56.4,
+// 800x600 41.4..80.2 / 43.2..67.3, each room between 16 % faster and 5 % slower apart; late
+// in a 300-frame stream, beside the frame's other kernels, 4,496 / 4,568 frames/s.  With
+// about a block a CU there is nothing to balance and the tiles' shared lines count: 256^3
+// FP32 at 319x241 19.6..36.1 / 19.8..33.7, the cheap rooms slower, the dear ones faster.
 constexpr int kSpreadBlocks = 384;
 
 struct RayArgs {
